@@ -41,11 +41,43 @@ __global__ __launch_bounds__(256) void k_eq_sample(const float* map, int mw, int
     }
 }
 
-// max |gy| as float bits (non-negative floats order like their bits)
-__global__ __launch_bounds__(256) void k_max_abs(const float* x, size_t count, uint32_t* out) {
+// Map VJP of EquirectSample (EquirectSampleBwd, f_ops.cpp:2823-2919): each
+// pixel's gy * tap weight (the reference's float product) is added to its
+// four texels in 64-bit fixed point, so any grouping of the adds gives the
+// same bits.
+//
+// What bounded the plain form (one global atomic per pixel, tap and channel)
+// was the atomics themselves: neighbouring pixels look at the same few
+// texels, and adds to one line follow each other at ~15 ns (512 x 512
+// pixels, 3 channels: 18.7 ms onto a 4 x 2 map, 1.6 ms onto 32 x 16, 0.9 ms
+// onto 128 x 64). Here a workgroup sums a tile of 1024 pixels in LDS and
+// sends each touched texel to memory once: 20-26 us on each of these maps,
+// most of it the LDS adds of one wave to the same texel.
+constexpr uint32_t kScatterPixels = 1024;
+// Entries (texel, channel) up to which a workgroup keeps the whole map in
+// LDS (48 KB, three workgroups per CU); above it a hash table of the texels
+// that the tile touches (at most 56 KB; a tile of a coherent direction image
+// touches tens to hundreds).
+constexpr uint32_t kScatterDirect = 6144;
+constexpr uint32_t kScatterEmpty = 0xffffffffu;
+constexpr uint32_t kScatterProbes = 8;
+inline uint32_t scatter_slots_log2(uint32_t n) { return n == 4 ? 10u : 11u; }
+// Workgroups (and partial maxima) of the preparation.
+constexpr uint32_t kScatterParts = 256;
+
+// max |gy| as float bits (non-negative floats order like their bits; inf and
+// NaN do not count), one partial per workgroup, and the cleared accumulators
+__global__ __launch_bounds__(256) void k_eq_scatter_prep(const float* x, size_t count,
+                                                         uint32_t* part,
+                                                         unsigned long long* acc, size_t n_acc) {
+    __shared__ uint32_t wmax[4];
+    const size_t t0 = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const size_t step = (size_t)gridDim.x * blockDim.x;
+    for (size_t i = t0; i < n_acc; i += step) {
+        acc[i] = 0ull;
+    }
     uint32_t m = 0;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < count;
-         i += (size_t)gridDim.x * blockDim.x) {
+    for (size_t i = t0; i < count; i += step) {
         const uint32_t b = __float_as_uint(fabsf(x[i]));
         m = b > m && b < 0x7f800000u ? b : m;
     }
@@ -55,8 +87,35 @@ __global__ __launch_bounds__(256) void k_max_abs(const float* x, size_t count, u
         m = other > m ? other : m;
     }
     if ((threadIdx.x & 63) == 0) {
-        atomicMax(out, m);
+        wmax[threadIdx.x >> 6] = m;
     }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int k = 1; k < 4; k++) {
+            m = wmax[k] > m ? wmax[k] : m;
+        }
+        part[blockIdx.x] = m;
+    }
+}
+
+// The largest of the partial maxima (n_part <= 256 = the workgroup's size).
+__device__ __forceinline__ uint32_t scatter_max(const uint32_t* part, uint32_t n_part,
+                                                uint32_t* wmax) {
+    uint32_t m = threadIdx.x < n_part ? part[threadIdx.x] : 0u;
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) {
+        const uint32_t other = (uint32_t)__shfl_xor((int)m, o);
+        m = other > m ? other : m;
+    }
+    if ((threadIdx.x & 63) == 0) {
+        wmax[threadIdx.x >> 6] = m;
+    }
+    __syncthreads();
+    m = wmax[0];
+    for (int k = 1; k < 4; k++) {
+        m = wmax[k] > m ? wmax[k] : m;
+    }
+    return m;
 }
 
 // Fixed-point exponent for sums bounded by max|x| * count: every partial
@@ -71,45 +130,102 @@ __device__ __forceinline__ int fixed_exponent(uint32_t max_bits, double count) {
     return 62 - e;
 }
 
-// Map VJP of EquirectSample (EquirectSampleBwd, f_ops.cpp:2823-2919): each
-// pixel's gy * tap weight (the reference's float product) added to its four
-// texels in fixed point at 2^k.
+// One workgroup per tile of tile_w x (1024 / tile_w) pixels. `slots_log2`:
+// 0 = the whole map in LDS, else the hash table's size.
 __global__ __launch_bounds__(256) void k_eq_scatter(const float* gy, uint32_t n, const float* dir,
-                                                    size_t npx, int mw, int mh,
-                                                    const uint32_t* max_bits,
+                                                    uint32_t dw, uint32_t dh, uint32_t tile_w,
+                                                    uint32_t tiles_x, int mw, int mh,
+                                                    const uint32_t* part, uint32_t n_part,
+                                                    uint32_t slots_log2,
                                                     unsigned long long* acc) {
-    const size_t p = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= npx) {
-        return;
+    extern __shared__ unsigned long long lds[];
+    __shared__ uint32_t wmax[4];
+    const uint32_t tid = threadIdx.x;
+    const uint32_t slots = 1u << slots_log2;
+    const uint32_t n_sum = slots_log2 ? slots * n : (uint32_t)(mw * mh) * n;
+    uint32_t* keys = (uint32_t*)(lds + n_sum);  // hash table only
+    for (uint32_t i = tid; i < n_sum; i += 256) {
+        lds[i] = 0ull;
     }
-    float u, v;
-    if (!dir_to_equirect(mk3(dir[p * 3 + 0], dir[p * 3 + 1], dir[p * 3 + 2]), &u, &v)) {
-        return;
+    if (slots_log2) {
+        for (uint32_t i = tid; i < slots; i += 256) {
+            keys[i] = kScatterEmpty;
+        }
     }
-    const int k = fixed_exponent(*max_bits, (double)npx);
-    const Taps t = taps_wrap(mw, mh, u, v);
-    for (uint32_t c = 0; c < n; c++) {
-        const float g = gy[p * n + c];
+    const int k = fixed_exponent(scatter_max(part, n_part, wmax), (double)((size_t)dw * dh));
+    __syncthreads();
+    const uint32_t x0 = (blockIdx.x % tiles_x) * tile_w;
+    const uint32_t y0 = (blockIdx.x / tiles_x) * (kScatterPixels / tile_w);
+    for (uint32_t q = tid; q < kScatterPixels; q += 256) {
+        const uint32_t x = x0 + q % tile_w, y = y0 + q / tile_w;
+        if (x >= dw || y >= dh) {
+            continue;
+        }
+        const size_t p = (size_t)y * dw + x;
+        float u, v;
+        if (!dir_to_equirect(mk3(dir[p * 3 + 0], dir[p * 3 + 1], dir[p * 3 + 2]), &u, &v)) {
+            continue;
+        }
+        const Taps t = taps_wrap(mw, mh, u, v);
+        float g[4];
+        for (uint32_t c = 0; c < n; c++) {
+            g[c] = gy[p * n + c];
+        }
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            const float prod = g * t.w[j];
-            const long long q = __double2ll_rn(ldexp((double)prod, k));
-            if (q) {
-                atomicAdd(&acc[(size_t)t.idx[j] * n + c], (unsigned long long)q);
+            const uint32_t texel = (uint32_t)t.idx[j];
+            uint32_t at = texel;
+            bool in_lds = true;
+            if (slots_log2) {
+                at = (texel * 2654435761u) >> (32 - slots_log2);
+                in_lds = false;
+                for (uint32_t tries = 0; tries < kScatterProbes; tries++) {
+                    uint32_t key = __hip_atomic_load(&keys[at], __ATOMIC_RELAXED,
+                                                     __HIP_MEMORY_SCOPE_WORKGROUP);
+                    if (key == kScatterEmpty) {
+                        key = atomicCAS(&keys[at], kScatterEmpty, texel);
+                        key = key == kScatterEmpty ? texel : key;
+                    }
+                    if (key == texel) {
+                        in_lds = true;
+                        break;
+                    }
+                    at = (at + 1) & (slots - 1);
+                }
             }
+            for (uint32_t c = 0; c < n; c++) {
+                const float prod = g[c] * t.w[j];
+                const long long fx = __double2ll_rn(ldexp((double)prod, k));
+                if (!fx) {
+                    continue;
+                }
+                if (in_lds) {
+                    atomicAdd(&lds[at * n + c], (unsigned long long)fx);
+                } else {
+                    atomicAdd(&acc[(size_t)texel * n + c], (unsigned long long)fx);
+                }
+            }
+        }
+    }
+    __syncthreads();
+    for (uint32_t i = tid; i < n_sum; i += 256) {
+        const unsigned long long a = lds[i];
+        if (a) {
+            const size_t texel = slots_log2 ? keys[i / n] : i / n;
+            atomicAdd(&acc[texel * n + i % n], a);
         }
     }
 }
 
 __global__ __launch_bounds__(256) void k_fixed_resolve(const unsigned long long* acc,
-                                                       size_t count, const uint32_t* max_bits,
-                                                       double npx, float* out) {
+                                                       size_t count, const uint32_t* part,
+                                                       uint32_t n_part, double npx, float* out) {
+    __shared__ uint32_t wmax[4];
+    const int k = fixed_exponent(scatter_max(part, n_part, wmax), npx);
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= count) {
-        return;
+    if (i < count) {
+        out[i] = (float)ldexp((double)(long long)acc[i], -k);
     }
-    const int k = fixed_exponent(*max_bits, npx);
-    out[i] = (float)ldexp((double)(long long)acc[i], -k);
 }
 
 // ---------------------------------------------------------------------------
@@ -358,23 +474,32 @@ int dressi_equirect_sample_bwd(dressi_ctx* ctx, const float* gy, uint32_t n_comp
     DRESSI_TRY_HIP(hipSetDevice(ctx->device));
     void *acc = nullptr, *mx = nullptr;
     if (int rc = ctx_workspace(ctx, 12, cnt * sizeof(unsigned long long), &acc)) return rc;
-    if (int rc = ctx_workspace(ctx, 13, sizeof(uint32_t), &mx)) return rc;
-    if (int rc = launch_zero(ctx->stream, acc, cnt * sizeof(unsigned long long))) return rc;
-    if (int rc = launch_zero(ctx->stream, mx, sizeof(uint32_t))) return rc;
+    if (int rc = ctx_workspace(ctx, 13, kScatterParts * sizeof(uint32_t), &mx)) return rc;
+    const size_t ng = npx * n_comp;
+    const uint32_t n_part =
+            (uint32_t)std::min<size_t>((std::max(ng, cnt) + 1023) / 1024, kScatterParts);
+    hipLaunchKernelGGL(k_eq_scatter_prep, dim3(n_part), dim3(256), 0, ctx->stream, gy, ng,
+                       (uint32_t*)mx, (unsigned long long*)acc, cnt);
+    DRESSI_CHECK_LAUNCH();
     if (npx) {
-        const size_t ng = npx * n_comp;
-        const uint32_t blocks = (uint32_t)std::min<size_t>((ng + 255) / 256, 1024);
-        hipLaunchKernelGGL(k_max_abs, dim3(blocks), dim3(256), 0, ctx->stream, gy, ng,
-                           (uint32_t*)mx);
-        DRESSI_CHECK_LAUNCH();
-        hipLaunchKernelGGL(k_eq_scatter, dim3((uint32_t)((npx + 255) / 256)), dim3(256), 0,
-                           ctx->stream, gy, n_comp, dir, npx, (int)mw, (int)mh,
-                           (const uint32_t*)mx, (unsigned long long*)acc);
+        // square tiles where the image has the rows for them, flatter ones
+        // for a list of directions
+        uint32_t tile_h = 1;
+        while (tile_h < 32 && tile_h < dh) tile_h *= 2;
+        const uint32_t tile_w = kScatterPixels / tile_h;
+        const uint32_t tiles_x = div_up(dw, tile_w);
+        const uint64_t tiles = (uint64_t)tiles_x * div_up(dh, tile_h);
+        DRESSI_REQUIRE(tiles < (1ull << 31), "too many pixels");
+        const uint32_t slots_log2 = cnt <= kScatterDirect ? 0u : scatter_slots_log2(n_comp);
+        const size_t lds = slots_log2 ? ((size_t)1 << slots_log2) * (8 * n_comp + 4) : cnt * 8;
+        hipLaunchKernelGGL(k_eq_scatter, dim3((uint32_t)tiles), dim3(256), lds, ctx->stream, gy,
+                           n_comp, dir, dw, dh, tile_w, tiles_x, (int)mw, (int)mh,
+                           (const uint32_t*)mx, n_part, slots_log2, (unsigned long long*)acc);
         DRESSI_CHECK_LAUNCH();
     }
     hipLaunchKernelGGL(k_fixed_resolve, dim3((uint32_t)((cnt + 255) / 256)), dim3(256), 0,
                        ctx->stream, (const unsigned long long*)acc, cnt, (const uint32_t*)mx,
-                       (double)npx, out);
+                       n_part, (double)npx, out);
     DRESSI_CHECK_LAUNCH();
     return DRESSI_OK;
 }

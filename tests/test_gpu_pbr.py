@@ -139,6 +139,39 @@ def test_equirect_sample_smooth_map_and_vjp(ctx, oracle):
     _exact(again, got, "equirect vjp rerun")
 
 
+@pytest.mark.parametrize("shape", [
+    # (map w, h, channels, dir rows, dir columns): the whole map in a workgroup's LDS, at its
+    # largest (6144 entries) and smallest; one entry past it (hash table) and with four channels;
+    # a list of directions; images smaller than a tile and one past its edges
+    (64, 32, 3, 33, 65), (1, 1, 1, 5, 7), (4, 2, 3, 70, 31), (2049, 1, 3, 40, 40),
+    (97, 49, 4, 64, 33), (3073, 2, 1, 1, 1500), (128, 64, 3, 1, 1), (128, 64, 2, 1025, 1)])
+@pytest.mark.parametrize("coherent", [True, False])
+def test_equirect_vjp_tiles(ctx, oracle, shape, coherent):
+    """The map VJP over the forms of its tile sums: against the oracle's ordered float sums within
+    their rounding, 2^-24 of the sum of magnitudes for each of a texel's (at most 4 pixels each)
+    terms, and the same bits on a second run. Incoherent directions overflow the hash table."""
+    from opendressi_amd import ops
+    mw, mh, nc, h, w = shape
+    print(f"[equirect vjp] map {mw}x{mh}x{nc} dirs {h}x{w} coherent {coherent}", flush=True)
+    rng = np.random.default_rng(mw + h)
+    if coherent:
+        y, x = np.meshgrid(np.arange(h) / 40.0, np.arange(w) / 50.0, indexing="ij")
+        d = np.stack([np.cos(x), 0.3 + y, np.sin(x) + 0.1], -1).astype(np.float32)
+    else:
+        d = rng.standard_normal((h, w, 3)).astype(np.float32)
+    d[0, 0] = 0.0  # no direction: no contribution
+    gy = (rng.standard_normal((h, w, nc)) * 10.0 ** rng.uniform(-3, 3, (h, w, 1))).astype(np.float32)
+    zero = np.zeros((mh, mw, nc), np.float32)
+    got = host(ops.equirect_sample_bwd(ctx, dev(gy), dev(d), mw, mh))
+    ref = oracle.equirect_sample(zero, d, gy)
+    size = oracle.equirect_sample(zero, d, np.abs(gy)).astype(np.float64)
+    # the fixed point itself rounds each term to 2^-62 of max|gy| times the pixels
+    bar = 4.0 * h * w * (2.0 ** -24 * size + 2.0 ** -61 * h * w * float(np.abs(gy).max()))
+    err = np.abs(got.astype(np.float64) - ref)
+    assert (err <= bar).all(), (float(err.max()), float((err - bar).max()))
+    _exact(host(ops.equirect_sample_bwd(ctx, dev(gy), dev(d), mw, mh)), got, "rerun")
+
+
 # ---- the fused C5 plan -------------------------------------------------------
 
 def _scene(g):
