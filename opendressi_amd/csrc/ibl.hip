@@ -3,9 +3,9 @@
 // IrradianceConv / PrefilterConv and their transposes, PrefilterEnv and
 // BrdfIntegrationLut (src/core/f_ops.cpp:2785-3415, src/core/ibl_math.h).
 //
-// The dense convolutions run one thread per output texel over the source
-// texels in the reference's loop order, so with the reference's direction
-// tables (ibl_core.h) their sums are the reference's bit for bit. The map
+// The dense convolutions add each output texel's terms in the reference's
+// loop order, so with the reference's direction tables (ibl_core.h) their
+// sums are the reference's bit for bit. The map
 // VJP of EquirectSample scatters in 64-bit fixed point (exact, so the
 // result does not depend on the order of the atomics).
 #include <hip/hip_runtime.h>
@@ -278,66 +278,171 @@ enum ConvMode : int {
     kPrefBwd = 4,  // out(s) = sin_s sum_t gy(t) ggx(r_t . d_s) / max(W_t, 1e-12)
 };
 
-// One thread per output texel, the other side in the reference's loop order
-// (f_ops.cpp:2970-3087, 3166-3348). `odir` are the output-map directions,
-// `sdir` the source (env) directions; `in` is the env (forward modes) or the
-// output-map gradient (backward modes), n <= 4 channels.
-template <int MODE>
-__global__ __launch_bounds__(64) void k_eq_conv(const float4* odir, uint32_t n_o,
-                                                const float4* sdir, uint32_t n_s,
-                                                const float* in, const float* norm, uint32_t n,
-                                                float alpha, float scale, float* out) {
+// Each output texel's sum runs over the other side in the reference's loop
+// order (f_ops.cpp:2970-3087, 3166-3348), one float add after the other, so
+// the terms can be formed in parallel but not added so. A workgroup takes
+// kConvOut outputs: four waves form the terms (weight times value, one
+// rounding each, as the reference) of a chunk of kConvChunk sources into one
+// LDS buffer while the fifth adds the chunk before from the other, one lane
+// per output and channel, in order.
+//
+// One thread per output that did both (the form before) had 8192 / 64 waves
+// and less, each at the latency of a weight, a load and an add per source:
+// 2.4-3.2 ms from an 8192-texel source whatever the output's size. Now
+// 128 x 64 from 128 x 64 takes 69 us (67 M weights of ~40 VALU instructions:
+// issue), its transpose 103 us (one division more), and every smaller output
+// 40-47 us, which is the chain of 8192 adds (8 cycles each) and 64 barriers.
+// 256 sources a chunk: smaller outputs 37 us, but 112 us for the largest,
+// where the LDS then leaves three workgroups per CU.
+// Eight outputs: enough workgroups for a 64 x 32 map to reach all 256 CUs.
+constexpr uint32_t kConvOut = 8;
+constexpr uint32_t kConvChunk = 128;
+// A row of terms, padded so that the adding lanes' 16-byte reads start 4
+// banks apart.
+constexpr uint32_t kConvRow = kConvChunk + 4;
+constexpr uint32_t kConvThreads = 5 * 64;
+
+// `odir` are the output-map directions, `sdir` the source (env) directions;
+// `in` is the env (forward modes) or the output-map gradient (backward
+// modes), N channels.
+template <int MODE, int N>
+__global__ __launch_bounds__(kConvThreads) void k_eq_conv(const float4* odir, uint32_t n_o,
+                                                          const float4* sdir, uint32_t n_s,
+                                                          const float* in, const float* norm,
+                                                          float alpha, float scale, float* out) {
     constexpr bool kBwd = MODE == kIrrBwd || MODE == kPrefBwd;
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    __shared__ alignas(16) float term[2][kConvOut][N][kConvRow];
     const uint32_t n_i = kBwd ? n_s : n_o;
     const uint32_t n_j = kBwd ? n_o : n_s;
-    if (i >= n_i) {
+    const float4* idir = kBwd ? sdir : odir;
+    const float4* jdir = kBwd ? odir : sdir;
+    const uint32_t i0 = blockIdx.x * kConvOut;
+    const uint32_t n_chunks = (n_j + kConvChunk - 1) / kConvChunk;
+    const uint32_t tid = threadIdx.x;
+    const bool adds = tid >= 256;  // the fifth wave
+
+    // forming: one source per thread, every second output (two waves take the
+    // even ones, so an output's direction is the wave's: scalar loads)
+    const uint32_t src = tid & (kConvChunk - 1);
+    const uint32_t half = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 7)) & 1u;
+    float4 me[kConvOut / 2];
+#pragma unroll
+    for (uint32_t o = 0; o < kConvOut / 2; o++) {
+        const uint32_t i = i0 + 2 * o + half;
+        me[o] = idir[i < n_i ? i : n_i - 1];
+    }
+    struct Source {
+        float4 d;
+        float norm, val[N];
+    };
+    const auto load = [&](uint32_t chunk, Source* s) {
+        const uint32_t j = chunk * kConvChunk + src;
+        const uint32_t jc = j < n_j ? j : n_j - 1;
+        s->d = jdir[jc];
+        if (MODE == kPrefBwd) {
+            s->norm = norm[jc];
+        }
+        if (MODE != kPrefNorm) {
+#pragma unroll
+            for (int c = 0; c < N; c++) {
+                s->val[c] = in[(size_t)jc * N + c];
+            }
+        }
+    };
+    // a term past the last source is +0: a sum that starts at +0 is never -0,
+    // so adding +0 leaves it as it is
+    const auto form = [&](uint32_t chunk, const Source& s) {
+        const float nj = MODE == kPrefBwd && s.norm > 1e-12f ? s.norm : 1e-12f;
+        const bool live = chunk * kConvChunk + src < n_j;
+#pragma unroll
+        for (uint32_t o = 0; o < kConvOut / 2; o++) {
+            const float4 ot = kBwd ? s.d : me[o];
+            const float4 sd = kBwd ? me[o] : s.d;
+            const float dt = ot.x * sd.x + ot.y * sd.y + ot.z * sd.z;
+            float w;
+            bool used = live;
+            if (MODE == kIrrFwd || MODE == kIrrBwd) {
+                w = (dt > 0.f ? dt : 0.f) * sd.w;
+            } else if (MODE == kPrefNorm || MODE == kPrefFwd) {
+                w = ggx_conv_weight(dt, alpha) * sd.w;
+            } else {
+                const float w0 = ggx_conv_weight(dt, alpha);
+                used = used && !(w0 <= 0.f);  // the reference skips these
+                w = w0 / nj;
+            }
+            float(*row)[kConvRow] = term[chunk & 1u][2 * o + half];
+            if (MODE == kPrefNorm) {
+                row[0][src] = used ? w : 0.f;
+            } else {
+#pragma unroll
+                for (int c = 0; c < N; c++) {
+                    row[c][src] = used ? s.val[c] * w : 0.f;
+                }
+            }
+        }
+    };
+
+    const uint32_t lane = tid & 63u;
+    const bool sums = adds && lane < kConvOut * N;
+    const uint32_t so = lane / N, sc = lane % N;
+    float acc = 0.f;
+    Source cur{}, next{};
+    if (!adds) {
+        load(0, &cur);
+        load(n_chunks > 1 ? 1 : 0, &next);
+        form(0, cur);
+        cur = next;
+    }
+    __syncthreads();
+    for (uint32_t chunk = 0; chunk < n_chunks; chunk++) {
+        if (!adds) {
+            if (chunk + 1 < n_chunks) {
+                load(chunk + 2 < n_chunks ? chunk + 2 : chunk + 1, &next);
+                form(chunk + 1, cur);
+                cur = next;
+            }
+        } else if (sums) {
+            // the next 16 terms' reads in flight while these 16 are added
+            const float4* t = (const float4*)term[chunk & 1u][so][sc];
+            float4 now[4], next[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                now[k] = t[k];
+            }
+#pragma unroll
+            for (uint32_t q = 4; q <= kConvChunk / 4; q += 4) {
+                if (q < kConvChunk / 4) {
+#pragma unroll
+                    for (int k = 0; k < 4; k++) {
+                        next[k] = t[q + k];
+                    }
+                }
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    acc += now[k].x;
+                    acc += now[k].y;
+                    acc += now[k].z;
+                    acc += now[k].w;
+                    now[k] = next[k];
+                }
+            }
+        }
+        __syncthreads();
+    }
+    const uint32_t i = i0 + so;
+    if (!sums || i >= n_i) {
         return;
     }
-    const float4 me = kBwd ? sdir[i] : odir[i];
-    float acc[4] = {0.f, 0.f, 0.f, 0.f};
-    for (uint32_t j = 0; j < n_j; j++) {
-        const float4 ot = kBwd ? odir[j] : me;
-        const float4 sd = kBwd ? me : sdir[j];
-        const float dt = ot.x * sd.x + ot.y * sd.y + ot.z * sd.z;
-        float w;
-        if (MODE == kIrrFwd || MODE == kIrrBwd) {
-            w = (dt > 0.f ? dt : 0.f) * sd.w;
-        } else if (MODE == kPrefNorm || MODE == kPrefFwd) {
-            w = ggx_conv_weight(dt, alpha) * sd.w;
-        } else {
-            const float w0 = ggx_conv_weight(dt, alpha);
-            if (w0 <= 0.f) {
-                continue;
-            }
-            const float nt = norm[j];
-            w = w0 / (nt > 1e-12f ? nt : 1e-12f);
-        }
-        if (MODE == kPrefNorm) {
-            acc[0] += w;
-        } else {
-            const float* src = in + (size_t)j * n;
-            for (uint32_t c = 0; c < n; c++) {
-                acc[c] += src[c] * w;
-            }
-        }
+    float r = acc;
+    if (MODE == kIrrFwd || MODE == kIrrBwd) {
+        r *= scale;
+    } else if (MODE == kPrefFwd) {
+        const float nt = norm[i];
+        r /= (nt > 1e-12f ? nt : 1e-12f);
+    } else if (MODE == kPrefBwd) {
+        r *= idir[i].w;
     }
-    if (MODE == kPrefNorm) {
-        out[i] = acc[0];
-        return;
-    }
-    for (uint32_t c = 0; c < n; c++) {
-        float r = acc[c];
-        if (MODE == kIrrFwd || MODE == kIrrBwd) {
-            r *= scale;
-        } else if (MODE == kPrefFwd) {
-            const float nt = norm[i];
-            r /= (nt > 1e-12f ? nt : 1e-12f);
-        } else {
-            r *= me.w;
-        }
-        out[(size_t)i * n + c] = r;
-    }
+    out[(size_t)i * N + sc] = r;
 }
 
 // PrefilterEnv (f_ops.cpp:3089-3157): per output texel, n_samples GGX
@@ -431,8 +536,20 @@ int run_conv(dressi_ctx* ctx, const float* in, uint32_t sw, uint32_t sh, uint32_
     constexpr bool kBwd = MODE == kIrrBwd || MODE == kPrefBwd;
     const uint32_t n_i = kBwd ? sw * sh : ow * oh;
     const float scale = kIblTwoPi / ((float)sw * (float)sh);
-    hipLaunchKernelGGL(k_eq_conv<MODE>, dim3(div_up(n_i, 64)), dim3(64), 0, ctx->stream, od,
-                       ow * oh, sd, sw * sh, in, norm, n, alpha, scale, out);
+    const auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(div_up(n_i, kConvOut)), dim3(kConvThreads), 0, ctx->stream,
+                           od, ow * oh, sd, sw * sh, in, norm, alpha, scale, out);
+    };
+    if constexpr (MODE == kPrefNorm) {
+        launch(k_eq_conv<MODE, 1>);
+    } else {
+        switch (n) {
+            case 1: launch(k_eq_conv<MODE, 1>); break;
+            case 2: launch(k_eq_conv<MODE, 2>); break;
+            case 3: launch(k_eq_conv<MODE, 3>); break;
+            default: launch(k_eq_conv<MODE, 4>); break;
+        }
+    }
     DRESSI_CHECK_LAUNCH();
     return DRESSI_OK;
 }

@@ -119,6 +119,37 @@ def test_ibl_convs_match_oracle_at_map_sizes(ctx, oracle, shape):
            oracle.irradiance_conv(env, ow // 2, oh // 2), "irradiance")
 
 
+@pytest.mark.parametrize("shape", [
+    # (source w, h, output w, h, channels): workgroups of 8 outputs and chunks of 128 sources,
+    # whole, one past and one short of them; single texels; every channel count
+    (16, 8, 4, 2, 3), (43, 3, 1, 1, 4), (129, 1, 3, 3, 1), (128, 2, 9, 1, 2), (127, 3, 17, 5, 3),
+    (1, 1, 16, 8, 3)])
+def test_ibl_conv_chunks_match_oracle(ctx, oracle, shape):
+    """Bit for bit, forward and back; an infinite and a NaN source value reach the sums that the
+    reference's order brings them to."""
+    from opendressi_amd import ops
+    sw, sh, ow, oh, nc = shape
+    print(f"[ibl conv chunks] {shape}", flush=True)
+    rng = np.random.default_rng(sw)
+    env = rng.random((sh, sw, nc), dtype=np.float32)
+    gy = rng.standard_normal((oh, ow, nc)).astype(np.float32)
+
+    def check(env, gy):
+        for rough in (0.0, 0.7):
+            _exact(np.nan_to_num(host(ops.prefilter_conv(ctx, dev(env), ow, oh, rough))),
+                   np.nan_to_num(oracle.prefilter_conv(env, ow, oh, rough)), f"pref {rough}")
+            _exact(np.nan_to_num(host(ops.prefilter_conv_bwd(ctx, dev(gy), sw, sh, rough))),
+                   np.nan_to_num(oracle.prefilter_conv(env, ow, oh, rough, gy)), f"bwd {rough}")
+        _exact(np.nan_to_num(host(ops.irradiance_conv(ctx, dev(env), ow, oh))),
+               np.nan_to_num(oracle.irradiance_conv(env, ow, oh)), "irradiance")
+        _exact(np.nan_to_num(host(ops.irradiance_conv_bwd(ctx, dev(gy), sw, sh))),
+               np.nan_to_num(oracle.irradiance_conv(env, ow, oh, gy)), "irradiance bwd")
+
+    check(env, gy)
+    env.flat[0], gy.flat[-1] = np.inf, np.nan
+    check(env, gy)
+
+
 def test_equirect_sample_smooth_map_and_vjp(ctx, oracle):
     """A 512 x 256 smooth map sampled at 96 x 80 random directions (bit for
     bit), and the map VJP of 1024 x 8 directions (gradients 1e-5)."""
