@@ -527,12 +527,79 @@ int upload(dressi_ctx* ctx, int slot, const std::vector<float4>& v, const float4
     return DRESSI_OK;
 }
 
+enum TableKind : int { kDirs = 0, kSamples = 1 };
+
+// The texel directions of an (a, b) map (kDirs) or the a angles of a sample
+// count (kSamples). They depend on the sizes alone, but the C library's sinf
+// and cosf per texel, the copy and the wait for it took 40-150 us of host
+// time per table and call (28 tables, ~1 ms, in the chain of a 512 x 256
+// environment whose kernels take 0.8 ms). So the context keeps them: up to
+// kTablesMax tables of kTableBytesMax each and kTablesBytes together, the
+// longest unused given back first. A call uses at most two, and two always
+// fit, so the second never takes the first's place. Larger ones go through
+// the workspace `slot` on each call, as all did.
+constexpr size_t kTableBytesMax = 16u << 20;
+constexpr size_t kTablesBytes = 64u << 20;
+constexpr size_t kTablesMax = 64;
+
+int device_table(dressi_ctx* ctx, int slot, TableKind kind, uint32_t a, uint32_t b,
+                 const float4** out) {
+    // a graph would keep the table's address past its place here
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    DRESSI_TRY_HIP(hipStreamIsCapturing(ctx->stream, &capture));
+    if (capture != hipStreamCaptureStatusNone) {
+        set_error("the IBL convolutions and sample tables cannot be captured");
+        return DRESSI_ERR_HIP;
+    }
+    auto& tables = ctx->tables;
+    for (dressi_ctx::Table& t : tables) {
+        if (t.kind == kind && t.a == a && t.b == b) {
+            t.used = ++ctx->table_clock;
+            *out = (const float4*)t.ptr;
+            return DRESSI_OK;
+        }
+    }
+    const std::vector<float4> v = kind == kDirs ? host_equirect_dirs(a, b) : host_hammersley(a);
+    const size_t bytes = v.size() * sizeof(float4);
+    if (bytes > kTableBytesMax) {
+        return upload(ctx, slot, v, out);
+    }
+    size_t total = bytes;
+    for (const dressi_ctx::Table& t : tables) total += t.bytes;
+    while (tables.size() >= kTablesMax || total > kTablesBytes) {
+        const auto old = std::min_element(
+                tables.begin(), tables.end(),
+                [](const dressi_ctx::Table& x, const dressi_ctx::Table& y) {
+                    return x.used < y.used;
+                });
+        // whatever stream last read it
+        DRESSI_TRY_HIP(hipDeviceSynchronize());
+        DRESSI_TRY_HIP(hipFree(old->ptr));
+        total -= old->bytes;
+        tables.erase(old);
+    }
+    void* p = nullptr;
+    DRESSI_TRY_HIP(hipMalloc(&p, bytes));
+    // complete before the call returns, so that a later call may read it on
+    // any stream
+    hipError_t e = hipMemcpyAsync(p, v.data(), bytes, hipMemcpyHostToDevice, ctx->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
+    if (e != hipSuccess) {
+        hipFree(p);
+        set_error("table upload failed: %s", hipGetErrorString(e));
+        return DRESSI_ERR_HIP;
+    }
+    tables.push_back({kind, a, b, p, bytes, ++ctx->table_clock});
+    *out = (const float4*)p;
+    return DRESSI_OK;
+}
+
 template <int MODE>
 int run_conv(dressi_ctx* ctx, const float* in, uint32_t sw, uint32_t sh, uint32_t n,
              uint32_t ow, uint32_t oh, float alpha, const float* norm, float* out) {
     const float4 *od = nullptr, *sd = nullptr;
-    if (int rc = upload(ctx, 10, host_equirect_dirs(ow, oh), &od)) return rc;
-    if (int rc = upload(ctx, 11, host_equirect_dirs(sw, sh), &sd)) return rc;
+    if (int rc = device_table(ctx, 10, kDirs, ow, oh, &od)) return rc;
+    if (int rc = device_table(ctx, 11, kDirs, sw, sh, &sd)) return rc;
     constexpr bool kBwd = MODE == kIrrBwd || MODE == kPrefBwd;
     const uint32_t n_i = kBwd ? sw * sh : ow * oh;
     const float scale = kIblTwoPi / ((float)sw * (float)sh);
@@ -703,8 +770,8 @@ int dressi_prefilter_env(dressi_ctx* ctx, const float* env, uint32_t sw, uint32_
     if (int rc = check_map(ow, oh, n_comp)) return rc;
     DRESSI_TRY_HIP(hipSetDevice(ctx->device));
     const float4 *od = nullptr, *smp = nullptr;
-    if (int rc = upload(ctx, 10, host_equirect_dirs(ow, oh), &od)) return rc;
-    if (int rc = upload(ctx, 11, host_hammersley(n_samples), &smp)) return rc;
+    if (int rc = device_table(ctx, 10, kDirs, ow, oh, &od)) return rc;
+    if (int rc = device_table(ctx, 11, kSamples, n_samples, 0, &smp)) return rc;
     hipLaunchKernelGGL(k_prefilter_env, dim3(div_up(ow * oh, 64)), dim3(64), 0, ctx->stream, od,
                        ow * oh, env, (int)sw, (int)sh, n_comp, smp, n_samples, roughness, out);
     DRESSI_CHECK_LAUNCH();
@@ -717,7 +784,7 @@ int dressi_brdf_lut(dressi_ctx* ctx, uint32_t w, uint32_t h, uint32_t n_samples,
     if (int rc = check_map(w, h, 2)) return rc;
     DRESSI_TRY_HIP(hipSetDevice(ctx->device));
     const float4* smp = nullptr;
-    if (int rc = upload(ctx, 11, host_hammersley(n_samples), &smp)) return rc;
+    if (int rc = device_table(ctx, 11, kSamples, n_samples, 0, &smp)) return rc;
     hipLaunchKernelGGL(k_brdf_lut, dim3(div_up(w * h, 64)), dim3(64), 0, ctx->stream, (int)w,
                        (int)h, smp, n_samples, (float2*)out);
     DRESSI_CHECK_LAUNCH();

@@ -30,6 +30,17 @@ struct dressi_ctx {
     // bumped whenever a slot is freed and reallocated: a captured hipGraph
     // holding the old addresses is stale once this changes
     uint64_t ws_generation = 0;
+    // host-built tables of the IBL ops (texel directions, sample angles) kept
+    // on the device by their sizes (ibl.hip: device_table)
+    struct Table {
+        int kind;
+        uint32_t a, b;
+        void* ptr;
+        size_t bytes;
+        uint64_t used;
+    };
+    std::vector<Table> tables;
+    uint64_t table_clock = 0;
 };
 
 namespace dressi {

@@ -144,6 +144,9 @@ int dressi_ctx_destroy(dressi_ctx* ctx) {
             hipEventDestroy(ctx->ws_event[i]);
         }
     }
+    for (const dressi_ctx::Table& t : ctx->tables) {
+        hipFree(t.ptr);
+    }
     if (ctx->d_err) {
         hipFree(ctx->d_err);
     }

@@ -150,6 +150,23 @@ def test_ibl_conv_chunks_match_oracle(ctx, oracle, shape):
     check(env, gy)
 
 
+def test_ibl_tables_beyond_the_kept_ones(oracle):
+    """More map sizes than a context keeps tables for (64), the first ones again after they had to
+    give place, and the tables of one context after another's end: the oracle's bits each time."""
+    import opendressi_amd as od
+    from opendressi_amd import ops
+    print("[ibl tables] 70 sizes", flush=True)
+    env = smooth_map(4, 8, 3, 9)
+    for _ in range(2):
+        c = od.Context(0)
+        for w in list(range(1, 71)) + [1, 2, 70]:
+            _exact(host(ops.irradiance_conv(c, dev(env), w, 1)), oracle.irradiance_conv(env, w, 1),
+                   f"irradiance {w}x1")
+        _exact(host(ops.prefilter_env(c, dev(env), 8, 4, 0.5, 64)),
+               oracle.prefilter_env(env, 8, 4, 0.5, 64), "prefilter env")
+        c.close()
+
+
 def test_equirect_sample_smooth_map_and_vjp(ctx, oracle):
     """A 512 x 256 smooth map sampled at 96 x 80 random directions (bit for
     bit), and the map VJP of 1024 x 8 directions (gradients 1e-5)."""
