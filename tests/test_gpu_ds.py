@@ -73,3 +73,38 @@ def test_gather_dist_grad_matches_oracle(ctx, oracle, level, s, seed):
         _exact(got, oracle.gather_dist_grad(gy, rs, clip, faces, vf, wide=wide),
                f"wide={wide}")
     ctx.synchronize()
+
+
+@pytest.mark.parametrize("h,w", [(8, 8), (37, 129), (80, 50)])
+def test_gather_dist_grad_boxes_and_rows(ctx, oracle, h, w):
+    """Faces whose boxes are the whole screen (many steps of 512 pixels, more than 64 hits a
+    step) or a few pixels, a vertex of more than 64 faces, faces that repeat a vertex, rows that
+    hold a face twice or one that is not theirs: bit for bit against the oracle."""
+    from opendressi_amd import ops
+    print(f"[dist grad] boxes {h}x{w}", flush=True)
+    rng = np.random.default_rng(h)
+    n_fan = 70
+    ang = np.linspace(0.0, 2.0 * np.pi, n_fan, endpoint=False)
+    pos = np.concatenate([[[0.0, 0.0, 0.5]],
+                          np.stack([0.9 * np.cos(ang), 0.9 * np.sin(ang), 0 * ang + 0.4], 1),
+                          rng.uniform(-1, 1, (12, 3)) * [1.2, 1.2, 0.4] + [0, 0, 0.5]])
+    clip = np.concatenate([pos, np.ones((len(pos), 1))], 1).astype(np.float32)
+    clip *= rng.uniform(0.5, 2.0, (len(pos), 1)).astype(np.float32)
+    fan = [(0, 1 + i, 1 + (i + 1) % n_fan) for i in range(n_fan)]
+    k = 1 + n_fan
+    faces = np.array(fan + [(k, k + 1, k + 2), (k + 3, k + 4, k + 5), (k + 6, k + 6, k + 7),
+                            (k + 8, k + 9, k + 8), (0, k + 10, 0)], np.float32)
+    nf = len(faces)
+    fid = np.repeat(np.arange(nf, dtype=np.float32), 3)[:, None]
+    fs = np.arange(3 * nf, dtype=np.float32).reshape(nf, 3)
+    vf = oracle.vertex_faces_tex(faces, len(pos))
+    vf = np.concatenate([vf, vf[:1], np.full_like(vf[:1], nf - 1)]).astype(np.float32)
+    assert vf.shape[0] > 64
+    rs = oracle.rasterize_soft(oracle.soft_clip(clip, faces, w, h, 3.0), fid, fs, clip, faces, w, h,
+                               3.0)
+    gy = rng.standard_normal((h, w, 4)).astype(np.float32)
+    got = host(ops.gather_dist_grad(ctx, dev(gy), dev(rs), dev(clip), dev(faces), dev(vf), 3.0))
+    ref = oracle.gather_dist_grad(gy, rs, clip, faces, vf, wide=True)
+    assert np.abs(ref).max() > 0
+    _exact(got, ref, "wide")
+    ctx.synchronize()
