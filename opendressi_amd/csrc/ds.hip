@@ -10,12 +10,14 @@
 namespace dressi {
 namespace {
 
-// cpu_raster.cpp:114-151 (SignedDistToTri) with the argmin edge and its
-// clamped parameter.
+// cpu_raster.cpp:114-151 (SignedDistToTri) with the argmin edge, its clamped
+// parameter and its nearest point (kept here: found again from the edge's
+// run-time index it would put the corner arrays in scratch).
 struct TriDistE {
     float dist;
     int edge;
     float t;
+    float qx, qy;
 };
 
 __device__ __forceinline__ TriDistE signed_dist_edge(float px, float py, const float sx[3],
@@ -24,6 +26,7 @@ __device__ __forceinline__ TriDistE signed_dist_edge(float px, float py, const f
     best.dist = 0.f;
     best.edge = 0;
     best.t = 0.f;
+    best.qx = best.qy = 0.f;
     float best_d2 = -1.f;
     int n_pos = 0, n_neg = 0;
 #pragma unroll
@@ -46,6 +49,8 @@ __device__ __forceinline__ TriDistE signed_dist_edge(float px, float py, const f
             best_d2 = d2;
             best.edge = k;
             best.t = t;
+            best.qx = qx;
+            best.qy = qy;
         }
         const float cr = ex * (py - sy[k]) - ey * (px - sx[k]);
         n_pos += (cr >= 0.f);
@@ -72,11 +77,9 @@ __device__ __forceinline__ void signed_dist_grad_k(float px, float py, const flo
     if (k != ia && k != ib) {
         return;
     }
-    const float qx = sx[ia] + td.t * (sx[ib] - sx[ia]);
-    const float qy = sy[ia] + td.t * (sy[ib] - sy[ia]);
     const float sgn = td.dist >= 0.f ? 1.f : -1.f;
-    const float nx = (px - qx) / d;
-    const float ny = (py - qy) / d;
+    const float nx = (px - td.qx) / d;
+    const float ny = (py - td.qy) / d;
     if (k == ia) {
         *gx = -sgn * (1.f - td.t) * nx;
         *gy = -sgn * (1.f - td.t) * ny;
@@ -168,9 +171,12 @@ __device__ __forceinline__ void add_corner(const FaceCorners& fc, const TriDistE
 //
 // One thread per row scanned its face's box alone: each face three times,
 // one pixel after another at a memory latency each, and the last threads'
-// boxes (long edge-on faces) set the time: 3.8 ms at 512 x 512, 5120 faces.
-// The wave looks at 8 x 64 pixels at once; what follows for the few that the
-// face won is the evaluation side by side, and only the adds one by one.
+// boxes (edge-on faces, up to 12 k pixels) set the time: 3.8 ms at 512 x 512,
+// 5120 faces. The wave looks at 8 x 64 pixels at once and keeps the few that
+// the face won (at most ~250 here); these are evaluated side by side, and
+// only the adds go one by one: 56 us, set by the largest boxes' steps at a
+// memory latency each (124 us when each step's hits were evaluated at once;
+// four waves to a face 93 us: the setup's divisions repeat per wave).
 __global__ __launch_bounds__(256) void k_gather_dist_grad_rows(const float* faces, uint32_t n_verts,
                                                                uint32_t n_faces, const float* vf,
                                                                uint32_t max_deg, uint32_t* err,
@@ -193,25 +199,35 @@ __global__ __launch_bounds__(256) void k_gather_dist_grad_rows(const float* face
     }
 }
 
-// Pixels per lane and step (loads in flight).
-constexpr int kDistPx = 8;
+// Pixels per lane and step (loads in flight); pixels that the face won kept
+// before they are evaluated.
+constexpr uint32_t kDistPx = 8;
+constexpr uint32_t kDistHits = 1024;
+static_assert(kDistHits >= 2 * 64 * kDistPx, "a step's hits fit beside those kept");
+
+// Orders the (one-wave) workgroup's LDS accesses.
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 
 __global__ __launch_bounds__(64) void k_gather_dist_grad_faces(
         const float4* gy, const float4* rs, const float4* clip, uint32_t n_verts,
         const float* faces, const float* vf, uint32_t max_deg, float radius, uint32_t w,
         uint32_t h, float4* out) {
-    __shared__ uint32_t hit_px[64 * kDistPx];
+    __shared__ uint32_t hit_px[kDistHits];
     // per hit: corner k's x, y, w contributions
     __shared__ float term[64][9];
     const uint32_t f = blockIdx.x, lane = threadIdx.x;
     const float W = (float)w, H = (float)h;
-    FaceCorners fc;
     // (bad indices are the row kernel's to report)
     for (int k = 0; k < 3; k++) {
         if ((uint32_t)(int64_t)(faces[(size_t)f * 3 + k] + 0.5f) >= n_verts) {
             return;
         }
     }
+    FaceCorners fc;
     int bx0, by0, bx1, by1;
     if (!load_face(faces, clip, n_verts, f, W, H, &fc, nullptr) ||
         !soft_bbox(fc, w, h, radius, &bx0, &by0, &bx1, &by1)) {
@@ -221,16 +237,15 @@ __global__ __launch_bounds__(64) void k_gather_dist_grad_faces(
     const uint32_t n_px = bw * (uint32_t)(by1 - by0 + 1);
     // lane 3 r + c < 9 sums component c of corner r's row
     const uint32_t r = lane < 9 ? lane / 3 : 0, comp = lane < 9 ? lane % 3 : 0;
-    bool mine[3];
-    for (int k = 0; k < 3; k++) {
-        mine[k] = fc.idx[k] == fc.idx[r];
-    }
+    const uint32_t my = r == 0 ? fc.idx[0] : r == 1 ? fc.idx[1] : fc.idx[2];
+    const bool twice = fc.idx[0] == fc.idx[1] || fc.idx[1] == fc.idx[2] || fc.idx[2] == fc.idx[0];
     float acc = 0.f;
+    uint32_t n_hits = 0;
     for (uint32_t p0 = 0; p0 < n_px; p0 += 64 * kDistPx) {
         uint32_t o[kDistPx];
         float2 yw[kDistPx];  // the winner's face id, coverage
 #pragma unroll
-        for (int s = 0; s < kDistPx; s++) {
+        for (uint32_t s = 0; s < kDistPx; s++) {
             const uint32_t p = p0 + s * 64 + lane;
             const uint32_t q = p < n_px ? p : 0;
             const uint32_t row = q / bw;
@@ -238,9 +253,8 @@ __global__ __launch_bounds__(64) void k_gather_dist_grad_faces(
             const float4 v = rs[o[s]];
             yw[s] = make_float2(v.y, p < n_px ? v.w : 0.f);
         }
-        uint32_t n_hits = 0;
 #pragma unroll
-        for (int s = 0; s < kDistPx; s++) {
+        for (uint32_t s = 0; s < kDistPx; s++) {
             const bool hit = !(yw[s].y < 0.5f) && (uint32_t)(int64_t)(yw[s].x + 0.5f) == f;
             const uint64_t m = __ballot(hit);
             if (hit) {
@@ -248,7 +262,11 @@ __global__ __launch_bounds__(64) void k_gather_dist_grad_faces(
             }
             n_hits += (uint32_t)__popcll(m);
         }
-        __syncthreads();
+        const bool last = p0 + 64 * kDistPx >= n_px;
+        if (!last && n_hits + 64 * kDistPx <= kDistHits) {
+            continue;
+        }
+        wave_lds_sync();
         for (uint32_t h0 = 0; h0 < n_hits; h0 += 64) {
             const uint32_t n = min(64u, n_hits - h0);
             if (lane < n) {
@@ -271,37 +289,45 @@ __global__ __launch_bounds__(64) void k_gather_dist_grad_faces(
                     term[lane][k * 3 + 2] = t[k].w;
                 }
             }
-            __syncthreads();
-            if (lane < 9) {
-                // a contribution that the reference leaves out is +0 here: a
-                // sum that starts at +0 is never -0, and +0 leaves it as it is
+            wave_lds_sync();
+            // a contribution that the reference leaves out is +0 here: a sum
+            // that starts at +0 is never -0, and +0 leaves it as it is
+            if (lane < 9 && !twice) {
+#pragma unroll 8
+                for (uint32_t q = 0; q < n; q++) {
+                    acc += term[q][lane];
+                }
+            } else if (lane < 9) {
                 for (uint32_t q = 0; q < n; q++) {
 #pragma unroll
                     for (int k = 0; k < 3; k++) {
-                        if (mine[k]) {
+                        if (fc.idx[k] == my) {
                             acc += term[q][k * 3 + comp];
                         }
                     }
                 }
             }
-            __syncthreads();
+            wave_lds_sync();
         }
+        n_hits = 0;
     }
     // the corner's row: the first of its vertex's that holds f
-    uint32_t row[3];
+    uint32_t row = max_deg;
+#pragma unroll
     for (int k = 0; k < 3; k++) {
-        row[k] = max_deg;
-        for (uint32_t d0 = 0; d0 < max_deg && row[k] == max_deg; d0 += 64) {
+        uint32_t at = max_deg;
+        for (uint32_t d0 = 0; d0 < max_deg && at == max_deg; d0 += 64) {
             const uint32_t d = d0 + lane;
             const float fv = d < max_deg ? vf[(size_t)d * n_verts + fc.idx[k]] : -1.f;
             const uint64_t m = __ballot(fv >= -0.5f && (uint32_t)(int64_t)(fv + 0.5f) == f);
             if (m) {
-                row[k] = d0 + (uint32_t)__builtin_ctzll(m);
+                at = d0 + (uint32_t)__builtin_ctzll(m);
             }
         }
+        row = (int)r == k ? at : row;
     }
-    if (lane < 9 && row[r] < max_deg) {
-        float* dst = (float*)&out[(size_t)row[r] * n_verts + fc.idx[r]];
+    if (lane < 9 && row < max_deg) {
+        float* dst = (float*)&out[(size_t)row * n_verts + my];
         dst[comp == 2 ? 3 : comp] = acc;
     }
 }
