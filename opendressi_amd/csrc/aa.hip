@@ -156,32 +156,6 @@ __global__ __launch_bounds__(256) void k_antialias_bwd_img_op(const float* gy, u
     }
 }
 
-// One active pair's contribution to vertex v's row (f_ops.cpp:2345-2386,
-// only_v): gr = dot(gy(s), c(s) - c(n)) / 9, then each endpoint equal to v.
-__device__ __forceinline__ void aa_accumulate_v(const float* gy, const float* img,
-                                                uint32_t n_comp, const float4* clip, float W,
-                                                float H, uint32_t w, uint32_t v, int x, int y,
-                                                int nx, int ny, const AaPair& pr, float4* dst) {
-    const size_t so = ((size_t)y * w + x) * n_comp;
-    const size_t no = ((size_t)ny * w + nx) * n_comp;
-    float gr = 0.f;
-    for (uint32_t c = 0; c < n_comp; c++) {
-        gr += gy[so + c] * (img[so + c] - img[no + c]);
-    }
-    gr /= 9.f;
-    if (gr == 0.f) {
-        return;
-    }
-    float dqa[2], dqb[2];
-    aa_pair_dq(pr, x, y, dqa, dqb);
-    if (pr.ia == v) {
-        aa_add_endpoint(gr, dqa, clip[pr.ia], W, H, dst);
-    }
-    if (pr.ib == v) {
-        aa_add_endpoint(gr, dqb, clip[pr.ib], W, H, dst);
-    }
-}
-
 // AntiAliasBwdVtx, n_samples > 0 (f_ops.cpp:2410-2472): one 8-lane group per
 // (vertex, slot) row when `wide` (out {V, deg} VEC4, row d * V + v), else
 // per vertex accumulating its slots in order (out {V,1}). The group walks
@@ -312,14 +286,28 @@ __global__ __launch_bounds__(256) void k_antialias_bwd_vtx_op(
 // so every vertex's sum has the reference's order. An active pair's edge
 // belongs to a face covering s or its neighbour, so no pair of v's lies
 // outside those pixels.
-__global__ __launch_bounds__(128) void k_antialias_bwd_vtx_exact_op(
+//
+// One workgroup per vertex. Its pairs were one thread's serial chain (a few
+// thousand pairs at a memory latency each: 12 ms at 61 x 97 pixels, 162
+// vertices, on three wavefronts). Now 256 pixels a step: each thread tests
+// its pixel's eight pairs by what needs no geometry (the faces differ, and
+// dot(gy(s), c(s) - c(n)) / 9 is not 0: else the pair adds nothing), the
+// pairs left are listed in raster and neighbour order, evaluated side by
+// side, and their terms added one by one: 21 us, a handful of dependent
+// loads and barriers per step.
+constexpr uint32_t kAaExactThreads = 256;
+
+__global__ __launch_bounds__(kAaExactThreads) void k_antialias_bwd_vtx_exact_op(
         const float* gy, const float* img, uint32_t n_comp, const float* tri, const float4* clip,
         uint32_t n_verts, int clip_per_item, const float* faces, uint32_t n_faces,
         const float* vtx_faces, uint32_t max_deg, uint32_t w, uint32_t h, float4* out) {
-    const uint32_t v = blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= n_verts) {
-        return;
-    }
+    constexpr uint32_t T = kAaExactThreads;
+    __shared__ int box[4];
+    __shared__ uint32_t wave_pairs[T / 64];
+    __shared__ uint16_t pair[T * 8];  // thread of the pixel << 3 | neighbour
+    __shared__ float term[T][6];      // endpoint a's x, y, w, then b's
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+    const uint32_t v = blockIdx.x;
     const AaItem it(w, h);
     gy = it.img(gy, n_comp);
     img = it.img(img, n_comp);
@@ -327,8 +315,14 @@ __global__ __launch_bounds__(128) void k_antialias_bwd_vtx_exact_op(
     clip = it.clip(clip, n_verts, clip_per_item);
     out += (size_t)it.item * n_verts;
     const float W = (float)w, H = (float)h;
-    int bx0 = (int)w, by0 = (int)h, bx1 = -1, by1 = -1;
-    for (uint32_t d = 0; d < max_deg; d++) {
+    if (tid == 0) {
+        box[0] = (int)w;
+        box[1] = (int)h;
+        box[2] = -1;
+        box[3] = -1;
+    }
+    __syncthreads();
+    for (uint32_t d = tid; d < max_deg; d += T) {
         const float fv = vtx_faces[(size_t)d * n_verts + v];
         if (fv < -0.5f) {
             continue;
@@ -337,53 +331,137 @@ __global__ __launch_bounds__(128) void k_antialias_bwd_vtx_exact_op(
         if (f >= n_faces) {
             continue;
         }
+        uint32_t vi[3];
         float qx[3], qy[3];
-        bool ok = true;
-        for (int k = 0; k < 3 && ok; k++) {
-            const uint32_t vi = FloatFaces{faces}(f, k);
-            ok = vi < n_verts && clip_w_valid(clip[vi].w);
-            if (ok) {
-                const float4 c = clip[vi];
-                const ScreenVert s = project_to_screen(c.x, c.y, c.z, c.w, W, H);
-                qx[k] = s.x;
-                qy[k] = s.y;
-            }
-        }
-        if (!ok) {
+        if (!TriFromClip{faces, clip, n_verts, W, H}(f, vi, qx, qy)) {
             continue;  // never an owner (EvalAaPair skips it)
         }
         int fx0, fy0, fx1, fy1;
         pixel_bbox(qx[0], qx[1], qx[2], qy[0], qy[1], qy[2], (int)w, (int)h, &fx0, &fy0, &fx1,
                    &fy1);
-        bx0 = min(bx0, fx0 - 1);
-        by0 = min(by0, fy0 - 1);
-        bx1 = max(bx1, fx1 + 1);
-        by1 = max(by1, fy1 + 1);
+        atomicMin(&box[0], fx0 - 1);
+        atomicMin(&box[1], fy0 - 1);
+        atomicMax(&box[2], fx1 + 1);
+        atomicMax(&box[3], fy1 + 1);
     }
-    bx0 = max(bx0, 0);
-    by0 = max(by0, 0);
-    bx1 = min(bx1, (int)w - 1);
-    by1 = min(by1, (int)h - 1);
-    float4 dst = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int y = by0; y <= by1; y++) {
-        for (int x = bx0; x <= bx1; x++) {
-            const uint32_t its = tri_id(tri, (size_t)y * w + x);
+    __syncthreads();
+    const int bx0 = max(box[0], 0), by0 = max(box[1], 0);
+    const int bx1 = min(box[2], (int)w - 1), by1 = min(box[3], (int)h - 1);
+    float acc = 0.f;  // threads 0, 1, 2: the row's x, y, w
+    const uint32_t bw = bx1 >= bx0 ? (uint32_t)(bx1 - bx0 + 1) : 0u;
+    const uint32_t n_px = by1 >= by0 ? bw * (uint32_t)(by1 - by0 + 1) : 0u;
+    for (uint32_t p0 = 0; p0 < n_px; p0 += T) {
+        uint32_t mask = 0;
+        if (p0 + tid < n_px) {
+            const uint32_t row = (p0 + tid) / bw;
+            const int x = bx0 + (int)(p0 + tid - row * bw), y = by0 + (int)row;
+            const size_t s = (size_t)y * w + x;
+            const uint32_t its = tri_id(tri, s);
+            float gs[4], cs[4];
+            for (uint32_t c = 0; c < n_comp; c++) {
+                gs[c] = gy[s * n_comp + c];
+                cs[c] = img[s * n_comp + c];
+            }
+#pragma unroll
             for (int k = 0; k < 8; k++) {
-                const int nx = x + kAaOffX[k], ny = y + kAaOffY[k];
+                const int nx = x + kAaOffXh[k], ny = y + kAaOffYh[k];
                 if (nx < 0 || ny < 0 || nx >= (int)w || ny >= (int)h) {
                     continue;
                 }
-                AaPair pr;
-                if (!eval_aa_pair(its, tri_id(tri, (size_t)ny * w + nx), x, y, nx, ny, n_faces,
-                                  TriFromClip{faces, clip, n_verts, W, H}, &pr) ||
-                    pr.r >= 1.f || (pr.ia != v && pr.ib != v)) {
-                    continue;
+                const size_t n = (size_t)ny * w + nx;
+                float gr = 0.f;
+                for (uint32_t c = 0; c < n_comp; c++) {
+                    gr += gs[c] * (cs[c] - img[n * n_comp + c]);
                 }
-                aa_accumulate_v(gy, img, n_comp, clip, W, H, w, v, x, y, nx, ny, pr, &dst);
+                gr /= 9.f;
+                if (tri_id(tri, n) != its && gr != 0.f) {
+                    mask |= 1u << k;
+                }
             }
         }
+        // the pairs in raster order: waves, lanes, neighbours
+        uint32_t before = 0, own = 0;
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            const uint64_t m = __ballot((mask >> k) & 1u);
+            before += (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
+            own += (uint32_t)__popcll(m);
+        }
+        if (lane == 0) {
+            wave_pairs[wave] = own;
+        }
+        __syncthreads();
+        uint32_t n_pairs = 0;
+#pragma unroll
+        for (uint32_t q = 0; q < T / 64; q++) {
+            before += q < wave ? wave_pairs[q] : 0u;
+            n_pairs += wave_pairs[q];
+        }
+        for (uint32_t m = mask; m; m &= m - 1) {
+            pair[before++] = (uint16_t)(tid << 3 | (uint32_t)__builtin_ctz(m));
+        }
+        __syncthreads();
+        for (uint32_t q0 = 0; q0 < n_pairs; q0 += T) {
+            const uint32_t n_now = min(T, n_pairs - q0);
+            float t[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+            if (tid < n_now) {
+                const uint32_t pk = pair[q0 + tid];
+                const uint32_t p = p0 + (pk >> 3), k = pk & 7u;
+                const uint32_t row = p / bw;
+                const int x = bx0 + (int)(p - row * bw), y = by0 + (int)row;
+                const int nx = x + kAaOffX[k], ny = y + kAaOffY[k];
+                const size_t s = (size_t)y * w + x, n = (size_t)ny * w + nx;
+                AaPair pr;
+                if (eval_aa_pair(tri_id(tri, s), tri_id(tri, n), x, y, nx, ny, n_faces,
+                                 TriFromClip{faces, clip, n_verts, W, H}, &pr) &&
+                    !(pr.r >= 1.f) && (pr.ia == v || pr.ib == v)) {
+                    float gr = 0.f;
+                    for (uint32_t c = 0; c < n_comp; c++) {
+                        gr += gy[s * n_comp + c] * (img[s * n_comp + c] - img[n * n_comp + c]);
+                    }
+                    gr /= 9.f;
+                    float dqa[2], dqb[2];
+                    aa_pair_dq(pr, x, y, dqa, dqb);
+                    float4 g = make_float4(0.f, 0.f, 0.f, 0.f);
+                    if (pr.ia == v) {
+                        aa_add_endpoint(gr, dqa, clip[v], W, H, &g);
+                        t[0] = g.x;
+                        t[1] = g.y;
+                        t[2] = g.w;
+                        g = make_float4(0.f, 0.f, 0.f, 0.f);
+                    }
+                    if (pr.ib == v) {
+                        aa_add_endpoint(gr, dqb, clip[v], W, H, &g);
+                        t[3] = g.x;
+                        t[4] = g.y;
+                        t[5] = g.w;
+                    }
+                }
+            }
+#pragma unroll
+            for (int c = 0; c < 6; c++) {
+                term[tid][c] = t[c];
+            }
+            __syncthreads();
+            if (tid < 3) {
+                // a pair or endpoint that is not v's is +0 here: a sum that
+                // starts at +0 is never -0, and +0 leaves it as it is
+#pragma unroll 4
+                for (uint32_t q = 0; q < n_now; q++) {
+                    acc += term[q][tid];
+                    acc += term[q][3 + tid];
+                }
+            }
+            __syncthreads();
+        }
     }
-    out[v] = dst;
+    if (tid < 3) {
+        float* dst = (float*)&out[v];
+        dst[tid == 2 ? 3 : tid] = acc;
+        if (tid == 0) {
+            dst[2] = 0.f;
+        }
+    }
 }
 
 // ColSum (f_ops.cpp:1227-1244): rows summed in order per column and component.
@@ -1341,8 +1419,8 @@ int dressi_antialias_bwd_vtx_batch(dressi_ctx* ctx, const float* gy, const float
         return DRESSI_OK;
     }
     if (n_samples == 0) {
-        hipLaunchKernelGGL(k_antialias_bwd_vtx_exact_op, dim3(div_up(n_verts, 128), n_items),
-                           dim3(128), 0, ctx->stream, gy, img, n_comp, tri, (const float4*)clip,
+        hipLaunchKernelGGL(k_antialias_bwd_vtx_exact_op, dim3(n_verts, n_items),
+                           dim3(kAaExactThreads), 0, ctx->stream, gy, img, n_comp, tri, (const float4*)clip,
                            n_verts, clip_per_item, faces, n_faces, vtx_faces, max_deg, width,
                            height, (float4*)out);
     } else {

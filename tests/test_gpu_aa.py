@@ -106,6 +106,29 @@ def test_aa_ops_match_oracle(ctx, oracle, seed, level, s):
         _exact(got, want, f"bwd vtx n={n}")
 
 
+@pytest.mark.parametrize("level,h,w,nc", [(3, 97, 90, 3), (1, 150, 211, 1), (0, 16, 16, 4),
+                                          (2, 5, 70, 2)])
+def test_aa_exact_vertex_gradient_steps(ctx, oracle, level, h, w, nc):
+    """The exact vertex gradient over its steps of 256 pixels and lists of 256 pairs: an image
+    without equal neighbours (every pair of two faces counts, hundreds a step), boxes of many
+    steps, of less than one and cut by the screen, a vertex of no face; bit for bit."""
+    from opendressi_amd import ops
+    print(f"[aa exact steps] level={level} {h}x{w}x{nc}", flush=True)
+    clip, faces = _random_scene(oracle, level, level, w)
+    clip = np.concatenate([clip, clip[:1]])
+    tri = oracle.rasterize_face_id(clip, faces, w, h)
+    vf = oracle.vertex_faces_tex(faces, len(clip))
+    rng = np.random.default_rng(nc)
+    img = rng.random((h, w, nc), dtype=np.float32)
+    gy = rng.standard_normal((h, w, nc)).astype(np.float32)
+    got = host(ops.antialias_bwd_vtx(ctx, dev(gy), dev(img), dev(tri), dev(clip), dev(faces),
+                                     dev(vf), None, 0))
+    want = oracle.antialias_bwd_vtx(gy, img, tri, clip, faces, vf, 0.0, 0)
+    assert np.abs(want[:-1]).max() > 0
+    _exact(got, want, "exact")
+    ctx.synchronize()
+
+
 def test_aa_batch_ops_match_oracle(ctx, oracle):
     """The batched AntiAlias / AntiAliasBwdImg / AntiAliasBwdVtx / ColSum
     entry points: three items (own cameras; per-item clips, and one clip
