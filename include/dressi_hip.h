@@ -459,6 +459,29 @@ int dressi_pbr_profile(dressi_pbr_plan* plan, uint32_t iters, char* names,
                        size_t name_stride, float* usec, uint32_t cap,
                        uint32_t* n);
 
+/* ---- the torch surface's ops (python/dressi/torch/ops.py:95-698) ---- */
+/* Each is one call of opendressi_amd.torch in one or two launches, with the
+ * float operations (and their order) of the per-op kernels that the reference
+ * surface composes. `rast` {N,H,W} VEC4 = (u, v, z / w, face + 1). */
+/* rasterize: pos {N,V} VEC4, z in [-w, w]; faces int32 {F,3}; clip_vk
+ * {N,V} VEC4 gets pos with z remapped to [0, w]. */
+int dressi_surface_rasterize(dressi_ctx* ctx, const float* pos, uint32_t n_verts,
+                             uint32_t n_items, const int32_t* faces, uint32_t n_faces,
+                             uint32_t width, uint32_t height, float* clip_vk, float* rast);
+/* interpolate: attr {n_attr} VEC n_comp, shared or per item -> {N,H,W}. */
+int dressi_surface_interpolate(dressi_ctx* ctx, const float* attr, uint32_t n_attr,
+                               uint32_t n_comp, int attr_per_item, const float* rast,
+                               uint32_t width, uint32_t height, uint32_t n_items,
+                               const float* faces, uint32_t n_faces, float* out);
+/* ... and d/d attr: g_face is scratch of N * F * 3 * n_comp floats; g_attr
+ * {V} (shared_attr: summed over the items) or {N,V}. */
+int dressi_surface_interpolate_bwd(dressi_ctx* ctx, const float* gy, uint32_t n_comp,
+                                   const float* rast, uint32_t width, uint32_t height,
+                                   uint32_t n_items, const float* clip, uint32_t n_clip,
+                                   int clip_per_item, const float* faces, uint32_t n_faces,
+                                   const float* vtx_faces, uint32_t n_verts, uint32_t max_deg,
+                                   int shared_attr, float* g_face, float* g_attr);
+
 /* ---- texture path (C3) ---- */
 /* F::TextureBilinear forward (src/core/f_ops.cpp:2736-2780, BilerpClamp
  * src/core/ibl_math.h:91-115): tex {tw,th} x n_comp (1..4) sampled at

@@ -103,6 +103,10 @@ _SIGS = {
                                             _I, _U, _U, _U, _P]),
     "dressi_col_sum_batch": (_I, [_P, _P, _U, _U, _U, _U, _P]),
     "dressi_gather_dist_grad": (_I, [_P, _P, _P, _P, _U, _P, _U, _P, _U, _F, _I, _U, _U, _P]),
+    "dressi_surface_rasterize": (_I, [_P, _P, _U, _U, _P, _U, _U, _U, _P, _P]),
+    "dressi_surface_interpolate": (_I, [_P, _P, _U, _U, _I, _P, _U, _U, _U, _P, _U, _P]),
+    "dressi_surface_interpolate_bwd": (_I, [_P, _P, _U, _P, _U, _U, _U, _P, _U, _I, _P, _U, _P, _U,
+                                            _U, _I, _P, _P]),
     "dressi_equirect_sample": (_I, [_P, _P, _U, _U, _U, _P, _U, _U, _P]),
     "dressi_equirect_sample_bwd": (_I, [_P, _P, _U, _P, _U, _U, _U, _U, _P]),
     "dressi_avg_pool2x2": (_I, [_P, _P, _U, _U, _U, _P]),

@@ -21,7 +21,7 @@ PKG = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(PKG)
 CSRC = os.path.join(PKG, "csrc")
 LIB = os.path.join(PKG, "libdressi_hip.so")
-SOURCES = ["runtime.hip", "raster.hip", "hsr.hip", "aa.hip", "tex.hip", "ds.hip", "ibl.hip", "pbr.hip",
+SOURCES = ["runtime.hip", "raster.hip", "hsr.hip", "aa.hip", "tex.hip", "ds.hip", "surface.hip", "ibl.hip", "pbr.hip",
            "graph.hip", "executor.hip", "builders.hip", "route.hip"]
 # host-only sources (the examples' asset, geometry and PBR-graph helpers), built with g++;
 # zlib is linked for their deflate streams

@@ -960,33 +960,6 @@ __device__ __forceinline__ void hard_fragment(const HardRec& r, uint32_t f, int 
     }
 }
 
-// Walks the faces binned to one (view, tile) of the hard rasterizer (scan
-// based bins): chunks of up to 256 records are staged through LDS and every
-// lane folds each record via `frag(rec, f)`. When the bin's list overflowed
-// the capacity the walk covers all faces.
-template <typename Rec, typename Frag>
-__device__ __forceinline__ void walk_bin(const Rec* recs, const BinBuffers& b, uint32_t bin,
-                                         uint32_t n_faces, Rec* lds_rec, uint32_t* lds_face,
-                                         Frag&& frag) {
-    const uint32_t beg = b.offsets[bin];
-    const uint32_t end = b.offsets[bin + 1];
-    const bool implicit = end > b.cap;
-    const uint32_t n = implicit ? n_faces : end - beg;
-    for (uint32_t base = 0; base < n; base += kTileThreads) {
-        const uint32_t cnt = (n - base) < (uint32_t)kTileThreads ? (n - base) : kTileThreads;
-        __syncthreads();
-        if (threadIdx.x < cnt) {
-            const uint32_t f = implicit ? base + threadIdx.x : b.list[beg + base + threadIdx.x];
-            lds_face[threadIdx.x] = f;
-            lds_rec[threadIdx.x] = recs[f];
-        }
-        __syncthreads();
-        for (uint32_t j = 0; j < cnt; j++) {
-            frag(lds_rec[j], lds_face[j]);
-        }
-    }
-}
-
 // ---------------------------------------------------------------------------
 // Fixed-capacity soft bins, appended from the setup kernels. A face goes to
 // the tiles of its pixel bbox that its triangle reaches (the separating-axis

@@ -413,6 +413,55 @@ def gather_dist_grad(ctx: Context, gy: torch.Tensor, rs: torch.Tensor, clip: tor
     return out if wide else out[0]
 
 
+# ---- the torch surface's ops (opendressi_amd.torch) -------------------------
+
+def surface_rasterize(ctx: Context, pos: torch.Tensor, faces: torch.Tensor, width: int,
+                      height: int):
+    """dressi_surface_rasterize: pos (N, V, 4), z in [-w, w]; faces (F, 3)
+    int32 -> (rast (N, H, W, 4), pos with z in [0, w])."""
+    _prep(ctx)
+    n, nv = pos.shape[0], pos.shape[1]
+    clip_vk = torch.empty_like(pos)
+    rast = torch.empty((n, height, width, 4), dtype=torch.float32, device=pos.device)
+    check(lib.dressi_surface_rasterize(ctx.handle, _ptr(pos, "pos"), nv, n,
+                                       C.c_void_p(faces.data_ptr()), faces.shape[0], width,
+                                       height, _ptr(clip_vk, "clip"), _ptr(rast, "rast")))
+    return rast, clip_vk
+
+
+def surface_interpolate(ctx: Context, attr: torch.Tensor, rast: torch.Tensor,
+                        faces: torch.Tensor) -> torch.Tensor:
+    """dressi_surface_interpolate: attr (V, C) shared or (N, V, C), rast
+    (N, H, W, 4), faces (F, 3) float ids -> (N, H, W, C)."""
+    _prep(ctx)
+    n, h, w = rast.shape[:3]
+    nv, nc = attr.shape[-2], attr.shape[-1]
+    out = torch.empty((n, h, w, nc), dtype=torch.float32, device=rast.device)
+    check(lib.dressi_surface_interpolate(ctx.handle, _ptr(attr, "attr"), nv, nc,
+                                         1 if attr.dim() == 3 else 0, _ptr(rast, "rast"), w, h, n,
+                                         _ptr(faces, "faces"), faces.shape[0], _ptr(out, "out")))
+    return out
+
+
+def surface_interpolate_bwd(ctx: Context, gy: torch.Tensor, rast: torch.Tensor,
+                            clip: torch.Tensor, faces: torch.Tensor, vtx_faces: torch.Tensor,
+                            shared: bool) -> torch.Tensor:
+    """dressi_surface_interpolate_bwd: gy (N, H, W, C), clip (N, V, 4) ->
+    d/d attr (V, C) when `shared`, else (N, V, C)."""
+    _prep(ctx)
+    n, h, w, nc = gy.shape
+    deg, nv = vtx_faces.shape
+    nf = faces.shape[0]
+    g_face = torch.empty((n, nf, 3, nc), dtype=torch.float32, device=gy.device)
+    out = torch.empty((nv, nc) if shared else (n, nv, nc), dtype=torch.float32, device=gy.device)
+    check(lib.dressi_surface_interpolate_bwd(
+        ctx.handle, _ptr(gy, "gy"), nc, _ptr(rast, "rast"), w, h, n, _ptr(clip, "clip"),
+        clip.shape[1], 1 if clip.shape[0] > 1 else 0, _ptr(faces, "faces"), nf,
+        _ptr(vtx_faces, "vtx_faces"), nv, deg, 1 if shared else 0, _ptr(g_face, "g_face"),
+        _ptr(out, "out")))
+    return out
+
+
 # ---- split-sum IBL ops (maps are (H, W, C) equirect images) ----------------
 
 def _map_nc(m: torch.Tensor) -> int:

@@ -23,9 +23,9 @@ def tri_int32(tri: torch.Tensor) -> torch.Tensor:
 
 class MeshData:
     """Static-topology arrays of one triangle list, on the device
-    (python/dressi/torch/meshdata.py:11-43): faces as float ids, the unweld
-    gather index, sequential faces of the unwelded corners, the per-corner
-    face id, the {max_deg, V} vertex -> face adjacency."""
+    (python/dressi/torch/meshdata.py:11-43): faces as float ids and as int32,
+    sequential faces of the unwelded corners, the per-corner face id, the
+    {max_deg, V} vertex -> face adjacency."""
 
     def __init__(self, tri: torch.Tensor, device: torch.device):
         # the source tensor is pinned: the cache key holds its data_ptr
@@ -35,7 +35,7 @@ class MeshData:
         self.n_verts = int(t.max().item()) + 1 if self.n_faces else 0
         faces_np = t.numpy().astype(np.float32)
         self.faces_f = torch.from_numpy(faces_np).to(device)
-        self.unweld = t.reshape(-1).long().to(device)
+        self.faces_i = t.to(device)
         self.faces_seq = torch.arange(self.n_faces * 3, dtype=torch.float32).reshape(-1, 3).to(device)
         self.corner_face_id = torch.arange(self.n_faces, dtype=torch.float32).repeat_interleave(3).to(device)
         vft = vertex_faces_tex(faces_np, self.n_verts)

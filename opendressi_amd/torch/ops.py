@@ -8,9 +8,9 @@ device, with no host round trip. The backward of every op composes the
 reference's backward kernels exactly as the reference's backward builder does
 (src/core/build_backward.cpp:62-149): the same kernels, the same operand
 order, gradient contributions summed in descending creation order of the
-nodes that produced them. rasterize runs the whole batch in one raster
-pass; the other ops run their per-item kernels for each item; per-signature
-constants live in the context's `_engines`.
+nodes that produced them. rasterize, interpolate and antialias run the whole
+batch at once; the other ops run their per-item kernels for each item;
+per-signature state lives in the context's `_engines`.
 """
 from __future__ import annotations
 
@@ -53,11 +53,10 @@ def rasterize(ctx: RasterizeHipContext, pos: torch.Tensor, tri: torch.Tensor, re
     returns (rast, rast_db) with rast[..., :] = (u, v, z/w, triangle_id + 1),
     0 = background, rast_db zeros.
 
-    The mesh is unwelded per corner and rasterized with the corner
-    barycentric constants (1,0), (0,1), (0,0) plus (z, w) as perspective-
-    correct attributes; z/w is guarded by the coverage mask (0 on
-    background). Not differentiable w.r.t. `pos` (geometry gradients come
-    from antialias / rasterize_soft)."""
+    The raster carries the corner barycentric constants (1,0), (0,1), (0,0)
+    and (z, w) as perspective-correct attributes; z/w is 0 on background. Not
+    differentiable w.r.t. `pos` (geometry gradients come from antialias /
+    rasterize_soft)."""
     if ranges is not None:
         raise NotImplementedError("opendressi_amd.torch: range mode is not supported")
     del grad_db
@@ -66,38 +65,18 @@ def rasterize(ctx: RasterizeHipContext, pos: torch.Tensor, tri: torch.Tensor, re
     if pos_b.shape[2] != 4:
         raise ValueError(f"pos must have 4 components, got {pos_b.shape[2]}")
     md = ctx.mesh(tri)
-    n = pos_b.shape[0]
-
-    def build():
-        corner = torch.tensor([[1.0, 0.0], [0.0, 1.0], [0.0, 0.0]], dtype=torch.float32)
-        return _Engine(corner_uv=corner.repeat(md.n_faces, 1).to(ctx.device))
-
-    eng = ctx.engine(("rasterize", h, w, md.n_faces, md.n_verts, n), build)
-    clip_vk = clip_gl_to_vk(pos_b)
+    if md.n_verts > pos_b.shape[1]:
+        raise IndexError(f"tri names vertex {md.n_verts - 1}, pos has {pos_b.shape[1]}")
+    ctx.engine(("rasterize", h, w, md.n_faces, md.n_verts, pos_b.shape[0]), _Engine)
     with ctx.lock:
-        # every item in one pass: attributes and face ids from the same raster
-        clip3 = clip_vk[:, md.unweld].contiguous()
-        attr4 = torch.cat([eng.corner_uv.expand(n, -1, -1), pos_b[:, md.unweld][:, :, 2:4]],
-                          dim=2).contiguous()
-        g, tid = K.rasterize_batch(ctx._ctx, clip3, attr4, md.faces_seq, w, h,
-                                   with_face_id=True)
-        mask = (tid > 0.5).to(torch.float32)
-        zw = g[..., 2] / (g[..., 3] + (1.0 - mask))
-        rast = torch.stack([g[..., 0], g[..., 1], zw, tid], dim=-1)
+        # every item in one pass
+        rast, clip_vk = K.surface_rasterize(ctx._ctx, pos_b, md.faces_i, w, h)
     rast = rast.to(pos.device)
     stamp(rast, RasterOrigin(clip_vk=clip_vk, tri=tri, resolution=(h, w), ctx=ctx))
     return rast, torch.zeros_like(rast)
 
 
 # ------------------------------ interpolate --------------------------------
-
-
-def _faces_of(ctx, attr: torch.Tensor, faces: torch.Tensor, corner: int, n: int) -> torch.Tensor:
-    """LookupFaces of a shared (V, C) attribute -> (F, C), or of per-item
-    (N, V, C) attributes -> (N, F, C), in one launch."""
-    if attr.dim() == 2:
-        return K.lookup_faces(ctx, attr, faces, corner)
-    return K.lookup_faces_batch(ctx, attr, faces, corner, n)
 
 
 class _InterpolateFn(torch.autograd.Function):
@@ -107,50 +86,27 @@ class _InterpolateFn(torch.autograd.Function):
         attr_d = to_dev(attr, dev, "attr")
         rast_d = to_dev(rast, dev, "rast")
         shared = attr_d.dim() == 2
-        c = channels(attr_d.shape[-1], "attr")
-        n = rast_d.shape[0]
+        channels(attr_d.shape[-1], "attr")
+        if attr_d.dim() not in (2, 3) or (not shared and attr_d.shape[0] != rast_d.shape[0]):
+            raise ValueError(f"attr must be [V, C] or [{rast_d.shape[0]}, V, C], got "
+                             f"{tuple(attr.shape)}")
         with vctx.lock:
-            # each op once for the whole batch
-            a = attr_d.contiguous()
-            tid = rast_d[..., 3].contiguous()
-            pix = [K.face_fetch_batch(vctx._ctx, _faces_of(vctx._ctx, a, md.faces_f, k, n), tid)
-                   for k in range(3)]
-        u = rast_d[..., 0:1]
-        v = rast_d[..., 1:2]
-        out = u * pix[0] + v * pix[1] + ((1.0 - u) - v) * pix[2]
-        fctx.dressi = (vctx, md, rinfo, shared, c)
+            # the whole batch in one launch
+            out = K.surface_interpolate(vctx._ctx, attr_d, rast_d, md.faces_f)
+        fctx.dressi = (vctx, md, rinfo, shared)
         fctx.save_for_backward(attr, rast)
         return out.to(attr.device)
 
     @staticmethod
     def backward(fctx, grad_out):
-        vctx, md, rinfo, shared, c = fctx.dressi
+        vctx, md, rinfo, shared = fctx.dressi
         attr, rast = fctx.saved_tensors
         dev = vctx.device
         rast_d = to_dev(rast, dev, "rast")
         g = to_dev(grad_out, dev, "grad_out")
-        n = rast_d.shape[0]
-        clip_vk = rinfo.clip_vk
-        u = rast_d[..., 0:1]
-        v = rast_d[..., 1:2]
-        g_pix = [g * u, g * v, g * ((1.0 - u) - v)]
-        seeds = torch.zeros(n, dtype=torch.float32, device=dev)
         with vctx.lock:
-            clip = clip_vk.contiguous() if clip_vk.shape[0] > 1 else clip_vk[0].contiguous()
-            prj = [_faces_of(vctx._ctx, clip, md.faces_f, k, n) for k in range(3)]
-            tid = rast_d[..., 3].contiguous()
-            # per corner k = 2, 1, 0: the (N, V, C) vertex contributions
-            contribs = []
-            for k in (2, 1, 0):
-                g_face = K.face_fetch_bwd_batch(vctx._ctx, g_pix[k].contiguous(), tid, prj[0],
-                                                prj[1], prj[2], seeds, 1.0, 0)
-                contribs.append(K.lookup_faces_bwd_batch(vctx._ctx, g_face, md.faces_f, md.vft, k))
-        per_item = [[cb[i] for cb in contribs] for i in range(n)]
-        if shared:
-            # the shared leaf's consumers, latest-created (last item) first
-            g_attr = sum_contribs([cb for contribs in reversed(per_item) for cb in contribs])
-        else:
-            g_attr = torch.stack([sum_contribs(cb) for cb in per_item], 0)
+            g_attr = K.surface_interpolate_bwd(vctx._ctx, g, rast_d, rinfo.clip_vk, md.faces_f,
+                                               md.vft, shared)
         return g_attr.to(attr.device), None, None, None, None
 
 
