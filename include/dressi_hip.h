@@ -482,6 +482,28 @@ int dressi_surface_interpolate_bwd(dressi_ctx* ctx, const float* gy, uint32_t n_
                                    const float* vtx_faces, uint32_t n_verts, uint32_t max_deg,
                                    int shared_attr, float* g_face, float* g_attr);
 
+/* antialias and its backward: img, gy {N,H,W} VEC n_comp, pos {V} VEC4
+ * (shared) or {N,V}, z not read. d/d pos {N,n_rows} VEC4, for an adjacency of
+ * the same faces, times `boost`: the exact gradient (n_samples = 0) or the
+ * stochastic one of item i's seed float(seed + i); g_corner is scratch of
+ * N * F * 9 floats (n_samples > 0). */
+int dressi_surface_antialias(dressi_ctx* ctx, const float* img, uint32_t n_comp,
+                             const float* rast, const float* pos, uint32_t n_verts,
+                             int pos_per_item, const float* faces, uint32_t n_faces,
+                             uint32_t width, uint32_t height, uint32_t n_items, float* out);
+int dressi_surface_antialias_bwd_img(dressi_ctx* ctx, const float* gy, uint32_t n_comp,
+                                     const float* rast, const float* pos, uint32_t n_verts,
+                                     int pos_per_item, const float* faces, uint32_t n_faces,
+                                     uint32_t width, uint32_t height, uint32_t n_items,
+                                     float* out);
+int dressi_surface_antialias_bwd_pos(dressi_ctx* ctx, const float* gy, const float* img,
+                                     uint32_t n_comp, const float* rast, const float* pos,
+                                     uint32_t n_verts, int pos_per_item, const float* faces,
+                                     uint32_t n_faces, const float* vtx_faces, uint32_t n_rows,
+                                     uint32_t max_deg, uint64_t seed, uint32_t n_samples,
+                                     float boost, uint32_t width, uint32_t height,
+                                     uint32_t n_items, float* g_corner, float* out);
+
 /* ---- texture path (C3) ---- */
 /* F::TextureBilinear forward (src/core/f_ops.cpp:2736-2780, BilerpClamp
  * src/core/ibl_math.h:91-115): tex {tw,th} x n_comp (1..4) sampled at

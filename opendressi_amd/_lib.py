@@ -107,6 +107,11 @@ _SIGS = {
     "dressi_surface_interpolate": (_I, [_P, _P, _U, _U, _I, _P, _U, _U, _U, _P, _U, _P]),
     "dressi_surface_interpolate_bwd": (_I, [_P, _P, _U, _P, _U, _U, _U, _P, _U, _I, _P, _U, _P, _U,
                                             _U, _I, _P, _P]),
+    "dressi_surface_antialias": (_I, [_P, _P, _U, _P, _P, _U, _I, _P, _U, _U, _U, _U, _P]),
+    "dressi_surface_antialias_bwd_img": (_I, [_P, _P, _U, _P, _P, _U, _I, _P, _U, _U, _U, _U,
+                                              _P]),
+    "dressi_surface_antialias_bwd_pos": (_I, [_P, _P, _P, _U, _P, _P, _U, _I, _P, _U, _P, _U, _U,
+                                              C.c_uint64, _U, _F, _U, _U, _U, _P, _P]),
     "dressi_equirect_sample": (_I, [_P, _P, _U, _U, _U, _P, _U, _U, _P]),
     "dressi_equirect_sample_bwd": (_I, [_P, _P, _U, _P, _U, _U, _U, _U, _P]),
     "dressi_avg_pool2x2": (_I, [_P, _P, _U, _U, _U, _P]),

@@ -9,10 +9,6 @@ namespace dressi {
 
 namespace {
 
-__device__ __forceinline__ uint32_t tri_id(const float* tri, size_t o) {
-    return (uint32_t)(int)(tri[o] + 0.5f);  // int(tri + 0.5f) (cpu_raster.cpp:374-375)
-}
-
 // Reference-layout accessors of the per-op kernels: faces as float ids
 // (int64(v + 0.5f), cpu_raster.cpp:395), clip {V,1} VEC4.
 struct FloatFaces {
@@ -40,6 +36,15 @@ struct TriFromRecs {
     }
 };
 
+// A face-id image: face + 1 as int(tri + 0.5f) (cpu_raster.cpp:374-375).
+struct TriIds {
+    const float* p;
+    uint32_t stride;
+    __device__ uint32_t operator()(size_t o) const {
+        return (uint32_t)(int)(p[o * stride] + 0.5f);
+    }
+};
+
 // kAaOffX / kAaOffY as compile-time constants (register-array indices)
 constexpr int kAaOffXh[8] = {-1, 0, 1, -1, 1, -1, 0, 1};
 constexpr int kAaOffYh[8] = {-1, -1, -1, 0, 0, 1, 1, 1};
@@ -51,7 +56,8 @@ constexpr int kAaOffYh[8] = {-1, -1, -1, 0, 0, 1, 1, 1};
 // ---------------------------------------------------------------------------
 
 // Batched per-op kernels: blockIdx.y is the item; images are [item][H][W]
-// (x n_comp), clips [item][V] when `clip_per_item`, else shared.
+// (x n_comp), clips [item][V] when `clip_per_item`, else shared; face ids are
+// `tri_stride` floats apart (1, or 4 in the torch surface's raster).
 struct AaItem {
     uint32_t item;
     size_t npx;
@@ -61,45 +67,100 @@ struct AaItem {
     __device__ const float4* clip(const float4* p, uint32_t n_verts, int per_item) const {
         return per_item ? p + (size_t)item * n_verts : p;
     }
+    __device__ TriIds tri(const float* p, uint32_t stride) const {
+        return TriIds{p + item * npx * stride, stride};
+    }
 };
 
-// AntiAlias forward (f_ops.cpp:2544-2576), one thread per pixel.
+// AntiAlias forward (f_ops.cpp:2544-2576), one thread per pixel for the sum.
+// Its pairs of two faces are listed in LDS and evaluated densely by the
+// workgroup: evaluated by the pixel's own thread, one neighbour after the
+// other, each waits for face, corner and clip loads while the lanes of
+// pixels without such a pair idle (28 us for 61 x 97 pixels, 43 us for eight
+// images of 256 x 256; so 14 and 26).
 __global__ __launch_bounds__(256) void k_antialias_op(const float* img, uint32_t n_comp,
-                                                      const float* tri, const float4* clip,
-                                                      uint32_t n_verts, int clip_per_item,
-                                                      const float* faces, uint32_t n_faces,
-                                                      uint32_t w, uint32_t h, float* out) {
-    const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
+                                                      const float* tri_f, uint32_t tri_stride,
+                                                      const float4* clip, uint32_t n_verts,
+                                                      int clip_per_item, const float* faces,
+                                                      uint32_t n_faces, uint32_t w, uint32_t h,
+                                                      float* out) {
+    __shared__ uint16_t pair[256 * 8];  // pixel's thread << 3 | neighbour
+    __shared__ float ratio[256 * 8];    // its r, < 0: no active edge
+    __shared__ uint32_t n_pairs;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+    const uint32_t p0 = blockIdx.x * 256, p = p0 + tid;
+    const AaItem it(w, h);
+    img = it.img(img, n_comp);
+    out = it.img(out, n_comp);
+    const TriIds tri = it.tri(tri_f, tri_stride);
+    clip = it.clip(clip, n_verts, clip_per_item);
+    const float W = (float)w, H = (float)h;
+    if (tid == 0) {
+        n_pairs = 0;
+    }
+    __syncthreads();
+    const int x = (int)(p % w), y = (int)(p / w);
+    uint32_t mask = 0;
+    if (p < w * h) {
+        const uint32_t its = tri(p);
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            const int nx = x + kAaOffXh[k], ny = y + kAaOffYh[k];
+            if (!(nx < 0 || ny < 0 || nx >= (int)w || ny >= (int)h) &&
+                tri((size_t)ny * w + nx) != its) {
+                mask |= 1u << k;
+            }
+        }
+    }
+    uint32_t own = 0, before = 0;
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        const uint64_t m = __ballot((mask >> k) & 1u);
+        before += (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
+        own += (uint32_t)__popcll(m);
+    }
+    if (own) {
+        uint32_t base = 0;
+        if (lane == 0) {
+            base = atomicAdd(&n_pairs, own);
+        }
+        before += (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
+        for (uint32_t m = mask; m; m &= m - 1) {
+            pair[before++] = (uint16_t)(tid << 3 | (uint32_t)__builtin_ctz(m));
+        }
+    }
+    __syncthreads();
+    for (uint32_t q = tid; q < n_pairs; q += 256) {
+        const uint32_t pk = pair[q], ps = p0 + (pk >> 3), k = pk & 7u;
+        const int sx = (int)(ps % w), sy = (int)(ps / w);
+        const int nx = sx + kAaOffX[k], ny = sy + kAaOffY[k];
+        AaPair pr;
+        ratio[pk] = eval_aa_pair(tri(ps), tri((size_t)ny * w + nx), sx, sy, nx, ny, n_faces,
+                                 TriFromClip{faces, clip, n_verts, W, H}, &pr)
+                            ? pr.r
+                            : -1.f;
+    }
+    __syncthreads();
     if (p >= w * h) {
         return;
     }
-    const AaItem it(w, h);
-    img = it.img(img, n_comp);
-    tri = it.img(tri, 1);
-    out = it.img(out, n_comp);
-    clip = it.clip(clip, n_verts, clip_per_item);
-    const int x = (int)(p % w), y = (int)(p / w);
-    const float W = (float)w, H = (float)h;
     const size_t so = (size_t)p * n_comp;
-    float dst[4];
+    float src[4], dst[4];
     for (uint32_t c = 0; c < n_comp; c++) {
-        dst[c] = img[so + c];
+        dst[c] = src[c] = img[so + c];
     }
-    const uint32_t its = tri_id(tri, p);
+#pragma unroll
     for (int k = 0; k < 8; k++) {
-        const int nx = x + kAaOffX[k], ny = y + kAaOffY[k];
-        AaPair pr;
-        const bool in = !(nx < 0 || ny < 0 || nx >= (int)w || ny >= (int)h);
-        if (!in || !eval_aa_pair(its, tri_id(tri, (size_t)ny * w + nx), x, y, nx, ny, n_faces,
-                                 TriFromClip{faces, clip, n_verts, W, H}, &pr)) {
+        const float r = (mask >> k) & 1u ? ratio[tid * 8 + k] : -1.f;
+        if (r < 0.f) {
             for (uint32_t c = 0; c < n_comp; c++) {
-                dst[c] += img[so + c];
+                dst[c] += src[c];
             }
             continue;
         }
-        const size_t no = ((size_t)ny * w + nx) * n_comp;
+        const size_t no = ((size_t)(y + kAaOffYh[k]) * w + (x + kAaOffXh[k])) * n_comp;
         for (uint32_t c = 0; c < n_comp; c++) {
-            dst[c] += pr.r * img[so + c] + (1.f - pr.r) * img[no + c];
+            dst[c] += r * src[c] + (1.f - r) * img[no + c];
         }
     }
     for (uint32_t c = 0; c < n_comp; c++) {
@@ -109,7 +170,9 @@ __global__ __launch_bounds__(256) void k_antialias_op(const float* img, uint32_t
 
 // AntiAliasBwdImg (f_ops.cpp:2231-2275), one thread per pixel.
 __global__ __launch_bounds__(256) void k_antialias_bwd_img_op(const float* gy, uint32_t n_comp,
-                                                              const float* tri, const float4* clip,
+                                                              const float* tri_f,
+                                                              uint32_t tri_stride,
+                                                              const float4* clip,
                                                               uint32_t n_verts, int clip_per_item,
                                                               const float* faces,
                                                               uint32_t n_faces, uint32_t w,
@@ -120,7 +183,7 @@ __global__ __launch_bounds__(256) void k_antialias_bwd_img_op(const float* gy, u
     }
     const AaItem it(w, h);
     gy = it.img(gy, n_comp);
-    tri = it.img(tri, 1);
+    const TriIds tri = it.tri(tri_f, tri_stride);
     out = it.img(out, n_comp);
     clip = it.clip(clip, n_verts, clip_per_item);
     const int x = (int)(p % w), y = (int)(p / w);
@@ -128,14 +191,14 @@ __global__ __launch_bounds__(256) void k_antialias_bwd_img_op(const float* gy, u
     const size_t so = (size_t)p * n_comp;
     float dst[4] = {0.f, 0.f, 0.f, 0.f};
     float alpha_sum = 0.f;
-    const uint32_t its = tri_id(tri, p);
+    const uint32_t its = tri(p);
     for (int k = 0; k < 8; k++) {
         const int nx = x + kAaOffX[k], ny = y + kAaOffY[k];
         if (nx < 0 || ny < 0 || nx >= (int)w || ny >= (int)h) {
             alpha_sum += 1.f;
             continue;
         }
-        const uint32_t itn = tri_id(tri, (size_t)ny * w + nx);
+        const uint32_t itn = tri((size_t)ny * w + nx);
         AaPair pr;
         alpha_sum += eval_aa_pair(its, itn, x, y, nx, ny, n_faces,
                                   TriFromClip{faces, clip, n_verts, W, H}, &pr)
@@ -165,7 +228,7 @@ __global__ __launch_bounds__(256) void k_antialias_bwd_img_op(const float* gy, u
 // so the row sums its terms in the reference's (slot, sample, neighbour)
 // order.
 __global__ __launch_bounds__(256) void k_antialias_bwd_vtx_op(
-        const float* gy, const float* img, uint32_t n_comp, const float* tri, const float4* clip,
+        const float* gy, const float* img, uint32_t n_comp, const float* tri_f, const float4* clip,
         uint32_t n_verts, int clip_per_item, const float* faces, uint32_t n_faces,
         const float* vtx_faces, uint32_t max_deg, const float* seed, uint32_t n_samples, int wide,
         uint32_t w, uint32_t h, float4* out) {
@@ -179,7 +242,7 @@ __global__ __launch_bounds__(256) void k_antialias_bwd_vtx_op(
     const AaItem it(w, h);
     gy = it.img(gy, n_comp);
     img = it.img(img, n_comp);
-    tri = it.img(tri, 1);
+    const TriIds tri = it.tri(tri_f, 1);
     clip = it.clip(clip, n_verts, clip_per_item);
     seed += it.item;
     out += (size_t)it.item * rows * n_verts;
@@ -225,9 +288,9 @@ __global__ __launch_bounds__(256) void k_antialias_bwd_vtx_op(
             int has = 0;
             const int nx = x + kAaOffX[k], ny = y + kAaOffY[k];
             if (!(nx < 0 || ny < 0 || nx >= (int)w || ny >= (int)h)) {
-                const uint32_t its = tri_id(tri, (size_t)y * w + x);
+                const uint32_t its = tri((size_t)y * w + x);
                 AaPair pr;
-                if (eval_aa_pair(its, tri_id(tri, (size_t)ny * w + nx), x, y, nx, ny, n_faces,
+                if (eval_aa_pair(its, tri((size_t)ny * w + nx), x, y, nx, ny, n_faces,
                                  TriFromClip{faces, clip, n_verts, W, H}, &pr) &&
                     pr.r < 1.f && (pr.ia == v || pr.ib == v)) {
                     const size_t so = ((size_t)y * w + x) * n_comp;
@@ -298,9 +361,10 @@ __global__ __launch_bounds__(256) void k_antialias_bwd_vtx_op(
 constexpr uint32_t kAaExactThreads = 256;
 
 __global__ __launch_bounds__(kAaExactThreads) void k_antialias_bwd_vtx_exact_op(
-        const float* gy, const float* img, uint32_t n_comp, const float* tri, const float4* clip,
-        uint32_t n_verts, int clip_per_item, const float* faces, uint32_t n_faces,
-        const float* vtx_faces, uint32_t max_deg, uint32_t w, uint32_t h, float4* out) {
+        const float* gy, const float* img, uint32_t n_comp, const float* tri_f, uint32_t tri_stride,
+        const float4* clip, uint32_t n_verts, int clip_per_item, const float* faces,
+        uint32_t n_faces, const float* vtx_faces, uint32_t n_rows, uint32_t max_deg, uint32_t w,
+        uint32_t h, float scale, float4* out) {
     constexpr uint32_t T = kAaExactThreads;
     __shared__ int box[4];
     __shared__ uint32_t wave_pairs[T / 64];
@@ -311,9 +375,9 @@ __global__ __launch_bounds__(kAaExactThreads) void k_antialias_bwd_vtx_exact_op(
     const AaItem it(w, h);
     gy = it.img(gy, n_comp);
     img = it.img(img, n_comp);
-    tri = it.img(tri, 1);
+    const TriIds tri = it.tri(tri_f, tri_stride);
     clip = it.clip(clip, n_verts, clip_per_item);
-    out += (size_t)it.item * n_verts;
+    out += (size_t)it.item * n_rows;
     const float W = (float)w, H = (float)h;
     if (tid == 0) {
         box[0] = (int)w;
@@ -323,7 +387,7 @@ __global__ __launch_bounds__(kAaExactThreads) void k_antialias_bwd_vtx_exact_op(
     }
     __syncthreads();
     for (uint32_t d = tid; d < max_deg; d += T) {
-        const float fv = vtx_faces[(size_t)d * n_verts + v];
+        const float fv = vtx_faces[(size_t)d * n_rows + v];
         if (fv < -0.5f) {
             continue;
         }
@@ -356,7 +420,7 @@ __global__ __launch_bounds__(kAaExactThreads) void k_antialias_bwd_vtx_exact_op(
             const uint32_t row = (p0 + tid) / bw;
             const int x = bx0 + (int)(p0 + tid - row * bw), y = by0 + (int)row;
             const size_t s = (size_t)y * w + x;
-            const uint32_t its = tri_id(tri, s);
+            const uint32_t its = tri(s);
             float gs[4], cs[4];
             for (uint32_t c = 0; c < n_comp; c++) {
                 gs[c] = gy[s * n_comp + c];
@@ -374,7 +438,7 @@ __global__ __launch_bounds__(kAaExactThreads) void k_antialias_bwd_vtx_exact_op(
                     gr += gs[c] * (cs[c] - img[n * n_comp + c]);
                 }
                 gr /= 9.f;
-                if (tri_id(tri, n) != its && gr != 0.f) {
+                if (tri(n) != its && gr != 0.f) {
                     mask |= 1u << k;
                 }
             }
@@ -412,7 +476,7 @@ __global__ __launch_bounds__(kAaExactThreads) void k_antialias_bwd_vtx_exact_op(
                 const int nx = x + kAaOffX[k], ny = y + kAaOffY[k];
                 const size_t s = (size_t)y * w + x, n = (size_t)ny * w + nx;
                 AaPair pr;
-                if (eval_aa_pair(tri_id(tri, s), tri_id(tri, n), x, y, nx, ny, n_faces,
+                if (eval_aa_pair(tri(s), tri(n), x, y, nx, ny, n_faces,
                                  TriFromClip{faces, clip, n_verts, W, H}, &pr) &&
                     !(pr.r >= 1.f) && (pr.ia == v || pr.ib == v)) {
                     float gr = 0.f;
@@ -457,11 +521,146 @@ __global__ __launch_bounds__(kAaExactThreads) void k_antialias_bwd_vtx_exact_op(
     }
     if (tid < 3) {
         float* dst = (float*)&out[v];
-        dst[tid == 2 ? 3 : tid] = acc;
+        dst[tid == 2 ? 3 : tid] = acc * scale;
         if (tid == 0) {
-            dst[2] = 0.f;
+            dst[2] = 0.f * scale;
         }
     }
+}
+
+// The torch surface's stochastic vertex gradient: k_antialias_bwd_vtx_op's
+// rows and ColSum for an adjacency that is the faces' own (VertexFacesTex), so
+// that the rows of one face are its three corners'. One wave per face and item
+// takes eight samples at once, a lane per (sample, neighbour), tests each pair
+// by what needs no geometry (two faces, dot(gy(s), c(s) - c(n)) / 9 not 0),
+// evaluates the few left and adds their terms per corner in (sample,
+// neighbour, endpoint) order into g_corner {N,F,3} (x, y, w).
+//
+// The row form repeats every face's samples for its three corners and waits
+// for each sample's loads in turn: 66 us for eight views of 642 vertices
+// and eight samples, this 17 + 6.
+__global__ __launch_bounds__(64) void k_surface_aa_bwd_faces(
+        const float* gy, const float* img, uint32_t n_comp, const float* tri_f,
+        uint32_t tri_stride, const float4* clip, uint32_t n_verts, int clip_per_item,
+        const float* faces, uint32_t n_faces, uint64_t seed0, uint32_t n_samples, uint32_t w,
+        uint32_t h, float* g_corner) {
+    __shared__ float term[64][6];   // endpoint a's x, y, w, then b's
+    __shared__ uint32_t end[64][2];  // their vertices
+    const uint32_t f = blockIdx.x, lane = threadIdx.x;
+    const AaItem it(w, h);
+    gy = it.img(gy, n_comp);
+    img = it.img(img, n_comp);
+    const TriIds tri = it.tri(tri_f, tri_stride);
+    clip = it.clip(clip, n_verts, clip_per_item);
+    g_corner += ((size_t)it.item * n_faces + f) * 9;
+    const float W = (float)w, H = (float)h;
+    // the sampler's seed: an integer held in float32, as the image {1,1} the
+    // reference reads it from
+    const uint32_t seed_u = (uint32_t)(int64_t)((float)(seed0 + it.item) + 0.5f);
+    uint32_t vi[3];
+    float4 c[3];
+    bool ok = true;
+#pragma unroll
+    for (int q = 0; q < 3; q++) {
+        vi[q] = FloatFaces{faces}(f, q);
+        ok = ok && vi[q] < n_verts;
+        c[q] = ok ? clip[vi[q]] : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+    float s3x[3], s3y[3];
+    ok = ok && aa_face_screen(c, W, H, s3x, s3y);
+    // lane 3 r + comp < 9 sums corner r's component
+    const uint32_t comp = lane % 3;
+    const uint32_t my = lane < 3 ? vi[0] : lane < 6 ? vi[1] : vi[2];
+    float acc = 0.f;
+    for (uint32_t smp0 = 0; ok && smp0 < n_samples; smp0 += 8) {
+        const uint32_t smp = smp0 + (lane >> 3), k = lane & 7u;
+        int x = 0, y = 0;
+        bool cand = smp < n_samples && aa_sample_px(s3x, s3y, f, smp, seed_u, &x, &y) && x >= 0 &&
+                    y >= 0 && x < (int)w && y < (int)h;
+        const int nx = x + kAaOffX[k], ny = y + kAaOffY[k];
+        cand = cand && nx >= 0 && ny >= 0 && nx < (int)w && ny < (int)h;
+        uint32_t its = 0, itn = 0;
+        float gr = 0.f;
+        if (cand) {
+            const size_t so = (size_t)y * w + x, no = (size_t)ny * w + nx;
+            its = tri(so);
+            itn = tri(no);
+            for (uint32_t cc = 0; cc < n_comp; cc++) {
+                gr += gy[so * n_comp + cc] * (img[so * n_comp + cc] - img[no * n_comp + cc]);
+            }
+            gr /= 9.f;
+            cand = its != itn && gr != 0.f;
+        }
+        AaPair pr;
+        cand = cand && eval_aa_pair(its, itn, x, y, nx, ny, n_faces,
+                                    TriFromClip{faces, clip, n_verts, W, H}, &pr) &&
+               pr.r < 1.f;
+        const uint64_t m = __ballot(cand);
+        if (!m) {
+            continue;
+        }
+        if (cand) {
+            const uint32_t at = (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
+            float dqa[2], dqb[2];
+            aa_pair_dq(pr, x, y, dqa, dqb);
+            float4 ta = make_float4(0.f, 0.f, 0.f, 0.f), tb = ta;
+            aa_add_endpoint(gr, dqa, clip[pr.ia], W, H, &ta);
+            aa_add_endpoint(gr, dqb, clip[pr.ib], W, H, &tb);
+            end[at][0] = pr.ia;
+            end[at][1] = pr.ib;
+            term[at][0] = ta.x;
+            term[at][1] = ta.y;
+            term[at][2] = ta.w;
+            term[at][3] = tb.x;
+            term[at][4] = tb.y;
+            term[at][5] = tb.w;
+        }
+        __syncthreads();
+        if (lane < 9) {
+            const uint32_t n = (uint32_t)__popcll(m);
+            for (uint32_t q = 0; q < n; q++) {
+                // another vertex's term is left out by adding +0: a sum that
+                // starts at +0 is never -0
+                acc += end[q][0] == my ? term[q][comp] : 0.f;
+                acc += end[q][1] == my ? term[q][3 + comp] : 0.f;
+            }
+        }
+        __syncthreads();
+    }
+    if (lane < 9) {
+        g_corner[lane] = acc;
+    }
+}
+
+// ColSum of the vertex's rows in adjacency order, the z remap's transpose
+// (z 0.5 z, w + 0.5 z; the gradient's z is 0) and the boost.
+__global__ __launch_bounds__(256) void k_surface_aa_bwd_vtx(const float* g_corner,
+                                                            const float* faces, uint32_t n_faces,
+                                                            const float* vf, uint32_t n_verts,
+                                                            uint32_t max_deg, float boost,
+                                                            float4* out) {
+    const uint32_t v = blockIdx.x * blockDim.x + threadIdx.x;
+    if (v >= n_verts) {
+        return;
+    }
+    g_corner += (size_t)blockIdx.y * n_faces * 9;
+    float acc[3] = {0.f, 0.f, 0.f};
+    for (uint32_t d = 0; d < max_deg; d++) {
+        const float fv = vf[(size_t)d * n_verts + v];
+        const uint32_t f = fv < -0.5f ? n_faces : fid_u(fv);
+        if (f >= n_faces) {
+            continue;
+        }
+        int k = 2;
+        k = fid_u(faces[(size_t)f * 3 + 1]) == v ? 1 : k;
+        k = fid_u(faces[(size_t)f * 3 + 0]) == v ? 0 : k;
+#pragma unroll
+        for (int q = 0; q < 3; q++) {
+            acc[q] += g_corner[(size_t)f * 9 + k * 3 + q];
+        }
+    }
+    out[(size_t)blockIdx.y * n_verts + v] =
+            make_float4(acc[0] * boost, acc[1] * boost, 0.f * boost, acc[2] * boost);
 }
 
 // ColSum (f_ops.cpp:1227-1244): rows summed in order per column and component.
@@ -1362,8 +1561,8 @@ int dressi_antialias_batch(dressi_ctx* ctx, const float* img, uint32_t n_comp, c
     }
     const uint32_t npx = width * height;
     hipLaunchKernelGGL(k_antialias_op, dim3(div_up(npx, 256), n_items), dim3(256), 0,
-                       ctx->stream, img, n_comp, tri, (const float4*)clip, n_verts, clip_per_item,
-                       faces, n_faces, width, height, out);
+                       ctx->stream, img, n_comp, tri, 1u, (const float4*)clip, n_verts,
+                       clip_per_item, faces, n_faces, width, height, out);
     DRESSI_CHECK_LAUNCH();
     return DRESSI_OK;
 }
@@ -1389,8 +1588,8 @@ int dressi_antialias_bwd_img_batch(dressi_ctx* ctx, const float* gy, uint32_t n_
     }
     const uint32_t npx = width * height;
     hipLaunchKernelGGL(k_antialias_bwd_img_op, dim3(div_up(npx, 256), n_items), dim3(256), 0,
-                       ctx->stream, gy, n_comp, tri, (const float4*)clip, n_verts, clip_per_item,
-                       faces, n_faces, width, height, out);
+                       ctx->stream, gy, n_comp, tri, 1u, (const float4*)clip, n_verts,
+                       clip_per_item, faces, n_faces, width, height, out);
     DRESSI_CHECK_LAUNCH();
     return DRESSI_OK;
 }
@@ -1420,9 +1619,9 @@ int dressi_antialias_bwd_vtx_batch(dressi_ctx* ctx, const float* gy, const float
     }
     if (n_samples == 0) {
         hipLaunchKernelGGL(k_antialias_bwd_vtx_exact_op, dim3(n_verts, n_items),
-                           dim3(kAaExactThreads), 0, ctx->stream, gy, img, n_comp, tri, (const float4*)clip,
-                           n_verts, clip_per_item, faces, n_faces, vtx_faces, max_deg, width,
-                           height, (float4*)out);
+                           dim3(kAaExactThreads), 0, ctx->stream, gy, img, n_comp, tri, 1u,
+                           (const float4*)clip, n_verts, clip_per_item, faces, n_faces, vtx_faces,
+                           n_verts, max_deg, width, height, 1.f, (float4*)out);
     } else {
         const uint32_t rows = wide ? max_deg : 1u;
         DRESSI_REQUIRE((uint64_t)n_verts * rows * 8 < (1ull << 32), "AntiAliasBwdVtx: too many rows");
@@ -1464,6 +1663,83 @@ int dressi_col_sum_batch(dressi_ctx* ctx, const float* x, uint32_t n_comp, uint3
 int dressi_col_sum(dressi_ctx* ctx, const float* x, uint32_t n_comp, uint32_t width,
                    uint32_t height, float* out) {
     return dressi_col_sum_batch(ctx, x, n_comp, width, height, 1, out);
+}
+
+// The torch surface's antialias: ids from the raster's fourth channel, pos
+// as the caller's clip positions (z is not read).
+int dressi_surface_antialias(dressi_ctx* ctx, const float* img, uint32_t n_comp,
+                             const float* rast, const float* pos, uint32_t n_verts,
+                             int pos_per_item, const float* faces, uint32_t n_faces,
+                             uint32_t width, uint32_t height, uint32_t n_items, float* out) {
+    if (int rc = check_aa_args(ctx, n_comp, width, height)) return rc;
+    DRESSI_REQUIRE(img && rast && pos && (faces || n_faces == 0) && out, "antialias: NULL buffer");
+    DRESSI_REQUIRE(n_items <= kMaxBatchItems, "batch of %u items exceeds %u", n_items,
+                   kMaxBatchItems);
+    if (n_items == 0) {
+        return DRESSI_OK;
+    }
+    hipLaunchKernelGGL(k_antialias_op, dim3(div_up(width * height, 256), n_items), dim3(256), 0,
+                       ctx->stream, img, n_comp, rast + 3, 4u, (const float4*)pos, n_verts,
+                       pos_per_item, faces, n_faces, width, height, out);
+    DRESSI_CHECK_LAUNCH();
+    return DRESSI_OK;
+}
+
+int dressi_surface_antialias_bwd_img(dressi_ctx* ctx, const float* gy, uint32_t n_comp,
+                                     const float* rast, const float* pos, uint32_t n_verts,
+                                     int pos_per_item, const float* faces, uint32_t n_faces,
+                                     uint32_t width, uint32_t height, uint32_t n_items,
+                                     float* out) {
+    if (int rc = check_aa_args(ctx, n_comp, width, height)) return rc;
+    DRESSI_REQUIRE(gy && rast && pos && (faces || n_faces == 0) && out,
+                   "antialias backward: NULL buffer");
+    DRESSI_REQUIRE(n_items <= kMaxBatchItems, "batch of %u items exceeds %u", n_items,
+                   kMaxBatchItems);
+    if (n_items == 0) {
+        return DRESSI_OK;
+    }
+    hipLaunchKernelGGL(k_antialias_bwd_img_op, dim3(div_up(width * height, 256), n_items),
+                       dim3(256), 0, ctx->stream, gy, n_comp, rast + 3, 4u, (const float4*)pos,
+                       n_verts, pos_per_item, faces, n_faces, width, height, out);
+    DRESSI_CHECK_LAUNCH();
+    return DRESSI_OK;
+}
+
+int dressi_surface_antialias_bwd_pos(dressi_ctx* ctx, const float* gy, const float* img,
+                                     uint32_t n_comp, const float* rast, const float* pos,
+                                     uint32_t n_verts, int pos_per_item, const float* faces,
+                                     uint32_t n_faces, const float* vtx_faces, uint32_t n_rows,
+                                     uint32_t max_deg, uint64_t seed, uint32_t n_samples,
+                                     float boost, uint32_t width, uint32_t height,
+                                     uint32_t n_items, float* g_corner, float* out) {
+    if (int rc = check_aa_args(ctx, n_comp, width, height)) return rc;
+    DRESSI_REQUIRE(gy && img && rast && pos && (faces || n_faces == 0) && vtx_faces && out &&
+                           (g_corner || n_faces == 0 || n_samples == 0),
+                   "antialias backward: NULL buffer");
+    DRESSI_REQUIRE(n_items <= kMaxBatchItems, "batch of %u items exceeds %u", n_items,
+                   kMaxBatchItems);
+    if (n_rows == 0 || n_items == 0) {
+        return DRESSI_OK;
+    }
+    if (n_samples == 0) {
+        hipLaunchKernelGGL(k_antialias_bwd_vtx_exact_op, dim3(n_rows, n_items),
+                           dim3(kAaExactThreads), 0, ctx->stream, gy, img, n_comp, rast + 3, 4u,
+                           (const float4*)pos, n_verts, pos_per_item, faces, n_faces, vtx_faces,
+                           n_rows, max_deg, width, height, boost, (float4*)out);
+        DRESSI_CHECK_LAUNCH();
+        return DRESSI_OK;
+    }
+    if (n_faces) {
+        hipLaunchKernelGGL(k_surface_aa_bwd_faces, dim3(n_faces, n_items), dim3(64), 0,
+                           ctx->stream, gy, img, n_comp, rast + 3, 4u, (const float4*)pos, n_verts,
+                           pos_per_item, faces, n_faces, seed, n_samples, width, height, g_corner);
+        DRESSI_CHECK_LAUNCH();
+    }
+    hipLaunchKernelGGL(k_surface_aa_bwd_vtx, dim3(div_up(n_rows, 256), n_items), dim3(256), 0,
+                       ctx->stream, g_corner, faces, n_faces, vtx_faces, n_rows, max_deg, boost,
+                       (float4*)out);
+    DRESSI_CHECK_LAUNCH();
+    return DRESSI_OK;
 }
 
 }  // extern "C"

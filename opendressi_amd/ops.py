@@ -462,6 +462,53 @@ def surface_interpolate_bwd(ctx: Context, gy: torch.Tensor, rast: torch.Tensor,
     return out
 
 
+def surface_antialias(ctx: Context, img: torch.Tensor, rast: torch.Tensor, pos: torch.Tensor,
+                      faces: torch.Tensor) -> torch.Tensor:
+    """dressi_surface_antialias: img (N, H, W, C), rast (N, H, W, 4), pos
+    (V, 4) shared or (N, V, 4) -> (N, H, W, C)."""
+    _prep(ctx)
+    n, h, w, nc = img.shape
+    nv, per_item = _batch_clip(pos, n)
+    out = torch.empty_like(img)
+    check(lib.dressi_surface_antialias(ctx.handle, _ptr(img, "img"), nc, _ptr(rast, "rast"),
+                                       _ptr(pos, "pos"), nv, per_item, _ptr(faces, "faces"),
+                                       faces.shape[0], w, h, n, _ptr(out, "out")))
+    return out
+
+
+def surface_antialias_bwd_img(ctx: Context, gy: torch.Tensor, rast: torch.Tensor,
+                              pos: torch.Tensor, faces: torch.Tensor) -> torch.Tensor:
+    """dressi_surface_antialias_bwd_img: gy (N, H, W, C) -> like gy."""
+    _prep(ctx)
+    n, h, w, nc = gy.shape
+    nv, per_item = _batch_clip(pos, n)
+    out = torch.empty_like(gy)
+    check(lib.dressi_surface_antialias_bwd_img(
+        ctx.handle, _ptr(gy, "gy"), nc, _ptr(rast, "rast"), _ptr(pos, "pos"), nv, per_item,
+        _ptr(faces, "faces"), faces.shape[0], w, h, n, _ptr(out, "out")))
+    return out
+
+
+def surface_antialias_bwd_pos(ctx: Context, gy: torch.Tensor, img: torch.Tensor,
+                              rast: torch.Tensor, pos: torch.Tensor, faces: torch.Tensor,
+                              vtx_faces: torch.Tensor, seed: int, n_samples: int,
+                              boost: float) -> torch.Tensor:
+    """dressi_surface_antialias_bwd_pos: gy, img (N, H, W, C) -> (N, V, 4)."""
+    _prep(ctx)
+    n, h, w, nc = gy.shape
+    nv, per_item = _batch_clip(pos, n)
+    deg, rows = vtx_faces.shape
+    nf = faces.shape[0]
+    scratch = (torch.empty((n, nf, 9), dtype=torch.float32, device=gy.device)
+               if n_samples > 0 else None)
+    out = torch.empty((n, rows, 4), dtype=torch.float32, device=gy.device)
+    check(lib.dressi_surface_antialias_bwd_pos(
+        ctx.handle, _ptr(gy, "gy"), _ptr(img, "img"), nc, _ptr(rast, "rast"), _ptr(pos, "pos"),
+        nv, per_item, _ptr(faces, "faces"), nf, _ptr(vtx_faces, "vtx_faces"), rows, deg, seed,
+        n_samples, boost, w, h, n, _ptr(scratch, "scratch"), _ptr(out, "out")))
+    return out
+
+
 # ---- split-sum IBL ops (maps are (H, W, C) equirect images) ----------------
 
 def _map_nc(m: torch.Tensor) -> int:

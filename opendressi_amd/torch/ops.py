@@ -207,9 +207,10 @@ def texture(tex, uv, uv_da=None, mip_level_bias=None, mip=None, filter_mode="aut
 # ------------------------------- antialias ---------------------------------
 
 
-def _batch_clip(clip_vk: torch.Tensor) -> torch.Tensor:
-    """Per-item clips (N, V, 4), or the one (V, 4) every item shares."""
-    return clip_vk.contiguous() if clip_vk.shape[0] > 1 else clip_vk[0].contiguous()
+def _batch_pos(pos: torch.Tensor, device) -> torch.Tensor:
+    """Per-item clip positions (N, V, 4), or the one (V, 4) every item shares."""
+    pos_b = vertex_batch(to_dev(pos, device, "pos"))
+    return pos_b if pos_b.shape[0] > 1 else pos_b[0]
 
 
 class _AntiAliasFn(torch.autograd.Function):
@@ -219,11 +220,12 @@ class _AntiAliasFn(torch.autograd.Function):
         col_d = image_batch(to_dev(color, dev, "color"), "color")
         rast_d = to_dev(rast, dev, "rast")
         channels(col_d.shape[3], "color")
-        clip_vk = clip_gl_to_vk(vertex_batch(to_dev(pos, dev, "pos")))
+        if col_d.shape[1:3] != rast_d.shape[1:3] or col_d.shape[0] > rast_d.shape[0]:
+            raise ValueError(f"color {tuple(color.shape)} does not match rast {tuple(rast.shape)}")
+        pos_d = _batch_pos(pos, dev)
         with vctx.lock:
             # the whole batch in one launch
-            out = K.antialias_batch(vctx._ctx, col_d.contiguous(), rast_d[..., 3].contiguous(),
-                                    _batch_clip(clip_vk), md.faces_f)
+            out = K.surface_antialias(vctx._ctx, col_d, rast_d, pos_d, md.faces_f)
         fctx.dressi = (vctx, md, n_samples, boost)
         fctx.save_for_backward(color, rast, pos)
         return out.to(color.device)
@@ -236,7 +238,7 @@ class _AntiAliasFn(torch.autograd.Function):
         dev = vctx.device
         col_d = image_batch(to_dev(color, dev, "color"), "color")
         rast_d = to_dev(rast, dev, "rast")
-        clip_vk = clip_gl_to_vk(vertex_batch(to_dev(pos, dev, "pos")))
+        pos_d = _batch_pos(pos, dev)
         g = image_batch(to_dev(grad_out, dev, "grad_out"), "grad_out")
         n, h, w, c = col_d.shape
         key = ("antialias", h, w, md.n_faces, md.n_verts, c, n, n_samples)
@@ -245,26 +247,15 @@ class _AntiAliasFn(torch.autograd.Function):
             # each backward pass advances the stochastic sampler's jitter;
             # items get distinct seeds so their sample patterns decorrelate
             eng.iter_seed += 1
-            tid = rast_d[..., 3].contiguous()
-            clip = _batch_clip(clip_vk)
-            gc = g.contiguous()
             if need_color:
-                g_col = K.antialias_bwd_img_batch(vctx._ctx, gc, tid, clip, md.faces_f)
+                g_col = K.surface_antialias_bwd_img(vctx._ctx, g, rast_d, pos_d, md.faces_f)
             if need_pos:
-                seeds = torch.tensor([float(eng.iter_seed * n + i) for i in range(n)],
-                                     dtype=torch.float32, device=dev)
-                if n_samples > 0:
-                    wide = K.antialias_bwd_vtx_batch(vctx._ctx, gc, col_d.contiguous(), tid, clip,
-                                                     md.faces_f, md.vft, seeds, n_samples, True)
-                    g_clip = K.col_sum_batch(vctx._ctx, wide)
-                else:
-                    g_clip = K.antialias_bwd_vtx_batch(vctx._ctx, gc, col_d.contiguous(), tid,
-                                                       clip, md.faces_f, md.vft, seeds, 0, False)
+                gp = K.surface_antialias_bwd_pos(vctx._ctx, g, col_d, rast_d, pos_d, md.faces_f,
+                                                 md.vft, eng.iter_seed * n, n_samples, boost)
         out_gc = out_gp = None
         if need_color:
             out_gc = (g_col[0] if color.dim() == 3 else g_col).to(color.device)
         if need_pos:
-            gp = clip_grad_vk_to_gl(g_clip) * boost
             out_gp = (gp.sum(dim=0) if pos.dim() == 2 else gp).to(pos.device)
         return out_gc, None, out_gp, None, None, None, None, None
 
@@ -279,7 +270,7 @@ def antialias(color, rast, pos, tri, topology_hash=None, pos_gradient_boost=1.0,
     rinfo = origin(rast, RasterOrigin, "rasterize")
     vctx = rinfo.ctx
     md = vctx.mesh(tri)
-    return _AntiAliasFn.apply(color, rast, pos, vctx, md, rinfo, int(n_samples),
+    return _AntiAliasFn.apply(color, rast, pos, vctx, md, rinfo, max(int(n_samples), 0),
                               float(pos_gradient_boost))
 
 

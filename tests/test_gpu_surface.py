@@ -1,0 +1,135 @@
+"""The torch surface's fused ops (dressi_surface_*) against the per-op entry points they stand
+for, composed as the reference's surface composes them: the same bits at the edges of the fused
+kernels' steps (boxes of several steps, screens that end inside a workgroup, sample counts that
+are no multiple of eight, batches whose contributions take several summation levels)."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    import opendressi_amd as od
+    c = od.Context(0)
+    yield c
+    c.close()
+
+
+def _same(a, b, what):
+    torch.cuda.synchronize()
+    assert a.shape == b.shape, (what, a.shape, b.shape)
+    assert torch.equal(torch.nan_to_num(a), torch.nan_to_num(b)), \
+        f"{what}: {int((a != b).sum())} values differ, max {float((a - b).abs().max()):.3g}"
+
+
+def _scene(level, n, seed, spread=0.1):
+    """n random orbit views of an icosphere: clip positions (n, V, 4) with z in [-w, w], faces
+    as int32 and float ids, the adjacency."""
+    import opendressi_amd as od
+    pos, faces = od.icosphere(level)
+    rng = np.random.default_rng(seed)
+    pos = pos * (1.0 + spread * rng.standard_normal((len(pos), 1)))
+    mvp = od.orbit_cameras(1, n, seed)[0].reshape(n, 4, 4).astype(np.float64)
+    clip = np.concatenate([pos, np.ones((len(pos), 1))], 1)[None] @ mvp
+    clip[..., 2] = 2.0 * clip[..., 2] - clip[..., 3]
+    vf = od.vertex_faces_tex(faces, len(pos))
+    dev = lambda a, t: torch.from_numpy(np.ascontiguousarray(a, t)).cuda()
+    return (dev(clip, np.float32), dev(faces, np.int32), dev(faces, np.float32),
+            dev(vf, np.float32))
+
+
+def _to_vk(clip):
+    out = clip.clone()
+    out[..., 2] = 0.5 * (clip[..., 2] + clip[..., 3])
+    return out
+
+
+SCENES = [(0, 1, 40, 64), (2, 3, 61, 97), (4, 7, 33, 18), (3, 2, 1, 200), (1, 5, 130, 131)]
+
+
+@pytest.mark.parametrize("level,n,h,w", SCENES)
+def test_surface_rasterize(ctx, level, n, h, w):
+    """Against Rasterize of the unwelded mesh with the corner constants and (z, w)."""
+    from opendressi_amd import ops as K
+    print(f"[surface rasterize] level {level} {n}x{h}x{w}", flush=True)
+    clip, fi, ff, _ = _scene(level, n, level + n)
+    nf = len(fi)
+    rast, vk = K.surface_rasterize(ctx, clip, fi, w, h)
+    _same(vk, _to_vk(clip), "clip")
+    idx = fi.reshape(-1).long()
+    corner = torch.tensor([[1.0, 0.0], [0.0, 1.0], [0.0, 0.0]]).repeat(nf, 1).cuda()
+    attr = torch.cat([corner.expand(n, -1, -1), clip[:, idx][:, :, 2:4]], 2).contiguous()
+    seq = torch.arange(nf * 3, dtype=torch.float32).reshape(-1, 3).cuda()
+    g, tid = K.rasterize_batch(ctx, _to_vk(clip)[:, idx].contiguous(), attr, seq, w, h,
+                               with_face_id=True)
+    zw = g[..., 2] / (g[..., 3] + (1.0 - (tid > 0.5).float()))
+    _same(rast, torch.stack([g[..., 0], g[..., 1], zw, tid], -1), "rast")
+    assert (tid > 0).any()
+    ctx.synchronize()
+
+
+@pytest.mark.parametrize("level,n,h,w", SCENES)
+@pytest.mark.parametrize("nc,shared", [(1, True), (2, False), (3, True), (4, False), (4, True)])
+def test_surface_interpolate(ctx, level, n, h, w, nc, shared):
+    from opendressi_amd import ops as K
+    from opendressi_amd.torch.convert import sum_contribs
+    print(f"[surface interpolate] level {level} {n}x{h}x{w}x{nc} shared {shared}", flush=True)
+    clip, fi, ff, vf = _scene(level, n, level + n)
+    rast, vk = K.surface_rasterize(ctx, clip, fi, w, h)
+    gen = torch.Generator(device="cuda").manual_seed(nc)
+    nv = clip.shape[1]
+    attr = torch.randn((nv, nc) if shared else (n, nv, nc), device="cuda", generator=gen)
+    u, v, tid = rast[..., 0:1], rast[..., 1:2], rast[..., 3].contiguous()
+
+    def per_face(a, k):
+        return (K.lookup_faces(ctx, a, ff, k) if a.dim() == 2
+                else K.lookup_faces_batch(ctx, a, ff, k, n))
+
+    pix = [K.face_fetch_batch(ctx, per_face(attr, k), tid) for k in range(3)]
+    _same(K.surface_interpolate(ctx, attr, rast, ff),
+          u * pix[0] + v * pix[1] + ((1.0 - u) - v) * pix[2], "forward")
+    g = torch.randn((n, h, w, nc), device="cuda", generator=gen)
+    gp = [g * u, g * v, g * ((1.0 - u) - v)]
+    prj = [per_face(vk, k) for k in range(3)]
+    seeds = torch.zeros(n, device="cuda")
+    parts = [K.lookup_faces_bwd_batch(ctx, K.face_fetch_bwd_batch(
+        ctx, gp[k].contiguous(), tid, prj[0], prj[1], prj[2], seeds, 1.0, 0), ff, vf, k)
+        for k in (2, 1, 0)]
+    per_item = [[p[i] for p in parts] for i in range(n)]
+    ref = (sum_contribs([p for parts_i in reversed(per_item) for p in parts_i]) if shared
+           else torch.stack([sum_contribs(p) for p in per_item], 0))
+    _same(K.surface_interpolate_bwd(ctx, g, rast, vk, ff, vf, shared), ref, "backward")
+    ctx.synchronize()
+
+
+@pytest.mark.parametrize("level,n,h,w", SCENES)
+@pytest.mark.parametrize("nc,samples,shared", [(1, 8, False), (3, 0, False), (2, 5, True),
+                                               (4, 17, False)])
+def test_surface_antialias(ctx, level, n, h, w, nc, samples, shared):
+    """Forward and colour gradient against the per-op batch, the position gradient against the
+    wide partials, ColSum, the z remap's transpose and the boost."""
+    from opendressi_amd import ops as K
+    print(f"[surface antialias] level {level} {n}x{h}x{w}x{nc} n={samples} {shared}", flush=True)
+    clip, fi, ff, vf = _scene(level, 1 if shared else n, level + n)
+    rast, vk = K.surface_rasterize(ctx, clip.expand(n, -1, -1).contiguous(), fi, w, h)
+    pos, vk = (clip[0], vk[0].contiguous()) if shared else (clip, vk)
+    tid = rast[..., 3].contiguous()
+    gen = torch.Generator(device="cuda").manual_seed(nc)
+    img = torch.rand((n, h, w, nc), device="cuda", generator=gen)
+    g = torch.randn((n, h, w, nc), device="cuda", generator=gen)
+    _same(K.surface_antialias(ctx, img, rast, pos, ff), K.antialias_batch(ctx, img, tid, vk, ff),
+          "forward")
+    _same(K.surface_antialias_bwd_img(ctx, g, rast, pos, ff),
+          K.antialias_bwd_img_batch(ctx, g, tid, vk, ff), "colour gradient")
+    got = K.surface_antialias_bwd_pos(ctx, g, img, rast, pos, ff, vf, 3 * n, samples, 1.5)
+    seeds = torch.tensor([float(3 * n + i) for i in range(n)], device="cuda")
+    ref = K.antialias_bwd_vtx_batch(ctx, g, img, tid, vk, ff, vf, seeds, samples, samples > 0)
+    if samples:
+        ref = K.col_sum_batch(ctx, ref)
+    ref[..., 3] += 0.5 * ref[..., 2]
+    ref[..., 2] *= 0.5
+    assert float(ref.abs().max()) > 0 or h == 1
+    _same(got, ref * 1.5, "position gradient")
+    ctx.synchronize()
