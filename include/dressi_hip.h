@@ -504,6 +504,22 @@ int dressi_surface_antialias_bwd_pos(dressi_ctx* ctx, const float* gy, const flo
                                      float boost, uint32_t width, uint32_t height,
                                      uint32_t n_items, float* g_corner, float* out);
 
+/* rasterize_soft: pos {N,V} VEC4, z in [-w, w] -> out {N,K,H,W} VEC4 (signed
+ * dist, face id, hard z, coverage) of K = peels layers; threshold is scratch
+ * of N * H * W floats (K > 1), neg_inv_radius = -1 / radius_px. Its backward:
+ * gy, rs {N,K,H,W} VEC4 -> d/d pos {N,n_rows} VEC4 for an adjacency of the
+ * same faces; g_corner is scratch of N * K * F * 9 floats. */
+int dressi_surface_rasterize_soft(dressi_ctx* ctx, const float* pos, uint32_t n_verts,
+                                  uint32_t n_items, const float* faces, uint32_t n_faces,
+                                  uint32_t width, uint32_t height, float radius_px,
+                                  float neg_inv_radius, uint32_t peels, float* threshold,
+                                  float* out);
+int dressi_surface_soft_bwd(dressi_ctx* ctx, const float* gy, const float* rs, uint32_t peels,
+                            const float* pos, uint32_t n_verts, uint32_t n_items,
+                            const float* faces, uint32_t n_faces, const float* vtx_faces,
+                            uint32_t n_rows, uint32_t max_deg, float radius_px, uint32_t width,
+                            uint32_t height, float* g_corner, float* out);
+
 /* ---- texture path (C3) ---- */
 /* F::TextureBilinear forward (src/core/f_ops.cpp:2736-2780, BilerpClamp
  * src/core/ibl_math.h:91-115): tex {tw,th} x n_comp (1..4) sampled at

@@ -112,6 +112,9 @@ _SIGS = {
                                               _P]),
     "dressi_surface_antialias_bwd_pos": (_I, [_P, _P, _P, _U, _P, _P, _U, _I, _P, _U, _P, _U, _U,
                                               C.c_uint64, _U, _F, _U, _U, _U, _P, _P]),
+    "dressi_surface_rasterize_soft": (_I, [_P, _P, _U, _U, _P, _U, _U, _U, _F, _F, _U, _P, _P]),
+    "dressi_surface_soft_bwd": (_I, [_P, _P, _P, _U, _P, _U, _U, _P, _U, _P, _U, _U, _F, _U, _U,
+                                     _P, _P]),
     "dressi_equirect_sample": (_I, [_P, _P, _U, _U, _U, _P, _U, _U, _P]),
     "dressi_equirect_sample_bwd": (_I, [_P, _P, _U, _P, _U, _U, _U, _U, _P]),
     "dressi_avg_pool2x2": (_I, [_P, _P, _U, _U, _U, _P]),

@@ -28,7 +28,7 @@ SOURCES = ["runtime.hip", "raster.hip", "hsr.hip", "aa.hip", "tex.hip", "ds.hip"
 HOST_SOURCES = ["assets.cpp", "jpeg.cpp", "geometry.cpp", "pbr_graph.cpp"]
 HEADERS = ["internal.h", "dressi_math.h", "raster_core.h", "soft_clip.h", "hsr_chain.h",
            "aa_core.h", "plan.h", "ibl_core.h", "graph_ir.h", "route.h", "libm_f32.h",
-           "libm_pow5_table.h", "image_codecs.h"]
+           "libm_pow5_table.h", "image_codecs.h", "surface_core.h"]
 ARCH = os.environ.get("DRESSI_OFFLOAD_ARCH", "gfx950")
 
 FLAGS = [

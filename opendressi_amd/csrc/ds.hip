@@ -6,6 +6,7 @@
 
 #include "internal.h"
 #include "soft_clip.h"
+#include "surface_core.h"
 
 namespace dressi {
 namespace {
@@ -205,37 +206,19 @@ constexpr uint32_t kDistPx = 8;
 constexpr uint32_t kDistHits = 1024;
 static_assert(kDistHits >= 2 * 64 * kDistPx, "a step's hits fit beside those kept");
 
-// Orders the (one-wave) workgroup's LDS accesses.
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
+struct DistLds {
+    uint32_t hit_px[kDistHits];
+    float term[64][9];  // per hit: corner k's x, y, w contributions
+};
 
-__global__ __launch_bounds__(64) void k_gather_dist_grad_faces(
-        const float4* gy, const float4* rs, const float4* clip, uint32_t n_verts,
-        const float* faces, const float* vf, uint32_t max_deg, float radius, uint32_t w,
-        uint32_t h, float4* out) {
-    __shared__ uint32_t hit_px[kDistHits];
-    // per hit: corner k's x, y, w contributions
-    __shared__ float term[64][9];
-    const uint32_t f = blockIdx.x, lane = threadIdx.x;
-    const float W = (float)w, H = (float)h;
-    // (bad indices are the row kernel's to report)
-    for (int k = 0; k < 3; k++) {
-        if ((uint32_t)(int64_t)(faces[(size_t)f * 3 + k] + 0.5f) >= n_verts) {
-            return;
-        }
-    }
-    FaceCorners fc;
-    int bx0, by0, bx1, by1;
-    if (!load_face(faces, clip, n_verts, f, W, H, &fc, nullptr) ||
-        !soft_bbox(fc, w, h, radius, &bx0, &by0, &bx1, &by1)) {
-        return;
-    }
-    const uint32_t bw = (uint32_t)(bx1 - bx0 + 1);
-    const uint32_t n_px = bw * (uint32_t)(by1 - by0 + 1);
-    // lane 3 r + c < 9 sums component c of corner r's row
+// The sum of one face's pixels' contributions by one wave, in raster order:
+// lane 3 r + c < 9 gets component c (x, y, w) of corner r's row. rs and gy are
+// the item's images.
+__device__ __forceinline__ float dist_face_sum(const FaceCorners& fc, uint32_t f, int bx0, int by0,
+                                               uint32_t bw, uint32_t n_px, const float4* rs,
+                                               const float4* gy, uint32_t w, float W, float H,
+                                               DistLds& lds) {
+    const uint32_t lane = threadIdx.x;
     const uint32_t r = lane < 9 ? lane / 3 : 0, comp = lane < 9 ? lane % 3 : 0;
     const uint32_t my = r == 0 ? fc.idx[0] : r == 1 ? fc.idx[1] : fc.idx[2];
     const bool twice = fc.idx[0] == fc.idx[1] || fc.idx[1] == fc.idx[2] || fc.idx[2] == fc.idx[0];
@@ -258,7 +241,7 @@ __global__ __launch_bounds__(64) void k_gather_dist_grad_faces(
             const bool hit = !(yw[s].y < 0.5f) && (uint32_t)(int64_t)(yw[s].x + 0.5f) == f;
             const uint64_t m = __ballot(hit);
             if (hit) {
-                hit_px[n_hits + __popcll(m & ((1ull << lane) - 1ull))] = o[s];
+                lds.hit_px[n_hits + __popcll(m & ((1ull << lane) - 1ull))] = o[s];
             }
             n_hits += (uint32_t)__popcll(m);
         }
@@ -270,7 +253,7 @@ __global__ __launch_bounds__(64) void k_gather_dist_grad_faces(
         for (uint32_t h0 = 0; h0 < n_hits; h0 += 64) {
             const uint32_t n = min(64u, n_hits - h0);
             if (lane < n) {
-                const uint32_t at = hit_px[h0 + lane];
+                const uint32_t at = lds.hit_px[h0 + lane];
                 const uint32_t y = at / w, x = at - y * w;
                 const float g = gy[at].x;
                 float4 t[3] = {};
@@ -284,9 +267,9 @@ __global__ __launch_bounds__(64) void k_gather_dist_grad_faces(
                 }
 #pragma unroll
                 for (int k = 0; k < 3; k++) {
-                    term[lane][k * 3 + 0] = t[k].x;
-                    term[lane][k * 3 + 1] = t[k].y;
-                    term[lane][k * 3 + 2] = t[k].w;
+                    lds.term[lane][k * 3 + 0] = t[k].x;
+                    lds.term[lane][k * 3 + 1] = t[k].y;
+                    lds.term[lane][k * 3 + 2] = t[k].w;
                 }
             }
             wave_lds_sync();
@@ -295,14 +278,14 @@ __global__ __launch_bounds__(64) void k_gather_dist_grad_faces(
             if (lane < 9 && !twice) {
 #pragma unroll 8
                 for (uint32_t q = 0; q < n; q++) {
-                    acc += term[q][lane];
+                    acc += lds.term[q][lane];
                 }
             } else if (lane < 9) {
                 for (uint32_t q = 0; q < n; q++) {
 #pragma unroll
                     for (int k = 0; k < 3; k++) {
                         if (fc.idx[k] == my) {
-                            acc += term[q][k * 3 + comp];
+                            acc += lds.term[q][k * 3 + comp];
                         }
                     }
                 }
@@ -311,6 +294,34 @@ __global__ __launch_bounds__(64) void k_gather_dist_grad_faces(
         }
         n_hits = 0;
     }
+    return acc;
+}
+
+__global__ __launch_bounds__(64) void k_gather_dist_grad_faces(
+        const float4* gy, const float4* rs, const float4* clip, uint32_t n_verts,
+        const float* faces, const float* vf, uint32_t max_deg, float radius, uint32_t w,
+        uint32_t h, float4* out) {
+    __shared__ DistLds lds;
+    const uint32_t f = blockIdx.x, lane = threadIdx.x;
+    const float W = (float)w, H = (float)h;
+    // (bad indices are the row kernel's to report)
+    for (int k = 0; k < 3; k++) {
+        if ((uint32_t)(int64_t)(faces[(size_t)f * 3 + k] + 0.5f) >= n_verts) {
+            return;
+        }
+    }
+    FaceCorners fc;
+    int bx0, by0, bx1, by1;
+    if (!load_face(faces, clip, n_verts, f, W, H, &fc, nullptr) ||
+        !soft_bbox(fc, w, h, radius, &bx0, &by0, &bx1, &by1)) {
+        return;
+    }
+    const uint32_t bw = (uint32_t)(bx1 - bx0 + 1);
+    const uint32_t n_px = bw * (uint32_t)(by1 - by0 + 1);
+    // lane 3 r + c < 9 sums component c of corner r's row
+    const uint32_t r = lane < 9 ? lane / 3 : 0, comp = lane < 9 ? lane % 3 : 0;
+    const uint32_t my = r == 0 ? fc.idx[0] : r == 1 ? fc.idx[1] : fc.idx[2];
+    const float acc = dist_face_sum(fc, f, bx0, by0, bw, n_px, rs, gy, w, W, H, lds);
     // the corner's row: the first of its vertex's that holds f
     uint32_t row = max_deg;
 #pragma unroll
@@ -330,6 +341,78 @@ __global__ __launch_bounds__(64) void k_gather_dist_grad_faces(
         float* dst = (float*)&out[(size_t)row * n_verts + my];
         dst[comp == 2 ? 3 : comp] = acc;
     }
+}
+
+// The torch surface's form: every item and peel, corner sums {N,K,F,3}
+// (x, y, w) for an adjacency of the same faces. A face's setup serves its
+// peels.
+__global__ __launch_bounds__(64) void k_surface_soft_bwd_faces(
+        const float4* gy, const float4* rs, uint32_t peels, const float4* pos, uint32_t n_verts,
+        const float* faces, uint32_t n_faces, float radius, uint32_t w, uint32_t h,
+        float* g_corner) {
+    __shared__ DistLds lds;
+    const uint32_t f = blockIdx.x, lane = threadIdx.x;
+    const float W = (float)w, H = (float)h;
+    const size_t npx = (size_t)w * h;
+    pos += (size_t)blockIdx.y * n_verts;
+    bool ok = true;
+    for (int k = 0; k < 3; k++) {
+        ok = ok && fid_u(faces[(size_t)f * 3 + k]) < n_verts;
+    }
+    FaceCorners fc;
+    int bx0 = 1, by0 = 1, bx1 = 0, by1 = 0;
+    ok = ok && load_face(faces, pos, n_verts, f, W, H, &fc, nullptr) &&
+         soft_bbox(fc, w, h, radius, &bx0, &by0, &bx1, &by1);
+    const uint32_t bw = (uint32_t)(bx1 - bx0 + 1);
+    const uint32_t n_px = ok ? bw * (uint32_t)(by1 - by0 + 1) : 0u;
+    for (uint32_t k = 0; k < peels; k++) {
+        const size_t layer = (size_t)blockIdx.y * peels + k;
+        float acc = 0.f;
+        if (n_px) {
+            acc = dist_face_sum(fc, f, bx0, by0, bw, n_px, rs + layer * npx, gy + layer * npx, w,
+                                W, H, lds);
+        }
+        if (lane < 9) {
+            g_corner[(layer * n_faces + f) * 9 + lane] = acc;
+        }
+    }
+}
+
+// ColSum of the vertex's rows per peel, the peels' contributions (the last
+// peel first), the z remap's transpose (the gradient's z is 0). One thread
+// per vertex and component.
+__global__ __launch_bounds__(256) void k_surface_soft_bwd_vtx(
+        const float* g_corner, uint32_t peels, const float* faces, uint32_t n_faces,
+        const float* vf, uint32_t n_verts, uint32_t max_deg, float* out) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n_verts * 4) {
+        return;
+    }
+    const uint32_t v = i >> 2, comp = i & 3u;
+    float* dst = out + (size_t)blockIdx.y * n_verts * 4 + i;
+    if (comp == 2) {
+        *dst = 0.f;
+        return;
+    }
+    const uint32_t c = comp == 3 ? 2u : comp;
+    ContribSum total;
+    for (uint32_t k = peels; k-- > 0;) {
+        const float* g = g_corner + ((size_t)blockIdx.y * peels + k) * n_faces * 9;
+        float acc = 0.f;
+        for (uint32_t d = 0; d < max_deg; d++) {
+            const float fv = vf[(size_t)d * n_verts + v];
+            const uint32_t f = fv < -0.5f ? n_faces : fid_u(fv);
+            if (f >= n_faces) {
+                continue;
+            }
+            uint32_t q = 2;
+            q = fid_u(faces[(size_t)f * 3 + 1]) == v ? 1u : q;
+            q = fid_u(faces[(size_t)f * 3 + 0]) == v ? 0u : q;
+            acc += g[(size_t)f * 9 + q * 3 + c];
+        }
+        total.push(acc);
+    }
+    *dst = total.sum();
 }
 
 // {V,1} layout, one thread per vertex: the union of its incident faces'
@@ -429,6 +512,36 @@ extern "C" int dressi_gather_dist_grad(dressi_ctx* ctx, const float* gy, const f
                            n_verts, faces, n_faces, vtx_faces, max_deg, radius_px, width, height,
                            ctx->d_err, (float4*)out);
     }
+    DRESSI_CHECK_LAUNCH();
+    return DRESSI_OK;
+}
+
+extern "C" int dressi_surface_soft_bwd(dressi_ctx* ctx, const float* gy, const float* rs,
+                                       uint32_t peels, const float* pos, uint32_t n_verts,
+                                       uint32_t n_items, const float* faces, uint32_t n_faces,
+                                       const float* vtx_faces, uint32_t n_rows, uint32_t max_deg,
+                                       float radius_px, uint32_t width, uint32_t height,
+                                       float* g_corner, float* out) {
+    DRESSI_REQUIRE(ctx && gy && rs && pos && (faces || n_faces == 0) && vtx_faces && out &&
+                           (g_corner || n_faces == 0),
+                   "rasterize_soft backward: NULL buffer");
+    DRESSI_REQUIRE(radius_px > 0.f, "radius_px must be > 0");
+    DRESSI_REQUIRE(peels >= 1 && n_items <= kMaxBatchItems, "batch of %u items exceeds %u",
+                   n_items, kMaxBatchItems);
+    DRESSI_REQUIRE((uint64_t)width * height < (1ull << 31) && n_rows < (1u << 30),
+                   "rasterize_soft backward: too large");
+    if (!n_items || !n_rows) return DRESSI_OK;
+    DRESSI_TRY_HIP(hipSetDevice(ctx->device));
+    if (n_faces) {
+        hipLaunchKernelGGL(k_surface_soft_bwd_faces, dim3(n_faces, n_items), dim3(64), 0,
+                           ctx->stream, (const float4*)gy, (const float4*)rs, peels,
+                           (const float4*)pos, n_verts, faces, n_faces, radius_px, width, height,
+                           g_corner);
+        DRESSI_CHECK_LAUNCH();
+    }
+    hipLaunchKernelGGL(k_surface_soft_bwd_vtx, dim3(div_up(n_rows * 4, 256), n_items), dim3(256),
+                       0, ctx->stream, (const float*)g_corner, peels, faces, n_faces, vtx_faces,
+                       n_rows, max_deg, out);
     DRESSI_CHECK_LAUNCH();
     return DRESSI_OK;
 }

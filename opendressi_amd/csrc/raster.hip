@@ -458,6 +458,93 @@ __global__ __launch_bounds__(64) void k_raster_soft_op(RasterGeom g, const SoftR
     out[(size_t)py * g.width + px] = o;
 }
 
+// The torch surface's soft raster: SoftClip and the soft setup of every item's
+// faces from its clip positions (z in [-w, w], remapped), binned per item.
+__global__ __launch_bounds__(256) void k_surface_soft_setup(RasterGeom g, const float4* pos,
+                                                            uint32_t n_verts, const float* faces,
+                                                            float radius, BinBuffers b,
+                                                            uint32_t* err, SoftRec* recs,
+                                                            CullRec* cull) {
+    __shared__ BinLds blds;
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    const bool live = i < g.n_views * g.n_faces;
+    const uint32_t view = live ? i / g.n_faces : 0;
+    const uint32_t f = live ? i - view * g.n_faces : 0;
+    SoftRec r;
+    r.bx0 = 1;
+    r.bx1 = 0;
+    r.by0 = 1;
+    r.by1 = 0;
+    r.flags = 0;
+    if (live) {
+        float4 hc[3], sc[3];
+        bool ok = true;
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            const uint32_t v = fid_u(faces[(size_t)f * 3 + k]);
+            ok = ok && v < n_verts;
+            hc[k] = ok ? pos[(size_t)view * n_verts + v] : make_float4(0.f, 0.f, 0.f, 0.f);
+            hc[k].z = 0.5f * (hc[k].z + hc[k].w);
+        }
+        if (ok) {
+            soft_clip_face(hc, g.width, g.height, radius, sc);
+            soft_setup(sc, hc, (float)f, g.width, g.height, &r);
+        } else {
+            atomicOr(err, 8u);
+        }
+        recs[i] = r;
+        cull[i] = cull_setup(r);
+    }
+    const bool valid = live && r.bx0 <= r.bx1 && r.by0 <= r.by1;
+    bin_append(b, g, valid, view, f, r.bx0, r.by0, r.bx1, r.by1, soft_bin_tri(r), blds);
+}
+
+// One peel of every item: k_raster_soft_op's resolve and outputs, and, where
+// another peel follows, its depth threshold (this layer's shifted depth
+// rebuilt from its channels, python/dressi/torch/ops.py:608-615).
+// blockIdx.y: the item. neg_inv_radius = -1 / radius.
+__global__ __launch_bounds__(64) void k_surface_raster_soft(
+        RasterGeom g, const SoftRec* recs, const CullRec* cull, BinBuffers b, float radius,
+        float neg_inv_radius, const float* prev, uint32_t layer, uint32_t peels, float4* out,
+        float* threshold) {
+    const BlockPos blk = block_pos(blockIdx.x, g);
+    if (!blk.valid) {
+        return;
+    }
+    const size_t npx = (size_t)g.width * g.height;
+    const uint32_t item = blockIdx.y;
+    recs += (size_t)item * g.n_faces;
+    cull += (size_t)item * g.n_faces;
+    prev = prev ? prev + item * npx : nullptr;
+    const int lane = threadIdx.x & 63;
+    const int px = blk.bx + (lane & 7);
+    const int py = blk.by + (lane >> 3);
+    const BinView bv = bin_view(b, item * g.n_tiles + blk.tile, g.n_faces);
+    __shared__ ResolveLds lds;
+    const PixelBest best =
+            resolve_block(recs, cull, bv, blk.bx, blk.by, radius, prev, g.width, lds);
+    if (px >= (int)g.width || py >= (int)g.height) {
+        return;
+    }
+    float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (best.key != kEmptyKey) {
+        const SoftRec& r = recs[key_face(best.key)];
+        const float p0 = (float)px + 0.5f;
+        const float p1 = (float)py + 0.5f;
+        const float dist = signed_dist(p0, p1, r.hx, r.hy, r.ex, r.ey, r.len2);
+        o = make_float4(dist, r.fid, hard_z_at(r, p0, p1), 1.f);
+    }
+    const size_t at = (size_t)py * g.width + px;
+    out[((size_t)item * peels + layer) * npx + at] = o;
+    if (threshold) {
+        const auto clamp01 = [](float x) { return x < 0.f ? 0.f : x > 1.f ? 1.f : x; };
+        const float ge = o.x >= 0.f ? 1.f : 0.f;
+        const float near = clamp01(o.z) * 0.5f;
+        const float far = clamp01(o.x * neg_inv_radius) * 0.5f + 0.5f;
+        threshold[item * npx + at] = o.w * (ge * near + (1.f - ge) * far);
+    }
+}
+
 __global__ void k_soft_clip(const float4* clip, uint32_t n_verts, const float* faces,
                             uint32_t n_faces, uint32_t w, uint32_t h, float radius,
                             uint32_t* err, float4* out) {
@@ -772,6 +859,66 @@ int dressi_surface_rasterize(dressi_ctx* ctx, const float* pos, uint32_t n_verts
     DRESSI_CHECK_LAUNCH();
     return launch_hard_op(ctx, g, hb, pos, n_verts, nullptr, faces, 1, pos, 4, 2, rast,
                           (size_t)n_verts * 4, nullptr);
+}
+
+// The torch surface's rasterize_soft: pos {N,V} VEC4, z in [-w, w] -> out
+// {N,K,H,W} VEC4. Items go through in groups whose bins fit kSoftGroupBytes.
+int dressi_surface_rasterize_soft(dressi_ctx* ctx, const float* pos, uint32_t n_verts,
+                                  uint32_t n_items, const float* faces, uint32_t n_faces,
+                                  uint32_t width, uint32_t height, float radius_px,
+                                  float neg_inv_radius, uint32_t peels, float* threshold,
+                                  float* out) {
+    constexpr size_t kSoftGroupBytes = (size_t)256 << 20;
+    if (int rc = check_ctx(ctx)) return rc;
+    DRESSI_REQUIRE((pos || n_verts == 0) && (faces || n_faces == 0) && out &&
+                           (threshold || peels == 1),
+                   "rasterize_soft: NULL buffer");
+    DRESSI_REQUIRE(radius_px > 0.f, "RasterizeSoft: radius_px must be > 0");
+    DRESSI_REQUIRE(width > 0 && height > 0, "RasterizeSoft: empty screen");
+    DRESSI_REQUIRE(peels >= 1, "RasterizeSoft: peels must be >= 1");
+    if (n_items == 0) return DRESSI_OK;
+    const size_t npx = (size_t)width * height;
+    const size_t item_bytes = fixed_bin_bytes(make_geom(width, height, 1, n_faces).n_tiles,
+                                              kSoftBinCap);
+    uint32_t group = (uint32_t)std::min<size_t>(
+            std::max<size_t>(kSoftGroupBytes / item_bytes, 1), n_items);
+    group = std::min(group, kMaxBatchItems);
+    while (group > 1 && (uint64_t)group * n_faces >= (1ull << 31)) group /= 2;
+    for (uint32_t i0 = 0; i0 < n_items; i0 += group) {
+        const uint32_t n = std::min(group, n_items - i0);
+        const RasterGeom g = make_geom(width, height, n, n_faces);
+        // (the raster takes an item on the grid's y: tiles of one view)
+        const RasterGeom g1 = make_geom(width, height, 1, n_faces);
+        void *recs = nullptr, *bins = nullptr, *cull = nullptr;
+        const size_t nf = (size_t)(n_faces ? n_faces : 1) * n;
+        if (int rc = ctx_workspace(ctx, 0, sizeof(SoftRec) * nf, &recs)) return rc;
+        if (int rc = ctx_workspace(ctx, 1, fixed_bin_bytes(g.n_tiles * n, kSoftBinCap), &bins))
+            return rc;
+        if (int rc = ctx_workspace(ctx, 3, sizeof(CullRec) * nf, &cull)) return rc;
+        BinBuffers b;
+        fixed_bin_carve(bins, g.n_tiles * n, kSoftBinCap, &b);
+        if (int rc = launch_zero(ctx->stream, b.counts, sizeof(uint32_t) * g.n_tiles * n))
+            return rc;
+        const float* p = pos + (size_t)i0 * n_verts * 4;
+        if (n_faces) {
+            hipLaunchKernelGGL(k_surface_soft_setup, dim3(div_up(n * n_faces, 256)), dim3(256), 0,
+                               ctx->stream, g, (const float4*)p, n_verts, faces, radius_px, b,
+                               ctx->d_err, (SoftRec*)recs, (CullRec*)cull);
+            DRESSI_CHECK_LAUNCH();
+        }
+        for (uint32_t k = 0; k < peels; k++) {
+            // layer k reads layer k - 1's threshold and writes its own over it
+            // (each pixel its own)
+            float* thr = threshold ? threshold + i0 * npx : nullptr;
+            hipLaunchKernelGGL(k_surface_raster_soft, dim3(block_grid(g1), n), dim3(64), 0,
+                               ctx->stream, g1, (const SoftRec*)recs, (const CullRec*)cull, b,
+                               radius_px, neg_inv_radius, k ? thr : (const float*)nullptr, k, peels,
+                               (float4*)out + (size_t)i0 * peels * npx,
+                               k + 1 < peels ? thr : nullptr);
+            DRESSI_CHECK_LAUNCH();
+        }
+    }
+    return DRESSI_OK;
 }
 
 }  // extern "C"

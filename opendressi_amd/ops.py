@@ -509,6 +509,39 @@ def surface_antialias_bwd_pos(ctx: Context, gy: torch.Tensor, img: torch.Tensor,
     return out
 
 
+def surface_rasterize_soft(ctx: Context, pos: torch.Tensor, faces: torch.Tensor, width: int,
+                           height: int, radius_px: float, peels: int) -> torch.Tensor:
+    """dressi_surface_rasterize_soft: pos (N, V, 4), z in [-w, w] ->
+    (N, K, H, W, 4)."""
+    _prep(ctx)
+    n, nv = pos.shape[0], pos.shape[1]
+    out = torch.empty((n, peels, height, width, 4), dtype=torch.float32, device=pos.device)
+    thr = (torch.empty((n, height, width), dtype=torch.float32, device=pos.device)
+           if peels > 1 else None)
+    check(lib.dressi_surface_rasterize_soft(
+        ctx.handle, _ptr(pos, "pos"), nv, n, _ptr(faces, "faces"), faces.shape[0], width, height,
+        radius_px, -1.0 / radius_px if radius_px else 0.0, peels, _ptr(thr, "threshold"),
+        _ptr(out, "out")))
+    return out
+
+
+def surface_soft_bwd(ctx: Context, gy: torch.Tensor, rs: torch.Tensor, pos: torch.Tensor,
+                     faces: torch.Tensor, vtx_faces: torch.Tensor,
+                     radius_px: float) -> torch.Tensor:
+    """dressi_surface_soft_bwd: gy, rs (N, K, H, W, 4) -> (N, V, 4)."""
+    _prep(ctx)
+    n, peels, h, w = rs.shape[:4]
+    deg, rows = vtx_faces.shape
+    nf = faces.shape[0]
+    scratch = torch.empty((n, peels, nf, 9), dtype=torch.float32, device=rs.device)
+    out = torch.empty((n, rows, 4), dtype=torch.float32, device=rs.device)
+    check(lib.dressi_surface_soft_bwd(
+        ctx.handle, _ptr(gy, "gy"), _ptr(rs, "rs"), peels, _ptr(pos, "pos"), pos.shape[1], n,
+        _ptr(faces, "faces"), nf, _ptr(vtx_faces, "vtx_faces"), rows, deg, radius_px, w, h,
+        _ptr(scratch, "scratch"), _ptr(out, "out")))
+    return out
+
+
 # ---- split-sum IBL ops (maps are (H, W, C) equirect images) ----------------
 
 def _map_nc(m: torch.Tensor) -> int:

@@ -20,8 +20,6 @@ from .. import ops as K
 from .context import RasterizeHipContext
 from .convert import (
     channels,
-    clip_grad_vk_to_gl,
-    clip_gl_to_vk,
     image_batch,
     resolution_hw,
     sum_contribs,
@@ -281,22 +279,12 @@ class _RasterizeSoftFn(torch.autograd.Function):
     @staticmethod
     def forward(fctx, pos, vctx, md, resolution, radius_px, peels):
         h, w = resolution
-        dev = vctx.device
-        clip_vk = clip_gl_to_vk(vertex_batch(to_dev(pos, dev, "pos")))
-        n = clip_vk.shape[0]
-        layers = []
+        pos_b = vertex_batch(to_dev(pos, vctx.device, "pos"))
+        if md.n_verts > pos_b.shape[1]:
+            raise IndexError(f"tri names vertex {md.n_verts - 1}, pos has {pos_b.shape[1]}")
         with vctx.lock:
-            for i in range(n):
-                clip = clip_vk[i].contiguous()
-                sc = K.soft_clip(vctx._ctx, clip, md.faces_f, w, h, radius_px)
-                prev = None
-                for k in range(peels):
-                    rs = K.rasterize_soft(vctx._ctx, sc, md.corner_face_id, md.faces_seq, clip,
-                                          md.faces_f, w, h, radius_px, prev)
-                    layers.append(rs)
-                    if k + 1 < peels:
-                        prev = _peel_threshold(rs, radius_px)
-        out = torch.stack(layers, 0).reshape(n, peels, h, w, 4)
+            # every item and peel from one setup
+            out = K.surface_rasterize_soft(vctx._ctx, pos_b, md.faces_f, w, h, radius_px, peels)
         fctx.dressi = (vctx, md, radius_px)
         fctx.save_for_backward(pos, out)
         return out.to(pos.device)
@@ -306,34 +294,14 @@ class _RasterizeSoftFn(torch.autograd.Function):
         vctx, md, radius_px = fctx.dressi
         pos, out = fctx.saved_tensors
         dev = vctx.device
-        clip_vk = clip_gl_to_vk(vertex_batch(to_dev(pos, dev, "pos")))
+        pos_b = vertex_batch(to_dev(pos, dev, "pos"))
         g = to_dev(grad_out, dev, "grad_out")
-        n, peels = out.shape[:2]
-        g_clip = []
         with vctx.lock:
-            for i in range(n):
-                clip = clip_vk[i].contiguous()
-                contribs = []
-                for k in reversed(range(peels)):
-                    wide = K.gather_dist_grad(vctx._ctx, g[i, k].contiguous(), out[i, k], clip,
-                                              md.faces_f, md.vft, radius_px, True)
-                    contribs.append(K.col_sum(vctx._ctx, wide))
-                g_clip.append(sum_contribs(contribs))
-        g_pos = clip_grad_vk_to_gl(torch.stack(g_clip, 0))
+            g_pos = K.surface_soft_bwd(vctx._ctx, g, to_dev(out, dev, "out"), pos_b, md.faces_f,
+                                       md.vft, radius_px)
         if pos.dim() == 2:
             g_pos = g_pos.sum(dim=0)
         return g_pos.to(pos.device), None, None, None, None, None
-
-
-def _peel_threshold(rs: torch.Tensor, radius_px: float) -> torch.Tensor:
-    """The next peel's depth threshold: this layer's shifted depth rebuilt
-    from its output channels, 0 on background
-    (python/dressi/torch/ops.py:608-615)."""
-    dist, z, cov = rs[..., 0], rs[..., 2], rs[..., 3]
-    ge = (dist >= 0.0).to(torch.float32)
-    near = torch.clamp(z, 0.0, 1.0) * 0.5
-    far = torch.clamp(dist * (-1.0 / radius_px), 0.0, 1.0) * 0.5 + 0.5
-    return (cov * (ge * near + (1.0 - ge) * far)).contiguous()
 
 
 def rasterize_soft(ctx, pos, tri, resolution, radius_px=3.0, peels=1):

@@ -133,3 +133,44 @@ def test_surface_antialias(ctx, level, n, h, w, nc, samples, shared):
     assert float(ref.abs().max()) > 0 or h == 1
     _same(got, ref * 1.5, "position gradient")
     ctx.synchronize()
+
+
+def _peel_threshold(rs, radius_px):
+    dist, z, cov = rs[..., 0], rs[..., 2], rs[..., 3]
+    ge = (dist >= 0.0).to(torch.float32)
+    near = torch.clamp(z, 0.0, 1.0) * 0.5
+    far = torch.clamp(dist * (-1.0 / radius_px), 0.0, 1.0) * 0.5 + 0.5
+    return (cov * (ge * near + (1.0 - ge) * far)).contiguous()
+
+
+@pytest.mark.parametrize("level,n,h,w,peels,radius", [
+    (0, 1, 40, 64, 1, 3.0), (2, 3, 61, 97, 6, 2.7), (3, 2, 33, 130, 2, 3.0), (1, 4, 1, 200, 3, 0.4),
+    # 65 screens' bins: a second group of items
+    (0, 65, 512, 512, 2, 3.0)])
+def test_surface_rasterize_soft(ctx, level, n, h, w, peels, radius):
+    """Every item and peel against SoftClip / RasterizeSoft with the peel thresholds, and the
+    position gradient against GatherDistGrad, ColSum, the peels' sum and the remap's transpose."""
+    from opendressi_amd import ops as K
+    from opendressi_amd.torch.convert import clip_grad_vk_to_gl, sum_contribs
+    print(f"[surface soft] level {level} {n}x{h}x{w} peels {peels} r {radius}", flush=True)
+    clip, fi, ff, vf = _scene(level, n, level + n, 0.0)
+    nf = len(fi)
+    fid = torch.arange(nf, dtype=torch.float32).repeat_interleave(3).cuda()
+    seq = torch.arange(nf * 3, dtype=torch.float32).reshape(-1, 3).cuda()
+    got = K.surface_rasterize_soft(ctx, clip, ff, w, h, radius, peels)
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    gy = torch.randn(got.shape, device="cuda", generator=gen)
+    g_pos = K.surface_soft_bwd(ctx, gy, got, clip, ff, vf, radius)
+    for i in (range(n) if n < 10 else (0, n - 2, n - 1)):
+        vk = _to_vk(clip[i])
+        sc = K.soft_clip(ctx, vk, ff, w, h, radius)
+        prev, parts = None, []
+        for k in range(peels):
+            rs = K.rasterize_soft(ctx, sc, fid, seq, vk, ff, w, h, radius, prev)
+            _same(got[i, k], rs, f"item {i} peel {k}")
+            prev = _peel_threshold(rs, radius)
+            parts.insert(0, K.col_sum(ctx, K.gather_dist_grad(ctx, gy[i, k].contiguous(), rs, vk,
+                                                              ff, vf, radius, True)))
+        _same(g_pos[i], clip_grad_vk_to_gl(sum_contribs(parts)), f"item {i} gradient")
+    assert float(g_pos.abs().max()) > 0
+    ctx.synchronize()
