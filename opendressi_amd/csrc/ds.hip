@@ -224,17 +224,18 @@ __device__ __forceinline__ float dist_face_sum(const FaceCorners& fc, uint32_t f
     const bool twice = fc.idx[0] == fc.idx[1] || fc.idx[1] == fc.idx[2] || fc.idx[2] == fc.idx[0];
     float acc = 0.f;
     uint32_t n_hits = 0;
+    const uint32_t origin = (uint32_t)by0 * w + (uint32_t)bx0;
+    BoxWalk at((uint32_t)bx0, (uint32_t)by0, bw, w, lane);
     for (uint32_t p0 = 0; p0 < n_px; p0 += 64 * kDistPx) {
         uint32_t o[kDistPx];
         float2 yw[kDistPx];  // the winner's face id, coverage
 #pragma unroll
         for (uint32_t s = 0; s < kDistPx; s++) {
-            const uint32_t p = p0 + s * 64 + lane;
-            const uint32_t q = p < n_px ? p : 0;
-            const uint32_t row = q / bw;
-            o[s] = (by0 + row) * w + bx0 + (q - row * bw);
+            const bool in = p0 + s * 64 + lane < n_px;
+            o[s] = in ? at.o : origin;
+            at.next();
             const float4 v = rs[o[s]];
-            yw[s] = make_float2(v.y, p < n_px ? v.w : 0.f);
+            yw[s] = make_float2(v.y, in ? v.w : 0.f);
         }
 #pragma unroll
         for (uint32_t s = 0; s < kDistPx; s++) {
@@ -253,9 +254,9 @@ __device__ __forceinline__ float dist_face_sum(const FaceCorners& fc, uint32_t f
         for (uint32_t h0 = 0; h0 < n_hits; h0 += 64) {
             const uint32_t n = min(64u, n_hits - h0);
             if (lane < n) {
-                const uint32_t at = lds.hit_px[h0 + lane];
-                const uint32_t y = at / w, x = at - y * w;
-                const float g = gy[at].x;
+                const uint32_t px_o = lds.hit_px[h0 + lane];
+                const uint32_t y = px_o / w, x = px_o - y * w;
+                const float g = gy[px_o].x;
                 float4 t[3] = {};
                 if (g != 0.f) {
                     const float px = (float)x + 0.5f, py = (float)y + 0.5f;

@@ -117,17 +117,18 @@ __global__ __launch_bounds__(64) void k_surface_interp_bwd_faces(
         y1 = y1 < (int)h - 1 ? y1 : (int)h - 1;
         const uint32_t bw = x1 >= x0 ? (uint32_t)(x1 - x0 + 1) : 0u;
         const uint32_t n_px = y1 >= y0 ? bw * (uint32_t)(y1 - y0 + 1) : 0u;
+        const uint32_t origin = (uint32_t)y0 * w + (uint32_t)x0;
+        BoxWalk at((uint32_t)x0, (uint32_t)y0, bw ? bw : 1u, w, lane);
         for (uint32_t p0 = 0; p0 < n_px; p0 += 64 * kInterpPx) {
             float4 r[kInterpPx];
             uint32_t o[kInterpPx];
 #pragma unroll
             for (uint32_t q = 0; q < kInterpPx; q++) {
-                const uint32_t p = p0 + q * 64 + lane;
-                const uint32_t pc = p < n_px ? p : 0u;
-                const uint32_t row = pc / bw;
-                o[q] = (y0 + row) * w + x0 + (pc - row * bw);
+                const bool in = p0 + q * 64 + lane < n_px;
+                o[q] = in ? at.o : origin;
+                at.next();
                 r[q] = rast[o[q]];
-                r[q].w = p < n_px ? r[q].w : 0.f;
+                r[q].w = in ? r[q].w : 0.f;
             }
             uint32_t n_hits = 0;
 #pragma unroll
@@ -135,14 +136,14 @@ __global__ __launch_bounds__(64) void k_surface_interp_bwd_faces(
                 const bool hit = fid_u(r[q].w) == f + 1;
                 const uint64_t m = __ballot(hit);
                 if (hit) {
-                    const uint32_t at = n_hits + __popcll(m & ((1ull << lane) - 1ull));
+                    const uint32_t slot = n_hits + __popcll(m & ((1ull << lane) - 1ull));
                     const float w2 = (1.f - r[q].x) - r[q].y;
 #pragma unroll
                     for (int c = 0; c < C; c++) {
                         const float g = gy[(size_t)o[q] * C + c];
-                        term[at][c] = g * r[q].x;
-                        term[at][C + c] = g * r[q].y;
-                        term[at][2 * C + c] = g * w2;
+                        term[slot][c] = g * r[q].x;
+                        term[slot][C + c] = g * r[q].y;
+                        term[slot][2 * C + c] = g * w2;
                     }
                 }
                 n_hits += (uint32_t)__popcll(m);

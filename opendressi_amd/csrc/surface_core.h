@@ -14,6 +14,31 @@ __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// A lane's way through a box of an image in raster order, 64 pixels a step:
+// an add and a carry in place of a division per pixel.
+struct BoxWalk {
+    uint32_t o;  // the pixel's index in the image
+    uint32_t col, bw, step_col, step_o, wrap;
+    __device__ __forceinline__ BoxWalk(uint32_t x0, uint32_t y0, uint32_t box_w, uint32_t img_w,
+                                       uint32_t lane)
+        : bw(box_w) {
+        const uint32_t row = lane / bw, rows = 64u / bw;
+        col = lane - row * bw;
+        o = (y0 + row) * img_w + x0 + col;
+        step_col = 64u - rows * bw;
+        step_o = rows * img_w + step_col;
+        wrap = img_w - bw;
+    }
+    __device__ __forceinline__ void next() {
+        col += step_col;
+        o += step_o;
+        if (col >= bw) {
+            col -= bw;
+            o += wrap;
+        }
+    }
+};
+
 // The sum of gradient contributions as the reference's backward builder
 // forms it (src/core/build_backward.cpp:36-57): groups of at most four, each
 // summed left to right, level by level. Contributions come one at a time; a
