@@ -76,90 +76,102 @@ __global__ __launch_bounds__(256) void k_surface_interp(const float* attr, size_
 // that shows it, in raster order) of g u, g v and g ((1 - u) - v), the three
 // corners' gradients together: g_face {N,F,3} VEC C.
 //
-// A wave per face and item: 64 pixels of the box at once, the few that show
+// G lanes per face and item: PX G pixels of the box at once, the few that show
 // the face form their terms side by side, and one lane per corner and
 // channel adds them in order. One thread per face walked its box pixel by
 // pixel at a load latency each, three times over (one call per corner):
-// 3 x 515 us for four 1280 x 720 views of 20 480 faces, now 70.
-constexpr uint32_t kInterpPx = 2;  // pixels per lane and step
+// 3 x 515 us for four 1280 x 720 views of 20 480 faces, where a wave per face
+// takes 70. More pixels per step cost the LDS that keeps waves resident (four
+// per lane: 107 us there).
+//
+// Screen pixels per face from which a face gets a wave of its own. Below, its
+// box is a few steps of 32 pixels and four faces share a wave. Sixteen lanes
+// and a wave per face take (both kernels of the gradient) 41 and 62 us for
+// four 256 x 256 views at 3 pixels per face, 36 and 37 at 13, 49 and 35 at
+// 51; for four 1280 x 720 views 90 and 93 at 45, 459 and 163 at 720.
+constexpr uint32_t kInterpWavePx = 32;
 
-template <int C>
+template <int C, int G>
 __global__ __launch_bounds__(64) void k_surface_interp_bwd_faces(
         const float* gy, const float4* rast, uint32_t w, uint32_t h, const float4* clip,
         size_t clip_stride, const float* faces, uint32_t n_faces, uint32_t n_verts,
         float* g_face) {
-    __shared__ float term[64 * kInterpPx][3 * C];
-    const uint32_t f = blockIdx.x, lane = threadIdx.x;
+    static_assert(3 * C <= G, "a lane per corner and channel");
+    constexpr uint32_t PX = 2;  // pixels per lane and step
+    __shared__ float term[64 / G][G * PX][3 * C];
+    const uint32_t lane = threadIdx.x % G, grp = threadIdx.x / G;
+    const uint32_t f = blockIdx.x * (64 / G) + grp;
+    const bool live = f < n_faces;
     const size_t npx = (size_t)w * h;
     gy += blockIdx.y * npx * C;
     rast += blockIdx.y * npx;
     clip += blockIdx.y * clip_stride;
-    g_face += ((size_t)blockIdx.y * n_faces + f) * 3 * C;
-    float acc = 0.f;
     float s[3][2];
-    bool ok = true;
+    bool ok = live;
 #pragma unroll
     for (int k = 0; k < 3; k++) {
-        const uint32_t v = fid_u(faces[(size_t)f * 3 + k]);
+        const uint32_t v = live ? fid_u(faces[(size_t)f * 3 + k]) : n_verts;
         const float4 c = v < n_verts ? clip[v] : make_float4(0.f, 0.f, 0.f, 0.f);
         ok = ok && c.w > 1e-6f;
         s[k][0] = (c.x / c.w * 0.5f + 0.5f) * (float)w;
         s[k][1] = (c.y / c.w * 0.5f + 0.5f) * (float)h;
     }
-    if (ok) {
-        int x0 = (int)floorf(smin(smin(s[0][0], s[1][0]), s[2][0]) - 1.f);
-        int x1 = (int)ceilf(smax(smax(s[0][0], s[1][0]), s[2][0]) + 1.f);
-        int y0 = (int)floorf(smin(smin(s[0][1], s[1][1]), s[2][1]) - 1.f);
-        int y1 = (int)ceilf(smax(smax(s[0][1], s[1][1]), s[2][1]) + 1.f);
-        x0 = x0 > 0 ? x0 : 0;
-        y0 = y0 > 0 ? y0 : 0;
-        x1 = x1 < (int)w - 1 ? x1 : (int)w - 1;
-        y1 = y1 < (int)h - 1 ? y1 : (int)h - 1;
-        const uint32_t bw = x1 >= x0 ? (uint32_t)(x1 - x0 + 1) : 0u;
-        const uint32_t n_px = y1 >= y0 ? bw * (uint32_t)(y1 - y0 + 1) : 0u;
-        const uint32_t origin = (uint32_t)y0 * w + (uint32_t)x0;
-        BoxWalk at((uint32_t)x0, (uint32_t)y0, bw ? bw : 1u, w, lane);
-        for (uint32_t p0 = 0; p0 < n_px; p0 += 64 * kInterpPx) {
-            float4 r[kInterpPx];
-            uint32_t o[kInterpPx];
+    int x0 = (int)floorf(smin(smin(s[0][0], s[1][0]), s[2][0]) - 1.f);
+    int x1 = (int)ceilf(smax(smax(s[0][0], s[1][0]), s[2][0]) + 1.f);
+    int y0 = (int)floorf(smin(smin(s[0][1], s[1][1]), s[2][1]) - 1.f);
+    int y1 = (int)ceilf(smax(smax(s[0][1], s[1][1]), s[2][1]) + 1.f);
+    x0 = x0 > 0 ? x0 : 0;
+    y0 = y0 > 0 ? y0 : 0;
+    x1 = x1 < (int)w - 1 ? x1 : (int)w - 1;
+    y1 = y1 < (int)h - 1 ? y1 : (int)h - 1;
+    ok = ok && x1 >= x0 && y1 >= y0;
+    const uint32_t bw = ok ? (uint32_t)(x1 - x0 + 1) : 1u;
+    const uint32_t n_px = ok ? bw * (uint32_t)(y1 - y0 + 1) : 0u;
+    const uint32_t origin = ok ? (uint32_t)y0 * w + (uint32_t)x0 : 0u;
+    BoxWalk at(ok ? (uint32_t)x0 : 0u, ok ? (uint32_t)y0 : 0u, bw, w, lane, G);
+    const uint64_t below = (1ull << lane) - 1ull;
+    float acc = 0.f;
+    for (uint32_t p0 = 0; __any(p0 < n_px); p0 += G * PX) {
+        float4 r[PX];
+        uint32_t o[PX];
 #pragma unroll
-            for (uint32_t q = 0; q < kInterpPx; q++) {
-                const bool in = p0 + q * 64 + lane < n_px;
-                o[q] = in ? at.o : origin;
-                at.next();
-                r[q] = rast[o[q]];
-                r[q].w = in ? r[q].w : 0.f;
-            }
-            uint32_t n_hits = 0;
-#pragma unroll
-            for (uint32_t q = 0; q < kInterpPx; q++) {
-                const bool hit = fid_u(r[q].w) == f + 1;
-                const uint64_t m = __ballot(hit);
-                if (hit) {
-                    const uint32_t slot = n_hits + __popcll(m & ((1ull << lane) - 1ull));
-                    const float w2 = (1.f - r[q].x) - r[q].y;
-#pragma unroll
-                    for (int c = 0; c < C; c++) {
-                        const float g = gy[(size_t)o[q] * C + c];
-                        term[slot][c] = g * r[q].x;
-                        term[slot][C + c] = g * r[q].y;
-                        term[slot][2 * C + c] = g * w2;
-                    }
-                }
-                n_hits += (uint32_t)__popcll(m);
-            }
-            wave_lds_sync();
-            if (lane < 3 * C) {
-#pragma unroll 4
-                for (uint32_t q = 0; q < n_hits; q++) {
-                    acc += term[q][lane];
-                }
-            }
-            wave_lds_sync();
+        for (uint32_t q = 0; q < PX; q++) {
+            const bool in = p0 + q * G + lane < n_px;
+            o[q] = in ? at.o : origin;
+            at.next();
+            r[q] = rast[o[q]];
+            r[q].w = in ? r[q].w : 0.f;
         }
+        uint32_t n_hits = 0;
+#pragma unroll
+        for (uint32_t q = 0; q < PX; q++) {
+            const bool hit = live && fid_u(r[q].w) == f + 1;
+            // the group's lanes of the ballot
+            const uint64_t m = (__ballot(hit) >> (grp * G)) & (~0ull >> (64 - G));
+            if (hit) {
+                const uint32_t slot = n_hits + (uint32_t)__popcll(m & below);
+                const float w2 = (1.f - r[q].x) - r[q].y;
+#pragma unroll
+                for (int c = 0; c < C; c++) {
+                    const float g = gy[(size_t)o[q] * C + c];
+                    term[grp][slot][c] = g * r[q].x;
+                    term[grp][slot][C + c] = g * r[q].y;
+                    term[grp][slot][2 * C + c] = g * w2;
+                }
+            }
+            n_hits += (uint32_t)__popcll(m);
+        }
+        wave_lds_sync();
+        if (lane < 3 * C) {
+#pragma unroll 16
+            for (uint32_t q = 0; q < n_hits; q++) {
+                acc += term[grp][q][lane];
+            }
+        }
+        wave_lds_sync();
     }
-    if (lane < 3 * C) {
-        g_face[lane] = acc;
+    if (live && lane < 3 * C) {
+        g_face[((size_t)blockIdx.y * n_faces + f) * 3 * C + lane] = acc;
     }
 }
 
@@ -281,10 +293,17 @@ int dressi_surface_interpolate_bwd(dressi_ctx* ctx, const float* gy, uint32_t n_
     with_channels(n_comp, [&](auto c) {
         constexpr int C = decltype(c)::value;
         if (n_faces) {
-            hipLaunchKernelGGL(k_surface_interp_bwd_faces<C>, dim3(n_faces, n_items), dim3(64), 0,
-                               ctx->stream, gy, (const float4*)rast, width, height,
-                               (const float4*)clip, clip_per_item ? (size_t)n_clip : (size_t)0,
-                               faces, n_faces, n_clip, g_face);
+            const auto launch = [&](auto kernel, uint32_t per_wave) {
+                hipLaunchKernelGGL(kernel, dim3(div_up(n_faces, per_wave), n_items), dim3(64), 0,
+                                   ctx->stream, gy, (const float4*)rast, width, height,
+                                   (const float4*)clip, clip_per_item ? (size_t)n_clip : (size_t)0,
+                                   faces, n_faces, n_clip, g_face);
+            };
+            if ((uint64_t)width * height < (uint64_t)n_faces * kInterpWavePx) {
+                launch(k_surface_interp_bwd_faces<C, 16>, 4);
+            } else {
+                launch(k_surface_interp_bwd_faces<C, 64>, 1);
+            }
         }
         hipLaunchKernelGGL(k_surface_interp_bwd_vtx<C>,
                            dim3(div_up(n_verts * n_comp, 256), shared_attr ? 1 : n_items),

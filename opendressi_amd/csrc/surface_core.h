@@ -14,18 +14,19 @@ __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// A lane's way through a box of an image in raster order, 64 pixels a step:
-// an add and a carry in place of a division per pixel.
+// A lane's way through a box of an image in raster order, `stride` pixels a
+// step (the lanes that share the box): an add and a carry in place of a
+// division per pixel.
 struct BoxWalk {
     uint32_t o;  // the pixel's index in the image
     uint32_t col, bw, step_col, step_o, wrap;
     __device__ __forceinline__ BoxWalk(uint32_t x0, uint32_t y0, uint32_t box_w, uint32_t img_w,
-                                       uint32_t lane)
+                                       uint32_t lane, uint32_t stride = 64)
         : bw(box_w) {
-        const uint32_t row = lane / bw, rows = 64u / bw;
+        const uint32_t row = lane / bw, rows = stride / bw;
         col = lane - row * bw;
         o = (y0 + row) * img_w + x0 + col;
-        step_col = 64u - rows * bw;
+        step_col = stride - rows * bw;
         step_o = rows * img_w + step_col;
         wrap = img_w - bw;
     }
