@@ -227,7 +227,14 @@ int launch_hard_setup(hipStream_t s, const RasterGeom& g, const float* clip, uin
                       const int32_t* faces, HardRec* recs);
 int launch_raster_hard(hipStream_t s, const RasterGeom& g, const HardRec* recs,
                        const BinBuffers& b, const float* attr, uint32_t n_comp, int mode,
-                       float* out, size_t attr_view = 0, float* ids = nullptr);
+                       float* out, size_t attr_view = 0, float* ids = nullptr,
+                       uint32_t n_attr = 1);
+// The per-op hard raster of `n_views` clip sets [n_views][V] (or one) with
+// VEC4 attributes [n_attr][V], n_attr == n_views or n_views == 1: one image
+// per attribute set. Arguments are checked by the caller.
+int raster_attrs(dressi_ctx* ctx, const float* clip, uint32_t n_verts, uint32_t n_views,
+                 const float* attr, uint32_t n_attr, const float* faces, uint32_t n_faces,
+                 uint32_t width, uint32_t height, float* out);
 
 // Sizes of the binning buffers for a problem; `cap` = list capacity.
 size_t bin_bytes(uint32_t n_bins, uint32_t cap);

@@ -248,7 +248,9 @@ int launch_hard_setup(hipStream_t s, const RasterGeom& g, const float* clip, uin
 // One workgroup per (tile, view), a wave per 8x8 block of the tile. mode 0:
 // perspective-correct attribute of the winner (cpu_raster.cpp:205-223), mode
 // 1: face + 1, mode 2: (u, v, z / w, face + 1) of the torch surface's raster,
-// whose `attr` are the clip positions {V} VEC4 (z, w read).
+// whose `attr` are the clip positions {V} VEC4 (z, w read). n_attr > 1 (mode
+// 0, one view): that many attribute sets of the one raster, `attr_view`
+// floats apart, an image each.
 //
 // A wave folds only the records whose bbox meets its block, found by one
 // test per lane and a ballot; with each wave walking all of the tile's
@@ -258,7 +260,7 @@ __global__ __launch_bounds__(kTileThreads) void k_raster_hard(RasterGeom g, cons
                                                               BinBuffers b, const float* attr,
                                                               uint32_t n_comp, int mode,
                                                               float* out, size_t attr_view,
-                                                              float* ids) {
+                                                              float* ids, uint32_t n_attr) {
     __shared__ HardRec lds_rec[kTileThreads];
     __shared__ uint32_t lds_face[kTileThreads];
     const uint32_t tile = blockIdx.x;
@@ -306,9 +308,12 @@ __global__ __launch_bounds__(kTileThreads) void k_raster_hard(RasterGeom g, cons
         out[o] = id;
         return;
     }
+    const size_t out_attr = (size_t)g.width * g.height * n_comp;
     if (best == kEmptyKey) {
-        for (uint32_t c = 0; c < n_comp; c++) {
-            out[o * n_comp + c] = 0.f;
+        for (uint32_t a = 0; a < n_attr; a++) {
+            for (uint32_t c = 0; c < n_comp; c++) {
+                out[a * out_attr + o * n_comp + c] = 0.f;
+            }
         }
         return;
     }
@@ -334,20 +339,22 @@ __global__ __launch_bounds__(kTileThreads) void k_raster_hard(RasterGeom g, cons
                                         (num[2] / denom) / (num[3] / denom), id);
         return;
     }
-    for (uint32_t c = 0; c < n_comp; c++) {
-        float num = 0.f;
-        for (int k = 0; k < 3; k++) {
-            num += l[k] * r.inv_w[k] * attr[(size_t)r.idx[k] * n_comp + c];
+    for (uint32_t a = 0; a < n_attr; a++, attr += attr_view, out += out_attr) {
+        for (uint32_t c = 0; c < n_comp; c++) {
+            float num = 0.f;
+            for (int k = 0; k < 3; k++) {
+                num += l[k] * r.inv_w[k] * attr[(size_t)r.idx[k] * n_comp + c];
+            }
+            out[o * n_comp + c] = num / denom;
         }
-        out[o * n_comp + c] = num / denom;
     }
 }
 
 int launch_raster_hard(hipStream_t s, const RasterGeom& g, const HardRec* recs,
                        const BinBuffers& b, const float* attr, uint32_t n_comp, int mode,
-                       float* out, size_t attr_view, float* ids) {
+                       float* out, size_t attr_view, float* ids, uint32_t n_attr) {
     hipLaunchKernelGGL(k_raster_hard, dim3(g.n_tiles, g.n_views), dim3(kTileThreads), 0, s, g,
-                       recs, b, attr, n_comp, mode, out, attr_view, ids);
+                       recs, b, attr, n_comp, mode, out, attr_view, ids, n_attr);
     DRESSI_CHECK_LAUNCH();
     return DRESSI_OK;
 }
@@ -772,7 +779,8 @@ static int hard_bins(dressi_ctx* ctx, const RasterGeom& g, HardBins* hb) {
 static int launch_hard_op(dressi_ctx* ctx, const RasterGeom& g, const HardBins& hb,
                           const float* clip, uint32_t n_verts, const float* faces,
                           const int32_t* faces_i, int gl, const float* attr, uint32_t n_comp,
-                          int mode, float* out, size_t attr_view, float* ids) {
+                          int mode, float* out, size_t attr_view, float* ids,
+                          uint32_t n_attr = 1) {
     if (g.n_faces) {
         hipLaunchKernelGGL(k_hard_setup_count, dim3(div_up(g.n_views * g.n_faces, 256)), dim3(256),
                            0, ctx->stream, g, (const float4*)clip, n_verts, faces, faces_i, gl,
@@ -784,7 +792,7 @@ static int launch_hard_op(dressi_ctx* ctx, const RasterGeom& g, const HardBins& 
         if (int rc = launch_bin_hard(ctx->stream, g, hb.recs, hb.b)) return rc;
     }
     return launch_raster_hard(ctx->stream, g, hb.recs, hb.b, attr, n_comp, mode, out, attr_view,
-                              ids);
+                              ids, n_attr);
 }
 
 // `n_items` clip sets [n_items][n_verts] over one face list; attributes
@@ -922,3 +930,19 @@ int dressi_surface_rasterize_soft(dressi_ctx* ctx, const float* pos, uint32_t n_
 }
 
 }  // extern "C"
+
+namespace dressi {
+
+int raster_attrs(dressi_ctx* ctx, const float* clip, uint32_t n_verts, uint32_t n_views,
+                 const float* attr, uint32_t n_attr, const float* faces, uint32_t n_faces,
+                 uint32_t width, uint32_t height, float* out) {
+    const RasterGeom g = make_geom(width, height, n_views, n_faces);
+    HardBins hb;
+    if (int rc = hard_bins(ctx, g, &hb)) return rc;
+    if (int rc = launch_zero(ctx->stream, hb.b.counts, sizeof(uint32_t) * g.n_tiles * n_views))
+        return rc;
+    return launch_hard_op(ctx, g, hb, clip, n_verts, faces, nullptr, 0, attr, 4, 0, out,
+                          (size_t)n_verts * 4, nullptr, n_views > 1 ? 1 : n_attr);
+}
+
+}  // namespace dressi

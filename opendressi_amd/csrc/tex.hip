@@ -12,6 +12,7 @@
 #include <vector>
 
 #include "plan.h"
+#include "surface_core.h"
 
 namespace dressi {
 namespace {
@@ -194,7 +195,12 @@ __global__ __launch_bounds__(256) void k_texture_nearest_op(const float* tex, in
 // src/codegen/glsl_codegen.cpp:657-703): per texel the anchor's screen
 // pixel (truncated), then the first pixel of the 7 x 7 window around it
 // (row order) whose uv truncates to this texel; the texel takes that
-// pixel's gradient (zero when none).
+// pixel's gradient (zero when none). blockIdx.y: the item of a batch.
+//
+// A window row's seven uv are loaded together before the first is tested:
+// one after the other, up to the first match (the centre, 24 probes on, for
+// most texels), each waited for its load (32 us for a 512 x 512 texture and
+// screen; four of them now take 48).
 __global__ __launch_bounds__(256) void k_gather_nearest_op(const float* gy, uint32_t n_comp,
                                                            int sw, int sh, const float4* inv_uv,
                                                            int tw, int th, const float2* uv,
@@ -203,33 +209,81 @@ __global__ __launch_bounds__(256) void k_gather_nearest_op(const float* gy, uint
     if (q >= tw * th) {
         return;
     }
+    const size_t npx = (size_t)sw * sh, nt = (size_t)tw * th;
+    gy += blockIdx.y * npx * n_comp;
+    inv_uv += blockIdx.y * nt;
+    uv += blockIdx.y * npx;
+    out += blockIdx.y * nt * n_comp;
     const int ty = q / tw, tx = q - ty * tw;
     const float4 iv = inv_uv_anchor(inv_uv, tw, th, tx, ty);
     float o[4] = {0.f, 0.f, 0.f, 0.f};
     if (iv.z > 0.5f) {
         const int scx = (int)iv.x, scy = (int)iv.y;
-        bool found = false;
-        for (int dy = -3; dy <= 3 && !found; dy++) {
-            for (int dx = -3; dx <= 3; dx++) {
-                const int spx = scx + dx, spy = scy + dy;
-                if (spx < 0 || spy < 0 || spx >= sw || spy >= sh) {
-                    continue;
+        size_t found = npx;
+        for (int dy = -3; dy <= 3 && found == npx; dy++) {
+            const int spy = scy + dy;
+            if (spy < 0 || spy >= sh) {
+                continue;
+            }
+            float2 su[7];
+#pragma unroll
+            for (int k = 0; k < 7; k++) {
+                const int spx = min(max(scx + k - 3, 0), sw - 1);
+                su[k] = uv[(size_t)spy * sw + spx];
+            }
+#pragma unroll
+            for (int k = 6; k >= 0; k--) {
+                const int spx = scx + k - 3;
+                if (spx >= 0 && spx < sw && (int)(su[k].x * (float)tw) == tx &&
+                    (int)(su[k].y * (float)th) == ty) {
+                    found = (size_t)spy * sw + spx;
                 }
-                const size_t sp = (size_t)spy * sw + spx;
-                const float2 su = uv[sp];
-                if ((int)(su.x * (float)tw) == tx && (int)(su.y * (float)th) == ty) {
-                    for (uint32_t c = 0; c < n_comp; c++) {
-                        o[c] = gy[sp * n_comp + c];
-                    }
-                    found = true;
-                    break;
-                }
+            }
+        }
+        if (found < npx) {
+            for (uint32_t c = 0; c < n_comp; c++) {
+                o[c] = gy[found * n_comp + c];
             }
         }
     }
     for (uint32_t c = 0; c < n_comp; c++) {
         out[(size_t)q * n_comp + c] = o[c];
     }
+}
+
+// The torch surface's texture gradient: per vertex the uv as a clip position
+// (UvAsClip, mesh_utils.cpp:180-189) and, per item, its ScreenAttr.
+__global__ __launch_bounds__(256) void k_surface_tex_prep(const float2* uv, uint32_t n_uv,
+                                                          const float4* clip, uint32_t n_verts,
+                                                          uint32_t n_items, size_t clip_stride,
+                                                          float W, float H, float4* uv_clip,
+                                                          float4* sattr) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n_uv) {
+        const float2 q = uv[i];
+        uv_clip[i] = make_float4(q.x * 2.f - 1.f, q.y * 2.f - 1.f, 0.5f, 1.f);
+    }
+    if (i < n_items * n_verts) {
+        const uint32_t item = i / n_verts, v = i - item * n_verts;
+        const float4 c = clip[item * clip_stride + v];
+        const float ndc_x = c.x / c.w;
+        const float ndc_y = c.y / c.w;
+        sattr[i] = make_float4((ndc_x * 0.5f + 0.5f) * W, (ndc_y * 0.5f + 0.5f) * H, 1.f, 0.f);
+    }
+}
+
+// The items' contributions, the last item first.
+__global__ __launch_bounds__(256) void k_surface_item_sum(const float* part, size_t n,
+                                                          uint32_t n_items, float* out) {
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) {
+        return;
+    }
+    ContribSum total;
+    for (uint32_t k = n_items; k-- > 0;) {
+        total.push(part[k * n + i]);
+    }
+    out[i] = total.sum();
 }
 
 // ScreenAttr (src/core/mesh_utils.cpp:191-203).
@@ -887,6 +941,46 @@ int dressi_texture_nearest_bwd(dressi_ctx* ctx, const float* gy, uint32_t n_comp
                        ctx->stream, gy, n_comp, (int)sw, (int)sh, (const float4*)inv_uv, (int)tw,
                        (int)th, (const float2*)uv, out);
     DRESSI_CHECK_LAUNCH();
+    return DRESSI_OK;
+}
+
+int dressi_surface_texture_bwd(dressi_ctx* ctx, const float* gy, uint32_t n_comp, uint32_t sw,
+                               uint32_t sh, uint32_t n_items, const float* pix_uv,
+                               const float* vtx_uv, int uv_per_item, const float* clip,
+                               int clip_per_item, uint32_t n_verts, const float* faces,
+                               uint32_t n_faces, uint32_t tw, uint32_t th, float* uv_clip,
+                               float* sattr, float* inv_uv, float* part, float* out) {
+    DRESSI_REQUIRE(ctx && gy && pix_uv && vtx_uv && clip && (faces || n_faces == 0) && uv_clip &&
+                           sattr && inv_uv && (part || n_items <= 1) && out,
+                   "texture backward: NULL buffer");
+    DRESSI_REQUIRE(n_comp >= 1 && n_comp <= 4, "n_comp must be 1..4");
+    DRESSI_REQUIRE(n_items >= 1 && n_items <= kMaxBatchItems, "batch of %u items", n_items);
+    DRESSI_REQUIRE(tw > 0 && th > 0 && (uint64_t)tw * th < (1ull << 31) &&
+                           (uint64_t)sw * sh < (1ull << 31) &&
+                           (uint64_t)n_items * n_verts < (1ull << 31) &&
+                           (uint64_t)n_items * n_faces < (1ull << 31),
+                   "size too large");
+    DRESSI_TRY_HIP(hipSetDevice(ctx->device));
+    if (n_verts) {
+        hipLaunchKernelGGL(k_surface_tex_prep, dim3(div_up(n_items * n_verts, 256)), dim3(256), 0,
+                           ctx->stream, (const float2*)vtx_uv,
+                           uv_per_item ? n_items * n_verts : n_verts, (const float4*)clip, n_verts,
+                           n_items, clip_per_item ? (size_t)n_verts : (size_t)0, (float)sw,
+                           (float)sh, (float4*)uv_clip, (float4*)sattr);
+        DRESSI_CHECK_LAUNCH();
+    }
+    if (int rc = raster_attrs(ctx, uv_clip, n_verts, uv_per_item ? n_items : 1, sattr, n_items,
+                              faces, n_faces, tw, th, inv_uv)) return rc;
+    hipLaunchKernelGGL(k_gather_nearest_op, dim3(div_up(tw * th, 256), n_items), dim3(256), 0,
+                       ctx->stream, gy, n_comp, (int)sw, (int)sh, (const float4*)inv_uv, (int)tw,
+                       (int)th, (const float2*)pix_uv, n_items > 1 ? part : out);
+    DRESSI_CHECK_LAUNCH();
+    if (n_items > 1) {
+        const size_t n = (size_t)tw * th * n_comp;
+        hipLaunchKernelGGL(k_surface_item_sum, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0,
+                           ctx->stream, (const float*)part, n, n_items, out);
+        DRESSI_CHECK_LAUNCH();
+    }
     return DRESSI_OK;
 }
 

@@ -542,6 +542,26 @@ def surface_soft_bwd(ctx: Context, gy: torch.Tensor, rs: torch.Tensor, pos: torc
     return out
 
 
+def surface_texture_bwd(ctx: Context, gy: torch.Tensor, pix_uv: torch.Tensor,
+                        vtx_uv: torch.Tensor, clip: torch.Tensor, faces: torch.Tensor, tw: int,
+                        th: int) -> torch.Tensor:
+    """dressi_surface_texture_bwd: gy (N, H, W, C), pix_uv (N, H, W, 2),
+    vtx_uv (V, 2) or (N, V, 2), clip (1 or N, V, 4) -> d/d tex (th, tw, C)."""
+    _prep(ctx)
+    n, h, w, nc = gy.shape
+    nv = clip.shape[1]
+    new = lambda *shape: torch.empty(shape, dtype=torch.float32, device=gy.device)
+    uv_clip, sattr, inv_uv = new(*vtx_uv.shape[:-1], 4), new(n, nv, 4), new(n, th, tw, 4)
+    part = new(n, th, tw, nc) if n > 1 else None
+    out = new(th, tw, nc)
+    check(lib.dressi_surface_texture_bwd(
+        ctx.handle, _ptr(gy, "gy"), nc, w, h, n, _ptr(pix_uv, "uv"), _ptr(vtx_uv, "vtx_uv"),
+        1 if vtx_uv.dim() == 3 else 0, _ptr(clip, "clip"), 1 if clip.shape[0] > 1 else 0, nv,
+        _ptr(faces, "faces"), faces.shape[0], tw, th, _ptr(uv_clip, "uv_clip"),
+        _ptr(sattr, "sattr"), _ptr(inv_uv, "inv_uv"), _ptr(part, "part"), _ptr(out, "out")))
+    return out
+
+
 # ---- split-sum IBL ops (maps are (H, W, C) equirect images) ----------------
 
 def _map_nc(m: torch.Tensor) -> int:

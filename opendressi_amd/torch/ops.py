@@ -8,9 +8,8 @@ device, with no host round trip. The backward of every op composes the
 reference's backward kernels exactly as the reference's backward builder does
 (src/core/build_backward.cpp:62-149): the same kernels, the same operand
 order, gradient contributions summed in descending creation order of the
-nodes that produced them. rasterize, interpolate and antialias run the whole
-batch at once; the other ops run their per-item kernels for each item;
-per-signature state lives in the context's `_engines`.
+nodes that produced them. Every op runs the whole batch at once; per-signature
+state lives in the context's `_engines`.
 """
 from __future__ import annotations
 
@@ -22,7 +21,6 @@ from .convert import (
     channels,
     image_batch,
     resolution_hw,
-    sum_contribs,
     to_dev,
     vertex_batch,
 )
@@ -142,12 +140,15 @@ class _TextureFn(torch.autograd.Function):
             raise ValueError(f"tex must be [H, W, C] or [1, H, W, C], got {tuple(tex.shape)}")
         channels(tex_d.shape[2], "tex")
         uv_d = to_dev(uv, dev, "uv")
-        n = uv_d.shape[0]
+        n, h, w, c = uv_d.shape
+        if c != 2:
+            raise ValueError(f"uv must have 2 components, got {c}")
         with vctx.lock:
-            outs = [K.texture_nearest(vctx._ctx, tex_d, uv_d[i].contiguous()) for i in range(n)]
+            # the items' rows are one image's
+            out = K.texture_nearest(vctx._ctx, tex_d, uv_d.view(n * h, w, 2))
         fctx.dressi = (vctx, iinfo)
         fctx.save_for_backward(tex, uv)
-        return torch.stack(outs, 0).to(tex.device)
+        return out.view(n, h, w, tex_d.shape[2]).to(tex.device)
 
     @staticmethod
     def backward(fctx, grad_out):
@@ -158,24 +159,22 @@ class _TextureFn(torch.autograd.Function):
         uv_d = to_dev(uv, dev, "uv")
         g = to_dev(grad_out, dev, "grad_out")
         rinfo = iinfo.raster
-        h, w = rinfo.resolution
         md = vctx.mesh(rinfo.tri)
         vtx_uv = to_dev(iinfo.attr, dev, "uv attr")
         n = uv_d.shape[0]
-        contribs = []
+        if vtx_uv.shape[-1] != 2:
+            raise ValueError("texture backward: the interpolated uv attribute must be [V, 2]")
+        if vtx_uv.dim() == 3 and vtx_uv.shape[0] == 1:
+            vtx_uv = vtx_uv[0]
+        nv = min(vtx_uv.shape[-2], rinfo.clip_vk.shape[1])
+        if md.n_verts > nv:
+            raise IndexError(f"tri names vertex {md.n_verts - 1}, uv or pos has {nv}")
+        clip = rinfo.clip_vk
+        if vtx_uv.shape[-2] != clip.shape[1]:
+            # vertices that no face names
+            vtx_uv, clip = vtx_uv[..., :nv, :].contiguous(), clip[:, :nv].contiguous()
         with vctx.lock:
-            for i in reversed(range(n)):
-                vuv = vtx_uv if vtx_uv.dim() == 2 else vtx_uv[i if vtx_uv.shape[0] > 1 else 0]
-                if vuv.shape[-1] != 2:
-                    raise ValueError("texture backward: the interpolated uv attribute must be [V, 2]")
-                one = torch.ones_like(vuv[:, :1])
-                uv_clip = torch.cat([vuv * 2.0 - 1.0, one * 0.5, one], dim=1).contiguous()
-                clip = rinfo.clip_vk[i if rinfo.clip_vk.shape[0] > 1 else 0].contiguous()
-                sattr = K.screen_attr(vctx._ctx, clip, w, h)
-                inv_uv = K.rasterize(vctx._ctx, uv_clip, sattr, md.faces_f, tw, th)
-                contribs.append(K.texture_nearest_bwd(vctx._ctx, g[i].contiguous(), inv_uv,
-                                                      uv_d[i].contiguous()))
-        g_tex = sum_contribs(contribs)
+            g_tex = K.surface_texture_bwd(vctx._ctx, g, uv_d, vtx_uv, clip, md.faces_f, tw, th)
         if tex.dim() == 4:
             g_tex = g_tex.unsqueeze(0)
         return g_tex.to(tex.device), None, None, None

@@ -174,3 +174,40 @@ def test_surface_rasterize_soft(ctx, level, n, h, w, peels, radius):
         _same(g_pos[i], clip_grad_vk_to_gl(sum_contribs(parts)), f"item {i} gradient")
     assert float(g_pos.abs().max()) > 0
     ctx.synchronize()
+
+
+@pytest.mark.parametrize("n,h,w,tw,th,nc,shared", [
+    (1, 40, 64, 33, 17, 3, True), (5, 61, 97, 64, 64, 4, True), (3, 130, 33, 1, 7, 1, False),
+    (2, 1, 200, 129, 50, 2, True), (17, 20, 20, 40, 40, 3, False)])
+def test_surface_texture_bwd(ctx, n, h, w, tw, th, nc, shared):
+    """The nearest texture's gradient against UvAsClip / ScreenAttr / Rasterize /
+    GatherByInverseUV per item and the contributions' sum, shared and per-item uv, uv that leave
+    part of the texture to the dilation."""
+    import opendressi_amd as od
+    from opendressi_amd import ops as K
+    from opendressi_amd.torch.convert import sum_contribs
+    print(f"[surface texture] {n}x{h}x{w} tex {tw}x{th}x{nc} shared {shared}", flush=True)
+    pos, uv, faces = od.uv_sphere(12, 9)
+    mvp = od.orbit_cameras(1, n, n)[0].reshape(n, 4, 4).astype(np.float64)
+    clip = np.concatenate([pos, np.ones((len(pos), 1))], 1)[None] @ mvp
+    clip[..., 2] = 2.0 * clip[..., 2] - clip[..., 3]
+    dev = lambda a, t=np.float32: torch.from_numpy(np.ascontiguousarray(a, t)).cuda()
+    ff, fi = dev(faces), dev(faces, np.int32)
+    rast, vk = K.surface_rasterize(ctx, dev(clip), fi, w, h)
+    vtx_uv = dev(0.05 + 0.8 * uv)
+    if not shared:
+        vtx_uv = torch.stack([vtx_uv * (0.5 + 0.5 / (i + 1)) for i in range(n)])
+    pix_uv = K.surface_interpolate(ctx, vtx_uv, rast, ff)
+    gen = torch.Generator(device="cuda").manual_seed(nc)
+    g = torch.randn((n, h, w, nc), device="cuda", generator=gen)
+    parts = []
+    for i in reversed(range(n)):
+        vuv = vtx_uv if shared else vtx_uv[i]
+        one = torch.ones_like(vuv[:, :1])
+        uv_clip = torch.cat([vuv * 2.0 - 1.0, one * 0.5, one], 1).contiguous()
+        inv = K.rasterize(ctx, uv_clip, K.screen_attr(ctx, vk[i].contiguous(), w, h), ff, tw, th)
+        parts.append(K.texture_nearest_bwd(ctx, g[i].contiguous(), inv, pix_uv[i].contiguous()))
+    got = K.surface_texture_bwd(ctx, g, pix_uv, vtx_uv, vk, ff, tw, th)
+    _same(got, sum_contribs(parts), "texture gradient")
+    assert float(got.abs().max()) > 0 or h == 1
+    ctx.synchronize()
