@@ -12,6 +12,7 @@
 
 #include <algorithm>
 #include <cstdint>
+#include <type_traits>
 #include <vector>
 
 #include "dressi_hip.h"
@@ -289,18 +290,41 @@ enum ConvMode : int {
 // One thread per output that did both (the form before) had 8192 / 64 waves
 // and less, each at the latency of a weight, a load and an add per source:
 // 2.4-3.2 ms from an 8192-texel source whatever the output's size. Now
-// 128 x 64 from 128 x 64 takes 69 us (67 M weights of ~40 VALU instructions:
-// issue), its transpose 103 us (one division more), and every smaller output
-// 40-47 us, which is the chain of 8192 adds (8 cycles each) and 64 barriers.
-// 256 sources a chunk: smaller outputs 37 us, but 112 us for the largest,
-// where the LDS then leaves three workgroups per CU.
-// Eight outputs: enough workgroups for a 64 x 32 map to reach all 256 CUs.
+// 128 x 64 from 128 x 64 takes 64 us (67 M weights of ~40 VALU instructions:
+// issue), its transpose 86 us (one division more). Few outputs have the form
+// below.
 constexpr uint32_t kConvOut = 8;
 constexpr uint32_t kConvChunk = 128;
 // A row of terms, padded so that the adding lanes' 16-byte reads start 4
 // banks apart.
 constexpr uint32_t kConvRow = kConvChunk + 4;
 constexpr uint32_t kConvThreads = 5 * 64;
+
+// The weight of an output and a source (`nj`: PrefBwd's normaliser).
+template <int MODE>
+__device__ __forceinline__ float conv_weight(float dt, float sin_s, float nj, float alpha,
+                                             bool* used) {
+    if (MODE == kIrrFwd || MODE == kIrrBwd) {
+        return (dt > 0.f ? dt : 0.f) * sin_s;
+    }
+    const float w = ggx_conv_weight(dt, alpha);
+    if (MODE == kPrefNorm || MODE == kPrefFwd) {
+        return w * sin_s;
+    }
+    *used = *used && !(w <= 0.f);  // the reference skips these
+    return w / nj;
+}
+
+template <int MODE>
+__device__ __forceinline__ float conv_result(float sum, float scale, float norm, float sin_i) {
+    if (MODE == kIrrFwd || MODE == kIrrBwd) {
+        return sum * scale;
+    }
+    if (MODE == kPrefFwd) {
+        return sum / (norm > 1e-12f ? norm : 1e-12f);
+    }
+    return MODE == kPrefBwd ? sum * sin_i : sum;
+}
 
 // `odir` are the output-map directions, `sdir` the source (env) directions;
 // `in` is the env (forward modes) or the output-map gradient (backward
@@ -359,17 +383,8 @@ __global__ __launch_bounds__(kConvThreads) void k_eq_conv(const float4* odir, ui
             const float4 ot = kBwd ? s.d : me[o];
             const float4 sd = kBwd ? me[o] : s.d;
             const float dt = ot.x * sd.x + ot.y * sd.y + ot.z * sd.z;
-            float w;
             bool used = live;
-            if (MODE == kIrrFwd || MODE == kIrrBwd) {
-                w = (dt > 0.f ? dt : 0.f) * sd.w;
-            } else if (MODE == kPrefNorm || MODE == kPrefFwd) {
-                w = ggx_conv_weight(dt, alpha) * sd.w;
-            } else {
-                const float w0 = ggx_conv_weight(dt, alpha);
-                used = used && !(w0 <= 0.f);  // the reference skips these
-                w = w0 / nj;
-            }
+            const float w = conv_weight<MODE>(dt, sd.w, nj, alpha, &used);
             float(*row)[kConvRow] = term[chunk & 1u][2 * o + half];
             if (MODE == kPrefNorm) {
                 row[0][src] = used ? w : 0.f;
@@ -433,16 +448,158 @@ __global__ __launch_bounds__(kConvThreads) void k_eq_conv(const float4* odir, ui
     if (!sums || i >= n_i) {
         return;
     }
-    float r = acc;
-    if (MODE == kIrrFwd || MODE == kIrrBwd) {
-        r *= scale;
-    } else if (MODE == kPrefFwd) {
-        const float nt = norm[i];
-        r /= (nt > 1e-12f ? nt : 1e-12f);
-    } else if (MODE == kPrefBwd) {
-        r *= idir[i].w;
+    out[(size_t)i * N + sc] = conv_result<MODE>(acc, scale, MODE == kPrefFwd ? norm[i] : 0.f,
+                                                MODE == kPrefBwd ? idir[i].w : 0.f);
+}
+
+// The same sums for few outputs, where the chain of adds bounds (4.7 cycles
+// each by itself, 17 us for 8192). Four outputs to a workgroup, 256 sources a
+// chunk, three buffers: the adding wave starts a chunk's reads before it has
+// added the one before, and the forming waves' loads are up to four chunks
+// ahead and stay in flight across the barriers, which wait for LDS alone.
+// From an 8192-texel source 1 to 512 outputs take 27 us and 2048 take 30,
+// where the form above takes 37-41 and 43 (its adding wave waits for each
+// chunk's first reads, and its chunks for the loads of the next). Chunks of
+// 128 here 32-34 us, 16 reads in flight 33. From 8192 outputs the weights
+// bound and three buffers' LDS costs waves: 64 us above, 74 with them.
+constexpr uint32_t kFewMax = 2048;
+constexpr uint32_t kFewOut = 4;
+constexpr uint32_t kFewChunk = 256;
+constexpr uint32_t kFewRow = kFewChunk + 4;
+constexpr uint32_t kFewLoads = 4;  // chunks whose sources are on their way
+constexpr int kFewAhead = 8;        // the adding wave's 16-byte reads in flight
+
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+template <int MODE, int N>
+__global__ __launch_bounds__(kConvThreads) void k_eq_conv_few(const float4* odir, uint32_t n_o,
+                                                              const float4* sdir, uint32_t n_s,
+                                                              const float* in, const float* norm,
+                                                              float alpha, float scale,
+                                                              float* out) {
+    constexpr bool kBwd = MODE == kIrrBwd || MODE == kPrefBwd;
+    __shared__ alignas(16) float term[3][kFewOut][N][kFewRow];
+    const uint32_t n_i = kBwd ? n_s : n_o;
+    const uint32_t n_j = kBwd ? n_o : n_s;
+    const float4* idir = kBwd ? sdir : odir;
+    const float4* jdir = kBwd ? odir : sdir;
+    const uint32_t i0 = blockIdx.x * kFewOut;
+    const uint32_t n_chunks = (n_j + kFewChunk - 1) / kFewChunk;
+    const uint32_t src = threadIdx.x;
+    if (src < 256) {
+        float4 me[kFewOut];
+#pragma unroll
+        for (uint32_t o = 0; o < kFewOut; o++) {
+            const uint32_t i = i0 + o;
+            me[o] = idir[i < n_i ? i : n_i - 1];
+        }
+        struct Source {
+            float4 d;
+            float norm, val[N];
+        } s[kFewLoads];
+        const auto load = [&](uint32_t chunk, Source* to) {
+            const uint32_t j = (chunk < n_chunks ? chunk : n_chunks - 1) * kFewChunk + src;
+            const uint32_t jc = j < n_j ? j : n_j - 1;
+            to->d = jdir[jc];
+            if (MODE == kPrefBwd) {
+                to->norm = norm[jc];
+            }
+            if (MODE != kPrefNorm) {
+#pragma unroll
+                for (int c = 0; c < N; c++) {
+                    to->val[c] = in[(size_t)jc * N + c];
+                }
+            }
+        };
+#pragma unroll
+        for (uint32_t k = 0; k < kFewLoads; k++) {
+            load(k, &s[k]);
+        }
+        // Chunk c is formed before barrier c, its first terms are read after
+        // barrier c, the others after barrier c + 1, and its buffer is free
+        // after barrier c + 2. Two chunks too many, +0 terms that no sum
+        // takes: without a branch around the loads the waits are for one
+        // chunk's.
+        uint32_t buf = 0;
+        for (uint32_t c0 = 0;; c0 += kFewLoads) {
+#pragma unroll
+            for (uint32_t k = 0; k < kFewLoads; k++) {
+                const uint32_t c = c0 + k;
+                const float nj = MODE == kPrefBwd && s[k].norm > 1e-12f ? s[k].norm : 1e-12f;
+#pragma unroll
+                for (uint32_t o = 0; o < kFewOut; o++) {
+                    const float4 ot = kBwd ? s[k].d : me[o];
+                    const float4 sd = kBwd ? me[o] : s[k].d;
+                    const float dt = ot.x * sd.x + ot.y * sd.y + ot.z * sd.z;
+                    bool used = c * kFewChunk + src < n_j;
+                    const float w = conv_weight<MODE>(dt, sd.w, nj, alpha, &used);
+#pragma unroll
+                    for (int ch = 0; ch < N; ch++) {
+                        const float x = MODE == kPrefNorm ? w : s[k].val[ch] * w;
+                        term[buf][o][ch][src] = used ? x : 0.f;
+                    }
+                }
+                load(c + kFewLoads, &s[k]);
+                lds_barrier();
+                if (c > n_chunks) {
+                    return;
+                }
+                buf = buf == 2 ? 0 : buf + 1;
+            }
+        }
     }
-    out[(size_t)i * N + sc] = r;
+    const uint32_t lane = src & 63u;
+    const bool sums = lane < kFewOut * N;
+    const uint32_t so = sums ? lane / N : 0u, sc = sums ? lane % N : 0u;
+    __builtin_amdgcn_s_setprio(3);
+    float acc = 0.f;
+    float4 a[kFewAhead], b[kFewAhead];
+    const auto add = [&](const float4* x) {
+#pragma unroll
+        for (int k = 0; k < kFewAhead; k++) {
+            acc += x[k].x;
+            acc += x[k].y;
+            acc += x[k].z;
+            acc += x[k].w;
+        }
+    };
+    lds_barrier();
+    lds_barrier();
+#pragma unroll
+    for (int k = 0; k < kFewAhead; k++) {
+        a[k] = ((const float4*)term[0][so][sc])[k];
+    }
+    uint32_t buf = 0;
+    for (uint32_t chunk = 0; chunk < n_chunks; chunk++) {
+        const float4* t = (const float4*)term[buf][so][sc];
+        buf = buf == 2 ? 0 : buf + 1;
+        // formed before the last barrier (after the last chunk: +0 terms)
+        const float4* t_next = (const float4*)term[buf][so][sc];
+#pragma unroll
+        for (int q = 0; q < (int)kFewChunk / 4; q += 2 * kFewAhead) {
+#pragma unroll
+            for (int k = 0; k < kFewAhead; k++) {
+                b[k] = t[q + kFewAhead + k];
+            }
+            add(a);
+#pragma unroll
+            for (int k = 0; k < kFewAhead; k++) {
+                a[k] = q + 2 * kFewAhead < (int)kFewChunk / 4 ? t[q + 2 * kFewAhead + k]
+                                                              : t_next[k];
+            }
+            add(b);
+        }
+        lds_barrier();
+    }
+    const uint32_t i = i0 + so;
+    if (sums && i < n_i) {
+        out[(size_t)i * N + sc] = conv_result<MODE>(acc, scale, MODE == kPrefFwd ? norm[i] : 0.f,
+                                                    MODE == kPrefBwd ? idir[i].w : 0.f);
+    }
 }
 
 // PrefilterEnv (f_ops.cpp:3089-3157): per output texel, n_samples GGX
@@ -603,19 +760,19 @@ int run_conv(dressi_ctx* ctx, const float* in, uint32_t sw, uint32_t sh, uint32_
     constexpr bool kBwd = MODE == kIrrBwd || MODE == kPrefBwd;
     const uint32_t n_i = kBwd ? sw * sh : ow * oh;
     const float scale = kIblTwoPi / ((float)sw * (float)sh);
-    const auto launch = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3(div_up(n_i, kConvOut)), dim3(kConvThreads), 0, ctx->stream,
-                           od, ow * oh, sd, sw * sh, in, norm, alpha, scale, out);
+    const bool few = n_i <= kFewMax;
+    const auto launch = [&](auto n_comp) {
+        constexpr int N = decltype(n_comp)::value;
+        const auto kernel = few ? k_eq_conv_few<MODE, N> : k_eq_conv<MODE, N>;
+        hipLaunchKernelGGL(kernel, dim3(div_up(n_i, few ? kFewOut : kConvOut)),
+                           dim3(kConvThreads), 0, ctx->stream, od, ow * oh, sd, sw * sh, in, norm,
+                           alpha, scale, out);
     };
-    if constexpr (MODE == kPrefNorm) {
-        launch(k_eq_conv<MODE, 1>);
-    } else {
-        switch (n) {
-            case 1: launch(k_eq_conv<MODE, 1>); break;
-            case 2: launch(k_eq_conv<MODE, 2>); break;
-            case 3: launch(k_eq_conv<MODE, 3>); break;
-            default: launch(k_eq_conv<MODE, 4>); break;
-        }
+    switch (MODE == kPrefNorm ? 1u : n) {
+        case 1: launch(std::integral_constant<int, 1>()); break;
+        case 2: launch(std::integral_constant<int, 2>()); break;
+        case 3: launch(std::integral_constant<int, 3>()); break;
+        default: launch(std::integral_constant<int, 4>()); break;
     }
     DRESSI_CHECK_LAUNCH();
     return DRESSI_OK;

@@ -150,6 +150,30 @@ def test_ibl_conv_chunks_match_oracle(ctx, oracle, shape):
     check(env, gy)
 
 
+@pytest.mark.parametrize("shape", [
+    # (source w, h, output w, h, channels): the form for few outputs, its chunks of 256 sources
+    # (one, up to the four that are loaded ahead and past them) and workgroups of 4 outputs, on
+    # both sides of 2048 outputs
+    (255, 1, 5, 1, 3), (256, 1, 4, 1, 4), (257, 2, 3, 1, 2), (256, 4, 1, 1, 3), (205, 5, 7, 1, 1),
+    (128, 9, 2047, 1, 3), (33, 8, 2048, 1, 4), (33, 8, 2049, 1, 3)])
+def test_ibl_conv_few_outputs_match_oracle(ctx, oracle, shape):
+    """Bit for bit, forward and back (where the source's texels are the outputs)."""
+    from opendressi_amd import ops
+    sw, sh, ow, oh, nc = shape
+    print(f"[ibl conv few] {shape}", flush=True)
+    rng = np.random.default_rng(ow)
+    env = rng.random((sh, sw, nc), dtype=np.float32)
+    gy = rng.standard_normal((oh, ow, nc)).astype(np.float32)
+    _exact(host(ops.prefilter_conv(ctx, dev(env), ow, oh, 0.4)),
+           oracle.prefilter_conv(env, ow, oh, 0.4), "pref")
+    _exact(host(ops.prefilter_conv_bwd(ctx, dev(gy), sw, sh, 0.4)),
+           oracle.prefilter_conv(env, ow, oh, 0.4, gy), "bwd")
+    _exact(host(ops.irradiance_conv(ctx, dev(env), ow, oh)),
+           oracle.irradiance_conv(env, ow, oh), "irradiance")
+    _exact(host(ops.irradiance_conv_bwd(ctx, dev(gy), sw, sh)),
+           oracle.irradiance_conv(env, ow, oh, gy), "irradiance bwd")
+
+
 def test_ibl_tables_beyond_the_kept_ones(oracle):
     """More map sizes than a context keeps tables for (64), the first ones again after they had to
     give place, and the tables of one context after another's end: the oracle's bits each time."""
