@@ -52,9 +52,14 @@ __global__ __launch_bounds__(256) void k_eq_sample(const float* map, int mw, int
 // texels, and adds to one line follow each other at ~15 ns (512 x 512
 // pixels, 3 channels: 18.7 ms onto a 4 x 2 map, 1.6 ms onto 32 x 16, 0.9 ms
 // onto 128 x 64). Here a workgroup sums a tile of 1024 pixels in LDS and
-// sends each touched texel to memory once: 20-26 us on each of these maps,
-// most of it the LDS adds of one wave to the same texel.
+// sends each touched texel to memory once. The LDS adds of one wave to the
+// same texel follow each other as well (20-25 us on each of these maps with
+// one sum per texel and 256 threads), so a texel has up to 32 sums side by
+// side, each taking every such lane's adds: 9.4-15 us.
 constexpr uint32_t kScatterPixels = 1024;
+constexpr uint32_t kScatterThreads = 1024;
+// Sums per texel in the hash table (2^kScatterHashCopies).
+constexpr uint32_t kScatterHashCopies = 2;
 // Entries (texel, channel) up to which a workgroup keeps the whole map in
 // LDS (48 KB, three workgroups per CU); above it a hash table of the texels
 // that the tile touches (at most 56 KB; a tile of a coherent direction image
@@ -99,7 +104,7 @@ __global__ __launch_bounds__(256) void k_eq_scatter_prep(const float* x, size_t 
     }
 }
 
-// The largest of the partial maxima (n_part <= 256 = the workgroup's size).
+// The largest of the partial maxima (n_part <= 256 <= the workgroup's size).
 __device__ __forceinline__ uint32_t scatter_max(const uint32_t* part, uint32_t n_part,
                                                 uint32_t* wmax) {
     uint32_t m = threadIdx.x < n_part ? part[threadIdx.x] : 0u;
@@ -108,7 +113,7 @@ __device__ __forceinline__ uint32_t scatter_max(const uint32_t* part, uint32_t n
         const uint32_t other = (uint32_t)__shfl_xor((int)m, o);
         m = other > m ? other : m;
     }
-    if ((threadIdx.x & 63) == 0) {
+    if (threadIdx.x < 256 && (threadIdx.x & 63) == 0) {
         wmax[threadIdx.x >> 6] = m;
     }
     __syncthreads();
@@ -131,42 +136,37 @@ __device__ __forceinline__ int fixed_exponent(uint32_t max_bits, double count) {
     return 62 - e;
 }
 
-// One workgroup per tile of tile_w x (1024 / tile_w) pixels. `slots_log2`:
-// 0 = the whole map in LDS, else the hash table's size.
-__global__ __launch_bounds__(256) void k_eq_scatter(const float* gy, uint32_t n, const float* dir,
-                                                    uint32_t dw, uint32_t dh, uint32_t tile_w,
-                                                    uint32_t tiles_x, int mw, int mh,
-                                                    const uint32_t* part, uint32_t n_part,
-                                                    uint32_t slots_log2,
-                                                    unsigned long long* acc) {
+// One workgroup per tile of tile_w x (1024 / tile_w) pixels, a thread per
+// pixel. `slots_log2`: 0 = the whole map in LDS, else the hash table's size.
+// 2^copies_log2 sums per texel (and channel), neighbours in LDS: a lane adds
+// to the one of its number.
+__global__ __launch_bounds__(kScatterThreads) void k_eq_scatter(
+        const float* gy, uint32_t n, const float* dir, uint32_t dw, uint32_t dh, uint32_t tile_w,
+        uint32_t tiles_x, int mw, int mh, const uint32_t* part, uint32_t n_part,
+        uint32_t slots_log2, uint32_t copies_log2, unsigned long long* acc) {
     extern __shared__ unsigned long long lds[];
     __shared__ uint32_t wmax[4];
     const uint32_t tid = threadIdx.x;
     const uint32_t slots = 1u << slots_log2;
     const uint32_t n_sum = slots_log2 ? slots * n : (uint32_t)(mw * mh) * n;
-    uint32_t* keys = (uint32_t*)(lds + n_sum);  // hash table only
-    for (uint32_t i = tid; i < n_sum; i += 256) {
+    uint32_t* keys = (uint32_t*)(lds + ((size_t)n_sum << copies_log2));  // hash table only
+    for (uint32_t i = tid; i < n_sum << copies_log2; i += kScatterThreads) {
         lds[i] = 0ull;
     }
     if (slots_log2) {
-        for (uint32_t i = tid; i < slots; i += 256) {
+        for (uint32_t i = tid; i < slots; i += kScatterThreads) {
             keys[i] = kScatterEmpty;
         }
     }
+    const uint32_t x = (blockIdx.x % tiles_x) * tile_w + tid % tile_w;
+    const uint32_t y = (blockIdx.x / tiles_x) * (kScatterPixels / tile_w) + tid / tile_w;
+    const uint32_t copy = tid & ((1u << copies_log2) - 1u);
     const int k = fixed_exponent(scatter_max(part, n_part, wmax), (double)((size_t)dw * dh));
     __syncthreads();
-    const uint32_t x0 = (blockIdx.x % tiles_x) * tile_w;
-    const uint32_t y0 = (blockIdx.x / tiles_x) * (kScatterPixels / tile_w);
-    for (uint32_t q = tid; q < kScatterPixels; q += 256) {
-        const uint32_t x = x0 + q % tile_w, y = y0 + q / tile_w;
-        if (x >= dw || y >= dh) {
-            continue;
-        }
-        const size_t p = (size_t)y * dw + x;
-        float u, v;
-        if (!dir_to_equirect(mk3(dir[p * 3 + 0], dir[p * 3 + 1], dir[p * 3 + 2]), &u, &v)) {
-            continue;
-        }
+    const size_t p = (size_t)y * dw + x;
+    float u, v;
+    if (x < dw && y < dh &&
+        dir_to_equirect(mk3(dir[p * 3 + 0], dir[p * 3 + 1], dir[p * 3 + 2]), &u, &v)) {
         const Taps t = taps_wrap(mw, mh, u, v);
         float g[4];
         for (uint32_t c = 0; c < n; c++) {
@@ -201,7 +201,8 @@ __global__ __launch_bounds__(256) void k_eq_scatter(const float* gy, uint32_t n,
                     continue;
                 }
                 if (in_lds) {
-                    atomicAdd(&lds[at * n + c], (unsigned long long)fx);
+                    atomicAdd(&lds[((at * n + c) << copies_log2) + copy],
+                              (unsigned long long)fx);
                 } else {
                     atomicAdd(&acc[(size_t)texel * n + c], (unsigned long long)fx);
                 }
@@ -209,11 +210,18 @@ __global__ __launch_bounds__(256) void k_eq_scatter(const float* gy, uint32_t n,
         }
     }
     __syncthreads();
-    for (uint32_t i = tid; i < n_sum; i += 256) {
-        const unsigned long long a = lds[i];
-        if (a) {
-            const size_t texel = slots_log2 ? keys[i / n] : i / n;
-            atomicAdd(&acc[texel * n + i % n], a);
+    // a lane per sum; a texel's lanes meet by shuffles
+    const uint32_t n_all = n_sum << copies_log2;
+    for (uint32_t i0 = 0; i0 < n_all; i0 += kScatterThreads) {
+        const uint32_t i = i0 + tid;
+        unsigned long long a = i < n_all ? lds[i] : 0ull;
+        for (uint32_t o = 1u << copies_log2 >> 1; o >= 1; o >>= 1) {
+            a += (unsigned long long)__shfl_xor((long long)a, (int)o);
+        }
+        const uint32_t s = i >> copies_log2;
+        if (a && copy == 0) {
+            const size_t texel = slots_log2 ? keys[s / n] : s / n;
+            atomicAdd(&acc[texel * n + s % n], a);
         }
     }
 }
@@ -831,11 +839,22 @@ int dressi_equirect_sample_bwd(dressi_ctx* ctx, const float* gy, uint32_t n_comp
         const uint32_t tiles_x = div_up(dw, tile_w);
         const uint64_t tiles = (uint64_t)tiles_x * div_up(dh, tile_h);
         DRESSI_REQUIRE(tiles < (1ull << 31), "too many pixels");
-        const uint32_t slots_log2 = cnt <= kScatterDirect ? 0u : scatter_slots_log2(n_comp);
-        const size_t lds = slots_log2 ? ((size_t)1 << slots_log2) * (8 * n_comp + 4) : cnt * 8;
-        hipLaunchKernelGGL(k_eq_scatter, dim3((uint32_t)tiles), dim3(256), lds, ctx->stream, gy,
-                           n_comp, dir, dw, dh, tile_w, tiles_x, (int)mw, (int)mh,
-                           (const uint32_t*)mx, n_part, slots_log2, (unsigned long long*)acc);
+        uint32_t copies_log2 = 0, slots_log2 = 0;
+        if (cnt <= kScatterDirect) {
+            while (copies_log2 < 5 && cnt << (copies_log2 + 1) <= kScatterDirect) copies_log2++;
+        } else {
+            // four sums per texel in a quarter of the slots where an image
+            // that covers the map gives a texel 16 pixels and more; a tile
+            // with more texels than slots adds the rest in memory
+            copies_log2 = npx / 16 >= (size_t)mw * mh ? kScatterHashCopies : 0u;
+            slots_log2 = scatter_slots_log2(n_comp) - copies_log2;
+        }
+        const size_t sums = slots_log2 ? (size_t)n_comp << slots_log2 : cnt;
+        const size_t lds = (sums << copies_log2) * 8 + (slots_log2 ? 4ull << slots_log2 : 0);
+        hipLaunchKernelGGL(k_eq_scatter, dim3((uint32_t)tiles), dim3(kScatterThreads), lds,
+                           ctx->stream, gy, n_comp, dir, dw, dh, tile_w, tiles_x, (int)mw, (int)mh,
+                           (const uint32_t*)mx, n_part, slots_log2, copies_log2,
+                           (unsigned long long*)acc);
         DRESSI_CHECK_LAUNCH();
     }
     hipLaunchKernelGGL(k_fixed_resolve, dim3((uint32_t)((cnt + 255) / 256)), dim3(256), 0,
