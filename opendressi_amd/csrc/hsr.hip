@@ -1271,11 +1271,11 @@ int dressi_hsr_render_targets(dressi_hsr_plan* p, const float* tgt_pos, uint32_t
         return DRESSI_OK;
     }
     const RasterGeom g = make_geom(p->desc.width, p->desc.height, N, n_tfaces);
-    const uint32_t cap = default_bin_cap(g, 8);
+    const HardBinSizes z = hard_bin_sizes(g);
     dressi_ctx* ctx = p->ctx;
     void *dclip = nullptr, *dfi = nullptr, *recs = nullptr, *bins = nullptr, *ones = nullptr;
     if (int rc = ctx_workspace(ctx, 0, sizeof(HardRec) * (size_t)N * n_tfaces, &recs)) return rc;
-    if (int rc = ctx_workspace(ctx, 1, bin_bytes(g.n_tiles * N, cap), &bins)) return rc;
+    if (int rc = ctx_workspace(ctx, 1, z.bytes, &bins)) return rc;
     if (int rc = ctx_workspace(ctx, 2, fi.size() * 4, &dfi)) return rc;
     if (int rc = ctx_workspace(ctx, 3, clip.size() * 4, &dclip)) return rc;
     if (int rc = ctx_workspace(ctx, 4, (size_t)n_tverts * 4, &ones)) return rc;
@@ -1284,14 +1284,12 @@ int dressi_hsr_render_targets(dressi_hsr_plan* p, const float* tgt_pos, uint32_t
     DRESSI_TRY_HIP(hipMemcpyAsync(dfi, fi.data(), fi.size() * 4, hipMemcpyHostToDevice, s));
     DRESSI_TRY_HIP(hipMemcpyAsync(dclip, clip.data(), clip.size() * 4, hipMemcpyHostToDevice, s));
     DRESSI_TRY_HIP(hipMemcpyAsync(ones, one.data(), one.size() * 4, hipMemcpyHostToDevice, s));
-    BinBuffers b;
-    bin_carve(bins, g.n_tiles * N, cap, &b);
-    DRESSI_TRY_HIP(hipMemsetAsync(b.counts, 0, sizeof(uint32_t) * b.n_bins, s));
-    if (int rc = launch_hard_setup(s, g, (const float*)dclip, n_tverts, (const int32_t*)dfi,
-                                   (HardRec*)recs)) return rc;
-    if (int rc = launch_count_hard(s, g, (const HardRec*)recs, b)) return rc;
-    if (int rc = launch_scan_bins(s, b)) return rc;
-    if (int rc = launch_bin_hard(s, g, (const HardRec*)recs, b)) return rc;
+    HardBinBuffers b;
+    hard_bin_carve(bins, z, &b);
+    if (int rc = launch_zero(s, b.counts, sizeof(uint32_t) * (z.n_bins + 1))) return rc;
+    if (int rc = launch_hard_setup_bin(s, g, (const float*)dclip, n_tverts, nullptr,
+                                       (const int32_t*)dfi, 0, b, nullptr, (HardRec*)recs))
+        return rc;
     if (int rc = launch_raster_hard(s, g, (const HardRec*)recs, b, (const float*)ones, 1, 0,
                                     (float*)p->d.targets)) return rc;
     DRESSI_TRY_HIP(hipStreamSynchronize(s));

@@ -141,17 +141,27 @@ struct HardRec {
 };
 static_assert(sizeof(HardRec) == 20 * 4, "HardRec layout");
 
-// Device buffers of one binning problem: `n_bins` = views x tiles.
-// Scan-based bins (hard rasterizer): counts -> offsets -> list[cap].
-// Fixed-capacity bins (soft rasterizer): list[bin * cap + slot], counts
-// cleared by the consumer; offsets / cursor unused.
+// Device buffers of the soft rasterizer's bins, `n_bins` = views x tiles:
+// list[bin * cap + slot], counts cleared by the consumer.
 struct BinBuffers {
-    uint32_t* counts = nullptr;   // [n_bins], zero between uses
-    uint32_t* offsets = nullptr;  // [n_bins + 1]
-    uint32_t* cursor = nullptr;   // [n_bins]
-    uint32_t* list = nullptr;     // [cap] or [n_bins][cap] face indices
+    uint32_t* counts = nullptr;  // [n_bins], zero between uses
+    uint32_t* list = nullptr;    // [n_bins][cap] face indices
     uint32_t cap = 0;
     uint32_t n_bins = 0;
+};
+
+// The hard rasterizer's: counts and n_over (one word behind them) are cleared
+// before each use; faces that find their bin's list full go to `over`.
+struct HardBinBuffers {
+    uint32_t* counts = nullptr;  // [n_bins]
+    uint32_t* n_over = nullptr;  // counts + n_bins
+    uint2* over = nullptr;       // [over_cap] (bin, face)
+    uint32_t* list = nullptr;    // [n_bins][cap] face indices
+    uint32_t cap = 0, over_cap = 0, n_bins = 0;
+};
+struct HardBinSizes {
+    uint32_t n_bins, cap, over_cap;
+    size_t bytes;
 };
 
 // Fixed-capacity soft bins: n_bins counters + n_bins * cap entries.
@@ -161,8 +171,6 @@ inline size_t fixed_bin_bytes(uint32_t n_bins, uint32_t cap) {
 inline void fixed_bin_carve(void* base, uint32_t n_bins, uint32_t cap, BinBuffers* b) {
     uint32_t* p = (uint32_t*)base;
     b->counts = p;
-    b->offsets = nullptr;
-    b->cursor = nullptr;
     b->list = p + n_bins;
     b->cap = cap;
     b->n_bins = n_bins;
@@ -217,16 +225,14 @@ inline RasterGeom make_geom(uint32_t w, uint32_t h, uint32_t views, uint32_t fac
 }
 
 // Kernels shared between raster.hip and hsr.hip (launch helpers).
-int launch_scan_bins(hipStream_t s, const BinBuffers& b);
-int launch_bin_hard(hipStream_t s, const RasterGeom& g, const HardRec* recs, const BinBuffers& b);
-int launch_count_hard(hipStream_t s, const RasterGeom& g, const HardRec* recs, const BinBuffers& b);
 // Hard raster of a clip-space mesh into `out` ({views,S,S} x n_comp):
 // mode 0 = attribute interpolation, 1 = face id + 1. `clip` is [views][V]
-// float4, `faces` int32 [F][3].
-int launch_hard_setup(hipStream_t s, const RasterGeom& g, const float* clip, uint32_t n_verts,
-                      const int32_t* faces, HardRec* recs);
+// float4, `faces` float or `faces_i` int32 [F][3].
+int launch_hard_setup_bin(hipStream_t s, const RasterGeom& g, const float* clip, uint32_t n_verts,
+                          const float* faces, const int32_t* faces_i, int gl,
+                          const HardBinBuffers& b, uint32_t* err, HardRec* recs);
 int launch_raster_hard(hipStream_t s, const RasterGeom& g, const HardRec* recs,
-                       const BinBuffers& b, const float* attr, uint32_t n_comp, int mode,
+                       const HardBinBuffers& b, const float* attr, uint32_t n_comp, int mode,
                        float* out, size_t attr_view = 0, float* ids = nullptr,
                        uint32_t n_attr = 1);
 // The per-op hard raster of `n_views` clip sets [n_views][V] (or one) with
@@ -236,10 +242,8 @@ int raster_attrs(dressi_ctx* ctx, const float* clip, uint32_t n_verts, uint32_t 
                  const float* attr, uint32_t n_attr, const float* faces, uint32_t n_faces,
                  uint32_t width, uint32_t height, float* out);
 
-// Sizes of the binning buffers for a problem; `cap` = list capacity.
-size_t bin_bytes(uint32_t n_bins, uint32_t cap);
-void bin_carve(void* base, uint32_t n_bins, uint32_t cap, BinBuffers* b);
-// Default list capacity: `per_face` tile entries per face and view.
-uint32_t default_bin_cap(const RasterGeom& g, uint32_t per_face);
+// The hard bins' buffers for a problem.
+HardBinSizes hard_bin_sizes(const RasterGeom& g);
+void hard_bin_carve(void* base, const HardBinSizes& z, HardBinBuffers* b);
 
 }  // namespace dressi

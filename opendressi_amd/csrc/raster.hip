@@ -12,236 +12,157 @@ namespace dressi {
 // Binning
 // ---------------------------------------------------------------------------
 
-size_t bin_bytes(uint32_t n_bins, uint32_t cap) {
-    return sizeof(uint32_t) * ((size_t)n_bins * 3 + 1 + cap) + 256;
+// Entries of the hard bins' lists together (128 MB): a bin has room for the
+// whole mesh up to there, and at least kHardBinMin.
+constexpr uint64_t kHardListEntries = 32ull << 20;
+constexpr uint32_t kHardBinMin = 16;
+
+HardBinSizes hard_bin_sizes(const RasterGeom& g) {
+    const uint64_t n_bins = (uint64_t)g.n_tiles * g.n_views;
+    HardBinSizes z;
+    z.n_bins = (uint32_t)n_bins;
+    z.cap = (uint32_t)std::min<uint64_t>(
+            std::max<uint64_t>(kHardListEntries / n_bins, kHardBinMin),
+            std::max<uint64_t>(g.n_faces, 1));
+    z.over_cap = (uint32_t)std::min<uint64_t>((uint64_t)g.n_faces * g.n_views * 8 + 4096,
+                                              0x3fffffffull);
+    z.bytes = sizeof(uint32_t) * (n_bins + 2 + 2 * (size_t)z.over_cap + n_bins * z.cap) + 256;
+    return z;
 }
 
-void bin_carve(void* base, uint32_t n_bins, uint32_t cap, BinBuffers* b) {
+void hard_bin_carve(void* base, const HardBinSizes& z, HardBinBuffers* b) {
     uint32_t* p = (uint32_t*)base;
     b->counts = p;
-    b->offsets = p + n_bins;
-    b->cursor = p + 2 * (size_t)n_bins + 1;
-    b->list = p + 3 * (size_t)n_bins + 1;
-    b->cap = cap;
-    b->n_bins = n_bins;
-}
-
-uint32_t default_bin_cap(const RasterGeom& g, uint32_t per_face) {
-    const uint64_t c = (uint64_t)g.n_faces * g.n_views * per_face + 4096;
-    return c > 0x7fffffffull ? 0x7fffffffu : (uint32_t)c;
-}
-
-template <typename Rec>
-__global__ __launch_bounds__(256) void k_count(RasterGeom g, const Rec* recs, BinBuffers b) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= g.n_views * g.n_faces) {
-        return;
-    }
-    const Rec& r = recs[i];
-    if (r.bx0 > r.bx1 || r.by0 > r.by1) {
-        return;
-    }
-    const uint32_t view = i / g.n_faces;
-    uint32_t* cnt = b.counts + (size_t)view * g.n_tiles;
-    for (int ty = r.by0 / kTile; ty <= r.by1 / kTile; ty++) {
-        for (int tx = r.bx0 / kTile; tx <= r.bx1 / kTile; tx++) {
-            atomicAdd(&cnt[ty * g.tiles_x + tx], 1u);
-        }
-    }
-}
-
-template <typename Rec>
-__global__ __launch_bounds__(256) void k_bin(RasterGeom g, const Rec* recs, BinBuffers b) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= g.n_views * g.n_faces) {
-        return;
-    }
-    const Rec& r = recs[i];
-    if (r.bx0 > r.bx1 || r.by0 > r.by1) {
-        return;
-    }
-    const uint32_t view = i / g.n_faces;
-    const uint32_t f = i - view * g.n_faces;
-    uint32_t* cur = b.cursor + (size_t)view * g.n_tiles;
-    for (int ty = r.by0 / kTile; ty <= r.by1 / kTile; ty++) {
-        for (int tx = r.bx0 / kTile; tx <= r.bx1 / kTile; tx++) {
-            const uint32_t slot = atomicAdd(&cur[ty * g.tiles_x + tx], 1u);
-            if (slot < b.cap) {
-                b.list[slot] = f;
-            }
-        }
-    }
-}
-
-// Exclusive scan of the bin counts (one workgroup): writes offsets and
-// cursors and clears the counts for the next use. 4096 bins a step, four
-// neighbouring ones per thread, so that a wave's accesses are whole lines
-// (a contiguous run per thread, each access its own line, took 29 us for the
-// 14 400 tiles of four 1280 x 720 views; this takes 15).
-__global__ __launch_bounds__(1024) void k_scan(BinBuffers b) {
-    __shared__ uint32_t wave_sum[2][16];
-    const uint32_t n = b.n_bins;
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    uint32_t run = 0;
-    int buf = 0;
-    for (uint32_t base = 0; base < n; base += 4096, buf ^= 1) {
-        const uint32_t i0 = base + threadIdx.x * 4;
-        uint32_t c[4], s = 0;
-#pragma unroll
-        for (uint32_t k = 0; k < 4; k++) {
-            c[k] = i0 + k < n ? b.counts[i0 + k] : 0u;
-            s += c[k];
-        }
-        uint32_t incl = s;
-#pragma unroll
-        for (uint32_t o = 1; o < 64; o <<= 1) {
-            const uint32_t v = (uint32_t)__shfl_up((int)incl, o);
-            incl += lane >= o ? v : 0u;
-        }
-        if (lane == 63) {
-            wave_sum[buf][wave] = incl;
-        }
-        __syncthreads();
-        uint32_t at = run + incl - s;
-#pragma unroll
-        for (uint32_t q = 0; q < 16; q++) {
-            const uint32_t v = wave_sum[buf][q];
-            at += q < wave ? v : 0u;
-            run += v;
-        }
-#pragma unroll
-        for (uint32_t k = 0; k < 4; k++) {
-            if (i0 + k < n) {
-                b.offsets[i0 + k] = at;
-                b.cursor[i0 + k] = at;
-                b.counts[i0 + k] = 0;
-            }
-            at += c[k];
-        }
-    }
-    if (threadIdx.x == 0) {
-        b.offsets[n] = run;
-    }
-}
-
-int launch_scan_bins(hipStream_t s, const BinBuffers& b) {
-    hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, s, b);
-    DRESSI_CHECK_LAUNCH();
-    return DRESSI_OK;
-}
-
-int launch_count_hard(hipStream_t s, const RasterGeom& g, const HardRec* recs, const BinBuffers& b) {
-    const uint32_t n = g.n_views * g.n_faces;
-    hipLaunchKernelGGL(k_count<HardRec>, dim3(div_up(n, 256)), dim3(256), 0, s, g, recs, b);
-    DRESSI_CHECK_LAUNCH();
-    return DRESSI_OK;
-}
-
-int launch_bin_hard(hipStream_t s, const RasterGeom& g, const HardRec* recs, const BinBuffers& b) {
-    const uint32_t n = g.n_views * g.n_faces;
-    hipLaunchKernelGGL(k_bin<HardRec>, dim3(div_up(n, 256)), dim3(256), 0, s, g, recs, b);
-    DRESSI_CHECK_LAUNCH();
-    return DRESSI_OK;
+    b->n_over = p + z.n_bins;
+    const size_t at = ((size_t)z.n_bins + 2) & ~(size_t)1;  // pairs: 8-byte aligned
+    b->over = (uint2*)(p + at);
+    b->list = p + at + 2 * (size_t)z.over_cap;
+    b->cap = z.cap;
+    b->over_cap = z.over_cap;
+    b->n_bins = z.n_bins;
 }
 
 // ---------------------------------------------------------------------------
 // Hard rasterizer (Rasterize / RasterizeFaceId)
 // ---------------------------------------------------------------------------
 
-// clip [views][V] float4, faces int32 [F][3]; one thread per (view, face).
-__global__ __launch_bounds__(256) void k_hard_setup(RasterGeom g, const float4* clip,
-                                                     uint32_t n_verts, const int32_t* faces,
-                                                     HardRec* recs) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= g.n_views * g.n_faces) {
+// Adds face f to bin `bin`: to its list, or to the overflow that every tile
+// with a full list looks through.
+__device__ __forceinline__ void hard_append(const HardBinBuffers& b, uint32_t bin, uint32_t f,
+                                            uint32_t slot) {
+    if (slot < b.cap) {
+        b.list[(size_t)bin * b.cap + slot] = f;
         return;
     }
-    const uint32_t view = i / g.n_faces;
-    const uint32_t f = i - view * g.n_faces;
-    HardRec r;
-    int idx[3];
-    float4 c[3];
-    bool ok = true;
-    for (int k = 0; k < 3; k++) {
-        idx[k] = faces[(size_t)f * 3 + k];
-        ok = ok && idx[k] >= 0 && (uint32_t)idx[k] < n_verts;
+    const uint32_t o = atomicAdd(b.n_over, 1u);
+    if (o < b.over_cap) {
+        b.over[o] = make_uint2(bin, f);
     }
-    if (!ok) {
-        r.bx0 = 1;
-        r.bx1 = 0;
-        r.by0 = 1;
-        r.by1 = 0;
-        recs[i] = r;
-        return;
-    }
-    for (int k = 0; k < 3; k++) {
-        c[k] = clip[(size_t)view * n_verts + idx[k]];
-    }
-    hard_setup(c, idx, g.width, g.height, &r);
-    recs[i] = r;
 }
 
-// k_hard_setup and k_count in one: the per-op calls' setup, from the
-// reference's float face ids (decoded as RasterizeCore does,
-// uint32_t(int64_t(x)); a bad one is reported) or from int32 ones. `gl`: clip
-// z in [-w, w], remapped to 0.5 (z + w).
-__global__ __launch_bounds__(256) void k_hard_setup_count(RasterGeom g, const float4* clip,
-                                                          uint32_t n_verts, const float* faces,
-                                                          const int32_t* faces_i, int gl,
-                                                          BinBuffers b, uint32_t* err,
-                                                          HardRec* recs) {
+// Setup and binning, a thread per (view, face), from the reference's float
+// face ids (decoded as RasterizeCore does, uint32_t(int64_t(x)); a bad one is
+// reported) or from int32 ones. `gl`: clip z in [-w, w], remapped to
+// 0.5 (z + w). b.counts and b.n_over are zero.
+//
+// Lists of a fixed size take a face where it is set up. With lists sized by a
+// count and a scan (the form before) a raster had two launches more: 17 + 15
+// + 18 us for four 1280 x 720 views of 20 480 faces, now 21. What bounds is
+// the adds' round trip to memory: a wave shares its faces' tiles out evenly,
+// a lane has kBinPairs of them on their way at once (a thread that goes
+// through its own face's tiles, four at a time: 50 us). The lists' size makes
+// no difference there (128 entries or the whole mesh).
+constexpr uint32_t kBinPairs = 4;
+
+__global__ __launch_bounds__(256) void k_hard_setup_bin(RasterGeom g, const float4* clip,
+                                                        uint32_t n_verts, const float* faces,
+                                                        const int32_t* faces_i, int gl,
+                                                        HardBinBuffers b, uint32_t* err,
+                                                        HardRec* recs) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= g.n_views * g.n_faces) {
-        return;
-    }
-    const uint32_t view = i / g.n_faces;
-    const uint32_t f = i - view * g.n_faces;
+    const bool live = i < g.n_views * g.n_faces;
+    const uint32_t view = live ? i / g.n_faces : 0u;
+    const uint32_t f = live ? i - view * g.n_faces : 0u;
     HardRec r;
     r.bx0 = 1;
     r.bx1 = 0;
     r.by0 = 1;
     r.by1 = 0;
-    int idx[3];
-    float4 c[3];
-    bool ok = true;
+    if (live) {
+        int idx[3];
+        float4 c[3];
+        bool ok = true;
 #pragma unroll
-    for (int k = 0; k < 3; k++) {
-        const uint32_t v = faces ? (uint32_t)(int64_t)faces[(size_t)f * 3 + k]
-                                 : (uint32_t)faces_i[(size_t)f * 3 + k];
-        ok = ok && v < n_verts;
-        idx[k] = (int)v;
-    }
-    if (!ok) {
-        atomicOr(err, 16u);
-        recs[i] = r;
-        return;
-    }
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-        c[k] = clip[(size_t)view * n_verts + idx[k]];
-        if (gl) {
-            c[k].z = 0.5f * (c[k].z + c[k].w);
+        for (int k = 0; k < 3; k++) {
+            const uint32_t v = faces ? (uint32_t)(int64_t)faces[(size_t)f * 3 + k]
+                                     : (uint32_t)faces_i[(size_t)f * 3 + k];
+            ok = ok && v < n_verts;
+            idx[k] = (int)v;
         }
+        if (ok) {
+#pragma unroll
+            for (int k = 0; k < 3; k++) {
+                c[k] = clip[(size_t)view * n_verts + idx[k]];
+                if (gl) {
+                    c[k].z = 0.5f * (c[k].z + c[k].w);
+                }
+            }
+            hard_setup(c, idx, g.width, g.height, &r);
+        } else if (err) {
+            atomicOr(err, 16u);
+        }
+        recs[i] = r;
     }
-    hard_setup(c, idx, g.width, g.height, &r);
-    recs[i] = r;
-    if (r.bx0 > r.bx1 || r.by0 > r.by1) {
-        return;
+    const bool any = r.bx0 <= r.bx1 && r.by0 <= r.by1;
+    const uint32_t tx0 = any ? (uint32_t)r.bx0 / kTile : 0u;
+    const uint32_t ty0 = any ? (uint32_t)r.by0 / kTile : 0u;
+    const uint32_t tw = any ? (uint32_t)r.bx1 / kTile - tx0 + 1 : 1u;
+    const uint32_t n = any ? tw * ((uint32_t)r.by1 / kTile - ty0 + 1) : 0u;
+    const uint32_t first = view * g.n_tiles + ty0 * g.tiles_x + tx0;
+    // the wave's (face, tile) pairs, lane l's behind those of the lanes below
+    const uint32_t lane = threadIdx.x & 63u;
+    uint32_t incl = n;
+#pragma unroll
+    for (uint32_t o = 1; o < 64; o <<= 1) {
+        const uint32_t v = (uint32_t)__shfl_up((int)incl, o);
+        incl += lane >= o ? v : 0u;
     }
-    uint32_t* cnt = b.counts + (size_t)view * g.n_tiles;
-    for (int ty = r.by0 / kTile; ty <= r.by1 / kTile; ty++) {
-        for (int tx = r.bx0 / kTile; tx <= r.bx1 / kTile; tx++) {
-            atomicAdd(&cnt[ty * g.tiles_x + tx], 1u);
+    const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+    for (uint32_t t0 = 0; t0 < total; t0 += 64 * kBinPairs) {
+        uint32_t bin[kBinPairs], face[kBinPairs], slot[kBinPairs];
+#pragma unroll
+        for (uint32_t k = 0; k < kBinPairs; k++) {
+            const uint32_t t = t0 + k * 64 + lane;
+            uint32_t of = 0;  // the lanes whose pairs are all before t
+#pragma unroll
+            for (uint32_t step = 32; step >= 1; step >>= 1) {
+                of += (uint32_t)__shfl((int)incl, (int)(of + step - 1)) <= t ? step : 0u;
+            }
+            const uint32_t at = t - (uint32_t)__shfl((int)(incl - n), (int)of);
+            const uint32_t tw_of = (uint32_t)__shfl((int)tw, (int)of);
+            face[k] = (uint32_t)__shfl((int)f, (int)of);
+            const uint32_t ty = at / tw_of;
+            bin[k] = (uint32_t)__shfl((int)first, (int)of) + ty * g.tiles_x + (at - ty * tw_of);
+            slot[k] = t < total ? atomicAdd(&b.counts[bin[k]], 1u) : 0u;
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < kBinPairs; k++) {
+            if (t0 + k * 64 + lane < total) {
+                hard_append(b, bin[k], face[k], slot[k]);
+            }
         }
     }
 }
 
-int launch_hard_setup(hipStream_t s, const RasterGeom& g, const float* clip, uint32_t n_verts,
-                      const int32_t* faces, HardRec* recs) {
+int launch_hard_setup_bin(hipStream_t s, const RasterGeom& g, const float* clip, uint32_t n_verts,
+                          const float* faces, const int32_t* faces_i, int gl,
+                          const HardBinBuffers& b, uint32_t* err, HardRec* recs) {
     const uint32_t n = g.n_views * g.n_faces;
-    hipLaunchKernelGGL(k_hard_setup, dim3(div_up(n, 256)), dim3(256), 0, s, g,
-                       (const float4*)clip, n_verts, faces, recs);
-    DRESSI_CHECK_LAUNCH();
+    if (n) {
+        hipLaunchKernelGGL(k_hard_setup_bin, dim3(div_up(n, 256)), dim3(256), 0, s, g,
+                           (const float4*)clip, n_verts, faces, faces_i, gl, b, err, recs);
+        DRESSI_CHECK_LAUNCH();
+    }
     return DRESSI_OK;
 }
 
@@ -255,9 +176,11 @@ int launch_hard_setup(hipStream_t s, const RasterGeom& g, const float* clip, uin
 // A wave folds only the records whose bbox meets its block, found by one
 // test per lane and a ballot; with each wave walking all of the tile's
 // records the raster of four 1280 x 720 views of 20 480 faces took 71 us,
-// now 58: what is left is each tile's chain of dependent loads.
+// now 58: what is left is each tile's chain of dependent loads (a list's
+// first entries are read beside its count).
 __global__ __launch_bounds__(kTileThreads) void k_raster_hard(RasterGeom g, const HardRec* recs,
-                                                              BinBuffers b, const float* attr,
+                                                              HardBinBuffers b,
+                                                              const float* attr,
                                                               uint32_t n_comp, int mode,
                                                               float* out, size_t attr_view,
                                                               float* ids, uint32_t n_attr) {
@@ -272,18 +195,35 @@ __global__ __launch_bounds__(kTileThreads) void k_raster_hard(RasterGeom g, cons
     const int py = by + (int)(lane >> 3);
     const HardRec* vrec = recs + (size_t)view * g.n_faces;
     uint64_t best = kEmptyKey;
-    const uint32_t beg = b.offsets[view * g.n_tiles + tile];
-    const uint32_t end = b.offsets[view * g.n_tiles + tile + 1];
-    // a list that overflowed the capacity: every face of the view
-    const bool implicit = end > b.cap;
-    const uint32_t n = implicit ? g.n_faces : end - beg;
+    const uint32_t bin = view * g.n_tiles + tile;
+    const uint32_t* list = b.list + (size_t)bin * b.cap;
+    const uint32_t first = threadIdx.x < b.cap ? list[threadIdx.x] : 0u;
+    const uint32_t n_bin = b.counts[bin];
+    const uint32_t n_list = n_bin < b.cap ? n_bin : b.cap;
+    const uint32_t n_over = n_bin > b.cap ? *b.n_over : 0u;
+    // an overflow that overflowed: every face of the view
+    const bool implicit = n_over > b.over_cap;
+    const uint32_t n = implicit ? g.n_faces : n_list + n_over;
     for (uint32_t base = 0; base < n; base += kTileThreads) {
         const uint32_t cnt = (n - base) < (uint32_t)kTileThreads ? (n - base) : kTileThreads;
         __syncthreads();
         if (threadIdx.x < cnt) {
-            const uint32_t f = implicit ? base + threadIdx.x : b.list[beg + base + threadIdx.x];
-            lds_face[threadIdx.x] = f;
-            lds_rec[threadIdx.x] = vrec[f];
+            const uint32_t at = base + threadIdx.x;
+            uint2 e = make_uint2(bin, at);
+            if (!implicit) {
+                if (at >= n_list) {
+                    e = b.over[at - n_list];
+                } else {
+                    e.y = base == 0 ? first : list[at];
+                }
+            }
+            if (e.x == bin) {
+                lds_face[threadIdx.x] = e.y;
+                lds_rec[threadIdx.x] = vrec[e.y];
+            } else {
+                lds_rec[threadIdx.x].bx0 = 1 << 30;  // another tile's: meets no block
+                lds_rec[threadIdx.x].bx1 = -1;
+            }
         }
         __syncthreads();
         for (uint32_t q = 0; q < cnt; q += 64) {
@@ -351,7 +291,7 @@ __global__ __launch_bounds__(kTileThreads) void k_raster_hard(RasterGeom g, cons
 }
 
 int launch_raster_hard(hipStream_t s, const RasterGeom& g, const HardRec* recs,
-                       const BinBuffers& b, const float* attr, uint32_t n_comp, int mode,
+                       const HardBinBuffers& b, const float* attr, uint32_t n_comp, int mode,
                        float* out, size_t attr_view, float* ids, uint32_t n_attr) {
     hipLaunchKernelGGL(k_raster_hard, dim3(g.n_tiles, g.n_views), dim3(kTileThreads), 0, s, g,
                        recs, b, attr, n_comp, mode, out, attr_view, ids, n_attr);
@@ -761,36 +701,28 @@ int dressi_rasterize_soft_noalloc(dressi_ctx* ctx, const float* soft_clip, const
 // The per-op hard raster's workspaces.
 struct HardBins {
     HardRec* recs = nullptr;
-    BinBuffers b;
+    HardBinBuffers b;
 };
 
 static int hard_bins(dressi_ctx* ctx, const RasterGeom& g, HardBins* hb) {
-    const uint32_t cap = default_bin_cap(g, 8);
+    const HardBinSizes z = hard_bin_sizes(g);
     void *recs = nullptr, *bins = nullptr;
     const size_t nf1 = g.n_faces ? g.n_faces : 1;
     if (int rc = ctx_workspace(ctx, 0, sizeof(HardRec) * nf1 * g.n_views, &recs)) return rc;
-    if (int rc = ctx_workspace(ctx, 1, bin_bytes(g.n_tiles * g.n_views, cap), &bins)) return rc;
+    if (int rc = ctx_workspace(ctx, 1, z.bytes, &bins)) return rc;
     hb->recs = (HardRec*)recs;
-    bin_carve(bins, g.n_tiles * g.n_views, cap, &hb->b);
+    hard_bin_carve(bins, z, &hb->b);
     return DRESSI_OK;
 }
 
-// Setup, binning and raster; hb.b.counts are zero.
+// Setup, binning and raster; hb.b.counts and n_over (behind them) are zero.
 static int launch_hard_op(dressi_ctx* ctx, const RasterGeom& g, const HardBins& hb,
                           const float* clip, uint32_t n_verts, const float* faces,
                           const int32_t* faces_i, int gl, const float* attr, uint32_t n_comp,
                           int mode, float* out, size_t attr_view, float* ids,
                           uint32_t n_attr = 1) {
-    if (g.n_faces) {
-        hipLaunchKernelGGL(k_hard_setup_count, dim3(div_up(g.n_views * g.n_faces, 256)), dim3(256),
-                           0, ctx->stream, g, (const float4*)clip, n_verts, faces, faces_i, gl,
-                           hb.b, ctx->d_err, hb.recs);
-        DRESSI_CHECK_LAUNCH();
-    }
-    if (int rc = launch_scan_bins(ctx->stream, hb.b)) return rc;
-    if (g.n_faces) {
-        if (int rc = launch_bin_hard(ctx->stream, g, hb.recs, hb.b)) return rc;
-    }
+    if (int rc = launch_hard_setup_bin(ctx->stream, g, clip, n_verts, faces, faces_i, gl, hb.b,
+                                       ctx->d_err, hb.recs)) return rc;
     return launch_raster_hard(ctx->stream, g, hb.recs, hb.b, attr, n_comp, mode, out, attr_view,
                               ids, n_attr);
 }
@@ -814,7 +746,7 @@ static int rasterize_hard_common(dressi_ctx* ctx, const float* clip, uint32_t n_
     const RasterGeom g = make_geom(width, height, n_items, n_faces);
     HardBins hb;
     if (int rc = hard_bins(ctx, g, &hb)) return rc;
-    if (int rc = launch_zero(ctx->stream, hb.b.counts, sizeof(uint32_t) * g.n_tiles * n_items))
+    if (int rc = launch_zero(ctx->stream, hb.b.counts, sizeof(uint32_t) * (hb.b.n_bins + 1)))
         return rc;
     return launch_hard_op(ctx, g, hb, clip, n_verts, faces, nullptr, 0, attr,
                           mode == 1 ? 1 : n_comp, mode, out, attr_view, ids);
@@ -860,9 +792,9 @@ int dressi_surface_rasterize(dressi_ctx* ctx, const float* pos, uint32_t n_verts
     const RasterGeom g = make_geom(width, height, n_items, n_faces);
     HardBins hb;
     if (int rc = hard_bins(ctx, g, &hb)) return rc;
-    const uint32_t n_prep = std::max(n_verts * n_items, g.n_tiles * n_items);
+    const uint32_t n_prep = std::max(n_verts * n_items, hb.b.n_bins + 1);
     hipLaunchKernelGGL(k_surface_prep, dim3(div_up(n_prep, 256)), dim3(256), 0, ctx->stream,
-                       (const float4*)pos, n_verts * n_items, hb.b.counts, g.n_tiles * n_items,
+                       (const float4*)pos, n_verts * n_items, hb.b.counts, hb.b.n_bins + 1,
                        (float4*)clip_vk);
     DRESSI_CHECK_LAUNCH();
     return launch_hard_op(ctx, g, hb, pos, n_verts, nullptr, faces, 1, pos, 4, 2, rast,
@@ -939,7 +871,7 @@ int raster_attrs(dressi_ctx* ctx, const float* clip, uint32_t n_verts, uint32_t 
     const RasterGeom g = make_geom(width, height, n_views, n_faces);
     HardBins hb;
     if (int rc = hard_bins(ctx, g, &hb)) return rc;
-    if (int rc = launch_zero(ctx->stream, hb.b.counts, sizeof(uint32_t) * g.n_tiles * n_views))
+    if (int rc = launch_zero(ctx->stream, hb.b.counts, sizeof(uint32_t) * (hb.b.n_bins + 1)))
         return rc;
     return launch_hard_op(ctx, g, hb, clip, n_verts, faces, nullptr, 0, attr, 4, 0, out,
                           (size_t)n_verts * 4, nullptr, n_views > 1 ? 1 : n_attr);

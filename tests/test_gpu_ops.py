@@ -234,6 +234,31 @@ def test_raster_edge_cases(ctx, oracle):
     ctx.synchronize()
 
 
+@pytest.mark.parametrize("n,spread,size", [
+    (1500, 14, 1),     # one tile: its list of 512 is full, the rest in the overflow
+    (6000, 100, 12),   # small faces over 7 x 7 tiles: some lists full, some not
+    (2000, 100, 400),  # large ones: the overflow is full as well, every face is looked at
+])
+def test_raster_full_bins(ctx, oracle, n, spread, size):
+    """4096 x 4096 pixels, where a tile's list has 512 entries: more faces than that on a few
+    tiles, against the oracle and with the attribute raster beside the face ids."""
+    from opendressi_amd import ops
+    s = 4096
+    rng = np.random.default_rng(n)
+    print(f"[raster full bins] {n} faces of {size} px over {spread} px", flush=True)
+    at = 2000.0 + rng.random((n, 1, 2)) * spread
+    xy = np.clip(at + rng.standard_normal((n, 3, 2)) * size, 2000.0, 2001.0 + spread)
+    clip = np.concatenate([xy / s * 2.0 - 1.0, rng.random((n, 3, 1)), np.ones((n, 3, 1))], -1)
+    clip = clip.reshape(-1, 4).astype(np.float32)
+    faces = np.arange(3 * n, dtype=np.float32).reshape(n, 3)
+    attr = rng.random((3 * n, 2), dtype=np.float32)
+    ref = oracle.rasterize_face_id(clip, faces, s, s)
+    assert len(np.unique(ref)) > 20
+    _exact(host(ops.rasterize_face_id(ctx, dev(clip), dev(faces), s, s)), ref, "face id")
+    _exact(host(ops.rasterize(ctx, dev(clip), dev(attr), dev(faces), s, s)),
+           oracle.rasterize(clip, attr, faces, s, s), "attributes")
+
+
 def test_bad_indices_are_reported(ctx):
     import opendressi_amd as od
     from opendressi_amd import ops
