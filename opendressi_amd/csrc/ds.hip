@@ -2,6 +2,7 @@
 // backward of RasterizeSoft's dist channel w.r.t. the hard clip positions
 // (the backward RasterizeSoft builds, f_ops.cpp:1448-1455, and what
 // dressi.torch.rasterize_soft's VJP runs).
+#include <algorithm>
 #include <cstdint>
 
 #include "internal.h"
@@ -345,8 +346,10 @@ __global__ __launch_bounds__(64) void k_gather_dist_grad_faces(
 }
 
 // The torch surface's form: every item and peel, corner sums {N,K,F,3}
-// (x, y, w) for an adjacency of the same faces. A face's setup serves its
-// peels.
+// (x, y, w) for an adjacency of the same faces. A wave per face, item and
+// peel: what bounds is its chain of loads, and two peels in one wave after
+// one setup took 115 us for two 512 x 512 views of 5120 faces, side by side
+// 87.
 __global__ __launch_bounds__(64) void k_surface_soft_bwd_faces(
         const float4* gy, const float4* rs, uint32_t peels, const float4* pos, uint32_t n_verts,
         const float* faces, uint32_t n_faces, float radius, uint32_t w, uint32_t h,
@@ -366,7 +369,7 @@ __global__ __launch_bounds__(64) void k_surface_soft_bwd_faces(
          soft_bbox(fc, w, h, radius, &bx0, &by0, &bx1, &by1);
     const uint32_t bw = (uint32_t)(bx1 - bx0 + 1);
     const uint32_t n_px = ok ? bw * (uint32_t)(by1 - by0 + 1) : 0u;
-    for (uint32_t k = 0; k < peels; k++) {
+    for (uint32_t k = blockIdx.z; k < peels; k += gridDim.z) {
         const size_t layer = (size_t)blockIdx.y * peels + k;
         float acc = 0.f;
         if (n_px) {
@@ -534,8 +537,8 @@ extern "C" int dressi_surface_soft_bwd(dressi_ctx* ctx, const float* gy, const f
     if (!n_items || !n_rows) return DRESSI_OK;
     DRESSI_TRY_HIP(hipSetDevice(ctx->device));
     if (n_faces) {
-        hipLaunchKernelGGL(k_surface_soft_bwd_faces, dim3(n_faces, n_items), dim3(64), 0,
-                           ctx->stream, (const float4*)gy, (const float4*)rs, peels,
+        hipLaunchKernelGGL(k_surface_soft_bwd_faces, dim3(n_faces, n_items, std::min(peels, 16u)),
+                           dim3(64), 0, ctx->stream, (const float4*)gy, (const float4*)rs, peels,
                            (const float4*)pos, n_verts, faces, n_faces, radius_px, width, height,
                            g_corner);
         DRESSI_CHECK_LAUNCH();
