@@ -203,8 +203,15 @@ def col_sum(ctx: Context, x: torch.Tensor) -> torch.Tensor:
     return out
 
 
+def _vec4(t: torch.Tensor, name: str) -> None:
+    """The kernels read `t` as float4: any other row would be read past its end."""
+    if t.shape[-1] != 4:
+        raise ValueError(f"{name}: expected rows of 4 components, got {tuple(t.shape)}")
+
+
 def _batch_clip(clip: torch.Tensor, n: int) -> tuple[int, int]:
     """(n_verts, clip_per_item) of a (V, 4) shared or (N, V, 4) clip."""
+    _vec4(clip, "clip")
     if clip.dim() == 3:
         if clip.shape[0] != n:
             raise ValueError(f"clip: {clip.shape[0]} items for a batch of {n}")
@@ -216,9 +223,9 @@ def antialias_batch(ctx: Context, img: torch.Tensor, tri: torch.Tensor, clip: to
                     faces: torch.Tensor) -> torch.Tensor:
     """dressi_antialias_batch: img (N, H, W, C), tri (N, H, W), clip (V, 4)
     shared or (N, V, 4) -> (N, H, W, C); each item as antialias()."""
-    _prep(ctx)
     n, h, w, nc = img.shape
     nv, per_item = _batch_clip(clip, n)
+    _prep(ctx)
     out = torch.empty_like(img)
     check(lib.dressi_antialias_batch(ctx.handle, _ptr(img, "img"), nc, _ptr(tri, "tri"),
                                      _ptr(clip, "clip"), nv, per_item, _ptr(faces, "faces"),
@@ -229,9 +236,9 @@ def antialias_batch(ctx: Context, img: torch.Tensor, tri: torch.Tensor, clip: to
 def antialias_bwd_img_batch(ctx: Context, gy: torch.Tensor, tri: torch.Tensor,
                             clip: torch.Tensor, faces: torch.Tensor) -> torch.Tensor:
     """dressi_antialias_bwd_img_batch: gy (N, H, W, C) -> like gy."""
-    _prep(ctx)
     n, h, w, nc = gy.shape
     nv, per_item = _batch_clip(clip, n)
+    _prep(ctx)
     out = torch.empty_like(gy)
     check(lib.dressi_antialias_bwd_img_batch(ctx.handle, _ptr(gy, "gy"), nc, _ptr(tri, "tri"),
                                              _ptr(clip, "clip"), nv, per_item,
@@ -246,9 +253,9 @@ def antialias_bwd_vtx_batch(ctx: Context, gy: torch.Tensor, img: torch.Tensor,
                             wide: bool = True) -> torch.Tensor:
     """dressi_antialias_bwd_vtx_batch: gy, img (N, H, W, C), seeds (N,) ->
     (N, deg, V, 4) partials when n_samples > 0 and wide, else (N, V, 4)."""
-    _prep(ctx)
     n, h, w, nc = gy.shape
     nv, per_item = _batch_clip(clip, n)
+    _prep(ctx)
     deg = vtx_faces.shape[0]
     is_wide = bool(wide and n_samples > 0)
     out = torch.empty((n, deg if is_wide else 1, vtx_faces.shape[1], 4), dtype=torch.float32,
@@ -419,6 +426,7 @@ def surface_rasterize(ctx: Context, pos: torch.Tensor, faces: torch.Tensor, widt
                       height: int):
     """dressi_surface_rasterize: pos (N, V, 4), z in [-w, w]; faces (F, 3)
     int32 -> (rast (N, H, W, 4), pos with z in [0, w])."""
+    _vec4(pos, "pos")
     _prep(ctx)
     n, nv = pos.shape[0], pos.shape[1]
     clip_vk = torch.empty_like(pos)
@@ -448,6 +456,7 @@ def surface_interpolate_bwd(ctx: Context, gy: torch.Tensor, rast: torch.Tensor,
                             shared: bool) -> torch.Tensor:
     """dressi_surface_interpolate_bwd: gy (N, H, W, C), clip (N, V, 4) ->
     d/d attr (V, C) when `shared`, else (N, V, C)."""
+    _vec4(clip, "clip")
     _prep(ctx)
     n, h, w, nc = gy.shape
     deg, nv = vtx_faces.shape
@@ -466,9 +475,9 @@ def surface_antialias(ctx: Context, img: torch.Tensor, rast: torch.Tensor, pos: 
                       faces: torch.Tensor) -> torch.Tensor:
     """dressi_surface_antialias: img (N, H, W, C), rast (N, H, W, 4), pos
     (V, 4) shared or (N, V, 4) -> (N, H, W, C)."""
-    _prep(ctx)
     n, h, w, nc = img.shape
     nv, per_item = _batch_clip(pos, n)
+    _prep(ctx)
     out = torch.empty_like(img)
     check(lib.dressi_surface_antialias(ctx.handle, _ptr(img, "img"), nc, _ptr(rast, "rast"),
                                        _ptr(pos, "pos"), nv, per_item, _ptr(faces, "faces"),
@@ -479,9 +488,9 @@ def surface_antialias(ctx: Context, img: torch.Tensor, rast: torch.Tensor, pos: 
 def surface_antialias_bwd_img(ctx: Context, gy: torch.Tensor, rast: torch.Tensor,
                               pos: torch.Tensor, faces: torch.Tensor) -> torch.Tensor:
     """dressi_surface_antialias_bwd_img: gy (N, H, W, C) -> like gy."""
-    _prep(ctx)
     n, h, w, nc = gy.shape
     nv, per_item = _batch_clip(pos, n)
+    _prep(ctx)
     out = torch.empty_like(gy)
     check(lib.dressi_surface_antialias_bwd_img(
         ctx.handle, _ptr(gy, "gy"), nc, _ptr(rast, "rast"), _ptr(pos, "pos"), nv, per_item,
@@ -494,9 +503,9 @@ def surface_antialias_bwd_pos(ctx: Context, gy: torch.Tensor, img: torch.Tensor,
                               vtx_faces: torch.Tensor, seed: int, n_samples: int,
                               boost: float) -> torch.Tensor:
     """dressi_surface_antialias_bwd_pos: gy, img (N, H, W, C) -> (N, V, 4)."""
-    _prep(ctx)
     n, h, w, nc = gy.shape
     nv, per_item = _batch_clip(pos, n)
+    _prep(ctx)
     deg, rows = vtx_faces.shape
     nf = faces.shape[0]
     scratch = (torch.empty((n, nf, 9), dtype=torch.float32, device=gy.device)
@@ -513,6 +522,7 @@ def surface_rasterize_soft(ctx: Context, pos: torch.Tensor, faces: torch.Tensor,
                            height: int, radius_px: float, peels: int) -> torch.Tensor:
     """dressi_surface_rasterize_soft: pos (N, V, 4), z in [-w, w] ->
     (N, K, H, W, 4)."""
+    _vec4(pos, "pos")
     _prep(ctx)
     n, nv = pos.shape[0], pos.shape[1]
     out = torch.empty((n, peels, height, width, 4), dtype=torch.float32, device=pos.device)
@@ -529,6 +539,7 @@ def surface_soft_bwd(ctx: Context, gy: torch.Tensor, rs: torch.Tensor, pos: torc
                      faces: torch.Tensor, vtx_faces: torch.Tensor,
                      radius_px: float) -> torch.Tensor:
     """dressi_surface_soft_bwd: gy, rs (N, K, H, W, 4) -> (N, V, 4)."""
+    _vec4(pos, "pos")
     _prep(ctx)
     n, peels, h, w = rs.shape[:4]
     deg, rows = vtx_faces.shape
@@ -547,6 +558,7 @@ def surface_texture_bwd(ctx: Context, gy: torch.Tensor, pix_uv: torch.Tensor,
                         th: int) -> torch.Tensor:
     """dressi_surface_texture_bwd: gy (N, H, W, C), pix_uv (N, H, W, 2),
     vtx_uv (V, 2) or (N, V, 2), clip (1 or N, V, 4) -> d/d tex (th, tw, C)."""
+    _vec4(clip, "clip")
     _prep(ctx)
     n, h, w, nc = gy.shape
     nv = clip.shape[1]

@@ -61,6 +61,15 @@ def vertex_batch(t: torch.Tensor, name: str = "pos") -> torch.Tensor:
     return batched(t, 2, name, "V, C")
 
 
+def clip_batch(pos: torch.Tensor, device: torch.device) -> torch.Tensor:
+    """Clip positions [N, V, 4] on `device` from [V, 4] or [N, V, 4]. The
+    kernels read four components of each vertex, so no other count passes."""
+    pos_b = vertex_batch(to_dev(pos, device, "pos"))
+    if pos_b.shape[2] != 4:
+        raise ValueError(f"pos must have 4 components, got {pos_b.shape[2]}")
+    return pos_b
+
+
 def image_batch(t: torch.Tensor, name: str) -> torch.Tensor:
     """[N, H, W, C] from [H, W, C] or [N, H, W, C]."""
     return batched(t, 3, name, "H, W, C")

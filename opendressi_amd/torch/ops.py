@@ -19,10 +19,10 @@ from .. import ops as K
 from .context import RasterizeHipContext
 from .convert import (
     channels,
+    clip_batch,
     image_batch,
     resolution_hw,
     to_dev,
-    vertex_batch,
 )
 from .provenance import InterpOrigin, RasterOrigin, origin, stamp
 
@@ -57,9 +57,7 @@ def rasterize(ctx: RasterizeHipContext, pos: torch.Tensor, tri: torch.Tensor, re
         raise NotImplementedError("opendressi_amd.torch: range mode is not supported")
     del grad_db
     h, w = resolution_hw(resolution)
-    pos_b = vertex_batch(to_dev(pos, ctx.device, "pos"))
-    if pos_b.shape[2] != 4:
-        raise ValueError(f"pos must have 4 components, got {pos_b.shape[2]}")
+    pos_b = clip_batch(pos, ctx.device)
     md = ctx.mesh(tri)
     if md.n_verts > pos_b.shape[1]:
         raise IndexError(f"tri names vertex {md.n_verts - 1}, pos has {pos_b.shape[1]}")
@@ -206,7 +204,7 @@ def texture(tex, uv, uv_da=None, mip_level_bias=None, mip=None, filter_mode="aut
 
 def _batch_pos(pos: torch.Tensor, device) -> torch.Tensor:
     """Per-item clip positions (N, V, 4), or the one (V, 4) every item shares."""
-    pos_b = vertex_batch(to_dev(pos, device, "pos"))
+    pos_b = clip_batch(pos, device)
     return pos_b if pos_b.shape[0] > 1 else pos_b[0]
 
 
@@ -278,7 +276,7 @@ class _RasterizeSoftFn(torch.autograd.Function):
     @staticmethod
     def forward(fctx, pos, vctx, md, resolution, radius_px, peels):
         h, w = resolution
-        pos_b = vertex_batch(to_dev(pos, vctx.device, "pos"))
+        pos_b = clip_batch(pos, vctx.device)
         if md.n_verts > pos_b.shape[1]:
             raise IndexError(f"tri names vertex {md.n_verts - 1}, pos has {pos_b.shape[1]}")
         with vctx.lock:
@@ -293,7 +291,7 @@ class _RasterizeSoftFn(torch.autograd.Function):
         vctx, md, radius_px = fctx.dressi
         pos, out = fctx.saved_tensors
         dev = vctx.device
-        pos_b = vertex_batch(to_dev(pos, dev, "pos"))
+        pos_b = clip_batch(pos, dev)
         g = to_dev(grad_out, dev, "grad_out")
         with vctx.lock:
             g_pos = K.surface_soft_bwd(vctx._ctx, g, to_dev(out, dev, "out"), pos_b, md.faces_f,

@@ -1,6 +1,7 @@
 """Host-side logic of opendressi_amd.torch (no GPU): clip-space conventions,
 the gradient-sum order, provenance lifetime, argument checks."""
 import gc
+import threading
 import weakref
 
 import numpy as np
@@ -85,3 +86,67 @@ def test_vertex_adjacency_of_the_mesh_cache():
     assert vft[:, 2].tolist() == [0, 1, 2]
     assert vft[:, 0].tolist() == [0, -1, -1]
     assert vft[:, 3].tolist() == [1, 2, -1]
+
+
+class _Reached(Exception):
+    """Stands for a kernel launch."""
+
+
+def _host_context(monkeypatch):
+    """A context on the CPU whose launches raise _Reached."""
+    from types import SimpleNamespace
+
+    from opendressi_amd import ops as K
+    for name in [n for n in dir(K) if n.startswith(("surface_", "antialias"))]:
+        def launch(*args, **kw):
+            raise _Reached
+        monkeypatch.setattr(K, name, launch)
+    md = SimpleNamespace(n_verts=3, n_faces=1, faces_f=None, faces_i=None, vft=None)
+    return SimpleNamespace(device=torch.device("cpu"), _ctx=None, lock=threading.RLock(),
+                           mesh=lambda tri: md, engine=lambda key, build: build())
+
+
+@pytest.mark.parametrize("comps", [1, 2, 3, 5])
+@pytest.mark.parametrize("batched", [False, True])
+def test_positions_of_another_width_are_refused(monkeypatch, comps, batched):
+    """The kernels read a vertex as four floats: positions of any other width are refused before
+    one runs, by every op that takes them; four pass."""
+    import opendressi_amd.torch as dr
+    ctx = _host_context(monkeypatch)
+    tri = torch.tensor([[0, 1, 2]])
+    rast = torch.zeros(1, 4, 6, 4)
+    provenance.stamp(rast, provenance.RasterOrigin(clip_vk=None, tri=tri, resolution=(4, 6),
+                                                   ctx=ctx))
+    color = torch.zeros(1, 4, 6, 3)
+    calls = [lambda p: dr.rasterize(ctx, p, tri, [4, 6]),
+             lambda p: dr.rasterize_soft(ctx, p, tri, [4, 6]),
+             lambda p: dr.antialias(color, rast, p, tri)]
+    shape = (1, 3) if batched else (3,)
+    for call in calls:
+        with pytest.raises(ValueError, match="4 components"):
+            call(torch.zeros(*shape, comps))
+        with pytest.raises(_Reached):
+            call(torch.zeros(*shape, 4))
+
+
+@pytest.mark.parametrize("comps", [3, 5])
+def test_op_positions_of_another_width_are_refused(comps):
+    """The same for the entry points below, before they touch the context."""
+    from opendressi_amd import ops as K
+    p, img, rast = torch.zeros(2, 3, comps), torch.zeros(2, 4, 6, 3), torch.zeros(2, 4, 6, 4)
+    f, vf, uv = torch.zeros(1, 3), torch.zeros(1, 3), torch.zeros(2, 4, 6, 2)
+    rs = torch.zeros(2, 1, 4, 6, 4)
+    for call in (lambda: K.surface_rasterize(None, p, f.int(), 6, 4),
+                 lambda: K.surface_rasterize_soft(None, p, f, 6, 4, 3.0, 1),
+                 lambda: K.surface_soft_bwd(None, rs, rs, p, f, vf, 3.0),
+                 lambda: K.surface_interpolate_bwd(None, img, rast, p, f, vf, True),
+                 lambda: K.surface_texture_bwd(None, img, uv, torch.zeros(3, 2), p, f, 8, 8),
+                 lambda: K.surface_antialias(None, img, rast, p, f),
+                 lambda: K.surface_antialias_bwd_img(None, img, rast, p, f),
+                 lambda: K.surface_antialias_bwd_pos(None, img, img, rast, p, f, vf, 1, 8, 1.0),
+                 lambda: K.antialias_batch(None, img, rast[..., 3], p, f),
+                 lambda: K.antialias_bwd_img_batch(None, img, rast[..., 3], p, f),
+                 lambda: K.antialias_bwd_vtx_batch(None, img, img, rast[..., 3], p, f, vf, None, 8,
+                                                   True)):
+        with pytest.raises(ValueError, match="4 components"):
+            call()
