@@ -25,6 +25,13 @@ def _ptr(t: torch.Tensor | None, name: str) -> C.c_void_p:
     return C.c_void_p(t.data_ptr())
 
 
+def _ptr_i32(t: torch.Tensor, name: str) -> C.c_void_p:
+    if t.dtype != torch.int32 or not t.is_contiguous() or t.device.type != "cuda":
+        raise ValueError(f"{name}: expected a contiguous int32 device tensor, got "
+                         f"{t.dtype} {tuple(t.shape)} on {t.device}")
+    return C.c_void_p(t.data_ptr())
+
+
 def _prep(ctx: Context) -> None:
     ctx.use_torch_stream()
 
@@ -427,13 +434,14 @@ def surface_rasterize(ctx: Context, pos: torch.Tensor, faces: torch.Tensor, widt
     """dressi_surface_rasterize: pos (N, V, 4), z in [-w, w]; faces (F, 3)
     int32 -> (rast (N, H, W, 4), pos with z in [0, w])."""
     _vec4(pos, "pos")
+    faces_ptr = _ptr_i32(faces, "faces")
     _prep(ctx)
     n, nv = pos.shape[0], pos.shape[1]
     clip_vk = torch.empty_like(pos)
     rast = torch.empty((n, height, width, 4), dtype=torch.float32, device=pos.device)
     check(lib.dressi_surface_rasterize(ctx.handle, _ptr(pos, "pos"), nv, n,
-                                       C.c_void_p(faces.data_ptr()), faces.shape[0], width,
-                                       height, _ptr(clip_vk, "clip"), _ptr(rast, "rast")))
+                                       faces_ptr, faces.shape[0], width, height,
+                                       _ptr(clip_vk, "clip"), _ptr(rast, "rast")))
     return rast, clip_vk
 
 

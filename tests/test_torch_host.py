@@ -150,3 +150,14 @@ def test_op_positions_of_another_width_are_refused(comps):
                                                    True)):
         with pytest.raises(ValueError, match="4 components"):
             call()
+
+
+@pytest.mark.parametrize("faces", [torch.zeros(2, 3), torch.zeros(2, 3, dtype=torch.int64),
+                                   torch.zeros(3, 2, dtype=torch.int32).t(),
+                                   torch.zeros(2, 3, dtype=torch.int32)])
+def test_rasterize_faces_are_checked(faces):
+    """Float or 64-bit ids, strided ones and a host tensor are refused before the context is
+    touched: the kernel would read other memory."""
+    from opendressi_amd import ops as K
+    with pytest.raises(ValueError, match="faces: expected a contiguous int32 device tensor"):
+        K.surface_rasterize(None, torch.zeros(1, 3, 4), faces, 6, 4)
