@@ -449,8 +449,10 @@ def surface_interpolate(ctx: Context, attr: torch.Tensor, rast: torch.Tensor,
                         faces: torch.Tensor) -> torch.Tensor:
     """dressi_surface_interpolate: attr (V, C) shared or (N, V, C), rast
     (N, H, W, 4), faces (F, 3) float ids -> (N, H, W, C)."""
-    _prep(ctx)
     n, h, w = rast.shape[:3]
+    if attr.dim() == 3 and attr.shape[0] != n:
+        raise ValueError(f"attr: {attr.shape[0]} items for a batch of {n}")
+    _prep(ctx)
     nv, nc = attr.shape[-2], attr.shape[-1]
     out = torch.empty((n, h, w, nc), dtype=torch.float32, device=rast.device)
     check(lib.dressi_surface_interpolate(ctx.handle, _ptr(attr, "attr"), nv, nc,

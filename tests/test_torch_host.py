@@ -161,3 +161,13 @@ def test_rasterize_faces_are_checked(faces):
     from opendressi_amd import ops as K
     with pytest.raises(ValueError, match="faces: expected a contiguous int32 device tensor"):
         K.surface_rasterize(None, torch.zeros(1, 3, 4), faces, 6, 4)
+
+
+@pytest.mark.parametrize("items", [1, 2, 4])
+def test_interpolate_items_are_checked(items):
+    """Per-item attributes of another batch than the raster's are refused before the context is
+    touched: item i's would be read past their end, or another item's."""
+    from opendressi_amd import ops as K
+    with pytest.raises(ValueError, match=f"{items} items for a batch of 3"):
+        K.surface_interpolate(None, torch.zeros(items, 5, 2), torch.zeros(3, 4, 6, 4),
+                              torch.zeros(1, 3))
