@@ -211,3 +211,26 @@ def test_surface_texture_bwd(ctx, n, h, w, tw, th, nc, shared):
     _same(got, sum_contribs(parts), "texture gradient")
     assert float(got.abs().max()) > 0 or h == 1
     ctx.synchronize()
+
+
+@pytest.mark.parametrize("sw,sh", [(0, 4), (4, 0), (0, 0), (1, 1)])
+def test_texture_bwd_of_an_empty_screen(ctx, sw, sh):
+    """GatherByInverseUV of a screen without columns or rows, through the C entry point (a torch
+    tensor without elements has no address): anchors everywhere, yet zeros and no read; one pixel
+    finds its texel."""
+    from opendressi_amd import _lib as L
+    print(f"[texture bwd] empty screen {sw}x{sh}", flush=True)
+    tw, th, nc = 5, 3, 3
+    gy = torch.full((4, 4, nc), 7.0, device="cuda")
+    uv = torch.full((4, 4, 2), 0.5, device="cuda")
+    inv = torch.tensor([0.5, 1.5, 1.0, 0.0], device="cuda").repeat(th, tw, 1)
+    out = torch.full((th, tw, nc), 3.0, device="cuda")
+    ctx.use_torch_stream()
+    p = lambda t: L.C.c_void_p(t.data_ptr())
+    L.check(L.lib.dressi_texture_nearest_bwd(ctx.handle, p(gy), nc, sw, sh, p(inv), tw, th, p(uv),
+                                             p(out)))
+    ref = torch.zeros_like(out)
+    if sw and sh:
+        ref[1, 2] = 7.0  # uv (0.5, 0.5)
+    _same(out, ref, "out")
+    ctx.synchronize()
