@@ -1286,7 +1286,7 @@ int dressi_hsr_render_targets(dressi_hsr_plan* p, const float* tgt_pos, uint32_t
     DRESSI_TRY_HIP(hipMemcpyAsync(ones, one.data(), one.size() * 4, hipMemcpyHostToDevice, s));
     HardBinBuffers b;
     hard_bin_carve(bins, z, &b);
-    if (int rc = launch_zero(s, b.counts, sizeof(uint32_t) * (z.n_bins + 1))) return rc;
+    if (int rc = launch_zero(s, b.counts, b.clear_bytes())) return rc;
     if (int rc = launch_hard_setup_bin(s, g, (const float*)dclip, n_tverts, nullptr,
                                        (const int32_t*)dfi, 0, b, nullptr, (HardRec*)recs))
         return rc;

@@ -150,17 +150,22 @@ struct BinBuffers {
     uint32_t n_bins = 0;
 };
 
-// The hard rasterizer's: counts and n_over (one word behind them) are cleared
-// before each use; faces that find their bin's list full go to `over`.
+// The hard rasterizer's: a bin's first `cap` faces are in its list, those that
+// find it full in one of its kHardChains chains through `over`. The words from
+// `counts` on (n_bins + 2) are cleared before each use.
+constexpr uint32_t kHardChains = 64;
 struct HardBinBuffers {
     uint32_t* counts = nullptr;  // [n_bins]
-    uint32_t* n_over = nullptr;  // counts + n_bins
-    uint2* over = nullptr;       // [over_cap] (bin, face)
+    uint32_t* n_over = nullptr;  // entries of `over` taken
+    uint32_t* spilt = nullptr;   // != 0: `over` was full, some faces are nowhere
+    uint2* over = nullptr;       // [over_cap] (face, the chain's entry before)
+    uint32_t* heads = nullptr;   // [n_bins][kHardChains] a chain's last entry
     uint32_t* list = nullptr;    // [n_bins][cap] face indices
     uint32_t cap = 0, over_cap = 0, n_bins = 0;
+    size_t clear_bytes() const { return sizeof(uint32_t) * ((size_t)n_bins + 2); }
 };
 struct HardBinSizes {
-    uint32_t n_bins, cap, over_cap;
+    uint32_t n_bins, cap, over_cap;  // over_cap 0: a list holds the whole mesh
     size_t bytes;
 };
 

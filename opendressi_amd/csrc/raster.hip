@@ -12,21 +12,34 @@ namespace dressi {
 // Binning
 // ---------------------------------------------------------------------------
 
-// Entries of the hard bins' lists together (128 MB): a bin has room for the
-// whole mesh up to there, and at least kHardBinMin.
-constexpr uint64_t kHardListEntries = 32ull << 20;
-constexpr uint32_t kHardBinMin = 16;
+// A hard bin's list holds kHardBinShare times the faces that a bin would have
+// if every view's were spread evenly over its tiles, and kHardBinMin more: a
+// closed mesh that fills a third of the screen has about four times that
+// share on a tile and up to eleven at its limb. Small problems get what
+// kHardListEntries (16 MB) have room for, so that none of their lists fills up.
+// The overflow takes kHardOverShare entries per face and view. Four 1280 x 720
+// views of 20 480 faces take 23 MB, 64 of 1024 x 1024 and 81 920 faces 437 MB
+// (their records 6.6 and 419).
+constexpr uint64_t kHardBinShare = 8, kHardBinMin = 32, kHardOverShare = 4;
+constexpr uint64_t kHardListEntries = 4ull << 20;
+// Neither grows past these (4 GB each); a list keeps at least 16 entries.
+constexpr uint64_t kHardListMax = 1ull << 30, kHardOverMax = 1ull << 29;
 
 HardBinSizes hard_bin_sizes(const RasterGeom& g) {
     const uint64_t n_bins = (uint64_t)g.n_tiles * g.n_views;
+    const uint64_t faces = std::max<uint64_t>(g.n_faces, 1);
+    uint64_t cap = std::max(kHardBinMin + kHardBinShare * faces / g.n_tiles,
+                            kHardListEntries / n_bins);
+    cap = std::min(cap, std::max<uint64_t>(kHardListMax / n_bins, 16));
+    cap = std::min(cap, faces);
     HardBinSizes z;
     z.n_bins = (uint32_t)n_bins;
-    z.cap = (uint32_t)std::min<uint64_t>(
-            std::max<uint64_t>(kHardListEntries / n_bins, kHardBinMin),
-            std::max<uint64_t>(g.n_faces, 1));
-    z.over_cap = (uint32_t)std::min<uint64_t>((uint64_t)g.n_faces * g.n_views * 8 + 4096,
-                                              0x3fffffffull);
-    z.bytes = sizeof(uint32_t) * (n_bins + 2 + 2 * (size_t)z.over_cap + n_bins * z.cap) + 256;
+    z.cap = (uint32_t)cap;
+    z.over_cap = cap == faces ? 0u
+                              : (uint32_t)std::min(faces * g.n_views * kHardOverShare + 4096,
+                                                   kHardOverMax);
+    z.bytes = sizeof(uint32_t) * (n_bins + 4 + 2 * (size_t)z.over_cap +
+                                  n_bins * (cap + (z.over_cap ? kHardChains : 0u)));
     return z;
 }
 
@@ -34,9 +47,13 @@ void hard_bin_carve(void* base, const HardBinSizes& z, HardBinBuffers* b) {
     uint32_t* p = (uint32_t*)base;
     b->counts = p;
     b->n_over = p + z.n_bins;
-    const size_t at = ((size_t)z.n_bins + 2) & ~(size_t)1;  // pairs: 8-byte aligned
-    b->over = (uint2*)(p + at);
-    b->list = p + at + 2 * (size_t)z.over_cap;
+    b->spilt = b->n_over + 1;
+    p += ((size_t)z.n_bins + 3) & ~(size_t)1;  // pairs: 8-byte aligned
+    b->over = (uint2*)p;
+    p += 2 * (size_t)z.over_cap;
+    b->heads = p;
+    p += z.over_cap ? (size_t)z.n_bins * kHardChains : 0;
+    b->list = p;
     b->cap = z.cap;
     b->over_cap = z.over_cap;
     b->n_bins = z.n_bins;
@@ -46,24 +63,10 @@ void hard_bin_carve(void* base, const HardBinSizes& z, HardBinBuffers* b) {
 // Hard rasterizer (Rasterize / RasterizeFaceId)
 // ---------------------------------------------------------------------------
 
-// Adds face f to bin `bin`: to its list, or to the overflow that every tile
-// with a full list looks through.
-__device__ __forceinline__ void hard_append(const HardBinBuffers& b, uint32_t bin, uint32_t f,
-                                            uint32_t slot) {
-    if (slot < b.cap) {
-        b.list[(size_t)bin * b.cap + slot] = f;
-        return;
-    }
-    const uint32_t o = atomicAdd(b.n_over, 1u);
-    if (o < b.over_cap) {
-        b.over[o] = make_uint2(bin, f);
-    }
-}
-
 // Setup and binning, a thread per (view, face), from the reference's float
 // face ids (decoded as RasterizeCore does, uint32_t(int64_t(x)); a bad one is
 // reported) or from int32 ones. `gl`: clip z in [-w, w], remapped to
-// 0.5 (z + w). b.counts and b.n_over are zero.
+// 0.5 (z + w). b's counters are zero.
 //
 // Lists of a fixed size take a face where it is set up. With lists sized by a
 // count and a scan (the form before) a raster had two launches more: 17 + 15
@@ -72,6 +75,14 @@ __device__ __forceinline__ void hard_append(const HardBinBuffers& b, uint32_t bi
 // a lane has kBinPairs of them on their way at once (a thread that goes
 // through its own face's tiles, four at a time: 50 us). The lists' size makes
 // no difference there (128 entries or the whole mesh).
+//
+// What finds its list full goes to chains of its own bin, which its tile then
+// reads side by side, so that the work stays linear in the views (one overflow
+// for all tiles, as it was before, took 33 ms for 64 1024 x 1024 views of
+// 81 920 faces, which now take 2.3, and 169 ms for 128 of 512 x 512, now 4.3;
+// counted, scanned and filled lists 4.1 and 6.7). Where nearly everything
+// overflows, a mesh on nine tiles of each of 64 512 x 512 views: 7.6 ms, the
+// scanned lists 9.7.
 constexpr uint32_t kBinPairs = 4;
 
 __global__ __launch_bounds__(256) void k_hard_setup_bin(RasterGeom g, const float4* clip,
@@ -145,10 +156,39 @@ __global__ __launch_bounds__(256) void k_hard_setup_bin(RasterGeom g, const floa
             bin[k] = (uint32_t)__shfl((int)first, (int)of) + ty * g.tiles_x + (at - ty * tw_of);
             slot[k] = t < total ? atomicAdd(&b.counts[bin[k]], 1u) : 0u;
         }
+        uint64_t full[kBinPairs];  // the lanes whose bin's list is full
+        uint32_t n_full = 0;
 #pragma unroll
         for (uint32_t k = 0; k < kBinPairs; k++) {
-            if (t0 + k * 64 + lane < total) {
-                hard_append(b, bin[k], face[k], slot[k]);
+            const bool in = t0 + k * 64 + lane < total;
+            if (in && slot[k] < b.cap) {
+                b.list[(size_t)bin[k] * b.cap + slot[k]] = face[k];
+            }
+            full[k] = __ballot(in && slot[k] >= b.cap);
+            n_full += (uint32_t)__popcll(full[k]);
+        }
+        if (n_full) {
+            // Places in the overflow, one add for the wave's; then each into
+            // chain (slot - cap) % kHardChains of its bin. A chain's length
+            // follows from the bin's count, so heads need no initial value.
+            uint32_t at = 0;
+            if (lane == 0) {
+                at = atomicAdd(b.n_over, n_full);
+                if (at + n_full > b.over_cap) {
+                    *b.spilt = 1u;
+                }
+            }
+            at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at);
+#pragma unroll
+            for (uint32_t k = 0; k < kBinPairs; k++) {
+                const uint32_t o = at + (uint32_t)__popcll(full[k] & ((1ull << lane) - 1ull));
+                if ((full[k] >> lane & 1u) && o < b.over_cap) {
+                    const uint32_t chain = (slot[k] - b.cap) % kHardChains;
+                    b.over[o] = make_uint2(
+                            face[k],
+                            atomicExch(&b.heads[(size_t)bin[k] * kHardChains + chain], o));
+                }
+                at += (uint32_t)__popcll(full[k]);
             }
         }
     }
@@ -204,35 +244,12 @@ __global__ __launch_bounds__(kTileThreads) void k_raster_hard(RasterGeom g, cons
     const uint32_t first =
             threadIdx.x < kHardStage && threadIdx.x < b.cap ? list[threadIdx.x] : 0u;
     const uint32_t n_bin = b.counts[bin];
-    const uint32_t n_list = n_bin < b.cap ? n_bin : b.cap;
-    const uint32_t n_over = n_bin > b.cap ? *b.n_over : 0u;
-    // an overflow that overflowed: every face of the view
-    const bool implicit = n_over > b.over_cap;
-    const uint32_t n = implicit ? g.n_faces : n_list + n_over;
-    for (uint32_t base = 0; base < n; base += kHardStage) {
-        const uint32_t cnt = (n - base) < kHardStage ? (n - base) : kHardStage;
-        if (base) {
-            __syncthreads();
-        }
-        if (threadIdx.x < cnt) {
-            const uint32_t at = base + threadIdx.x;
-            uint2 e = make_uint2(bin, at);
-            if (!implicit) {
-                if (at >= n_list) {
-                    e = b.over[at - n_list];
-                } else {
-                    e.y = base == 0 ? first : list[at];
-                }
-            }
-            if (e.x == bin) {
-                lds_face[threadIdx.x] = e.y;
-                lds_rec[threadIdx.x] = vrec[e.y];
-            } else {
-                lds_rec[threadIdx.x].bx0 = 1 << 30;  // another tile's: meets no block
-                lds_rec[threadIdx.x].bx1 = -1;
-            }
-        }
-        __syncthreads();
+    // a full list and a full overflow: every face of the view
+    const bool full = n_bin > b.cap;
+    const bool implicit = full && *b.spilt;
+    const uint32_t n_list = implicit ? g.n_faces : full ? b.cap : n_bin;
+    // folds the `cnt` staged records
+    const auto fold = [&](uint32_t cnt) {
         for (uint32_t q = 0; q < cnt; q += 64) {
             const HardRec& mine = lds_rec[q + lane < cnt ? q + lane : q];
             uint64_t m = __ballot(q + lane < cnt && mine.bx0 <= bx + 7 && mine.bx1 >= bx &&
@@ -241,6 +258,41 @@ __global__ __launch_bounds__(kTileThreads) void k_raster_hard(RasterGeom g, cons
                 const uint32_t j = q + (uint32_t)__builtin_ctzll(m);
                 hard_fragment(lds_rec[j], lds_face[j], px, py, &best);
             }
+        }
+    };
+    for (uint32_t base = 0; base < n_list; base += kHardStage) {
+        const uint32_t cnt = (n_list - base) < kHardStage ? (n_list - base) : kHardStage;
+        if (base) {
+            __syncthreads();
+        }
+        if (threadIdx.x < cnt) {
+            const uint32_t at = base + threadIdx.x;
+            const uint32_t f = implicit ? at : base == 0 ? first : list[at];
+            lds_face[threadIdx.x] = f;
+            lds_rec[threadIdx.x] = vrec[f];
+        }
+        __syncthreads();
+        fold(cnt);
+    }
+    if (full && !implicit) {
+        // the bin's chains side by side: entry r of chain c is its overflow
+        // face c + r kHardChains, counted from the chain's head
+        static_assert(kHardChains <= kHardStage, "a record staged per chain");
+        const uint32_t n_over = n_bin - b.cap;
+        uint32_t at = threadIdx.x < kHardChains && threadIdx.x < n_over
+                              ? b.heads[(size_t)bin * kHardChains + threadIdx.x]
+                              : 0u;
+        for (uint32_t base = 0; base < n_over; base += kHardChains) {
+            const uint32_t cnt = (n_over - base) < kHardChains ? (n_over - base) : kHardChains;
+            __syncthreads();
+            if (threadIdx.x < cnt) {
+                const uint2 e = b.over[at];
+                at = e.y;
+                lds_face[threadIdx.x] = e.x;
+                lds_rec[threadIdx.x] = vrec[e.x];
+            }
+            __syncthreads();
+            fold(cnt);
         }
     }
     if (px >= (int)g.width || py >= (int)g.height) {
@@ -722,7 +774,7 @@ static int hard_bins(dressi_ctx* ctx, const RasterGeom& g, HardBins* hb) {
     return DRESSI_OK;
 }
 
-// Setup, binning and raster; hb.b.counts and n_over (behind them) are zero.
+// Setup, binning and raster; hb.b's counters are zero.
 static int launch_hard_op(dressi_ctx* ctx, const RasterGeom& g, const HardBins& hb,
                           const float* clip, uint32_t n_verts, const float* faces,
                           const int32_t* faces_i, int gl, const float* attr, uint32_t n_comp,
@@ -753,7 +805,7 @@ static int rasterize_hard_common(dressi_ctx* ctx, const float* clip, uint32_t n_
     const RasterGeom g = make_geom(width, height, n_items, n_faces);
     HardBins hb;
     if (int rc = hard_bins(ctx, g, &hb)) return rc;
-    if (int rc = launch_zero(ctx->stream, hb.b.counts, sizeof(uint32_t) * (hb.b.n_bins + 1)))
+    if (int rc = launch_zero(ctx->stream, hb.b.counts, hb.b.clear_bytes()))
         return rc;
     return launch_hard_op(ctx, g, hb, clip, n_verts, faces, nullptr, 0, attr,
                           mode == 1 ? 1 : n_comp, mode, out, attr_view, ids);
@@ -799,9 +851,10 @@ int dressi_surface_rasterize(dressi_ctx* ctx, const float* pos, uint32_t n_verts
     const RasterGeom g = make_geom(width, height, n_items, n_faces);
     HardBins hb;
     if (int rc = hard_bins(ctx, g, &hb)) return rc;
-    const uint32_t n_prep = std::max(n_verts * n_items, hb.b.n_bins + 1);
+    const uint32_t n_clear = (uint32_t)(hb.b.clear_bytes() / sizeof(uint32_t));
+    const uint32_t n_prep = std::max(n_verts * n_items, n_clear);
     hipLaunchKernelGGL(k_surface_prep, dim3(div_up(n_prep, 256)), dim3(256), 0, ctx->stream,
-                       (const float4*)pos, n_verts * n_items, hb.b.counts, hb.b.n_bins + 1,
+                       (const float4*)pos, n_verts * n_items, hb.b.counts, n_clear,
                        (float4*)clip_vk);
     DRESSI_CHECK_LAUNCH();
     return launch_hard_op(ctx, g, hb, pos, n_verts, nullptr, faces, 1, pos, 4, 2, rast,
@@ -878,7 +931,7 @@ int raster_attrs(dressi_ctx* ctx, const float* clip, uint32_t n_verts, uint32_t 
     const RasterGeom g = make_geom(width, height, n_views, n_faces);
     HardBins hb;
     if (int rc = hard_bins(ctx, g, &hb)) return rc;
-    if (int rc = launch_zero(ctx->stream, hb.b.counts, sizeof(uint32_t) * (hb.b.n_bins + 1)))
+    if (int rc = launch_zero(ctx->stream, hb.b.counts, hb.b.clear_bytes()))
         return rc;
     return launch_hard_op(ctx, g, hb, clip, n_verts, faces, nullptr, 0, attr, 4, 0, out,
                           (size_t)n_verts * 4, nullptr, n_views > 1 ? 1 : n_attr);

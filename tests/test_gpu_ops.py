@@ -235,12 +235,14 @@ def test_raster_edge_cases(ctx, oracle):
 
 
 @pytest.mark.parametrize("n,spread,size", [
-    (1500, 14, 1),     # one tile: its list of 512 is full, the rest in the overflow
-    (6000, 100, 12),   # small faces over 7 x 7 tiles: some lists full, some not
-    (2000, 100, 400),  # large ones: the overflow is full as well, every face is looked at
+    (1500, 14, 1),     # one tile: its list of 64 is full, the rest in its chains
+    (70, 14, 1),       # six faces too many: chains of one entry, most of them empty
+    (900, 100, 3),     # small faces over 7 x 7 tiles: some lists full, some not
+    (6000, 100, 12),   # the overflow is full as well: a full tile looks at every face
+    (2000, 100, 400),  # large ones, each on every one of these tiles
 ])
 def test_raster_full_bins(ctx, oracle, n, spread, size):
-    """4096 x 4096 pixels, where a tile's list has 512 entries: more faces than that on a few
+    """4096 x 4096 pixels, where a tile's list has 64 entries: more faces than that on a few
     tiles, against the oracle and with the attribute raster beside the face ids."""
     from opendressi_amd import ops
     s = 4096
@@ -257,6 +259,77 @@ def test_raster_full_bins(ctx, oracle, n, spread, size):
     _exact(host(ops.rasterize_face_id(ctx, dev(clip), dev(faces), s, s)), ref, "face id")
     _exact(host(ops.rasterize(ctx, dev(clip), dev(attr), dev(faces), s, s)),
            oracle.rasterize(clip, attr, faces, s, s), "attributes")
+
+
+def _full_bin_view(rng, s, n, spread, size):
+    """n random faces of `size` pixels over `spread` pixels of an s x s screen, as clip corners."""
+    at = 0.4 * s + rng.random((n, 1, 2)) * spread
+    xy = np.clip(at + rng.standard_normal((n, 3, 2)) * size, 0.0, 1.01 * s)
+    clip = np.concatenate([xy / s * 2.0 - 1.0, rng.random((n, 3, 1)), np.ones((n, 3, 1))], -1)
+    return clip.reshape(-1, 4).astype(np.float32)
+
+
+@pytest.mark.parametrize("views", [
+    # (spread, size) per view of 1500 faces; lists of 85 entries, an overflow of 22 096 for all.
+    # Views without a full list beside one with a single full tile, before it and behind it
+    [(1600, 1), (14, 1), (1600, 1)],
+    # full tiles in every view, a few and many
+    [(14, 1), (60, 2), (30, 1)],
+    # the large faces of one view fill the overflow up: the full tiles of the others, too, look
+    # at every face of their own view
+    [(14, 1), (100, 400), (30, 1)],
+])
+def test_raster_full_bins_of_several_views(ctx, oracle, views):
+    """Lists, chains and the look at every face, in views of one batch: each view's ids and
+    attributes are the oracle's."""
+    from opendressi_amd import ops
+    s, n = 2048, 1500
+    print(f"[raster full bins] views {views}", flush=True)
+    rng = np.random.default_rng(len(views))
+    clip = np.stack([_full_bin_view(rng, s, n, *v) for v in views])
+    faces = np.arange(3 * n, dtype=np.float32).reshape(n, 3)
+    attr = rng.random((3 * n, 2), dtype=np.float32)
+    for _ in range(2):  # the second time over the first one's workspace
+        out, ids = ops.rasterize_batch(ctx, dev(clip), dev(attr), dev(faces), s, s,
+                                       with_face_id=True)
+    for i in range(len(views)):
+        ref = oracle.rasterize_face_id(clip[i], faces, s, s)
+        assert len(np.unique(ref)) > 20
+        _exact(host(ids[i]), ref, f"view {i} face id")
+        _exact(host(out[i]), oracle.rasterize(clip[i], attr, faces, s, s), f"view {i} attributes")
+    ctx.synchronize()
+
+
+def test_raster_time_of_a_batch(ctx):
+    """A full tile reads its own overflow alone: eight times the views take about eight times as
+    long (64 times, where each full tile looked through every view's)."""
+    import torch
+
+    import opendressi_amd as od
+    from opendressi_amd import ops
+    pos, faces = od.icosphere(6)
+    faces = dev(faces)
+    attr = dev(pos)
+
+    def pass_ms(n):
+        # a mesh on a few tiles of its view, whose lists it fills
+        mvp = od.orbit_cameras(1, n, 1)[0].reshape(n, 4, 4).astype(np.float64)
+        clip = np.concatenate([pos, np.ones((len(pos), 1))], 1)[None] @ mvp
+        clip[..., :2] *= 0.15
+        clip = dev(clip)
+        best = math.inf
+        for _ in range(4):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            ops.rasterize_batch(ctx, clip, attr, faces, 512, 512)
+            b.record()
+            torch.cuda.synchronize()
+            best = min(best, a.elapsed_time(b))
+        return best
+
+    few, many = pass_ms(8), pass_ms(64)
+    print(f"[raster batch] 8 views {few:.3f} ms, 64 views {many:.3f} ms", flush=True)
+    assert many < 20.0 * few
 
 
 def test_bad_indices_are_reported(ctx):
