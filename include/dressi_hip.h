@@ -522,14 +522,16 @@ int dressi_surface_soft_bwd(dressi_ctx* ctx, const float* gy, const float* rs, u
 
 /* texture (nearest), d/d tex {th,tw} VEC n_comp: gy {N,sh,sw} VEC n_comp,
  * pix_uv {N,sh,sw} VEC2, the mesh's uv {V} VEC2 (or {N,V}) and clip {V} VEC4
- * (or {N,V}). Scratch: uv_clip {V} or {N,V} VEC4, sattr {N,V} VEC4, inv_uv
- * {N,th,tw} VEC4, part {N,th,tw} VEC n_comp (N > 1). */
+ * (or {N,V}). The items go through `group` at a time. Scratch, with G =
+ * min(group, N): uv_clip {V} or {G,V} VEC4, sattr {G,V} VEC4, inv_uv {G,th,tw}
+ * VEC4, and part {N,th,tw} VEC n_comp (N > 1). */
 int dressi_surface_texture_bwd(dressi_ctx* ctx, const float* gy, uint32_t n_comp, uint32_t sw,
                                uint32_t sh, uint32_t n_items, const float* pix_uv,
                                const float* vtx_uv, int uv_per_item, const float* clip,
                                int clip_per_item, uint32_t n_verts, const float* faces,
-                               uint32_t n_faces, uint32_t tw, uint32_t th, float* uv_clip,
-                               float* sattr, float* inv_uv, float* part, float* out);
+                               uint32_t n_faces, uint32_t tw, uint32_t th, uint32_t group,
+                               float* uv_clip, float* sattr, float* inv_uv, float* part,
+                               float* out);
 
 /* ---- texture path (C3) ---- */
 /* F::TextureBilinear forward (src/core/f_ops.cpp:2736-2780, BilerpClamp

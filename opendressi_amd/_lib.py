@@ -116,7 +116,7 @@ _SIGS = {
     "dressi_surface_soft_bwd": (_I, [_P, _P, _P, _U, _P, _U, _U, _P, _U, _P, _U, _U, _F, _U, _U,
                                      _P, _P]),
     "dressi_surface_texture_bwd": (_I, [_P, _P, _U, _U, _U, _U, _P, _P, _I, _P, _I, _U, _P, _U, _U,
-                                        _U, _P, _P, _P, _P, _P]),
+                                        _U, _U, _P, _P, _P, _P, _P]),
     "dressi_equirect_sample": (_I, [_P, _P, _U, _U, _U, _P, _U, _U, _P]),
     "dressi_equirect_sample_bwd": (_I, [_P, _P, _U, _P, _U, _U, _U, _U, _P]),
     "dressi_avg_pool2x2": (_I, [_P, _P, _U, _U, _U, _P]),

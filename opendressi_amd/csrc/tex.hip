@@ -948,37 +948,47 @@ int dressi_surface_texture_bwd(dressi_ctx* ctx, const float* gy, uint32_t n_comp
                                uint32_t sh, uint32_t n_items, const float* pix_uv,
                                const float* vtx_uv, int uv_per_item, const float* clip,
                                int clip_per_item, uint32_t n_verts, const float* faces,
-                               uint32_t n_faces, uint32_t tw, uint32_t th, float* uv_clip,
-                               float* sattr, float* inv_uv, float* part, float* out) {
+                               uint32_t n_faces, uint32_t tw, uint32_t th, uint32_t group,
+                               float* uv_clip, float* sattr, float* inv_uv, float* part,
+                               float* out) {
     DRESSI_REQUIRE(ctx && gy && pix_uv && vtx_uv && clip && (faces || n_faces == 0) && uv_clip &&
                            sattr && inv_uv && (part || n_items <= 1) && out,
                    "texture backward: NULL buffer");
     DRESSI_REQUIRE(n_comp >= 1 && n_comp <= 4, "n_comp must be 1..4");
-    DRESSI_REQUIRE(n_items >= 1 && n_items <= kMaxBatchItems, "batch of %u items", n_items);
+    DRESSI_REQUIRE(n_items >= 1 && group >= 1 && group <= kMaxBatchItems,
+                   "batch of %u items in groups of %u", n_items, group);
+    group = std::min(group, n_items);
     DRESSI_REQUIRE(tw > 0 && th > 0 && (uint64_t)tw * th < (1ull << 31) &&
                            (uint64_t)sw * sh < (1ull << 31) &&
-                           (uint64_t)n_items * n_verts < (1ull << 31) &&
-                           (uint64_t)n_items * n_faces < (1ull << 31),
+                           (uint64_t)group * n_verts < (1ull << 31) &&
+                           (uint64_t)group * n_faces < (1ull << 31),
                    "size too large");
     DRESSI_TRY_HIP(hipSetDevice(ctx->device));
-    if (n_verts) {
-        hipLaunchKernelGGL(k_surface_tex_prep, dim3(div_up(n_items * n_verts, 256)), dim3(256), 0,
-                           ctx->stream, (const float2*)vtx_uv,
-                           uv_per_item ? n_items * n_verts : n_verts, (const float4*)clip, n_verts,
-                           n_items, clip_per_item ? (size_t)n_verts : (size_t)0, (float)sw,
-                           (float)sh, (float4*)uv_clip, (float4*)sattr);
+    const size_t npx = (size_t)sw * sh, n_tex = (size_t)tw * th * n_comp;
+    for (uint32_t i0 = 0; i0 < n_items; i0 += group) {
+        const uint32_t n = std::min(group, n_items - i0);
+        if (n_verts) {
+            const size_t v0 = (size_t)i0 * n_verts;
+            hipLaunchKernelGGL(k_surface_tex_prep, dim3(div_up(n * n_verts, 256)), dim3(256), 0,
+                               ctx->stream, (const float2*)vtx_uv + (uv_per_item ? v0 : 0),
+                               uv_per_item ? n * n_verts : n_verts,
+                               (const float4*)clip + (clip_per_item ? v0 : 0), n_verts, n,
+                               clip_per_item ? (size_t)n_verts : (size_t)0, (float)sw, (float)sh,
+                               (float4*)uv_clip, (float4*)sattr);
+            DRESSI_CHECK_LAUNCH();
+        }
+        if (int rc = raster_attrs(ctx, uv_clip, n_verts, uv_per_item ? n : 1, sattr, n, faces,
+                                  n_faces, tw, th, inv_uv)) return rc;
+        hipLaunchKernelGGL(k_gather_nearest_op, dim3(div_up(tw * th, 256), n), dim3(256), 0,
+                           ctx->stream, gy + i0 * npx * n_comp, n_comp, (int)sw, (int)sh,
+                           (const float4*)inv_uv, (int)tw, (int)th,
+                           (const float2*)pix_uv + i0 * npx,
+                           n_items > 1 ? part + i0 * n_tex : out);
         DRESSI_CHECK_LAUNCH();
     }
-    if (int rc = raster_attrs(ctx, uv_clip, n_verts, uv_per_item ? n_items : 1, sattr, n_items,
-                              faces, n_faces, tw, th, inv_uv)) return rc;
-    hipLaunchKernelGGL(k_gather_nearest_op, dim3(div_up(tw * th, 256), n_items), dim3(256), 0,
-                       ctx->stream, gy, n_comp, (int)sw, (int)sh, (const float4*)inv_uv, (int)tw,
-                       (int)th, (const float2*)pix_uv, n_items > 1 ? part : out);
-    DRESSI_CHECK_LAUNCH();
     if (n_items > 1) {
-        const size_t n = (size_t)tw * th * n_comp;
-        hipLaunchKernelGGL(k_surface_item_sum, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0,
-                           ctx->stream, (const float*)part, n, n_items, out);
+        hipLaunchKernelGGL(k_surface_item_sum, dim3((uint32_t)((n_tex + 255) / 256)), dim3(256), 0,
+                           ctx->stream, (const float*)part, n_tex, n_items, out);
         DRESSI_CHECK_LAUNCH();
     }
     return DRESSI_OK;

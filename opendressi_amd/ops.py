@@ -429,6 +429,11 @@ def gather_dist_grad(ctx: Context, gy: torch.Tensor, rs: torch.Tensor, clip: tor
 
 # ---- the torch surface's ops (opendressi_amd.torch) -------------------------
 
+# Scratch for as many items as fit goes through at once: it does not grow with
+# the batch past this (a 2048 x 2048 texture's gradient takes 64 MB an item).
+_SCRATCH_BYTES = 256 << 20
+
+
 def surface_rasterize(ctx: Context, pos: torch.Tensor, faces: torch.Tensor, width: int,
                       height: int):
     """dressi_surface_rasterize: pos (N, V, 4), z in [-w, w]; faces (F, 3)
@@ -572,14 +577,16 @@ def surface_texture_bwd(ctx: Context, gy: torch.Tensor, pix_uv: torch.Tensor,
     _prep(ctx)
     n, h, w, nc = gy.shape
     nv = clip.shape[1]
+    group = min(n, max(1, _SCRATCH_BYTES // (16 * (th * tw + 2 * nv))))
     new = lambda *shape: torch.empty(shape, dtype=torch.float32, device=gy.device)
-    uv_clip, sattr, inv_uv = new(*vtx_uv.shape[:-1], 4), new(n, nv, 4), new(n, th, tw, 4)
+    uv_clip = new(*(() if vtx_uv.dim() == 2 else (group,)), nv, 4)
+    sattr, inv_uv = new(group, nv, 4), new(group, th, tw, 4)
     part = new(n, th, tw, nc) if n > 1 else None
     out = new(th, tw, nc)
     check(lib.dressi_surface_texture_bwd(
         ctx.handle, _ptr(gy, "gy"), nc, w, h, n, _ptr(pix_uv, "uv"), _ptr(vtx_uv, "vtx_uv"),
         1 if vtx_uv.dim() == 3 else 0, _ptr(clip, "clip"), 1 if clip.shape[0] > 1 else 0, nv,
-        _ptr(faces, "faces"), faces.shape[0], tw, th, _ptr(uv_clip, "uv_clip"),
+        _ptr(faces, "faces"), faces.shape[0], tw, th, group, _ptr(uv_clip, "uv_clip"),
         _ptr(sattr, "sattr"), _ptr(inv_uv, "inv_uv"), _ptr(part, "part"), _ptr(out, "out")))
     return out
 

@@ -179,10 +179,10 @@ def test_surface_rasterize_soft(ctx, level, n, h, w, peels, radius):
 @pytest.mark.parametrize("n,h,w,tw,th,nc,shared", [
     (1, 40, 64, 33, 17, 3, True), (5, 61, 97, 64, 64, 4, True), (3, 130, 33, 1, 7, 1, False),
     (2, 1, 200, 129, 50, 2, True), (17, 20, 20, 40, 40, 3, False)])
-def test_surface_texture_bwd(ctx, n, h, w, tw, th, nc, shared):
+def test_surface_texture_bwd(ctx, monkeypatch, n, h, w, tw, th, nc, shared):
     """The nearest texture's gradient against UvAsClip / ScreenAttr / Rasterize /
     GatherByInverseUV per item and the contributions' sum, shared and per-item uv, uv that leave
-    part of the texture to the dilation."""
+    part of the texture to the dilation; with the items all at once and in groups."""
     import opendressi_amd as od
     from opendressi_amd import ops as K
     from opendressi_amd.torch.convert import sum_contribs
@@ -210,6 +210,33 @@ def test_surface_texture_bwd(ctx, n, h, w, tw, th, nc, shared):
     got = K.surface_texture_bwd(ctx, g, pix_uv, vtx_uv, vk, ff, tw, th)
     _same(got, sum_contribs(parts), "texture gradient")
     assert float(got.abs().max()) > 0 or h == 1
+    item_bytes = 16 * (th * tw + 2 * len(pos))
+    for group in (1, 2, 3):
+        monkeypatch.setattr(K, "_SCRATCH_BYTES", group * item_bytes + 1)
+        _same(K.surface_texture_bwd(ctx, g, pix_uv, vtx_uv, vk, ff, tw, th), got,
+              f"groups of {group}")
+    ctx.synchronize()
+
+
+def test_surface_texture_bwd_scratch(ctx):
+    """The scratch of a batch stays within its bound: beside the items' contributions (half a
+    gigabyte here) 256 MB of the inverse uv images' two gigabytes."""
+    import opendressi_amd as od
+    from opendressi_amd import ops as K
+    print("[surface texture] scratch", flush=True)
+    n, t = 128, 1024
+    pos, uv, faces = od.uv_sphere(12, 9)
+    dev = lambda a, t=np.float32: torch.from_numpy(np.ascontiguousarray(a, t)).cuda()
+    clip = dev(np.concatenate([pos, np.ones((len(pos), 1))], 1)).expand(n, -1, -1).contiguous()
+    g = torch.ones((n, 8, 8, 1), device="cuda")
+    pix_uv = torch.full((n, 8, 8, 2), 0.5, device="cuda")
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    K.surface_texture_bwd(ctx, g, pix_uv, dev(uv), clip, dev(faces), t, t)
+    torch.cuda.synchronize()
+    took = torch.cuda.max_memory_allocated() - before
+    assert took <= 4 * n * t * t + (256 << 20) + (16 << 20), took
     ctx.synchronize()
 
 
