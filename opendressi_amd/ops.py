@@ -432,6 +432,12 @@ def gather_dist_grad(ctx: Context, gy: torch.Tensor, rs: torch.Tensor, clip: tor
 # Scratch for as many items as fit goes through at once: it does not grow with
 # the batch past this (a 2048 x 2048 texture's gradient takes 64 MB an item).
 _SCRATCH_BYTES = 256 << 20
+_MAX_ITEMS = 65535  # of a launch
+
+
+def _group(n: int, item_bytes: int) -> int:
+    """Items of a batch of n that go through at once."""
+    return max(1, min(n, _MAX_ITEMS, _SCRATCH_BYTES // max(item_bytes, 1)))
 
 
 def surface_rasterize(ctx: Context, pos: torch.Tensor, faces: torch.Tensor, width: int,
@@ -559,12 +565,16 @@ def surface_soft_bwd(ctx: Context, gy: torch.Tensor, rs: torch.Tensor, pos: torc
     n, peels, h, w = rs.shape[:4]
     deg, rows = vtx_faces.shape
     nf = faces.shape[0]
-    scratch = torch.empty((n, peels, nf, 9), dtype=torch.float32, device=rs.device)
+    group = _group(n, 36 * peels * nf)
+    scratch = torch.empty((group, peels, nf, 9), dtype=torch.float32, device=rs.device)
     out = torch.empty((n, rows, 4), dtype=torch.float32, device=rs.device)
-    check(lib.dressi_surface_soft_bwd(
-        ctx.handle, _ptr(gy, "gy"), _ptr(rs, "rs"), peels, _ptr(pos, "pos"), pos.shape[1], n,
-        _ptr(faces, "faces"), nf, _ptr(vtx_faces, "vtx_faces"), rows, deg, radius_px, w, h,
-        _ptr(scratch, "scratch"), _ptr(out, "out")))
+    for i in range(0, n, group):
+        gy_i, rs_i, pos_i, out_i = (gy, rs, pos, out) if group >= n else (
+            t[i:i + group] for t in (gy, rs, pos, out))
+        check(lib.dressi_surface_soft_bwd(
+            ctx.handle, _ptr(gy_i, "gy"), _ptr(rs_i, "rs"), peels, _ptr(pos_i, "pos"),
+            pos.shape[1], out_i.shape[0], _ptr(faces, "faces"), nf, _ptr(vtx_faces, "vtx_faces"),
+            rows, deg, radius_px, w, h, _ptr(scratch, "scratch"), _ptr(out_i, "out")))
     return out
 
 
@@ -577,7 +587,7 @@ def surface_texture_bwd(ctx: Context, gy: torch.Tensor, pix_uv: torch.Tensor,
     _prep(ctx)
     n, h, w, nc = gy.shape
     nv = clip.shape[1]
-    group = min(n, max(1, _SCRATCH_BYTES // (16 * (th * tw + 2 * nv))))
+    group = _group(n, 16 * (th * tw + 2 * nv))
     new = lambda *shape: torch.empty(shape, dtype=torch.float32, device=gy.device)
     uv_clip = new(*(() if vtx_uv.dim() == 2 else (group,)), nv, 4)
     sattr, inv_uv = new(group, nv, 4), new(group, th, tw, 4)

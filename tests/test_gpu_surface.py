@@ -147,9 +147,10 @@ def _peel_threshold(rs, radius_px):
     (0, 1, 40, 64, 1, 3.0), (2, 3, 61, 97, 6, 2.7), (3, 2, 33, 130, 2, 3.0), (1, 4, 1, 200, 3, 0.4),
     # 65 screens' bins: a second group of items
     (0, 65, 512, 512, 2, 3.0)])
-def test_surface_rasterize_soft(ctx, level, n, h, w, peels, radius):
+def test_surface_rasterize_soft(ctx, monkeypatch, level, n, h, w, peels, radius):
     """Every item and peel against SoftClip / RasterizeSoft with the peel thresholds, and the
-    position gradient against GatherDistGrad, ColSum, the peels' sum and the remap's transpose."""
+    position gradient against GatherDistGrad, ColSum, the peels' sum and the remap's transpose,
+    with the items' gradients all at once and in groups."""
     from opendressi_amd import ops as K
     from opendressi_amd.torch.convert import clip_grad_vk_to_gl, sum_contribs
     print(f"[surface soft] level {level} {n}x{h}x{w} peels {peels} r {radius}", flush=True)
@@ -173,6 +174,27 @@ def test_surface_rasterize_soft(ctx, level, n, h, w, peels, radius):
                                                               ff, vf, radius, True)))
         _same(g_pos[i], clip_grad_vk_to_gl(sum_contribs(parts)), f"item {i} gradient")
     assert float(g_pos.abs().max()) > 0
+    for group in (1, 3):
+        monkeypatch.setattr(K, "_SCRATCH_BYTES", group * 36 * peels * nf + 1)
+        _same(K.surface_soft_bwd(ctx, gy, got, clip, ff, vf, radius), g_pos, f"groups of {group}")
+    ctx.synchronize()
+
+
+def test_surface_soft_bwd_scratch(ctx):
+    """The gradient's scratch stays within 256 MB where the batch's corner sums would take 755."""
+    from opendressi_amd import ops as K
+    print("[surface soft] scratch", flush=True)
+    n, peels = 64, 4
+    clip, fi, ff, vf = _scene(6, n, 3, 0.0)
+    rs = torch.zeros((n, peels, 8, 8, 4), device="cuda")
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    out = K.surface_soft_bwd(ctx, rs, rs, clip, ff, vf, 3.0)
+    torch.cuda.synchronize()
+    took = torch.cuda.max_memory_allocated() - before
+    assert 36 * n * peels * len(fi) > 750e6
+    assert took <= out.numel() * 4 + (256 << 20) + (16 << 20), took
     ctx.synchronize()
 
 
