@@ -47,6 +47,9 @@ namespace dressi {
 
 // Items of a batched per-op launch (grid y dimension).
 constexpr uint32_t kMaxBatchItems = 65535;
+// Threads of one launch's x at most (its limit is 2^32 - 1); larger ones go in
+// pieces.
+constexpr uint64_t kLaunchThreads = 1ull << 31;
 
 // thread-local last error; every C entry point returns a dressi_status
 void set_error(const char* fmt, ...);

@@ -273,15 +273,15 @@ __global__ __launch_bounds__(256) void k_surface_tex_prep(const float2* uv, uint
 }
 
 // The items' contributions, the last item first.
-__global__ __launch_bounds__(256) void k_surface_item_sum(const float* part, size_t n,
-                                                          uint32_t n_items, float* out) {
+__global__ __launch_bounds__(256) void k_surface_item_sum(const float* part, size_t stride,
+                                                          uint32_t n_items, size_t n, float* out) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) {
         return;
     }
     ContribSum total;
     for (uint32_t k = n_items; k-- > 0;) {
-        total.push(part[k * n + i]);
+        total.push(part[k * stride + i]);
     }
     out[i] = total.sum();
 }
@@ -922,9 +922,13 @@ int dressi_texture_nearest(dressi_ctx* ctx, const float* tex, uint32_t tw, uint3
     const size_t n = (size_t)uw * uh;
     if (!n) return DRESSI_OK;
     DRESSI_TRY_HIP(hipSetDevice(ctx->device));
-    hipLaunchKernelGGL(k_texture_nearest_op, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0,
-                       ctx->stream, tex, (int)tw, (int)th, n_comp, (const float2*)uv, n, out);
-    DRESSI_CHECK_LAUNCH();
+    for (size_t p = 0; p < n; p += kLaunchThreads) {
+        const size_t m = std::min<size_t>(n - p, kLaunchThreads);
+        hipLaunchKernelGGL(k_texture_nearest_op, dim3((uint32_t)((m + 255) / 256)), dim3(256), 0,
+                           ctx->stream, tex, (int)tw, (int)th, n_comp, (const float2*)uv + p, m,
+                           out + p * n_comp);
+        DRESSI_CHECK_LAUNCH();
+    }
     return DRESSI_OK;
 }
 
@@ -987,9 +991,12 @@ int dressi_surface_texture_bwd(dressi_ctx* ctx, const float* gy, uint32_t n_comp
         DRESSI_CHECK_LAUNCH();
     }
     if (n_items > 1) {
-        hipLaunchKernelGGL(k_surface_item_sum, dim3((uint32_t)((n_tex + 255) / 256)), dim3(256), 0,
-                           ctx->stream, (const float*)part, n_tex, n_items, out);
-        DRESSI_CHECK_LAUNCH();
+        for (size_t t = 0; t < n_tex; t += kLaunchThreads) {
+            const size_t m = std::min<size_t>(n_tex - t, kLaunchThreads);
+            hipLaunchKernelGGL(k_surface_item_sum, dim3((uint32_t)((m + 255) / 256)), dim3(256), 0,
+                               ctx->stream, (const float*)part + t, n_tex, n_items, m, out + t);
+            DRESSI_CHECK_LAUNCH();
+        }
     }
     return DRESSI_OK;
 }

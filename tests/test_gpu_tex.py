@@ -182,3 +182,24 @@ def test_tex_c3_full_size_matches_oracle(ctx, oracle):
     _exact(tex, ref["tex"], "tex")
     _exact(m, ref["m"], "m")
     _exact(v, ref["v"], "v")
+
+
+def test_texture_nearest_of_many_pixels(ctx):
+    """A batch of 2^32 pixels and more (65 views of 8192 x 8192, looked up as one image), more
+    than a launch has threads: every pixel is written."""
+    import torch
+
+    from opendressi_amd import ops
+    n, s = 65, 8192
+    print(f"[texture] {n}x{s}x{s} pixels", flush=True)
+    tex = torch.tensor([[1.0, 2.0], [3.0, 4.0]], device="cuda").view(2, 2, 1)
+    uv = torch.full((n * s, s, 2), 0.25, device="cuda")
+    uv[-1, -1] = 0.75
+    uv[1 << 18, 0] = torch.tensor([0.75, 0.25])  # the second launch's first pixel
+    out = ops.texture_nearest(ctx, tex, uv)
+    assert float(out[-1, -1, 0]) == 4.0 and float(out[1 << 18, 0, 0]) == 2.0
+    del uv
+    for i in range(0, n * s, 1 << 16):
+        part = out[i:i + (1 << 16)]
+        ones = int((part == 1.0).sum())
+        assert ones == part.numel() - (i == 1 << 18) - (i + len(part) == n * s), i
