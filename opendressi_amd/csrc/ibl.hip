@@ -139,11 +139,11 @@ __device__ __forceinline__ int fixed_exponent(uint32_t max_bits, double count) {
 // One workgroup per tile of tile_w x (1024 / tile_w) pixels, a thread per
 // pixel. `slots_log2`: 0 = the whole map in LDS, else the hash table's size.
 // 2^copies_log2 sums per texel (and channel), neighbours in LDS: a lane adds
-// to the one of its number.
+// to the one of its number. The launch's tiles begin at `tile0`.
 __global__ __launch_bounds__(kScatterThreads) void k_eq_scatter(
         const float* gy, uint32_t n, const float* dir, uint32_t dw, uint32_t dh, uint32_t tile_w,
         uint32_t tiles_x, int mw, int mh, const uint32_t* part, uint32_t n_part,
-        uint32_t slots_log2, uint32_t copies_log2, unsigned long long* acc) {
+        uint32_t slots_log2, uint32_t copies_log2, uint32_t tile0, unsigned long long* acc) {
     extern __shared__ unsigned long long lds[];
     __shared__ uint32_t wmax[4];
     const uint32_t tid = threadIdx.x;
@@ -158,8 +158,9 @@ __global__ __launch_bounds__(kScatterThreads) void k_eq_scatter(
             keys[i] = kScatterEmpty;
         }
     }
-    const uint32_t x = (blockIdx.x % tiles_x) * tile_w + tid % tile_w;
-    const uint32_t y = (blockIdx.x / tiles_x) * (kScatterPixels / tile_w) + tid / tile_w;
+    const uint32_t tile = tile0 + blockIdx.x;
+    const uint32_t x = (tile % tiles_x) * tile_w + tid % tile_w;
+    const uint32_t y = (tile / tiles_x) * (kScatterPixels / tile_w) + tid / tile_w;
     const uint32_t copy = tid & ((1u << copies_log2) - 1u);
     const int k = fixed_exponent(scatter_max(part, n_part, wmax), (double)((size_t)dw * dh));
     __syncthreads();
@@ -336,19 +337,20 @@ __device__ __forceinline__ float conv_result(float sum, float scale, float norm,
 
 // `odir` are the output-map directions, `sdir` the source (env) directions;
 // `in` is the env (forward modes) or the output-map gradient (backward
-// modes), N channels.
+// modes), N channels. The launch's outputs begin at `first`.
 template <int MODE, int N>
 __global__ __launch_bounds__(kConvThreads) void k_eq_conv(const float4* odir, uint32_t n_o,
                                                           const float4* sdir, uint32_t n_s,
                                                           const float* in, const float* norm,
-                                                          float alpha, float scale, float* out) {
+                                                          float alpha, float scale,
+                                                          uint32_t first, float* out) {
     constexpr bool kBwd = MODE == kIrrBwd || MODE == kPrefBwd;
     __shared__ alignas(16) float term[2][kConvOut][N][kConvRow];
     const uint32_t n_i = kBwd ? n_s : n_o;
     const uint32_t n_j = kBwd ? n_o : n_s;
     const float4* idir = kBwd ? sdir : odir;
     const float4* jdir = kBwd ? odir : sdir;
-    const uint32_t i0 = blockIdx.x * kConvOut;
+    const uint32_t i0 = first + blockIdx.x * kConvOut;
     const uint32_t n_chunks = (n_j + kConvChunk - 1) / kConvChunk;
     const uint32_t tid = threadIdx.x;
     const bool adds = tid >= 256;  // the fifth wave
@@ -488,14 +490,14 @@ __global__ __launch_bounds__(kConvThreads) void k_eq_conv_few(const float4* odir
                                                               const float4* sdir, uint32_t n_s,
                                                               const float* in, const float* norm,
                                                               float alpha, float scale,
-                                                              float* out) {
+                                                              uint32_t first, float* out) {
     constexpr bool kBwd = MODE == kIrrBwd || MODE == kPrefBwd;
     __shared__ alignas(16) float term[3][kFewOut][N][kFewRow];
     const uint32_t n_i = kBwd ? n_s : n_o;
     const uint32_t n_j = kBwd ? n_o : n_s;
     const float4* idir = kBwd ? sdir : odir;
     const float4* jdir = kBwd ? odir : sdir;
-    const uint32_t i0 = blockIdx.x * kFewOut;
+    const uint32_t i0 = first + blockIdx.x * kFewOut;
     const uint32_t n_chunks = (n_j + kFewChunk - 1) / kFewChunk;
     const uint32_t src = threadIdx.x;
     if (src < 256) {
@@ -772,9 +774,13 @@ int run_conv(dressi_ctx* ctx, const float* in, uint32_t sw, uint32_t sh, uint32_
     const auto launch = [&](auto n_comp) {
         constexpr int N = decltype(n_comp)::value;
         const auto kernel = few ? k_eq_conv_few<MODE, N> : k_eq_conv<MODE, N>;
-        hipLaunchKernelGGL(kernel, dim3(div_up(n_i, few ? kFewOut : kConvOut)),
-                           dim3(kConvThreads), 0, ctx->stream, od, ow * oh, sd, sw * sh, in, norm,
-                           alpha, scale, out);
+        const uint32_t per = few ? kFewOut : kConvOut;
+        constexpr uint32_t kBlocks = (uint32_t)(kLaunchThreads / kConvThreads);
+        for (uint32_t first = 0; first < n_i; first += kBlocks * per) {
+            hipLaunchKernelGGL(kernel, dim3(std::min(div_up(n_i - first, per), kBlocks)),
+                               dim3(kConvThreads), 0, ctx->stream, od, ow * oh, sd, sw * sh, in,
+                               norm, alpha, scale, first, out);
+        }
     };
     switch (MODE == kPrefNorm ? 1u : n) {
         case 1: launch(std::integral_constant<int, 1>()); break;
@@ -831,10 +837,11 @@ int dressi_equirect_sample_bwd(dressi_ctx* ctx, const float* gy, uint32_t n_comp
                        (uint32_t*)mx, (unsigned long long*)acc, cnt);
     DRESSI_CHECK_LAUNCH();
     if (npx) {
-        // square tiles where the image has the rows for them, flatter ones
-        // for a list of directions
+        // square tiles where the image has the rows and columns for them,
+        // flat or narrow ones for a list of directions
         uint32_t tile_h = 1;
         while (tile_h < 32 && tile_h < dh) tile_h *= 2;
+        while (tile_h < kScatterPixels && kScatterPixels / tile_h >= 2ull * dw) tile_h *= 2;
         const uint32_t tile_w = kScatterPixels / tile_h;
         const uint32_t tiles_x = div_up(dw, tile_w);
         const uint64_t tiles = (uint64_t)tiles_x * div_up(dh, tile_h);
@@ -851,11 +858,14 @@ int dressi_equirect_sample_bwd(dressi_ctx* ctx, const float* gy, uint32_t n_comp
         }
         const size_t sums = slots_log2 ? (size_t)n_comp << slots_log2 : cnt;
         const size_t lds = (sums << copies_log2) * 8 + (slots_log2 ? 4ull << slots_log2 : 0);
-        hipLaunchKernelGGL(k_eq_scatter, dim3((uint32_t)tiles), dim3(kScatterThreads), lds,
-                           ctx->stream, gy, n_comp, dir, dw, dh, tile_w, tiles_x, (int)mw, (int)mh,
-                           (const uint32_t*)mx, n_part, slots_log2, copies_log2,
-                           (unsigned long long*)acc);
-        DRESSI_CHECK_LAUNCH();
+        constexpr uint32_t kBlocks = (uint32_t)(kLaunchThreads / kScatterThreads);
+        for (uint32_t tile0 = 0; tile0 < (uint32_t)tiles; tile0 += kBlocks) {
+            hipLaunchKernelGGL(k_eq_scatter, dim3(std::min((uint32_t)tiles - tile0, kBlocks)),
+                               dim3(kScatterThreads), lds, ctx->stream, gy, n_comp, dir, dw, dh,
+                               tile_w, tiles_x, (int)mw, (int)mh, (const uint32_t*)mx, n_part,
+                               slots_log2, copies_log2, tile0, (unsigned long long*)acc);
+            DRESSI_CHECK_LAUNCH();
+        }
     }
     hipLaunchKernelGGL(k_fixed_resolve, dim3((uint32_t)((cnt + 255) / 256)), dim3(256), 0,
                        ctx->stream, (const unsigned long long*)acc, cnt, (const uint32_t*)mx,

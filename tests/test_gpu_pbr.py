@@ -244,6 +244,37 @@ def test_equirect_vjp_tiles(ctx, oracle, shape, coherent):
     _exact(host(ops.equirect_sample_bwd(ctx, dev(gy), dev(d), mw, mh)), got, "rerun")
 
 
+def test_equirect_vjp_of_a_long_list(ctx):
+    """2^27 + 33 directions in one column and in one row: the same sums, so the same bits. A thread
+    per pixel of a square tile would pass a launch's 2^32 threads here."""
+    import torch
+
+    from opendressi_amd import ops
+    n = (1 << 27) + 33
+    print(f"[equirect vjp] list of {n}", flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    d = torch.randn((n, 3), device="cuda", generator=gen)
+    gy = torch.randn((n, 1), device="cuda", generator=gen)
+    column = ops.equirect_sample_bwd(ctx, gy.view(n, 1, 1), d.view(n, 1, 3), 8, 4)
+    row = ops.equirect_sample_bwd(ctx, gy.view(1, n, 1), d.view(1, n, 3), 8, 4)
+    _exact(host(column), host(row), "column and row")
+    assert float(row.abs().min()) > 0
+
+
+def test_ibl_conv_of_many_outputs(ctx):
+    """108 M outputs, more than a launch has threads for five waves of eight: the irradiance of
+    one texel, the cosine to its direction."""
+    from opendressi_amd import ops
+    ow, oh = 16384, 6600
+    print(f"[ibl conv] {ow}x{oh} outputs", flush=True)
+    got = ops.irradiance_conv(ctx, dev(np.full((1, 1, 1), 0.5, np.float32)), ow, oh)
+    phi = ((np.arange(ow) + 0.5) / ow - 0.5) * 2.0 * np.pi
+    for y in (0, 1, 3275, 3276, 3277, oh // 2, oh - 1):
+        want = np.pi * np.maximum(np.sin((y + 0.5) / oh * np.pi) * np.cos(phi), 0.0)
+        # float32 directions: a few ulp of 1, scaled
+        assert np.abs(host(got[y, :, 0]) - want).max() < 3e-6, y
+
+
 # ---- the fused C5 plan -------------------------------------------------------
 
 def _scene(g):
