@@ -3,6 +3,8 @@
 // AntiAliasBwdVtx / ColSum entry points and the kernels of the fused AA
 // silhouette iteration (hard raster -> AntiAlias -> L2 -> stochastic vertex
 // gather -> ColSum -> clip->pos -> Adam).
+#include <algorithm>
+
 #include "plan.h"
 
 namespace dressi {
@@ -364,14 +366,14 @@ __global__ __launch_bounds__(kAaExactThreads) void k_antialias_bwd_vtx_exact_op(
         const float* gy, const float* img, uint32_t n_comp, const float* tri_f, uint32_t tri_stride,
         const float4* clip, uint32_t n_verts, int clip_per_item, const float* faces,
         uint32_t n_faces, const float* vtx_faces, uint32_t n_rows, uint32_t max_deg, uint32_t w,
-        uint32_t h, float scale, float4* out) {
+        uint32_t h, float scale, uint32_t first, float4* out) {
     constexpr uint32_t T = kAaExactThreads;
     __shared__ int box[4];
     __shared__ uint32_t wave_pairs[T / 64];
     __shared__ uint16_t pair[T * 8];  // thread of the pixel << 3 | neighbour
     __shared__ float term[T][6];      // endpoint a's x, y, w, then b's
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-    const uint32_t v = blockIdx.x;
+    const uint32_t v = first + blockIdx.x;
     const AaItem it(w, h);
     gy = it.img(gy, n_comp);
     img = it.img(img, n_comp);
@@ -1515,6 +1517,24 @@ int check_aa_args(dressi_ctx* ctx, uint32_t n_comp, uint32_t w, uint32_t h) {
     return DRESSI_OK;
 }
 
+// A workgroup per vertex: pieces of 8 M vertices.
+int launch_vtx_exact(dressi_ctx* ctx, const float* gy, const float* img, uint32_t n_comp,
+                     const float* tri, uint32_t tri_stride, const float* clip, uint32_t n_verts,
+                     int clip_per_item, const float* faces, uint32_t n_faces,
+                     const float* vtx_faces, uint32_t n_rows, uint32_t max_deg, uint32_t w,
+                     uint32_t h, uint32_t n_items, float scale, float* out) {
+    constexpr uint32_t kBlocks = (uint32_t)(kLaunchThreads / kAaExactThreads);
+    for (uint32_t first = 0; first < n_rows; first += kBlocks) {
+        hipLaunchKernelGGL(k_antialias_bwd_vtx_exact_op,
+                           dim3(std::min(n_rows - first, kBlocks), n_items), dim3(kAaExactThreads),
+                           0, ctx->stream, gy, img, n_comp, tri, tri_stride, (const float4*)clip,
+                           n_verts, clip_per_item, faces, n_faces, vtx_faces, n_rows, max_deg, w,
+                           h, scale, first, (float4*)out);
+        DRESSI_CHECK_LAUNCH();
+    }
+    return DRESSI_OK;
+}
+
 }  // namespace
 
 namespace dressi {
@@ -1618,10 +1638,9 @@ int dressi_antialias_bwd_vtx_batch(dressi_ctx* ctx, const float* gy, const float
         return DRESSI_OK;
     }
     if (n_samples == 0) {
-        hipLaunchKernelGGL(k_antialias_bwd_vtx_exact_op, dim3(n_verts, n_items),
-                           dim3(kAaExactThreads), 0, ctx->stream, gy, img, n_comp, tri, 1u,
-                           (const float4*)clip, n_verts, clip_per_item, faces, n_faces, vtx_faces,
-                           n_verts, max_deg, width, height, 1.f, (float4*)out);
+        return launch_vtx_exact(ctx, gy, img, n_comp, tri, 1u, clip, n_verts, clip_per_item, faces,
+                                n_faces, vtx_faces, n_verts, max_deg, width, height, n_items, 1.f,
+                                out);
     } else {
         const uint32_t rows = wide ? max_deg : 1u;
         DRESSI_REQUIRE((uint64_t)n_verts * rows * 8 < (1ull << 32), "AntiAliasBwdVtx: too many rows");
@@ -1722,12 +1741,9 @@ int dressi_surface_antialias_bwd_pos(dressi_ctx* ctx, const float* gy, const flo
         return DRESSI_OK;
     }
     if (n_samples == 0) {
-        hipLaunchKernelGGL(k_antialias_bwd_vtx_exact_op, dim3(n_rows, n_items),
-                           dim3(kAaExactThreads), 0, ctx->stream, gy, img, n_comp, rast + 3, 4u,
-                           (const float4*)pos, n_verts, pos_per_item, faces, n_faces, vtx_faces,
-                           n_rows, max_deg, width, height, boost, (float4*)out);
-        DRESSI_CHECK_LAUNCH();
-        return DRESSI_OK;
+        return launch_vtx_exact(ctx, gy, img, n_comp, rast + 3, 4u, pos, n_verts, pos_per_item,
+                                faces, n_faces, vtx_faces, n_rows, max_deg, width, height, n_items,
+                                boost, out);
     }
     if (n_faces) {
         hipLaunchKernelGGL(k_surface_aa_bwd_faces, dim3(n_faces, n_items), dim3(64), 0,

@@ -47,8 +47,8 @@ namespace dressi {
 
 // Items of a batched per-op launch (grid y dimension).
 constexpr uint32_t kMaxBatchItems = 65535;
-// Threads of one launch's x at most (its limit is 2^32 - 1); larger ones go in
-// pieces.
+// Threads of one launch's x at most; larger ones go in pieces (past 2^32 - 1
+// the runtime takes the count modulo 2^32 and reports nothing).
 constexpr uint64_t kLaunchThreads = 1ull << 31;
 
 // thread-local last error; every C entry point returns a dressi_status

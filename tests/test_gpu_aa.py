@@ -129,6 +129,34 @@ def test_aa_exact_vertex_gradient_steps(ctx, oracle, level, h, w, nc):
     ctx.synchronize()
 
 
+def test_aa_exact_vertex_gradient_of_many_vertices(ctx, oracle):
+    """2^24 + 3 vertices, more than a launch has workgroups for: the first few are the small
+    scene's, every other one is written with zeros."""
+    import torch
+
+    from opendressi_amd import ops
+    n, h, w = (1 << 24) + 3, 40, 33
+    print(f"[aa exact] {n} vertices", flush=True)
+    clip, faces = _random_scene(oracle, 1, 1, w)
+    nv = len(clip)
+    tri = oracle.rasterize_face_id(clip, faces, w, h)
+    vf = oracle.vertex_faces_tex(faces, nv)
+    rng = np.random.default_rng(5)
+    img = rng.random((h, w, 2), dtype=np.float32)
+    gy = rng.standard_normal((h, w, 2)).astype(np.float32)
+    clips = torch.ones((n, 4), device="cuda")
+    clips[:nv] = dev(clip)
+    adj = torch.full((len(vf), n), -1.0, device="cuda")
+    adj[:, :nv] = dev(vf)
+    torch.full((n, 4), 7.0, device="cuda")  # what the output's memory may hold before
+    got = ops.antialias_bwd_vtx(ctx, dev(gy), dev(img), dev(tri), clips, dev(faces), adj, None, 0)
+    assert float(got[nv:].abs().max()) == 0.0
+    want = oracle.antialias_bwd_vtx(gy, img, tri, clip, faces, vf, 0.0, 0)
+    assert np.abs(want).max() > 0
+    _exact(host(got[:nv]), want, "exact")
+    ctx.synchronize()
+
+
 def test_aa_batch_ops_match_oracle(ctx, oracle):
     """The batched AntiAlias / AntiAliasBwdImg / AntiAliasBwdVtx / ColSum
     entry points: three items (own cameras; per-item clips, and one clip
