@@ -498,6 +498,7 @@ extern "C" int dressi_gather_dist_grad(dressi_ctx* ctx, const float* gy, const f
     DRESSI_REQUIRE(radius_px > 0.f, "radius_px must be > 0");
     DRESSI_REQUIRE(max_deg >= 1, "max_deg must be >= 1");
     DRESSI_REQUIRE((uint64_t)max_deg * n_verts < (1ull << 31), "adjacency too large");
+    DRESSI_REQUIRE(!wide || (uint64_t)width * height <= kMaxImagePixels, "screen too large");
     if (!n_verts) return DRESSI_OK;
     DRESSI_TRY_HIP(hipSetDevice(ctx->device));
     if (wide) {
@@ -532,7 +533,7 @@ extern "C" int dressi_surface_soft_bwd(dressi_ctx* ctx, const float* gy, const f
     DRESSI_REQUIRE(radius_px > 0.f, "radius_px must be > 0");
     DRESSI_REQUIRE(peels >= 1 && n_items <= kMaxBatchItems, "batch of %u items exceeds %u",
                    n_items, kMaxBatchItems);
-    DRESSI_REQUIRE((uint64_t)width * height < (1ull << 31) && n_rows < (1u << 30),
+    DRESSI_REQUIRE((uint64_t)width * height <= kMaxImagePixels && n_rows < (1u << 30),
                    "rasterize_soft backward: too large");
     if (!n_items || !n_rows) return DRESSI_OK;
     DRESSI_TRY_HIP(hipSetDevice(ctx->device));

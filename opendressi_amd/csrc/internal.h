@@ -47,6 +47,9 @@ namespace dressi {
 
 // Items of a batched per-op launch (grid y dimension).
 constexpr uint32_t kMaxBatchItems = 65535;
+// Pixels of an image up to which its indices, and a step's past the last one,
+// fit 32 bits: more than the rasterizers have threads for.
+constexpr uint64_t kMaxImagePixels = 0xffff0000ull;
 // Threads of one launch's x at most; larger ones go in pieces (past 2^32 - 1
 // the runtime takes the count modulo 2^32 and reports nothing).
 constexpr uint64_t kLaunchThreads = 1ull << 31;

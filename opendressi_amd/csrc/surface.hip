@@ -234,7 +234,7 @@ __global__ __launch_bounds__(256) void k_surface_interp_bwd_vtx(
 int check_surface(dressi_ctx* ctx, uint32_t n_comp, uint32_t w, uint32_t h, uint32_t n_items) {
     DRESSI_REQUIRE(ctx != nullptr, "NULL context");
     DRESSI_REQUIRE(n_comp >= 1 && n_comp <= 4, "n_comp must be 1..4");
-    DRESSI_REQUIRE((uint64_t)w * h < (1ull << 31), "screen too large");
+    DRESSI_REQUIRE((uint64_t)w * h <= kMaxImagePixels, "screen too large");
     DRESSI_REQUIRE(n_items <= kMaxBatchItems, "batch of %u items exceeds %u", n_items,
                    kMaxBatchItems);
     DRESSI_TRY_HIP(hipSetDevice(ctx->device));

@@ -963,7 +963,7 @@ int dressi_surface_texture_bwd(dressi_ctx* ctx, const float* gy, uint32_t n_comp
                    "batch of %u items in groups of %u", n_items, group);
     group = std::min(group, n_items);
     DRESSI_REQUIRE(tw > 0 && th > 0 && (uint64_t)tw * th < (1ull << 31) &&
-                           (uint64_t)sw * sh < (1ull << 31) &&
+                           (uint64_t)sw * sh < (1ull << 40) &&
                            (uint64_t)group * n_verts < (1ull << 31) &&
                            (uint64_t)group * n_faces < (1ull << 31),
                    "size too large");

@@ -283,3 +283,26 @@ def test_texture_bwd_of_an_empty_screen(ctx, sw, sh):
         ref[1, 2] = 7.0  # uv (0.5, 0.5)
     _same(out, ref, "out")
     ctx.synchronize()
+
+
+@pytest.mark.parametrize("w,h,ok", [(46341, 46341, True), (65535, 65534, True),
+                                    (65536, 65536, False)])
+def test_screen_limits(ctx, w, h, ok):
+    """Screens of 2^31 pixels and more, which the per-op entry points take, are no reason to
+    refuse a call; 2^32 are (a pixel's index would not fit). Batches and meshes of nothing, which
+    return after the checks."""
+    from opendressi_amd import _lib as L
+    print(f"[surface limits] {w}x{h}", flush=True)
+    some = torch.zeros(64, device="cuda")
+    p, lib = L.C.c_void_p(some.data_ptr()), L.lib
+    ctx.use_torch_stream()
+    calls = [
+        lambda: lib.dressi_surface_interpolate(ctx.handle, p, 1, 3, 0, p, w, h, 0, p, 1, p),
+        lambda: lib.dressi_surface_interpolate_bwd(ctx.handle, p, 3, p, w, h, 0, p, 1, 0, p, 1, p, 1,
+                                                   1, 1, p, p),
+        lambda: lib.dressi_surface_soft_bwd(ctx.handle, p, p, 1, p, 1, 0, p, 1, p, 1, 1, 3.0, w, h,
+                                            p, p),
+        lambda: lib.dressi_gather_dist_grad(ctx.handle, p, p, p, 0, p, 1, p, 1, 3.0, 1, w, h, p)]
+    for call in calls:
+        assert (call() == 0) == ok, lib.dressi_last_error()
+    ctx.synchronize()
