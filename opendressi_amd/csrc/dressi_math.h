@@ -61,6 +61,20 @@ DRESSI_HD void pixel_bbox(float x0f, float x1f, float x2f, float y0f, float y1f,
     *by1 = a < h - 1 ? a : h - 1;
 }
 
+// The screen pixel (truncated) that an inverse-UV anchor's window is around;
+// false for an anchor at infinity or next to it, whose window holds no pixel:
+// it would convert to the largest integer, and the window's indices would
+// wrap, past a clamp too (the compiler adds after it has clamped).
+DRESSI_HD bool anchor_pixel(float ax, float ay, int* x, int* y) {
+    constexpr float kFar = 2147483008.f;  // 2^31 - 640
+    if (fabsf(ax) >= kFar || fabsf(ay) >= kFar) {
+        return false;
+    }
+    *x = (int)ax;
+    *y = (int)ay;
+    return true;
+}
+
 // cpu_raster.cpp:177-193 (ScreenBarycentric) split into its per-triangle
 // part (area, 1/area) and per-pixel part; the values are identical to the
 // one-call form.

@@ -217,8 +217,9 @@ __global__ __launch_bounds__(256) void k_gather_nearest_op(const float* gy, uint
     const int ty = q / tw, tx = q - ty * tw;
     const float4 iv = inv_uv_anchor(inv_uv, tw, th, tx, ty);
     float o[4] = {0.f, 0.f, 0.f, 0.f};
-    if (iv.z > 0.5f && sw > 0) {  // (an empty screen has no column to clamp to)
-        const int scx = (int)iv.x, scy = (int)iv.y;
+    int scx, scy;
+    // (an empty screen has no column to clamp to)
+    if (iv.z > 0.5f && sw > 0 && anchor_pixel(iv.x, iv.y, &scx, &scy)) {
         size_t found = npx;
         for (int dy = -3; dy <= 3 && found == npx; dy++) {
             const int spy = scy + dy;

@@ -98,6 +98,39 @@ def test_texture_nearest_ops_match_oracle(ctx, oracle, seed):
                oracle.gather_inv_uv(gy, iv, uv2), f"gather nearest nc={nc}")
 
 
+FAR = (3.4e38, 1e20, 3e9, 2147483648.0, 2147483520.0, 2147483008.0, 2147482880.0, 1e6)
+
+
+@pytest.mark.parametrize("op", ["nearest"])
+def test_far_anchors(ctx, oracle, op):
+    """Inverse-UV anchors at infinity, at the largest integers and just off the screen beside
+    ordinary ones, on one axis or both: their windows hold no pixel, as one at (-100, -100)."""
+    from opendressi_amd import ops
+    print(f"[tex far anchors] {op}", flush=True)
+    rng = np.random.default_rng(3)
+    h, w, th, tw = 61, 47, 37, 53
+    gy = rng.standard_normal((h, w, 3)).astype(np.float32)
+    uv = rng.random((h, w, 2)).astype(np.float32)
+    iv = np.zeros((th, tw, 4), np.float32)
+    iv[..., 0] = rng.random((th, tw)) * 61 - 7
+    iv[..., 1] = rng.random((th, tw)) * 75 - 7
+    iv[..., 2] = (rng.random((th, tw)) < 0.7).astype(np.float32)
+    near = iv.copy()
+    far = np.array([np.inf, *FAR], np.float32)
+    far = np.concatenate([far, -far])
+    for axes in ((0,), (1,), (0, 1)):
+        at = rng.random((th, tw)) < 0.15
+        near[at, :2] = -100.0
+        for a in axes:
+            iv[at, a] = rng.choice(far, int(at.sum()))
+    gpu, ref = {"nearest": (ops.texture_nearest_bwd, oracle.gather_inv_uv),
+                "bilinear": (ops.texture_bilinear_bwd, oracle.gather_inv_uv_bilinear)}[op]
+    want = ref(gy, near, uv)
+    assert np.abs(want).max() > 0
+    _exact(host(gpu(ctx, dev(gy), dev(iv), dev(uv))), want, op)
+    ctx.synchronize()
+
+
 def _fit(ctx, g, images=True):
     import opendressi_amd as od
     return od.TextureFit(ctx, g["in_pos"], g["in_uv"], g["in_faces"], g["in_mvps"],
