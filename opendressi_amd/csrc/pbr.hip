@@ -346,10 +346,10 @@ __global__ __launch_bounds__(256) void k_pbr_csr(CsrArgs a) {
                 }
             }
         }
-        if (iv.z <= 0.5f) {
+        int scx, scy;
+        if (iv.z <= 0.5f || !anchor_pixel(iv.x, iv.y, &scx, &scy)) {
             continue;
         }
-        const int scx = (int)iv.x, scy = (int)iv.y;
         for (int dy = -3; dy <= 3; dy++) {
             for (int dx = -3; dx <= 3; dx++) {
                 const int spx = scx + dx, spy = scy + dy;

@@ -125,8 +125,8 @@ __global__ __launch_bounds__(256) void k_gather_bilinear_op(const float* gy, uin
         }
     }
     float o[4] = {0.f, 0.f, 0.f, 0.f};
-    if (iv.z > 0.5f) {
-        const int scx = (int)iv.x, scy = (int)iv.y;
+    int scx, scy;
+    if (iv.z > 0.5f && anchor_pixel(iv.x, iv.y, &scx, &scy)) {
         for (int dy = -3; dy <= 3; dy++) {
             for (int dx = -3; dx <= 3; dx++) {
                 const int spx = scx + dx, spy = scy + dy;

@@ -101,7 +101,7 @@ def test_texture_nearest_ops_match_oracle(ctx, oracle, seed):
 FAR = (3.4e38, 1e20, 3e9, 2147483648.0, 2147483520.0, 2147483008.0, 2147482880.0, 1e6)
 
 
-@pytest.mark.parametrize("op", ["nearest"])
+@pytest.mark.parametrize("op", ["nearest", "bilinear"])
 def test_far_anchors(ctx, oracle, op):
     """Inverse-UV anchors at infinity, at the largest integers and just off the screen beside
     ordinary ones, on one axis or both: their windows hold no pixel, as one at (-100, -100)."""
