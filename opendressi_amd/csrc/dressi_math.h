@@ -75,6 +75,15 @@ DRESSI_HD bool anchor_pixel(float ax, float ay, int* x, int* y) {
     return true;
 }
 
+// i + d clamped to [0, n), d = 0 or 1, for any i: one that converted to the
+// largest integer would wrap (past the clamp: it is compiled as an add after
+// the lower bound).
+DRESSI_HD int edge_tap(int i, int d, int n) {
+    const int x = (i < 0x7ffffffe ? i : 0x7ffffffe) + d;
+    const int lo = x > 0 ? x : 0;
+    return lo < n - 1 ? lo : n - 1;
+}
+
 // cpu_raster.cpp:177-193 (ScreenBarycentric) split into its per-triangle
 // part (area, 1/area) and per-pixel part; the values are identical to the
 // one-call form.

@@ -17,6 +17,7 @@
 #include <cstdint>
 #include <vector>
 
+#include "dressi_math.h"
 #include "libm_f32.h"
 
 namespace dressi {
@@ -143,10 +144,8 @@ __device__ __forceinline__ Taps taps_clamp(int w, int h, float u, float v) {
     for (int dy = 0; dy <= 1; dy++) {
 #pragma unroll
         for (int dx = 0; dx <= 1; dx++) {
-            int x = ix + dx;
-            x = x < 0 ? 0 : (x > w - 1 ? w - 1 : x);
-            int y = iy + dy;
-            y = y < 0 ? 0 : (y > h - 1 ? h - 1 : y);
+            const int x = edge_tap(ix, dx, w);
+            const int y = edge_tap(iy, dy, h);
             t.idx[dy * 2 + dx] = y * w + x;
             t.w[dy * 2 + dx] = (dx == 0 ? 1.f - fx : fx) * (dy == 0 ? 1.f - fy : fy);
         }

@@ -35,8 +35,8 @@ __device__ __forceinline__ void bilerp_clamp_n(const float* data, int w, int h, 
     for (int dy = 0; dy <= 1; dy++) {
 #pragma unroll
         for (int dx = 0; dx <= 1; dx++) {
-            const int x = min(max(ix + dx, 0), w - 1);
-            const int y = min(max(iy + dy, 0), h - 1);
+            const int x = edge_tap(ix, dx, w);
+            const int y = edge_tap(iy, dy, h);
             const float wgt = (dx == 0 ? 1.f - fx : fx) * (dy == 0 ? 1.f - fy : fy);
             const float* p = data + ((size_t)y * w + (size_t)x) * n;
             for (uint32_t c = 0; c < n; c++) {
@@ -46,7 +46,9 @@ __device__ __forceinline__ void bilerp_clamp_n(const float* data, int w, int h, 
     }
 }
 
-// The same for an RGBA texture (one 16-byte load per tap).
+// The same for an RGBA texture (one 16-byte load per tap), for indices within
+// 2^30 (dressi_tex_set_mesh sees to that: edge_tap's bound costs the fit's
+// forward 3 us of 136).
 __device__ __forceinline__ float4 bilerp_clamp4(const float4* tex, int w, int h, float u, float v) {
     const float sx = u * (float)w - 0.5f;
     const float sy = v * (float)h - 0.5f;
@@ -1208,6 +1210,11 @@ int dressi_tex_set_mesh(dressi_tex_plan* p, const float* pos, const float* uv,
         const float x = faces[i];
         DRESSI_REQUIRE(x >= 0.f && x < (float)V, "face index out of range at %zu", i);
         fi[i] = (int32_t)(uint32_t)(int64_t)(x + 0.5f);
+        // (a pixel's uv lies between its corners': see bilerp_clamp4)
+        const float* q = uv + (size_t)fi[i] * 2;
+        DRESSI_REQUIRE(!(std::fabs(q[0]) * (float)p->desc.tex_w > 0x1p30f) &&
+                               !(std::fabs(q[1]) * (float)p->desc.tex_h > 0x1p30f),
+                       "uv (%g, %g) of vertex %d is too large", q[0], q[1], fi[i]);
     }
     hipStream_t s = p->ctx->stream;
     TexDev& d = p->d;

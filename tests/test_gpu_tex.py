@@ -131,6 +131,46 @@ def test_far_anchors(ctx, oracle, op):
     ctx.synchronize()
 
 
+def test_far_bilinear_lookups(ctx, oracle):
+    """uv at infinity and at the largest integers beside ordinary ones: the pixels of the others
+    are the oracle's, those of the far ones read the texture's edge (whatever their weights)."""
+    from opendressi_amd import ops
+    print("[tex far uv] bilinear", flush=True)
+    rng = np.random.default_rng(4)
+    tex = rng.random((37, 53, 4)).astype(np.float32)
+    uv = (rng.random((61, 47, 2)) * 1.4 - 0.2).astype(np.float32)
+    uv[:3] = rng.choice(np.array([1e3, -1e3, 1e5, -1e5], np.float32), (3, 47, 2))
+    far = np.array([np.inf, *FAR[:-1]], np.float32)
+    at = rng.random((61, 47)) < 0.2
+    odd = uv.copy()
+    odd[at] = rng.choice(np.concatenate([far, -far]), (int(at.sum()), 2))
+    want = oracle.texture_bilinear(tex, uv)
+    got = host(ops.texture_bilinear(ctx, dev(tex), dev(odd)))
+    _exact(got[~at], want[~at], "bilinear")
+    ctx.synchronize()
+
+
+@pytest.mark.parametrize("value,ok", [(np.inf, False), (-1e20, False), (np.nan, True), (1e6, True)])
+def test_fit_refuses_uv_without_a_texel(ctx, value, ok):
+    """A texture fit's lookups take any finite texel index of ordinary size: a uv at infinity, or
+    whose index would pass 2^30, is refused where the mesh is set."""
+    import opendressi_amd as od
+    pos, uv, faces = od.uv_sphere(8, 6)
+    uv = uv.copy()
+    uv[7, 1] = value
+    tex = np.full((16, 16, 4), 0.5, np.float32)
+    print(f"[tex fit] uv {value}", flush=True)
+    make = lambda: od.TextureFit(ctx, pos, uv, faces, od.orbit_cameras(1, 2, 3), 32, tex, tex)
+    if ok:
+        fit = make()
+        fit.step(1)
+        ctx.synchronize()
+        fit.close()
+    else:
+        with pytest.raises(od.DressiError, match="uv"):
+            make()
+
+
 def _fit(ctx, g, images=True):
     import opendressi_amd as od
     return od.TextureFit(ctx, g["in_pos"], g["in_uv"], g["in_faces"], g["in_mvps"],
