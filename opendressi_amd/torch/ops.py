@@ -81,9 +81,11 @@ class _InterpolateFn(torch.autograd.Function):
         rast_d = to_dev(rast, dev, "rast")
         shared = attr_d.dim() == 2
         channels(attr_d.shape[-1], "attr")
-        if attr_d.dim() not in (2, 3) or (not shared and attr_d.shape[0] != rast_d.shape[0]):
-            raise ValueError(f"attr must be [V, C] or [{rast_d.shape[0]}, V, C], got "
-                             f"{tuple(attr.shape)}")
+        n = rast_d.shape[0]
+        if attr_d.dim() not in (2, 3) or (not shared and attr_d.shape[0] < n):
+            raise ValueError(f"attr must be [V, C] or [{n}, V, C], got {tuple(attr.shape)}")
+        if not shared:
+            attr_d = attr_d[:n]  # items past the raster's are not looked at
         with vctx.lock:
             # the whole batch in one launch
             out = K.surface_interpolate(vctx._ctx, attr_d, rast_d, md.faces_f)

@@ -565,6 +565,22 @@ def test_antialias_matches_oracle(dr, ctx, oracle, n_samples):
     assert np.abs(want_p).max() > 0
 
 
+def test_interpolate_more_items_than_the_raster(dr, ctx):
+    """Per-item attributes with items past the raster's: the first ones' images; fewer items are
+    refused (the last item's would be read past the tensor)."""
+    print("[torch] interpolate items", flush=True)
+    clip, faces = _sphere(level=1)
+    pos = torch.from_numpy(np.stack([clip, clip * np.float32(0.9)])).cuda()
+    tri = torch.from_numpy(faces).cuda()
+    rast, _ = dr.rasterize(ctx, pos, tri, resolution=[20, 31])
+    attr = torch.rand((3, len(clip), 2), device="cuda")
+    got, _ = dr.interpolate(attr, rast, tri)
+    want, _ = dr.interpolate(attr[:2], rast, tri)
+    assert torch.equal(got, want) and float(want.abs().max()) > 0
+    with pytest.raises(ValueError):
+        dr.interpolate(attr[:1], rast, tri)
+
+
 # ------------------------------ rasterize_soft -----------------------------
 
 
