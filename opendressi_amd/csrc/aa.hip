@@ -930,14 +930,6 @@ __global__ __launch_bounds__(64) void k_aa_raster(HsrDev d) {
     }
 }
 
-// Orders the LDS accesses of one wave around an exchange between its lanes
-// (a wave executes its LDS instructions in order).
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // Mask bits (1 = covered) of ids columns x0 .. x0+3 of one row.
 __device__ __forceinline__ uint32_t fg_bits4(uint32_t a, uint32_t b, uint32_t c, uint32_t e) {
     return (a != 0u ? 1u : 0u) | (b != 0u ? 2u : 0u) | (c != 0u ? 4u : 0u) | (e != 0u ? 8u : 0u);
@@ -1070,7 +1062,7 @@ __global__ __launch_bounds__(64 * NV) void k_aa_fwd(HsrDev d) {
             }
             n_q += (uint32_t)__popcll(m);
         }
-        wave_lds_sync();
+        wave_lds_fence();
         const TriFromRecs tris{d.faces, d.arecs + (size_t)view * d.g.n_faces};
         const int k = lane & 7;
         for (uint32_t q0 = 0; q0 < n_q; q0 += 8) {
@@ -1105,7 +1097,7 @@ __global__ __launch_bounds__(64 * NV) void k_aa_fwd(HsrDev d) {
                 epred[view][slot] = dst / 9.f;
             }
         }
-        wave_lds_sync();
+        wave_lds_fence();
 #pragma unroll
         for (int c = 0; c < 4; c++) {
             if ((edge >> c) & 1u) {

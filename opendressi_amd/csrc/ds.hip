@@ -251,7 +251,7 @@ __device__ __forceinline__ float dist_face_sum(const FaceCorners& fc, uint32_t f
         if (!last && n_hits + 64 * kDistPx <= kDistHits) {
             continue;
         }
-        wave_lds_sync();
+        wave_lds_fence();
         for (uint32_t h0 = 0; h0 < n_hits; h0 += 64) {
             const uint32_t n = min(64u, n_hits - h0);
             if (lane < n) {
@@ -274,7 +274,7 @@ __device__ __forceinline__ float dist_face_sum(const FaceCorners& fc, uint32_t f
                     lds.term[lane][k * 3 + 2] = t[k].w;
                 }
             }
-            wave_lds_sync();
+            wave_lds_fence();
             // a contribution that the reference leaves out is +0 here: a sum
             // that starts at +0 is never -0, and +0 leaves it as it is
             if (lane < 9 && !twice) {
@@ -292,7 +292,7 @@ __device__ __forceinline__ float dist_face_sum(const FaceCorners& fc, uint32_t f
                     }
                 }
             }
-            wave_lds_sync();
+            wave_lds_fence();
         }
         n_hits = 0;
     }

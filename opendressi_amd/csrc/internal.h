@@ -47,6 +47,14 @@ namespace dressi {
 
 // Items of a batched per-op launch (grid y dimension).
 constexpr uint32_t kMaxBatchItems = 65535;
+// Orders the LDS accesses of one wave around an exchange between its lanes
+// (a wave executes its LDS instructions in order).
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Pixels of an image up to which its indices, and a step's past the last one,
 // fit 32 bits: more than the rasterizers have threads for.
 constexpr uint64_t kMaxImagePixels = 0xffff0000ull;

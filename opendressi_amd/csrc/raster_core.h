@@ -663,14 +663,6 @@ struct ResolveLds {
     };
 };
 
-// Orders the LDS accesses of one wave around an exchange between its lanes
-// (a wave executes its LDS instructions in order).
-__device__ __forceinline__ void wave_lds_fence() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // Sorts key[0 .. n) descending (bitonic network over the next power of two,
 // padded with zeros, which sort last). One wave; n <= kFarCap.
 __device__ __forceinline__ void sort_desc(uint32_t* key, uint32_t n) {

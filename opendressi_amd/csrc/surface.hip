@@ -161,14 +161,14 @@ __global__ __launch_bounds__(64) void k_surface_interp_bwd_faces(
             }
             n_hits += (uint32_t)__popcll(m);
         }
-        wave_lds_sync();
+        wave_lds_fence();
         if (lane < 3 * C) {
 #pragma unroll 16
             for (uint32_t q = 0; q < n_hits; q++) {
                 acc += term[grp][q][lane];
             }
         }
-        wave_lds_sync();
+        wave_lds_fence();
     }
     if (live && lane < 3 * C) {
         g_face[((size_t)blockIdx.y * n_faces + f) * 3 * C + lane] = acc;

@@ -7,13 +7,6 @@
 
 namespace dressi {
 
-// Orders a one-wave workgroup's LDS accesses.
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // A lane's way through a box of an image in raster order, `stride` pixels a
 // step (the lanes that share the box): an add and a carry in place of a
 // division per pixel.
