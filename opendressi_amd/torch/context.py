@@ -24,8 +24,7 @@ def tri_int32(tri: torch.Tensor) -> torch.Tensor:
 class MeshData:
     """Static-topology arrays of one triangle list, on the device
     (python/dressi/torch/meshdata.py:11-43): faces as float ids and as int32,
-    sequential faces of the unwelded corners, the per-corner face id, the
-    {max_deg, V} vertex -> face adjacency."""
+    the {max_deg, V} vertex -> face adjacency."""
 
     def __init__(self, tri: torch.Tensor, device: torch.device):
         # the source tensor is pinned: the cache key holds its data_ptr
@@ -36,11 +35,8 @@ class MeshData:
         faces_np = t.numpy().astype(np.float32)
         self.faces_f = torch.from_numpy(faces_np).to(device)
         self.faces_i = t.to(device)
-        self.faces_seq = torch.arange(self.n_faces * 3, dtype=torch.float32).reshape(-1, 3).to(device)
-        self.corner_face_id = torch.arange(self.n_faces, dtype=torch.float32).repeat_interleave(3).to(device)
         vft = vertex_faces_tex(faces_np, self.n_verts)
         self.vft = torch.from_numpy(vft).to(device)
-        self.max_deg = int(vft.shape[0])
 
 
 def mesh_key(tri: torch.Tensor) -> tuple:
@@ -51,9 +47,9 @@ class RasterizeHipContext:
     """MI355X counterpart of nvdiffrast's RasterizeGLContext and of the
     reference's RasterizeVulkanContext: one HIP device (`device`: index or
     torch device, default the current one) shared by every op. Per-signature
-    constant buffers are cached in `_engines` (keyed by shape, as the
-    reference keys its compiled graphs) and per-topology data in `_meshes`;
-    `clear_cache()` frees both."""
+    state (the antialias gradient's iteration counters) is kept in `_engines`,
+    keyed by shape as the reference keys its compiled graphs, and per-topology
+    data in `_meshes`; `clear_cache()` frees both."""
 
     def __init__(self, device=None, debug: bool = False):
         del debug

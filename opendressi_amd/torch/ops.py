@@ -33,8 +33,8 @@ def _needs_grad(*tensors) -> bool:
 
 
 class _Engine:
-    """Per-signature device constants (and the antialias backward's
-    iteration counter), built once per key."""
+    """Per-signature state (the antialias backward's iteration counter), built
+    once per key."""
 
     def __init__(self, **kw):
         self.__dict__.update(kw)
@@ -61,7 +61,6 @@ def rasterize(ctx: RasterizeHipContext, pos: torch.Tensor, tri: torch.Tensor, re
     md = ctx.mesh(tri)
     if md.n_verts > pos_b.shape[1]:
         raise IndexError(f"tri names vertex {md.n_verts - 1}, pos has {pos_b.shape[1]}")
-    ctx.engine(("rasterize", h, w, md.n_faces, md.n_verts, pos_b.shape[0]), _Engine)
     with ctx.lock:
         # every item in one pass
         rast, clip_vk = K.surface_rasterize(ctx._ctx, pos_b, md.faces_i, w, h)

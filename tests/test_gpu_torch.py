@@ -137,18 +137,38 @@ def test_rasterize_depth_order(dr, ctx):
 
 
 def test_engine_cache_reuse(dr, ctx):
+    """What a context keeps: one MeshData for each triangle tensor and version of it, one antialias
+    engine for each signature, whose iteration counter continues from call to call; a forward pass
+    of any size adds nothing."""
     print("[torch] engine cache", flush=True)
     tri = torch.tensor([[0, 1, 2]], dtype=torch.int32)
     p1 = torch.tensor([[-0.5, -0.5, 0.0, 1.0], [0.5, -0.5, 0.0, 1.0], [-0.5, 0.5, 0.0, 1.0]])
     p2 = p1 * torch.tensor([1.5, 1.5, 1.0, 1.0])
-    n0 = len(ctx._engines)
+    n0, m0 = set(ctx._engines), len(ctx._meshes)
     r1, _ = dr.rasterize(ctx, p1, tri, resolution=[6, 6])
-    n1 = len(ctx._engines)
+    mesh = ctx.mesh(tri)
     r2, _ = dr.rasterize(ctx, p2, tri, resolution=[6, 6])
-    assert len(ctx._engines) == n1 == n0 + 1
+    assert len(ctx._meshes) == m0 + 1 and ctx.mesh(tri) is mesh
     assert not torch.equal(r1, r2)
     dr.rasterize(ctx, p1, tri, resolution=[12, 12])
-    assert len(ctx._engines) == n1 + 1
+    assert set(ctx._engines) == n0 and len(ctx._meshes) == m0 + 1
+
+    def backward(rast, size):
+        pos = p1.clone().requires_grad_(True)
+        out = dr.antialias(torch.rand(1, size, size, 1), rast, pos, tri, n_samples=4)
+        out.sum().backward()
+        return set(ctx._engines) - n0
+
+    keys = backward(r1, 6)
+    assert len(keys) == 1
+    eng = ctx._engines[next(iter(keys))]
+    assert eng.iter_seed == 1
+    assert backward(r1, 6) == keys and ctx._engines[next(iter(keys))] is eng
+    assert eng.iter_seed == 2
+    r12, _ = dr.rasterize(ctx, p1, tri, resolution=[12, 12])
+    assert len(backward(r12, 12)) == 2 and eng.iter_seed == 2
+    tri[0, 0] = 0  # another version of the tensor
+    assert ctx.mesh(tri) is not mesh and len(ctx._meshes) == m0 + 2
 
 
 def test_rasterize_batch(dr, ctx):
