@@ -186,6 +186,9 @@ void or_gather_dist_grad(const float* gy, const float* ro, const float* clip, ui
  * (EquirectSampleBwd + TileSum, f_ops.cpp:2786-2919) -> out {mw,mh} x n */
 int or_equirect_sample(const float* map, uint32_t mw, uint32_t mh, uint32_t n, const float* dir,
                        uint32_t dw, uint32_t dh, const float* gy, float* out);
+/* ... and that VJP summed in 64-bit fixed point -> out {mw,mh} x n */
+int or_equirect_vjp_fixed(const float* gy, uint32_t n, const float* dir, uint32_t dw, uint32_t dh,
+                          uint32_t mw, uint32_t mh, float* out);
 /* AvgPool2x2 (f_ops.cpp:3411-3415); with gy its VJP -> out {w,h} x n */
 int or_avg_pool2x2(const float* x, uint32_t w, uint32_t h, uint32_t n, const float* gy,
                    float* out);

@@ -209,6 +209,48 @@ int or_equirect_sample(const float* map, uint32_t mw, uint32_t mh, uint32_t n, c
     return 0;
 }
 
+/* The same map VJP with every gy * weight product (the reference's float)
+ * rounded to a multiple of 2^-k and summed in 64 bits, 2^k the largest scale
+ * at which npx * max|gy| stays below 2^62: no order, so one set of bits. */
+int or_equirect_vjp_fixed(const float* gy, uint32_t n, const float* dir, uint32_t dw, uint32_t dh,
+                          uint32_t mw, uint32_t mh, float* out) {
+    const size_t npx = (size_t)dw * dh, msz = (size_t)mw * mh * n;
+    int64_t* acc = (int64_t*)calloc(msz, sizeof(int64_t));
+    if (!acc) return -1;
+    float peak = 0.f;
+    for (size_t i = 0; i < npx * n; i++) {
+        if (isfinite(gy[i]) && fabsf(gy[i]) > peak) peak = fabsf(gy[i]);
+    }
+    int e = 62;
+    if (peak > 0.f) frexp((double)peak * (double)npx, &e);
+    const int k = 62 - e;
+    for (size_t p = 0; p < npx; p++) {
+        V3 d = v3(dir[p * 3 + 0], dir[p * 3 + 1], dir[p * 3 + 2]);
+        const float dlen = sqrtf(dot3(d, d));
+        if (dlen < 1e-8f) continue;
+        d = v3(d.x / dlen, d.y / dlen, d.z / dlen);
+        float u, v;
+        equirect_uv(d, &u, &v);
+        const float sx = u * (float)mw - 0.5f, sy = v * (float)mh - 0.5f;
+        const int ix = (int)floorf(sx), iy = (int)floorf(sy);
+        const float fx = sx - (float)ix, fy = sy - (float)iy;
+        for (int t = 0; t < 4; t++) {
+            int x = ix + (t & 1);
+            if (x < 0) x += (int)mw;
+            if (x >= (int)mw) x -= (int)mw;
+            const int y = clampi(iy + (t >> 1), 0, (int)mh - 1);
+            const float w = (t & 1 ? fx : 1.f - fx) * (t >> 1 ? fy : 1.f - fy);
+            for (uint32_t c = 0; c < n; c++) {
+                const float term = gy[p * n + c] * w;
+                acc[((size_t)y * mw + (uint32_t)x) * n + c] += llrint(ldexp((double)term, k));
+            }
+        }
+    }
+    for (size_t i = 0; i < msz; i++) out[i] = (float)ldexp((double)acc[i], -k);
+    free(acc);
+    return 0;
+}
+
 /* AvgPool2x2 = Reduce2x2Sum(x) * 0.25 (f_ops.cpp:3411-3415, 996-1033); its
  * VJP is UpsampleNearest2x(gy * 0.25) (f_ops.cpp:958-994). x {w,h} x n. */
 int or_avg_pool2x2(const float* x, uint32_t w, uint32_t h, uint32_t n, const float* gy,

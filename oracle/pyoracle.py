@@ -216,6 +216,15 @@ class _Lib:
                    _U32(dw), _U32(dh), _fp(gy), _fp(out))
         return out
 
+    def equirect_vjp_fixed(self, dirs, gy, mw, mh):
+        """The map VJP {mh, mw, n} summed in 64-bit fixed point."""
+        dirs, gy = _f32(dirs), _f32(gy)
+        dh, dw, n = gy.shape
+        out = np.zeros((mh, mw, n), np.float32)
+        self._call("equirect_vjp_fixed", _fp(gy), _U32(n), _fp(dirs), _U32(dw), _U32(dh), _U32(mw),
+                   _U32(mh), _fp(out))
+        return out
+
     def avg_pool2x2(self, x, gy=None):
         x = _f32(x)
         h, w, n = x.shape
@@ -291,8 +300,8 @@ class Oracle(_Lib):
         self.fn("vertex_faces_tex").restype = C.c_uint32
 
     # functions of the restatement that return a status (the rest are void)
-    _STATUS = frozenset(("equirect_sample", "avg_pool2x2", "irradiance_conv", "prefilter_conv",
-                         "prefilter_env", "brdf_lut", "pbr_fit"))
+    _STATUS = frozenset(("equirect_sample", "equirect_vjp_fixed", "avg_pool2x2", "irradiance_conv",
+                         "prefilter_conv", "prefilter_env", "brdf_lut", "pbr_fit"))
 
     def _call(self, name, *args):
         rc = self.fn(name)(*args)

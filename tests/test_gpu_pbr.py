@@ -119,11 +119,22 @@ def test_ibl_convs_match_oracle_at_map_sizes(ctx, oracle, shape):
            oracle.irradiance_conv(env, ow // 2, oh // 2), "irradiance")
 
 
+def _same_floats(a, b, what):
+    """The same bits, NaN (of any kind) in the same places."""
+    assert np.array_equal(np.isnan(a), np.isnan(b)), f"{what}: NaN in other places"
+    _exact(np.where(np.isnan(a), 0.0, a), np.where(np.isnan(b), 0.0, b), what)
+
+
 @pytest.mark.parametrize("shape", [
-    # (source w, h, output w, h, channels): workgroups of 8 outputs and chunks of 128 sources,
-    # whole, one past and one short of them; single texels; every channel count
-    (16, 8, 4, 2, 3), (43, 3, 1, 1, 4), (129, 1, 3, 3, 1), (128, 2, 9, 1, 2), (127, 3, 17, 5, 3),
-    (1, 1, 16, 8, 3)])
+    # (source w, h, output w, h, channels). More than 2048 outputs: workgroups of 8 and chunks of
+    # 128 sources, whole, one past and one short of them, single texels, every channel count,
+    # forward ...
+    (43, 3, 2051, 1, 4), (127, 1, 2050, 1, 1), (1, 1, 2049, 1, 2), (128, 2, 683, 3, 3),
+    # ... and back (the source's texels are the outputs)
+    (2049, 1, 1, 1, 4), (683, 3, 127, 1, 1), (2050, 1, 129, 1, 2), (2056, 1, 257, 1, 3),
+    # both; at most 2048 outputs, which take the other form
+    (2049, 1, 2049, 1, 1), (16, 8, 4, 2, 3), (43, 3, 1, 1, 4), (129, 1, 3, 3, 1),
+    (128, 2, 9, 1, 2), (127, 3, 17, 5, 3), (1, 1, 16, 8, 3)])
 def test_ibl_conv_chunks_match_oracle(ctx, oracle, shape):
     """Bit for bit, forward and back; an infinite and a NaN source value reach the sums that the
     reference's order brings them to."""
@@ -136,14 +147,14 @@ def test_ibl_conv_chunks_match_oracle(ctx, oracle, shape):
 
     def check(env, gy):
         for rough in (0.0, 0.7):
-            _exact(np.nan_to_num(host(ops.prefilter_conv(ctx, dev(env), ow, oh, rough))),
-                   np.nan_to_num(oracle.prefilter_conv(env, ow, oh, rough)), f"pref {rough}")
-            _exact(np.nan_to_num(host(ops.prefilter_conv_bwd(ctx, dev(gy), sw, sh, rough))),
-                   np.nan_to_num(oracle.prefilter_conv(env, ow, oh, rough, gy)), f"bwd {rough}")
-        _exact(np.nan_to_num(host(ops.irradiance_conv(ctx, dev(env), ow, oh))),
-               np.nan_to_num(oracle.irradiance_conv(env, ow, oh)), "irradiance")
-        _exact(np.nan_to_num(host(ops.irradiance_conv_bwd(ctx, dev(gy), sw, sh))),
-               np.nan_to_num(oracle.irradiance_conv(env, ow, oh, gy)), "irradiance bwd")
+            _same_floats(host(ops.prefilter_conv(ctx, dev(env), ow, oh, rough)),
+                         oracle.prefilter_conv(env, ow, oh, rough), f"pref {rough}")
+            _same_floats(host(ops.prefilter_conv_bwd(ctx, dev(gy), sw, sh, rough)),
+                         oracle.prefilter_conv(env, ow, oh, rough, gy), f"bwd {rough}")
+        _same_floats(host(ops.irradiance_conv(ctx, dev(env), ow, oh)),
+                     oracle.irradiance_conv(env, ow, oh), "irradiance")
+        _same_floats(host(ops.irradiance_conv_bwd(ctx, dev(gy), sw, sh)),
+                     oracle.irradiance_conv(env, ow, oh, gy), "irradiance bwd")
 
     check(env, gy)
     env.flat[0], gy.flat[-1] = np.inf, np.nan
@@ -216,12 +227,16 @@ def test_equirect_sample_smooth_map_and_vjp(ctx, oracle):
     # largest (6144 entries) and smallest; one entry past it (hash table) and with four channels;
     # a list of directions; images smaller than a tile and one past its edges
     (64, 32, 3, 33, 65), (1, 1, 1, 5, 7), (4, 2, 3, 70, 31), (2049, 1, 3, 40, 40),
-    (97, 49, 4, 64, 33), (3073, 2, 1, 1, 1500), (128, 64, 3, 1, 1), (128, 64, 2, 1025, 1)])
+    (97, 49, 4, 64, 33), (3073, 2, 1, 1, 1500), (128, 64, 3, 1, 1), (128, 64, 2, 1025, 1),
+    # 16 pixels per texel and more: the smaller hash table with four sums per texel, of 512 and
+    # (four channels) 256 texels; one pixel row short of it
+    (128, 64, 3, 512, 512), (97, 49, 4, 300, 260), (97, 49, 4, 292, 260)])
 @pytest.mark.parametrize("coherent", [True, False])
 def test_equirect_vjp_tiles(ctx, oracle, shape, coherent):
-    """The map VJP over the forms of its tile sums: against the oracle's ordered float sums within
-    their rounding, 2^-24 of the sum of magnitudes for each of a texel's (at most 4 pixels each)
-    terms, and the same bits on a second run. Incoherent directions overflow the hash table."""
+    """The map VJP over the forms of its tile sums: the bits of the same 64-bit sums on the host,
+    and the oracle's ordered float sums within their rounding, 2^-24 of the sum of magnitudes for
+    each of a texel's (at most 4 pixels each) terms. Incoherent directions overflow the hash
+    table."""
     from opendressi_amd import ops
     mw, mh, nc, h, w = shape
     print(f"[equirect vjp] map {mw}x{mh}x{nc} dirs {h}x{w} coherent {coherent}", flush=True)
@@ -241,7 +256,7 @@ def test_equirect_vjp_tiles(ctx, oracle, shape, coherent):
     bar = 4.0 * h * w * (2.0 ** -24 * size + 2.0 ** -61 * h * w * float(np.abs(gy).max()))
     err = np.abs(got.astype(np.float64) - ref)
     assert (err <= bar).all(), (float(err.max()), float((err - bar).max()))
-    _exact(host(ops.equirect_sample_bwd(ctx, dev(gy), dev(d), mw, mh)), got, "rerun")
+    _exact(got, oracle.equirect_vjp_fixed(d, gy, mw, mh), "64-bit sums")
 
 
 def test_equirect_vjp_of_a_long_list(ctx):
