@@ -532,53 +532,64 @@ __global__ __launch_bounds__(kAaExactThreads) void k_antialias_bwd_vtx_exact_op(
 
 // The torch surface's stochastic vertex gradient: k_antialias_bwd_vtx_op's
 // rows and ColSum for an adjacency that is the faces' own (VertexFacesTex), so
-// that the rows of one face are its three corners'. One wave per face and item
-// takes eight samples at once, a lane per (sample, neighbour), tests each pair
-// by what needs no geometry (two faces, dot(gy(s), c(s) - c(n)) / 9 not 0),
-// evaluates the few left and adds their terms per corner in (sample,
-// neighbour, endpoint) order into g_corner {N,F,3} (x, y, w).
+// that the rows of one face are its three corners'. S samples of a face and
+// item at once, a lane per (sample, neighbour), 8 / S faces to a wave: each
+// lane tests its pair by what needs no geometry (two faces, dot(gy(s), c(s) -
+// c(n)) / 9 not 0), the few left are evaluated and their terms added per
+// corner in (sample, neighbour, endpoint) order into g_corner {N,F,3} (x, y,
+// w).
 //
 // The row form repeats every face's samples for its three corners and waits
 // for each sample's loads in turn: 66 us for eight views of 642 vertices
-// and eight samples, this 17 + 6.
+// and eight samples, this 17 + 6. S follows the sample count: a wave for a
+// face of one sample is idle but for eight lanes, and many faces (327 680 on
+// 256 x 256 pixels) then take as long as their waves take to start, 400 us,
+// where the rows take 310.
+template <uint32_t S>
 __global__ __launch_bounds__(64) void k_surface_aa_bwd_faces(
         const float* gy, const float* img, uint32_t n_comp, const float* tri_f,
         uint32_t tri_stride, const float4* clip, uint32_t n_verts, int clip_per_item,
         const float* faces, uint32_t n_faces, uint64_t seed0, uint32_t n_samples, uint32_t w,
         uint32_t h, float* g_corner) {
+    constexpr uint32_t G = 8 * S;  // lanes of a face
+    static_assert(G >= 9 && 64 % G == 0, "a lane per corner and component");
     __shared__ float term[64][6];   // endpoint a's x, y, w, then b's
     __shared__ uint32_t end[64][2];  // their vertices
-    const uint32_t f = blockIdx.x, lane = threadIdx.x;
+    // (a wave's one face is the wave's: scalar loads)
+    const uint32_t grp = G == 64 ? 0u : threadIdx.x / G;
+    const uint32_t lane = G == 64 ? threadIdx.x : threadIdx.x % G;
+    const uint32_t f = blockIdx.x * (64 / G) + grp;
     const AaItem it(w, h);
     gy = it.img(gy, n_comp);
     img = it.img(img, n_comp);
     const TriIds tri = it.tri(tri_f, tri_stride);
     clip = it.clip(clip, n_verts, clip_per_item);
-    g_corner += ((size_t)it.item * n_faces + f) * 9;
     const float W = (float)w, H = (float)h;
     // the sampler's seed: an integer held in float32, as the image {1,1} the
     // reference reads it from
     const uint32_t seed_u = (uint32_t)(int64_t)((float)(seed0 + it.item) + 0.5f);
+    const bool live = G == 64 || f < n_faces;
     uint32_t vi[3];
     float4 c[3];
-    bool ok = true;
+    bool ok = live;
 #pragma unroll
     for (int q = 0; q < 3; q++) {
-        vi[q] = FloatFaces{faces}(f, q);
+        vi[q] = live ? FloatFaces{faces}(f, q) : n_verts;
         ok = ok && vi[q] < n_verts;
         c[q] = ok ? clip[vi[q]] : make_float4(0.f, 0.f, 0.f, 0.f);
     }
     float s3x[3], s3y[3];
     ok = ok && aa_face_screen(c, W, H, s3x, s3y);
-    // lane 3 r + comp < 9 sums corner r's component
+    // lane 3 r + comp < 9 of a face sums corner r's component
     const uint32_t comp = lane % 3;
     const uint32_t my = lane < 3 ? vi[0] : lane < 6 ? vi[1] : vi[2];
     float acc = 0.f;
-    for (uint32_t smp0 = 0; ok && smp0 < n_samples; smp0 += 8) {
+    for (uint32_t smp0 = 0; smp0 < n_samples && (G < 64 || ok); smp0 += S) {
         const uint32_t smp = smp0 + (lane >> 3), k = lane & 7u;
         int x = 0, y = 0;
-        bool cand = smp < n_samples && aa_sample_px(s3x, s3y, f, smp, seed_u, &x, &y) && x >= 0 &&
-                    y >= 0 && x < (int)w && y < (int)h;
+        bool cand = (G == 64 || ok) && smp < n_samples &&
+                    aa_sample_px(s3x, s3y, f, smp, seed_u, &x, &y) && x >= 0 && y >= 0 &&
+                    x < (int)w && y < (int)h;
         const int nx = x + kAaOffX[k], ny = y + kAaOffY[k];
         cand = cand && nx >= 0 && ny >= 0 && nx < (int)w && ny < (int)h;
         uint32_t its = 0, itn = 0;
@@ -597,12 +608,14 @@ __global__ __launch_bounds__(64) void k_surface_aa_bwd_faces(
         cand = cand && eval_aa_pair(its, itn, x, y, nx, ny, n_faces,
                                     TriFromClip{faces, clip, n_verts, W, H}, &pr) &&
                pr.r < 1.f;
-        const uint64_t m = __ballot(cand);
-        if (!m) {
+        const uint64_t all = __ballot(cand);
+        if (!all) {
             continue;
         }
+        // the face's lanes of the ballot
+        const uint64_t m = (all >> (grp * G)) & (~0ull >> (64 - G));
         if (cand) {
-            const uint32_t at = (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
+            const uint32_t at = grp * G + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
             float dqa[2], dqb[2];
             aa_pair_dq(pr, x, y, dqa, dqb);
             float4 ta = make_float4(0.f, 0.f, 0.f, 0.f), tb = ta;
@@ -620,7 +633,7 @@ __global__ __launch_bounds__(64) void k_surface_aa_bwd_faces(
         __syncthreads();
         if (lane < 9) {
             const uint32_t n = (uint32_t)__popcll(m);
-            for (uint32_t q = 0; q < n; q++) {
+            for (uint32_t q = grp * G; q < grp * G + n; q++) {
                 // another vertex's term is left out by adding +0: a sum that
                 // starts at +0 is never -0
                 acc += end[q][0] == my ? term[q][comp] : 0.f;
@@ -629,8 +642,8 @@ __global__ __launch_bounds__(64) void k_surface_aa_bwd_faces(
         }
         __syncthreads();
     }
-    if (lane < 9) {
-        g_corner[lane] = acc;
+    if (live && lane < 9) {
+        g_corner[((size_t)it.item * n_faces + f) * 9 + lane] = acc;
     }
 }
 
@@ -1738,9 +1751,19 @@ int dressi_surface_antialias_bwd_pos(dressi_ctx* ctx, const float* gy, const flo
                                 boost, out);
     }
     if (n_faces) {
-        hipLaunchKernelGGL(k_surface_aa_bwd_faces, dim3(n_faces, n_items), dim3(64), 0,
-                           ctx->stream, gy, img, n_comp, rast + 3, 4u, (const float4*)pos, n_verts,
-                           pos_per_item, faces, n_faces, seed, n_samples, width, height, g_corner);
+        const auto launch = [&](auto kernel, uint32_t per_wave) {
+            hipLaunchKernelGGL(kernel, dim3(div_up(n_faces, per_wave), n_items), dim3(64), 0,
+                               ctx->stream, gy, img, n_comp, rast + 3, 4u, (const float4*)pos,
+                               n_verts, pos_per_item, faces, n_faces, seed, n_samples, width,
+                               height, g_corner);
+        };
+        if (n_samples <= 2) {
+            launch(k_surface_aa_bwd_faces<2>, 4);
+        } else if (n_samples <= 4) {
+            launch(k_surface_aa_bwd_faces<4>, 2);
+        } else {
+            launch(k_surface_aa_bwd_faces<8>, 1);
+        }
         DRESSI_CHECK_LAUNCH();
     }
     hipLaunchKernelGGL(k_surface_aa_bwd_vtx, dim3(div_up(n_rows, 256), n_items), dim3(256), 0,

@@ -137,6 +137,32 @@ def test_surface_antialias(ctx, level, n, h, w, nc, samples, shared):
     ctx.synchronize()
 
 
+@pytest.mark.parametrize("samples", [1, 2, 3, 4, 5, 9])
+@pytest.mark.parametrize("drop", [0, 1, 2, 3])
+def test_surface_antialias_faces_of_a_wave(ctx, samples, drop):
+    """Four, two or one face to a wave by the sample count, face counts that leave a wave's last
+    groups empty, fewer samples than a group takes at once and more; against the wide partials
+    and ColSum."""
+    import opendressi_amd as od
+    from opendressi_amd import ops as K
+    print(f"[surface antialias] {samples} samples, {drop} faces dropped", flush=True)
+    n, h, w = 2, 61, 97
+    clip, fi, ff, _ = _scene(2, n, 11)
+    fi, ff = fi[:len(fi) - drop].contiguous(), ff[:len(ff) - drop].contiguous()
+    vf = torch.from_numpy(od.vertex_faces_tex(ff.cpu().numpy(), clip.shape[1])).cuda()
+    rast, vk = K.surface_rasterize(ctx, clip, fi, w, h)
+    gen = torch.Generator(device="cuda").manual_seed(samples)
+    img = torch.rand((n, h, w, 3), device="cuda", generator=gen)
+    g = torch.randn((n, h, w, 3), device="cuda", generator=gen)
+    got = K.surface_antialias_bwd_pos(ctx, g, img, rast, clip, ff, vf, 5 * n, samples, 1.0)
+    seeds = torch.tensor([float(5 * n + i) for i in range(n)], device="cuda")
+    ref = K.col_sum_batch(ctx, K.antialias_bwd_vtx_batch(ctx, g, img, rast[..., 3].contiguous(),
+                                                         vk, ff, vf, seeds, samples, True))
+    assert float(ref.abs().max()) > 0
+    _same(got, ref, "position gradient")
+    ctx.synchronize()
+
+
 def _peel_threshold(rs, radius_px):
     dist, z, cov = rs[..., 0], rs[..., 2], rs[..., 3]
     ge = (dist >= 0.0).to(torch.float32)
