@@ -352,28 +352,42 @@ __global__ __launch_bounds__(256) void k_antialias_bwd_vtx_op(
 // belongs to a face covering s or its neighbour, so no pair of v's lies
 // outside those pixels.
 //
-// One workgroup per vertex. Its pairs were one thread's serial chain (a few
-// thousand pairs at a memory latency each: 12 ms at 61 x 97 pixels, 162
-// vertices, on three wavefronts). Now 256 pixels a step: each thread tests
-// its pixel's eight pairs by what needs no geometry (the faces differ, and
-// dot(gy(s), c(s) - c(n)) / 9 is not 0: else the pair adds nothing), the
-// pairs left are listed in raster and neighbour order, evaluated side by
-// side, and their terms added one by one: 21 us, a handful of dependent
-// loads and barriers per step.
-constexpr uint32_t kAaExactThreads = 256;
+// G lanes of a T-thread workgroup per vertex. Its pairs were one thread's
+// serial chain (a few thousand pairs at a memory latency each: 12 ms at 61 x
+// 97 pixels, 162 vertices, on three wavefronts). Now G pixels a step: each
+// lane tests its pixel's eight pairs by what needs no geometry (the faces
+// differ, and dot(gy(s), c(s) - c(n)) / 9 is not 0: else the pair adds
+// nothing), the pairs left are listed in raster and neighbour order,
+// evaluated side by side, and their terms added one by one: 21 us, a handful
+// of dependent loads and barriers per step.
+//
+// Few vertices take 256 lanes each (one 512 x 512 view of 2562 vertices, every
+// pair counting: 212 us, 363 with a wave each). Where the vertices fill the
+// GPU as waves, so many workgroups of 256 take longer to start than to run,
+// and a wave each is faster (10 242 vertices on 64 x 64 pixels 136 -> 74 us,
+// 163 842 on 512 x 512 2070 -> 956). And where these are more than a pixel in
+// two each, eight lanes each (163 842 on 128 x 128 635 -> 551, 655 362 2225 ->
+// 1648; the thread per vertex 799 and 1397; 10 242 on 64 x 64, too few for it,
+// 74 -> 177).
+constexpr uint32_t kAaExactWaveVerts = 8192;     // vertices and items for a wave each
+constexpr uint32_t kAaExactLanesVerts = 131072;  // and for eight lanes each
 
-__global__ __launch_bounds__(kAaExactThreads) void k_antialias_bwd_vtx_exact_op(
+template <uint32_t T, uint32_t G>
+__global__ __launch_bounds__(T) void k_antialias_bwd_vtx_exact_op(
         const float* gy, const float* img, uint32_t n_comp, const float* tri_f, uint32_t tri_stride,
         const float4* clip, uint32_t n_verts, int clip_per_item, const float* faces,
         uint32_t n_faces, const float* vtx_faces, uint32_t n_rows, uint32_t max_deg, uint32_t w,
         uint32_t h, float scale, uint32_t first, float4* out) {
-    constexpr uint32_t T = kAaExactThreads;
-    __shared__ int box[4];
+    constexpr uint32_t NG = T / G;  // vertices of the workgroup
+    static_assert(NG == 1 || T == 64, "several vertices share one wave");
+    __shared__ int box[NG][4];
     __shared__ uint32_t wave_pairs[T / 64];
-    __shared__ uint16_t pair[T * 8];  // thread of the pixel << 3 | neighbour
-    __shared__ float term[T][6];      // endpoint a's x, y, w, then b's
+    __shared__ uint16_t pair[NG][G * 8];  // lane of the pixel << 3 | neighbour
+    __shared__ float term[T][6];          // endpoint a's x, y, w, then b's
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-    const uint32_t v = first + blockIdx.x;
+    const uint32_t grp = NG == 1 ? 0u : tid / G, gl = NG == 1 ? tid : tid % G;
+    const uint32_t v = first + blockIdx.x * NG + grp;
+    const bool live = NG == 1 || v < n_rows;
     const AaItem it(w, h);
     gy = it.img(gy, n_comp);
     img = it.img(img, n_comp);
@@ -381,14 +395,14 @@ __global__ __launch_bounds__(kAaExactThreads) void k_antialias_bwd_vtx_exact_op(
     clip = it.clip(clip, n_verts, clip_per_item);
     out += (size_t)it.item * n_rows;
     const float W = (float)w, H = (float)h;
-    if (tid == 0) {
-        box[0] = (int)w;
-        box[1] = (int)h;
-        box[2] = -1;
-        box[3] = -1;
+    if (gl == 0) {
+        box[grp][0] = (int)w;
+        box[grp][1] = (int)h;
+        box[grp][2] = -1;
+        box[grp][3] = -1;
     }
     __syncthreads();
-    for (uint32_t d = tid; d < max_deg; d += T) {
+    for (uint32_t d = gl; live && d < max_deg; d += G) {
         const float fv = vtx_faces[(size_t)d * n_rows + v];
         if (fv < -0.5f) {
             continue;
@@ -405,22 +419,28 @@ __global__ __launch_bounds__(kAaExactThreads) void k_antialias_bwd_vtx_exact_op(
         int fx0, fy0, fx1, fy1;
         pixel_bbox(qx[0], qx[1], qx[2], qy[0], qy[1], qy[2], (int)w, (int)h, &fx0, &fy0, &fx1,
                    &fy1);
-        atomicMin(&box[0], fx0 - 1);
-        atomicMin(&box[1], fy0 - 1);
-        atomicMax(&box[2], fx1 + 1);
-        atomicMax(&box[3], fy1 + 1);
+        atomicMin(&box[grp][0], fx0 - 1);
+        atomicMin(&box[grp][1], fy0 - 1);
+        atomicMax(&box[grp][2], fx1 + 1);
+        atomicMax(&box[grp][3], fy1 + 1);
     }
     __syncthreads();
-    const int bx0 = max(box[0], 0), by0 = max(box[1], 0);
-    const int bx1 = min(box[2], (int)w - 1), by1 = min(box[3], (int)h - 1);
-    float acc = 0.f;  // threads 0, 1, 2: the row's x, y, w
+    const int bx0 = max(box[grp][0], 0), by0 = max(box[grp][1], 0);
+    const int bx1 = min(box[grp][2], (int)w - 1), by1 = min(box[grp][3], (int)h - 1);
+    float acc = 0.f;  // a vertex's lanes 0, 1, 2: the row's x, y, w
     const uint32_t bw = bx1 >= bx0 ? (uint32_t)(bx1 - bx0 + 1) : 0u;
     const uint32_t n_px = by1 >= by0 ? bw * (uint32_t)(by1 - by0 + 1) : 0u;
-    for (uint32_t p0 = 0; p0 < n_px; p0 += T) {
+    // (a wave of several vertices goes on until the last is done)
+    const auto more = [](bool go) { return NG == 1 ? go : (bool)__any(go); };
+    // the vertex's lanes of a ballot
+    const auto lanes = [&](uint64_t m) {
+        return G < 64 ? (m >> (grp * G)) & ((1ull << (G & 63u)) - 1ull) : m;
+    };
+    for (uint32_t p0 = 0; more(p0 < n_px); p0 += G) {
         uint32_t mask = 0;
-        if (p0 + tid < n_px) {
-            const uint32_t row = (p0 + tid) / bw;
-            const int x = bx0 + (int)(p0 + tid - row * bw), y = by0 + (int)row;
+        if (p0 + gl < n_px) {
+            const uint32_t row = (p0 + gl) / bw;
+            const int x = bx0 + (int)(p0 + gl - row * bw), y = by0 + (int)row;
             const size_t s = (size_t)y * w + x;
             const uint32_t its = tri(s);
             float gs[4], cs[4];
@@ -446,41 +466,45 @@ __global__ __launch_bounds__(kAaExactThreads) void k_antialias_bwd_vtx_exact_op(
             }
         }
         // the pairs in raster order: waves, lanes, neighbours
-        uint32_t before = 0, own = 0;
+        uint32_t before = 0, n_pairs = 0;
 #pragma unroll
         for (int k = 0; k < 8; k++) {
-            const uint64_t m = __ballot((mask >> k) & 1u);
-            before += (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
-            own += (uint32_t)__popcll(m);
+            const uint64_t m = lanes(__ballot((mask >> k) & 1u));
+            before += (uint32_t)__popcll(m & ((1ull << (T == 64 ? gl : lane)) - 1ull));
+            n_pairs += (uint32_t)__popcll(m);
         }
-        if (lane == 0) {
-            wave_pairs[wave] = own;
-        }
-        __syncthreads();
-        uint32_t n_pairs = 0;
+        if (T > 64) {
+            if (lane == 0) {
+                wave_pairs[wave] = n_pairs;
+            }
+            __syncthreads();
+            n_pairs = 0;
 #pragma unroll
-        for (uint32_t q = 0; q < T / 64; q++) {
-            before += q < wave ? wave_pairs[q] : 0u;
-            n_pairs += wave_pairs[q];
+            for (uint32_t q = 0; q < T / 64; q++) {
+                before += q < wave ? wave_pairs[q] : 0u;
+                n_pairs += wave_pairs[q];
+            }
         }
         for (uint32_t m = mask; m; m &= m - 1) {
-            pair[before++] = (uint16_t)(tid << 3 | (uint32_t)__builtin_ctz(m));
+            pair[grp][before++] = (uint16_t)(gl << 3 | (uint32_t)__builtin_ctz(m));
         }
         __syncthreads();
-        for (uint32_t q0 = 0; q0 < n_pairs; q0 += T) {
-            const uint32_t n_now = min(T, n_pairs - q0);
+        for (uint32_t q0 = 0; more(q0 < n_pairs); q0 += G) {
+            uint32_t n_now = q0 < n_pairs ? min(G, n_pairs - q0) : 0u;
             float t[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-            if (tid < n_now) {
-                const uint32_t pk = pair[q0 + tid];
+            bool mine = false;
+            if (gl < n_now) {
+                const uint32_t pk = pair[grp][q0 + gl];
                 const uint32_t p = p0 + (pk >> 3), k = pk & 7u;
                 const uint32_t row = p / bw;
                 const int x = bx0 + (int)(p - row * bw), y = by0 + (int)row;
                 const int nx = x + kAaOffX[k], ny = y + kAaOffY[k];
                 const size_t s = (size_t)y * w + x, n = (size_t)ny * w + nx;
                 AaPair pr;
-                if (eval_aa_pair(tri(s), tri(n), x, y, nx, ny, n_faces,
-                                 TriFromClip{faces, clip, n_verts, W, H}, &pr) &&
-                    !(pr.r >= 1.f) && (pr.ia == v || pr.ib == v)) {
+                mine = eval_aa_pair(tri(s), tri(n), x, y, nx, ny, n_faces,
+                                    TriFromClip{faces, clip, n_verts, W, H}, &pr) &&
+                       !(pr.r >= 1.f) && (pr.ia == v || pr.ib == v);
+                if (mine) {
                     float gr = 0.f;
                     for (uint32_t c = 0; c < n_comp; c++) {
                         gr += gy[s * n_comp + c] * (img[s * n_comp + c] - img[n * n_comp + c]);
@@ -504,27 +528,36 @@ __global__ __launch_bounds__(kAaExactThreads) void k_antialias_bwd_vtx_exact_op(
                     }
                 }
             }
+            uint32_t at = tid;
+            if (T == 64) {
+                // the pairs that are not v's left out
+                const uint64_t m = lanes(__ballot(mine));
+                at = grp * G + (uint32_t)__popcll(m & ((1ull << gl) - 1ull));
+                n_now = (uint32_t)__popcll(m);
+            }
+            if (T > 64 || mine) {
 #pragma unroll
-            for (int c = 0; c < 6; c++) {
-                term[tid][c] = t[c];
+                for (int c = 0; c < 6; c++) {
+                    term[at][c] = t[c];
+                }
             }
             __syncthreads();
-            if (tid < 3) {
+            if (gl < 3) {
                 // a pair or endpoint that is not v's is +0 here: a sum that
                 // starts at +0 is never -0, and +0 leaves it as it is
 #pragma unroll 4
                 for (uint32_t q = 0; q < n_now; q++) {
-                    acc += term[q][tid];
-                    acc += term[q][3 + tid];
+                    acc += term[grp * G + q][gl];
+                    acc += term[grp * G + q][3 + gl];
                 }
             }
             __syncthreads();
         }
     }
-    if (tid < 3) {
+    if (live && gl < 3) {
         float* dst = (float*)&out[v];
-        dst[tid == 2 ? 3 : tid] = acc * scale;
-        if (tid == 0) {
+        dst[gl == 2 ? 3 : gl] = acc * scale;
+        if (gl == 0) {
             dst[2] = 0.f * scale;
         }
     }
@@ -1522,21 +1555,30 @@ int check_aa_args(dressi_ctx* ctx, uint32_t n_comp, uint32_t w, uint32_t h) {
     return DRESSI_OK;
 }
 
-// A workgroup per vertex: pieces of 8 M vertices.
 int launch_vtx_exact(dressi_ctx* ctx, const float* gy, const float* img, uint32_t n_comp,
                      const float* tri, uint32_t tri_stride, const float* clip, uint32_t n_verts,
                      int clip_per_item, const float* faces, uint32_t n_faces,
                      const float* vtx_faces, uint32_t n_rows, uint32_t max_deg, uint32_t w,
                      uint32_t h, uint32_t n_items, float scale, float* out) {
-    constexpr uint32_t kBlocks = (uint32_t)(kLaunchThreads / kAaExactThreads);
-    for (uint32_t first = 0; first < n_rows; first += kBlocks) {
-        hipLaunchKernelGGL(k_antialias_bwd_vtx_exact_op,
-                           dim3(std::min(n_rows - first, kBlocks), n_items), dim3(kAaExactThreads),
-                           0, ctx->stream, gy, img, n_comp, tri, tri_stride, (const float4*)clip,
-                           n_verts, clip_per_item, faces, n_faces, vtx_faces, n_rows, max_deg, w,
-                           h, scale, first, (float4*)out);
-        DRESSI_CHECK_LAUNCH();
+    const auto launch = [&](auto kernel, uint32_t threads, uint32_t verts) {
+        const uint32_t piece = (uint32_t)(kLaunchThreads / threads) * verts;
+        for (uint32_t first = 0; first < n_rows; first += piece) {
+            const uint32_t n = std::min(n_rows - first, piece);
+            hipLaunchKernelGGL(kernel, dim3(div_up(n, verts), n_items), dim3(threads), 0,
+                               ctx->stream, gy, img, n_comp, tri, tri_stride, (const float4*)clip,
+                               n_verts, clip_per_item, faces, n_faces, vtx_faces, n_rows, max_deg,
+                               w, h, scale, first, (float4*)out);
+        }
+    };
+    if ((uint64_t)n_rows * n_items < kAaExactWaveVerts) {
+        launch(k_antialias_bwd_vtx_exact_op<256, 256>, 256, 1);
+    } else if ((uint64_t)n_rows * n_items >= kAaExactLanesVerts &&
+               (uint64_t)w * h < 2ull * n_rows) {
+        launch(k_antialias_bwd_vtx_exact_op<64, 8>, 64, 8);
+    } else {
+        launch(k_antialias_bwd_vtx_exact_op<64, 64>, 64, 1);
     }
+    DRESSI_CHECK_LAUNCH();
     return DRESSI_OK;
 }
 

@@ -129,6 +129,30 @@ def test_aa_exact_vertex_gradient_steps(ctx, oracle, level, h, w, nc):
     ctx.synchronize()
 
 
+@pytest.mark.parametrize("level,h,w,nc,n", [
+    # a wave per vertex: 10 242 vertices, boxes of one step and several
+    (5, 40, 33, 3, 1), (5, 300, 211, 1, 1), (3, 61, 97, 4, 13),
+    # eight lanes per vertex: 163 842 vertices, and batches whose last wave is not full
+    (7, 64, 50, 3, 1), (5, 40, 33, 2, 13)])
+def test_aa_exact_vertex_gradient_forms(ctx, oracle, level, h, w, nc, n):
+    """The forms for many vertices, bit for bit: each item of a batch of one scene's images."""
+    from opendressi_amd import ops
+    print(f"[aa exact forms] level={level} {n}x{h}x{w}x{nc}", flush=True)
+    clip, faces = _random_scene(oracle, level, level, w)
+    tri = oracle.rasterize_face_id(clip, faces, w, h)
+    vf = oracle.vertex_faces_tex(faces, len(clip))
+    rng = np.random.default_rng(nc)
+    img = rng.random((n, h, w, nc), dtype=np.float32)
+    gy = rng.standard_normal((n, h, w, nc)).astype(np.float32)
+    got = host(ops.antialias_bwd_vtx_batch(ctx, dev(gy), dev(img), dev(np.stack([tri] * n)),
+                                           dev(clip), dev(faces), dev(vf), None, 0, False))
+    for i in sorted({0, n // 2, n - 1}):
+        want = oracle.antialias_bwd_vtx(gy[i], img[i], tri, clip, faces, vf, 0.0, 0)
+        assert np.abs(want).max() > 0
+        _exact(got[i], want, f"item {i}")
+    ctx.synchronize()
+
+
 def test_aa_exact_vertex_gradient_of_many_vertices(ctx, oracle):
     """2^24 + 3 vertices, more than a launch has workgroups for: the first few are the small
     scene's, every other one is written with zeros."""
