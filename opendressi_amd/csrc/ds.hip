@@ -299,6 +299,34 @@ __device__ __forceinline__ float dist_face_sum(const FaceCorners& fc, uint32_t f
     return acc;
 }
 
+// dist_face_sum's sums into the rows of face f's corners: of each vertex's rows
+// the first that holds f.
+__device__ __forceinline__ void dist_write_rows(const FaceCorners& fc, uint32_t f, float acc,
+                                                const float* vf, uint32_t n_verts,
+                                                uint32_t max_deg, float4* out) {
+    const uint32_t lane = threadIdx.x;
+    const uint32_t r = lane < 9 ? lane / 3 : 0, comp = lane < 9 ? lane % 3 : 0;
+    const uint32_t my = r == 0 ? fc.idx[0] : r == 1 ? fc.idx[1] : fc.idx[2];
+    uint32_t row = max_deg;
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        uint32_t at = max_deg;
+        for (uint32_t d0 = 0; d0 < max_deg && at == max_deg; d0 += 64) {
+            const uint32_t d = d0 + lane;
+            const float fv = d < max_deg ? vf[(size_t)d * n_verts + fc.idx[k]] : -1.f;
+            const uint64_t m = __ballot(fv >= -0.5f && (uint32_t)(int64_t)(fv + 0.5f) == f);
+            if (m) {
+                at = d0 + (uint32_t)__builtin_ctzll(m);
+            }
+        }
+        row = (int)r == k ? at : row;
+    }
+    if (lane < 9 && row < max_deg) {
+        float* dst = (float*)&out[(size_t)row * n_verts + my];
+        dst[comp == 2 ? 3 : comp] = acc;
+    }
+}
+
 __global__ __launch_bounds__(64) void k_gather_dist_grad_faces(
         const float4* gy, const float4* rs, const float4* clip, uint32_t n_verts,
         const float* faces, const float* vf, uint32_t max_deg, float radius, uint32_t w,
@@ -320,29 +348,8 @@ __global__ __launch_bounds__(64) void k_gather_dist_grad_faces(
     }
     const uint32_t bw = (uint32_t)(bx1 - bx0 + 1);
     const uint32_t n_px = bw * (uint32_t)(by1 - by0 + 1);
-    // lane 3 r + c < 9 sums component c of corner r's row
-    const uint32_t r = lane < 9 ? lane / 3 : 0, comp = lane < 9 ? lane % 3 : 0;
-    const uint32_t my = r == 0 ? fc.idx[0] : r == 1 ? fc.idx[1] : fc.idx[2];
     const float acc = dist_face_sum(fc, f, bx0, by0, bw, n_px, rs, gy, w, W, H, lds);
-    // the corner's row: the first of its vertex's that holds f
-    uint32_t row = max_deg;
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-        uint32_t at = max_deg;
-        for (uint32_t d0 = 0; d0 < max_deg && at == max_deg; d0 += 64) {
-            const uint32_t d = d0 + lane;
-            const float fv = d < max_deg ? vf[(size_t)d * n_verts + fc.idx[k]] : -1.f;
-            const uint64_t m = __ballot(fv >= -0.5f && (uint32_t)(int64_t)(fv + 0.5f) == f);
-            if (m) {
-                at = d0 + (uint32_t)__builtin_ctzll(m);
-            }
-        }
-        row = (int)r == k ? at : row;
-    }
-    if (lane < 9 && row < max_deg) {
-        float* dst = (float*)&out[(size_t)row * n_verts + my];
-        dst[comp == 2 ? 3 : comp] = acc;
-    }
+    dist_write_rows(fc, f, acc, vf, n_verts, max_deg, out);
 }
 
 // The torch surface's form: every item and peel, corner sums {N,K,F,3}
@@ -378,6 +385,182 @@ __global__ __launch_bounds__(64) void k_surface_soft_bwd_faces(
         }
         if (lane < 9) {
             g_corner[(layer * n_faces + f) * 9 + lane] = acc;
+        }
+    }
+}
+
+// Face f's corners and soft box; 0 pixels for a face that wins none.
+__device__ __forceinline__ uint32_t dist_face(const float* faces, const float4* clip,
+                                              uint32_t n_verts, uint32_t f, float radius,
+                                              uint32_t w, uint32_t h, FaceCorners* fc, int* bx0,
+                                              int* by0, uint32_t* bw) {
+    bool ok = true;
+    for (int k = 0; k < 3; k++) {
+        ok = ok && fid_u(faces[(size_t)f * 3 + k]) < n_verts;
+    }
+    int bx1, by1;
+    if (!ok || !load_face(faces, clip, n_verts, f, (float)w, (float)h, fc, nullptr) ||
+        !soft_bbox(*fc, w, h, radius, bx0, by0, &bx1, &by1)) {
+        return 0;
+    }
+    *bw = (uint32_t)(bx1 - *bx0 + 1);
+    return *bw * (uint32_t)(by1 - *by0 + 1);
+}
+
+// Faces whose boxes are too large for a lane of k_dist_lanes.
+struct DistBig {
+    uint32_t* n;  // zero before
+    uint2* list;  // (face, layer), room for all
+};
+
+// The listed faces, a wave at a time.
+template <bool ROWS>
+__global__ __launch_bounds__(64, 6) void k_dist_big(
+        const float4* gy, const float4* rs, uint32_t peels, const float4* clip, uint32_t n_verts,
+        const float* faces, uint32_t n_faces, const float* vf, uint32_t max_deg, float radius,
+        uint32_t w, uint32_t h, DistBig bigs, float* g_corner, float4* out) {
+    __shared__ DistLds lds;
+    const size_t npx = (size_t)w * h;
+    const uint32_t n = *bigs.n;
+    for (uint32_t i = blockIdx.x; i < n; i += gridDim.x) {
+        const uint2 e = bigs.list[i];
+        const float4* c = clip + (size_t)(e.y / peels) * n_verts;
+        FaceCorners fc;
+        int x0, y0;
+        uint32_t bw;
+        const uint32_t n_px = dist_face(faces, c, n_verts, e.x, radius, w, h, &fc, &x0, &y0, &bw);
+        const float acc = dist_face_sum(fc, e.x, x0, y0, bw, n_px, rs + e.y * npx, gy + e.y * npx,
+                                        w, (float)w, (float)h, lds);
+        if (ROWS) {
+            dist_write_rows(fc, e.x, acc, vf, n_verts, max_deg, out);
+        } else if (threadIdx.x < 9) {
+            g_corner[((size_t)e.y * n_faces + e.x) * 9 + threadIdx.x] = acc;
+        }
+    }
+}
+
+// Both forms for many small faces, a lane per face: lanes go through their own
+// boxes of up to kDistLaneBox pixels and list the few that the face won, and
+// evaluate them together; larger boxes are k_dist_big's.
+// ROWS: the wide layout's rows, else g_corner of every item and peel.
+constexpr uint32_t kDistLaneBox = 256;
+constexpr uint32_t kDistLaneHits = kDistHits / 64;
+static_assert(kDistLaneHits >= 2 * kDistPx, "a step's hits fit beside those kept");
+
+template <bool ROWS>
+__global__ __launch_bounds__(64) void k_dist_lanes(
+        const float4* gy, const float4* rs, uint32_t peels, const float4* clip, uint32_t n_verts,
+        const float* faces, uint32_t n_faces, const float* vf, uint32_t max_deg, float radius,
+        uint32_t w, uint32_t h, DistBig bigs, float* g_corner, float4* out) {
+    __shared__ DistLds lds;
+    const uint32_t lane = threadIdx.x, f = blockIdx.x * 64 + lane;
+    const float W = (float)w, H = (float)h;
+    const size_t npx = (size_t)w * h;
+    clip += (size_t)blockIdx.y * n_verts;
+    FaceCorners fc;
+    int bx0 = 0, by0 = 0;
+    uint32_t bw = 1;
+    const uint32_t n_box =
+            f < n_faces ? dist_face(faces, clip, n_verts, f, radius, w, h, &fc, &bx0, &by0, &bw)
+                        : 0u;
+    const bool big = n_box > kDistLaneBox;
+    const uint32_t n_px = big ? 0u : n_box;
+    const uint32_t origin = n_px ? (uint32_t)by0 * w + (uint32_t)bx0 : 0u;
+    for (uint32_t k = blockIdx.z; k < peels; k += gridDim.z) {
+        const size_t layer = (size_t)blockIdx.y * peels + k;
+        const float4 *rl = rs + layer * npx, *gl = gy + layer * npx;
+        float acc[3][3] = {};  // corner, component (x, y, w)
+        uint32_t n_hits = 0;
+        BoxWalk at((uint32_t)bx0, (uint32_t)by0, bw, w, 0, 1);
+        for (uint32_t p0 = 0; __any(p0 < n_px); p0 += kDistPx) {
+            if (p0 < n_px) {
+                uint32_t o[kDistPx];
+                float2 yw[kDistPx];
+#pragma unroll
+                for (uint32_t s = 0; s < kDistPx; s++) {
+                    const bool in = p0 + s < n_px;
+                    o[s] = in ? at.o : origin;
+                    at.next();
+                    const float4 v = rl[o[s]];
+                    yw[s] = make_float2(v.y, in ? v.w : 0.f);
+                }
+#pragma unroll
+                for (uint32_t s = 0; s < kDistPx; s++) {
+                    if (!(yw[s].y < 0.5f) && (uint32_t)(int64_t)(yw[s].x + 0.5f) == f) {
+                        lds.hit_px[n_hits * 64 + lane] = o[s];
+                        n_hits++;
+                    }
+                }
+            }
+            if (__any(p0 + kDistPx < n_px) && !__any(n_hits + kDistPx > kDistLaneHits)) {
+                continue;
+            }
+            // (a lane reads what it wrote itself)
+            for (uint32_t q = 0; __any(q < n_hits); q++) {
+                const uint32_t px_o = q < n_hits ? lds.hit_px[q * 64 + lane] : 0u;
+                const float g = q < n_hits ? gl[px_o].x : 0.f;
+                if (g != 0.f) {
+                    const uint32_t y = px_o / w, x = px_o - y * w;
+                    const float px = (float)x + 0.5f, py = (float)y + 0.5f;
+                    const TriDistE td = signed_dist_edge(px, py, fc.sx, fc.sy);
+                    float4 t[3] = {};
+#pragma unroll
+                    for (int c = 0; c < 3; c++) {
+                        add_corner(fc, td, px, py, c, g, W, H, &t[c]);
+                    }
+#pragma unroll
+                    for (int r = 0; r < 3; r++) {
+#pragma unroll
+                        for (int c = 0; c < 3; c++) {
+                            // a corner's row takes every corner of its vertex; a
+                            // contribution left out is +0, as above
+                            const bool add = c == r || fc.idx[c] == fc.idx[r];
+                            acc[r][0] += add ? t[c].x : 0.f;
+                            acc[r][1] += add ? t[c].y : 0.f;
+                            acc[r][2] += add ? t[c].w : 0.f;
+                        }
+                    }
+                }
+            }
+            n_hits = 0;
+        }
+        const uint64_t all = __ballot(big);
+        if (all) {
+            uint32_t at = 0;
+            if (lane == 0) {
+                at = atomicAdd(bigs.n, (uint32_t)__popcll(all));
+            }
+            at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at) +
+                 (uint32_t)__popcll(all & ((1ull << lane) - 1ull));
+            if (big) {
+                bigs.list[at] = make_uint2(f, (uint32_t)layer);
+            }
+        }
+        if (f >= n_faces || big) {
+            continue;
+        }
+        if (!ROWS) {
+#pragma unroll
+            for (int q = 0; q < 9; q++) {
+                g_corner[(layer * n_faces + f) * 9 + q] = acc[q / 3][q % 3];
+            }
+        } else if (n_box) {
+#pragma unroll
+            for (int r = 0; r < 3; r++) {
+                uint32_t d = 0;
+                for (; d < max_deg; d++) {
+                    const float fv = vf[(size_t)d * n_verts + fc.idx[r]];
+                    if (fv >= -0.5f && (uint32_t)(int64_t)(fv + 0.5f) == f) {
+                        break;
+                    }
+                }
+                if (d < max_deg) {
+                    float* dst = (float*)&out[(size_t)d * n_verts + fc.idx[r]];
+                    dst[0] = acc[r][0];
+                    dst[1] = acc[r][1];
+                    dst[3] = acc[r][2];
+                }
+            }
         }
     }
 }
@@ -489,6 +672,47 @@ __global__ __launch_bounds__(128) void k_gather_dist_grad_vtx(
 
 using namespace dressi;
 
+// Whether `n` faces (times items and peels) of a mesh go by lanes. A wave for
+// every face starts at about 1 ns, and that is what many small ones take: two
+// 256 x 256 views of 327 680 faces 792 us, the thread per row before the waves
+// 459, lanes 145; eight 64 x 64 ones of 20 480 219, 503 and 69. Where the boxes
+// are large the lanes' pass is in vain (one 2048 x 2048 view of 327 680 faces
+// 567 -> 678 us; the thread per row 5435), but their size is not known here (a
+// sixteenth of that screen 435 -> 211): below 131 072 lanes are taken where
+// the mesh has more faces than the screen has pixels.
+static bool dist_by_lane(uint64_t n, uint32_t n_faces, uint32_t w, uint32_t h) {
+    return n < (1ull << 32) &&
+           (n >= 131072 || (n >= 16384 && (uint64_t)w * h < n_faces));
+}
+// Waves of k_dist_big (8192 of them take 762 us for the 678 above).
+constexpr uint32_t kDistBigWaves = 32768;
+constexpr int kDistBigSlot = 14;
+
+template <bool ROWS>
+static int launch_dist_lanes(dressi_ctx* ctx, const float* gy, const float* rs, uint32_t peels,
+                             const float* clip, uint32_t n_verts, uint32_t n_items,
+                             const float* faces, uint32_t n_faces, const float* vf,
+                             uint32_t max_deg, float radius, uint32_t w, uint32_t h,
+                             float* g_corner, float* out) {
+    const uint64_t n = (uint64_t)n_faces * n_items * peels;
+    void* ws = nullptr;
+    if (int rc = ctx_workspace(ctx, kDistBigSlot, 8 + sizeof(uint2) * n, &ws)) return rc;
+    const DistBig bigs{(uint32_t*)ws, (uint2*)((char*)ws + 8)};
+    if (int rc = launch_zero(ctx->stream, ws, 8)) return rc;
+    hipLaunchKernelGGL(k_dist_lanes<ROWS>,
+                       dim3(div_up(n_faces, 64), n_items, std::min(peels, 16u)), dim3(64), 0,
+                       ctx->stream, (const float4*)gy, (const float4*)rs, peels,
+                       (const float4*)clip, n_verts, faces, n_faces, vf, max_deg, radius, w, h,
+                       bigs, g_corner, (float4*)out);
+    DRESSI_CHECK_LAUNCH();
+    hipLaunchKernelGGL(k_dist_big<ROWS>, dim3((uint32_t)std::min<uint64_t>(n, kDistBigWaves)), dim3(64), 0,
+                       ctx->stream, (const float4*)gy, (const float4*)rs, peels,
+                       (const float4*)clip, n_verts, faces, n_faces, vf, max_deg, radius, w, h,
+                       bigs, g_corner, (float4*)out);
+    DRESSI_CHECK_LAUNCH();
+    return DRESSI_OK;
+}
+
 extern "C" int dressi_gather_dist_grad(dressi_ctx* ctx, const float* gy, const float* rs,
                                        const float* clip, uint32_t n_verts, const float* faces,
                                        uint32_t n_faces, const float* vtx_faces, uint32_t max_deg,
@@ -507,9 +731,16 @@ extern "C" int dressi_gather_dist_grad(dressi_ctx* ctx, const float* gy, const f
                            ctx->d_err, (float4*)out);
         DRESSI_CHECK_LAUNCH();
         if (n_faces) {
-            hipLaunchKernelGGL(k_gather_dist_grad_faces, dim3(n_faces), dim3(64), 0, ctx->stream,
-                               (const float4*)gy, (const float4*)rs, (const float4*)clip, n_verts,
-                               faces, vtx_faces, max_deg, radius_px, width, height, (float4*)out);
+            if (dist_by_lane(n_faces, n_faces, width, height)) {
+                return launch_dist_lanes<true>(ctx, gy, rs, 1, clip, n_verts, 1, faces, n_faces,
+                                               vtx_faces, max_deg, radius_px, width, height,
+                                               nullptr, out);
+            } else {
+                hipLaunchKernelGGL(k_gather_dist_grad_faces, dim3(n_faces), dim3(64), 0,
+                                   ctx->stream, (const float4*)gy, (const float4*)rs,
+                                   (const float4*)clip, n_verts, faces, vtx_faces, max_deg,
+                                   radius_px, width, height, (float4*)out);
+            }
         }
     } else {
         hipLaunchKernelGGL(k_gather_dist_grad_vtx, dim3(div_up(n_verts, 128)), dim3(128), 0,
@@ -538,10 +769,17 @@ extern "C" int dressi_surface_soft_bwd(dressi_ctx* ctx, const float* gy, const f
     if (!n_items || !n_rows) return DRESSI_OK;
     DRESSI_TRY_HIP(hipSetDevice(ctx->device));
     if (n_faces) {
-        hipLaunchKernelGGL(k_surface_soft_bwd_faces, dim3(n_faces, n_items, std::min(peels, 16u)),
-                           dim3(64), 0, ctx->stream, (const float4*)gy, (const float4*)rs, peels,
-                           (const float4*)pos, n_verts, faces, n_faces, radius_px, width, height,
-                           g_corner);
+        const uint32_t z = std::min(peels, 16u);
+        if (dist_by_lane((uint64_t)n_faces * n_items * peels, n_faces, width, height)) {
+            if (int rc = launch_dist_lanes<false>(ctx, gy, rs, peels, pos, n_verts, n_items, faces,
+                                                  n_faces, nullptr, 0, radius_px, width, height,
+                                                  g_corner, nullptr)) return rc;
+        } else {
+            hipLaunchKernelGGL(k_surface_soft_bwd_faces, dim3(n_faces, n_items, z), dim3(64), 0,
+                               ctx->stream, (const float4*)gy, (const float4*)rs, peels,
+                               (const float4*)pos, n_verts, faces, n_faces, radius_px, width,
+                               height, g_corner);
+        }
         DRESSI_CHECK_LAUNCH();
     }
     hipLaunchKernelGGL(k_surface_soft_bwd_vtx, dim3(div_up(n_rows * 4, 256), n_items), dim3(256),

@@ -108,3 +108,85 @@ def test_gather_dist_grad_boxes_and_rows(ctx, oracle, h, w):
     assert np.abs(ref).max() > 0
     _exact(got, ref, "wide")
     ctx.synchronize()
+
+
+def _lanes_mesh(oracle, seed, level=5):
+    """A dense icosphere on a small part of the screen, a fan and single faces whose boxes are a
+    good part of it, faces that repeat a vertex: clip positions and faces."""
+    rng = np.random.default_rng(seed)
+    pos, sphere = oracle.icosphere(level)
+    n_fan = 40
+    ang = np.linspace(0.0, 2.0 * np.pi, n_fan, endpoint=False)
+    k = len(pos)
+    pos = np.concatenate([pos * [0.5, 0.5, 0.2] + [-0.2, 0.1, 0.5], [[0.0, 0.0, 0.2]],
+                          np.stack([0.9 * np.cos(ang), 0.9 * np.sin(ang), 0 * ang + 0.1], 1),
+                          rng.uniform(-1, 1, (9, 3)) * [1.2, 1.2, 0.4] + [0, 0, 0.5]])
+    clip = np.concatenate([pos, np.ones((len(pos), 1))], 1).astype(np.float32)
+    clip *= rng.uniform(0.5, 2.0, (len(pos), 1)).astype(np.float32)
+    a = k + 1 + n_fan
+    more = [(k, k + 1 + i, k + 1 + (i + 1) % n_fan) for i in range(0, n_fan, 3)] + [
+        (a, a + 1, a + 2), (a + 3, a + 3, a + 4), (a + 5, a + 6, a + 5), (k, a + 7, a + 8)]
+    return clip, np.concatenate([sphere, np.array(more)]).astype(np.float32)
+
+
+@pytest.mark.parametrize("h,w,radius", [(61, 97, 3.0), (50, 33, 8.0), (90, 90, 0.5)])
+def test_gather_dist_grad_many_faces(ctx, oracle, h, w, radius):
+    """More faces than pixels: a lane per face, more hits than a lane keeps, boxes too large for a
+    lane, a last wave that is not full: bit for bit against the oracle."""
+    from opendressi_amd import ops
+    print(f"[dist grad] many faces {h}x{w} r {radius}", flush=True)
+    clip, faces = _lanes_mesh(oracle, h)
+    nf = len(faces)
+    assert nf > max(16384, h * w) and nf % 64
+    vf = oracle.vertex_faces_tex(faces, len(clip))
+    vf = np.concatenate([vf, np.full_like(vf[:1], nf - 1)]).astype(np.float32)
+    fid = np.repeat(np.arange(nf, dtype=np.float32), 3)[:, None]
+    fs = np.arange(3 * nf, dtype=np.float32).reshape(nf, 3)
+    rs = oracle.rasterize_soft(oracle.soft_clip(clip, faces, w, h, radius), fid, fs, clip, faces, w,
+                               h, radius)
+    # faces of hundreds of pixels and of a few
+    ids, px = np.unique(rs[..., 1][rs[..., 3] > 0.5], return_counts=True)
+    assert px.max() > 100 and (px <= 2).any() and len(ids) > 100
+    gy = np.random.default_rng(w).standard_normal((h, w, 4)).astype(np.float32)
+    got = host(ops.gather_dist_grad(ctx, dev(gy), dev(rs), dev(clip), dev(faces), dev(vf), radius))
+    ref = oracle.gather_dist_grad(gy, rs, clip, faces, vf, wide=True)
+    assert np.abs(ref).max() > 0
+    _exact(got, ref, "wide")
+    ctx.synchronize()
+
+
+@pytest.mark.parametrize("peels,items", [(1, 7), (3, 3), (17, 1)])
+def test_surface_soft_gradient_many_faces(ctx, oracle, peels, items):
+    """The torch surface's gradient by lanes over items and peels (more than the launch's 16),
+    each layer with its own winners, against the wide form's rows, their column sums and the
+    contributions' sum."""
+    import torch
+
+    from opendressi_amd import ops
+    from opendressi_amd.torch.convert import sum_contribs
+    h, w = 61, 97
+    print(f"[dist grad] many faces, {items} items, {peels} peels", flush=True)
+    clip, faces = _lanes_mesh(oracle, 1)
+    faces = faces[np.array([len(set(f)) == 3 for f in faces])]
+    nf = len(faces)
+    assert nf * peels * items > 131072
+    clips = dev(np.stack([clip * np.float32(1.0 + 0.05 * i) for i in range(items)]))
+    vf = dev(oracle.vertex_faces_tex(faces, len(clip)))
+    gen = torch.Generator(device="cuda").manual_seed(peels)
+    shape = (items, peels, h, w)
+    rs = torch.zeros((*shape, 4), device="cuda")
+    rs[..., 1] = torch.randint(0, nf, shape, device="cuda", generator=gen).float()
+    rs[..., 3] = (torch.rand(shape, device="cuda", generator=gen) < 0.9).float()
+    # half of the pixels: the large faces
+    big = torch.randint(nf - 10, nf, shape, device="cuda", generator=gen).float()
+    rs[..., 1] = torch.where(torch.rand(shape, device="cuda", generator=gen) < 0.5, big, rs[..., 1])
+    gy = torch.randn((*shape, 4), device="cuda", generator=gen)
+    got = ops.surface_soft_bwd(ctx, gy, rs, clips, dev(faces), vf, 3.0)
+    for i in range(items):
+        parts = [ops.col_sum(ctx, ops.gather_dist_grad(ctx, gy[i, k], rs[i, k], clips[i],
+                                                       dev(faces), vf, 3.0, True))
+                 for k in reversed(range(peels))]
+        ref = sum_contribs(parts)
+        assert float(ref.abs().max()) > 0
+        _exact(host(got[i]), host(ref), f"item {i}")
+    ctx.synchronize()
