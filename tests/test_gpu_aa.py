@@ -154,8 +154,8 @@ def test_aa_exact_vertex_gradient_forms(ctx, oracle, level, h, w, nc, n):
 
 
 def test_aa_exact_vertex_gradient_of_many_vertices(ctx, oracle):
-    """2^24 + 3 vertices, more than a launch has workgroups for: the first few are the small
-    scene's, every other one is written with zeros."""
+    """2^24 + 3 vertices, for which a workgroup of 256 each passes a launch's 2^32 threads: the first
+    few are the small scene's, every other one is written with zeros."""
     import torch
 
     from opendressi_amd import ops
