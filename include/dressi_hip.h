@@ -460,7 +460,7 @@ int dressi_pbr_profile(dressi_pbr_plan* plan, uint32_t iters, char* names,
                        uint32_t* n);
 
 /* ---- the torch surface's ops (python/dressi/torch/ops.py:95-698) ---- */
-/* Each is one call of opendressi_amd.torch in one or two launches, with the
+/* Each is one call of opendressi_amd.torch for the whole batch, with the
  * float operations (and their order) of the per-op kernels that the reference
  * surface composes. `rast` {N,H,W} VEC4 = (u, v, z / w, face + 1). */
 /* rasterize: pos {N,V} VEC4, z in [-w, w]; faces int32 {F,3}; clip_vk

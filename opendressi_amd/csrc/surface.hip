@@ -1,11 +1,11 @@
 // surface.hip -- the torch surface's ops (opendressi_amd/torch) as kernels
-// of their own: each does in one or two launches what the surface composed
-// from the per-op entry points and torch's elementwise kernels, with the same
-// float operations in the same order (python/dressi/torch/ops.py:95-698 and
-// the reference's backward kernels it runs). Images are [item][H][W][C],
-// `rast` is the surface's raster, VEC4 (u, v, z / w, face + 1); face lists
-// are float ids {F,3}, adjacencies {max_deg, V} (VertexFacesTex) of the same
-// faces.
+// of their own: each does in a few launches (one for most, up to six for the
+// texture gradient) what the surface composed from the per-op entry points and
+// torch's elementwise kernels, with the same float operations in the same
+// order (python/dressi/torch/ops.py:95-698 and the reference's backward
+// kernels it runs). Images are [item][H][W][C], `rast` is the surface's
+// raster, VEC4 (u, v, z / w, face + 1); face lists are float ids {F,3},
+// adjacencies {max_deg, V} (VertexFacesTex) of the same faces.
 //
 // A call of the surface used to be 10-20 launches of a few microseconds each
 // (a slice, a product, a copy), bound by the host that issued them and by
