@@ -165,21 +165,21 @@ struct BinBuffers {
 };
 
 // The hard rasterizer's: a bin's first `cap` faces are in its list, those that
-// find it full in one of its kHardChains chains through `over`. The words from
+// find it full in one of its chains through `over`. The words from
 // `counts` on (n_bins + 2) are cleared before each use.
-constexpr uint32_t kHardChains = 64;
+constexpr uint32_t kHardChains = 64;  // a bin's at most
 struct HardBinBuffers {
     uint32_t* counts = nullptr;  // [n_bins]
     uint32_t* n_over = nullptr;  // entries of `over` taken
     uint32_t* spilt = nullptr;   // != 0: `over` was full, some faces are nowhere
     uint2* over = nullptr;       // [over_cap] (face, the chain's entry before)
-    uint32_t* heads = nullptr;   // [n_bins][kHardChains] a chain's last entry
+    uint32_t* heads = nullptr;   // [n_bins][chains] a chain's last entry
     uint32_t* list = nullptr;    // [n_bins][cap] face indices
-    uint32_t cap = 0, over_cap = 0, n_bins = 0;
+    uint32_t cap = 0, over_cap = 0, n_bins = 0, chains = 0;  // chains: a power of two
     size_t clear_bytes() const { return sizeof(uint32_t) * ((size_t)n_bins + 2); }
 };
 struct HardBinSizes {
-    uint32_t n_bins, cap, over_cap;  // over_cap 0: a list holds the whole mesh
+    uint32_t n_bins, cap, over_cap, chains;  // over_cap 0: a list holds the whole mesh
     size_t bytes;
 };
 

@@ -22,13 +22,18 @@ namespace dressi {
 // (their records 6.6 and 419).
 constexpr uint64_t kHardBinShare = 8, kHardBinMin = 32, kHardOverShare = 4;
 constexpr uint64_t kHardListEntries = 4ull << 20;
+// Bins from which a list's least is 16 entries, and words for the chains' heads
+// up to there (64 MB; a bin has at least eight): many bins are many pixels, of
+// which few have full lists.
+constexpr uint64_t kHardManyBins = 1ull << 20, kHardHeads = 1ull << 24;
 // Neither grows past these (4 GB each); a list keeps at least 16 entries.
 constexpr uint64_t kHardListMax = 1ull << 30, kHardOverMax = 1ull << 29;
 
 HardBinSizes hard_bin_sizes(const RasterGeom& g) {
     const uint64_t n_bins = (uint64_t)g.n_tiles * g.n_views;
     const uint64_t faces = std::max<uint64_t>(g.n_faces, 1);
-    uint64_t cap = std::max(kHardBinMin + kHardBinShare * faces / g.n_tiles,
+    uint64_t cap = std::max((n_bins > kHardManyBins ? 16 : kHardBinMin) +
+                                    kHardBinShare * faces / g.n_tiles,
                             kHardListEntries / n_bins);
     cap = std::min(cap, std::max<uint64_t>(kHardListMax / n_bins, 16));
     cap = std::min(cap, faces);
@@ -38,8 +43,10 @@ HardBinSizes hard_bin_sizes(const RasterGeom& g) {
     z.over_cap = cap == faces ? 0u
                               : (uint32_t)std::min(faces * g.n_views * kHardOverShare + 4096,
                                                    kHardOverMax);
+    z.chains = kHardChains;
+    while (z.chains > 8 && n_bins * z.chains > kHardHeads) z.chains /= 2;
     z.bytes = sizeof(uint32_t) * (n_bins + 4 + 2 * (size_t)z.over_cap +
-                                  n_bins * (cap + (z.over_cap ? kHardChains : 0u)));
+                                  n_bins * (cap + (z.over_cap ? z.chains : 0u)));
     return z;
 }
 
@@ -52,11 +59,12 @@ void hard_bin_carve(void* base, const HardBinSizes& z, HardBinBuffers* b) {
     b->over = (uint2*)p;
     p += 2 * (size_t)z.over_cap;
     b->heads = p;
-    p += z.over_cap ? (size_t)z.n_bins * kHardChains : 0;
+    p += z.over_cap ? (size_t)z.n_bins * z.chains : 0;
     b->list = p;
     b->cap = z.cap;
     b->over_cap = z.over_cap;
     b->n_bins = z.n_bins;
+    b->chains = z.chains;
 }
 
 // ---------------------------------------------------------------------------
@@ -169,7 +177,7 @@ __global__ __launch_bounds__(256) void k_hard_setup_bin(RasterGeom g, const floa
         }
         if (n_full) {
             // Places in the overflow, one add for the wave's; then each into
-            // chain (slot - cap) % kHardChains of its bin. A chain's length
+            // chain (slot - cap) % chains of its bin. A chain's length
             // follows from the bin's count, so heads need no initial value.
             uint32_t at = 0;
             if (lane == 0) {
@@ -183,10 +191,10 @@ __global__ __launch_bounds__(256) void k_hard_setup_bin(RasterGeom g, const floa
             for (uint32_t k = 0; k < kBinPairs; k++) {
                 const uint32_t o = at + (uint32_t)__popcll(full[k] & ((1ull << lane) - 1ull));
                 if ((full[k] >> lane & 1u) && o < b.over_cap) {
-                    const uint32_t chain = (slot[k] - b.cap) % kHardChains;
+                    const uint32_t chain = (slot[k] - b.cap) & (b.chains - 1);
                     b.over[o] = make_uint2(
                             face[k],
-                            atomicExch(&b.heads[(size_t)bin[k] * kHardChains + chain], o));
+                            atomicExch(&b.heads[(size_t)bin[k] * b.chains + chain], o));
                 }
                 at += (uint32_t)__popcll(full[k]);
             }
@@ -276,14 +284,14 @@ __global__ __launch_bounds__(kTileThreads) void k_raster_hard(RasterGeom g, cons
     }
     if (full && !implicit) {
         // the bin's chains side by side: entry r of chain c is its overflow
-        // face c + r kHardChains, counted from the chain's head
+        // face c + r chains, counted from the chain's head
         static_assert(kHardChains <= kHardStage, "a record staged per chain");
         const uint32_t n_over = n_bin - b.cap;
-        uint32_t at = threadIdx.x < kHardChains && threadIdx.x < n_over
-                              ? b.heads[(size_t)bin * kHardChains + threadIdx.x]
+        uint32_t at = threadIdx.x < b.chains && threadIdx.x < n_over
+                              ? b.heads[(size_t)bin * b.chains + threadIdx.x]
                               : 0u;
-        for (uint32_t base = 0; base < n_over; base += kHardChains) {
-            const uint32_t cnt = (n_over - base) < kHardChains ? (n_over - base) : kHardChains;
+        for (uint32_t base = 0; base < n_over; base += b.chains) {
+            const uint32_t cnt = (n_over - base) < b.chains ? (n_over - base) : b.chains;
             __syncthreads();
             if (threadIdx.x < cnt) {
                 const uint2 e = b.over[at];

@@ -300,6 +300,32 @@ def test_raster_full_bins_of_several_views(ctx, oracle, views):
     ctx.synchronize()
 
 
+@pytest.mark.parametrize("views,screen", [(20, 4096), (3, 16384)])
+def test_raster_full_bins_of_many_tiles(ctx, oracle, views, screen):
+    """More than 2^20 tiles: lists of 16 entries and eight chains to a bin instead of 64."""
+    from opendressi_amd import ops
+    n = 400
+    print(f"[raster full bins] {views} views of {screen}", flush=True)
+    rng = np.random.default_rng(views)
+    at = (0.25 + 0.001 * rng.random((n, 1, 2))) * screen
+    xy = at + rng.standard_normal((n, 3, 2)) * 6.0
+    clip = np.concatenate([xy / screen * 2.0 - 1.0, rng.random((n, 3, 1)), np.ones((n, 3, 1))], -1)
+    clip = clip.reshape(-1, 4).astype(np.float32)
+    faces = np.arange(3 * n, dtype=np.float32).reshape(n, 3)
+    ref = oracle.rasterize_face_id(clip, faces, screen, screen)
+    attr = rng.random((3 * n, 1), dtype=np.float32)
+    # the last views hold the mesh, the others nothing
+    clips = np.zeros((views, *clip.shape), np.float32)
+    clips[-2:] = clip
+    out, ids = ops.rasterize_batch(ctx, dev(clips), dev(attr), dev(faces), screen, screen,
+                                   with_face_id=True)
+    assert len(np.unique(ref)) > 50
+    for i in (views - 2, views - 1):
+        _exact(host(ids[i]), ref, f"view {i}")
+    assert float(ids[0].abs().max()) == 0.0
+    ctx.synchronize()
+
+
 def test_raster_time_of_a_batch(ctx):
     """A full tile reads its own overflow alone: eight times the views take about eight times as
     long (64 times, where each full tile looked through every view's)."""
